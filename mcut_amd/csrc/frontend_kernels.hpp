@@ -815,38 +815,71 @@ __global__ void k_edge_assign(const uint32_t* __restrict__ idx, CornerMap cm, ui
     }
 }
 
-// Packed edge table, for meshes whose vertex ids fit 21 bits and whose corner
-// ranks fit 22: one 64-bit word per edge holds (min vertex, max vertex) in
-// its top 42 bits and the smallest insertion rank in its low 22, so one
-// atomicCAS (plus an atomicMin when the edge is already there) replaces the
-// key and first-use tables: 53 us instead of 103 us for the 983,040 corners of
-// an icosphere-7.  Both meshes go through one launch per pass: corners
-// [0, K0) are the source's, [K0, K0 + K1) the cut mesh's (is_cut = 1).  The
-// insert leaves each corner's slot in its cedge entry; the flag pass reads
-// it instead of probing and replaces it with the edge's first rank, which the
-// assign pass then reads in corner order (the table word is a gather at a
-// hashed slot that brings a whole line; the first rank's eid entry lies near
-// the corner's own rank) before it overwrites the entry with the edge id.
-// Edge ids come from one exclusive scan over both meshes'
-// first-use flags, so a cut edge's id already counts the source's edges
-// (with a resident source only the cut mesh is scanned, after its ne edges).
-constexpr uint32_t kPackedVertexBits = 21, kPackedRankBits = 22;
-constexpr unsigned long long kPackedRankMask = (1ull << kPackedRankBits) - 1;
+// The edge numbering without a table in memory.  Every corner's word (its
+// undirected edge, insertion rank and direction) is scattered into the bucket
+// its edge hashes to; a block then resolves one bucket in LDS and writes, for
+// every corner, the rank of the edge's other corner (opp; kNoCorner on a
+// border); the first uses (no partner, or a later one) are counted per tile of
+// ranks, and the last pass numbers them by the prefix of those counts and
+// writes the edge table in order, each edge by its first corner.  A second
+// corner's edge is that of its partner's corner, which readers look up
+// (corner_edge) for the few corners they need.
+//
+// What bounds it: the corners' words (16 bytes a corner moved once each way)
+// and one scattered 4-byte store a corner.  The hash tables this replaces took
+// one device-scope compare-and-swap a corner, performed beyond the XCD's L2 at
+// about 20 G/s, then a gather of the table's line a corner.  LDS atomics have
+// no such limit.  On two subdivision-7 icospheres (2 M corners) the stage went
+// from 0.26 to 0.15 ms beside the other streams, on two of 1.3 M triangles from
+// 1.9 to 1.4 ms, on 320 uneven pairs (31 M corners) from 4.9 to 1.9 ms.
+//
+// Two levels of locality: vertex ids are grouped by 8 before they are hashed,
+// so the edges of a neighbourhood share a bucket and the block's stores to opp
+// meet in the same lines; and a segment (one mesh of one pair) has its own
+// buckets, so a batch's stores stay within the pair's.
+//
+// Words: the edge key is mixed by a bijection, whose top bits are the bucket,
+// so a word need not hold them: 2 vbits - bb key bits, kbits rank bits and the
+// direction fit 64 bits for any mesh the bucket limit admits (kTopoMaxBits).
+constexpr uint32_t kNoCorner = 0xffffffffu;
+constexpr int kTopoCapLog = 12;                    // words a bucket holds
+constexpr uint32_t kTopoCap = 1u << kTopoCapLog;
+constexpr uint32_t kTopoFillStride = 32;           // one counter per 128-byte line
+constexpr uint32_t kTopoFill = kTopoCap / 2;       // mean words of a bucket, at most: 4096 lies 6 sigma above
+constexpr int kTopoMaxBits = 12;                   // buckets a segment may have: 2^12 counters and a tile fill the LDS
+constexpr int kTopoBlock = 512;
+constexpr int kTopoScatterBlock = 1024;
+constexpr uint32_t kTopoTile = 4096;               // ranks per counting tile
+constexpr uint32_t kTopoDirectTiles = 2048;        // up to here a block sums the tiles before its own
 
-struct TopoMesh {
-    const uint32_t* idx;
-    CornerMap cm;
-    unsigned long long* keys;
-    uint64_t mask;
-    uint32_t* cedge;
-    uint64_t nk;
-    uint32_t vofs, fofs; // soup offsets of the mesh's vertices and faces
+// the corners of one mesh (of one pair) and their buckets
+struct TopoSeg {
+    unsigned long long c0; // first corner in its part
+    unsigned long long w0; // first word of its buckets
+    uint32_t k;            // corners
+    uint32_t vb;           // first vertex id in its part
+    uint32_t bucket0;      // first bucket
+    uint32_t tile0;        // first scatter tile (a segment of one bucket has none)
+    uint8_t bb, vbits, kbits, m;
 };
 
-__device__ __forceinline__ uint64_t packed_edge(uint32_t a, uint32_t b)
-{
-    return a < b ? ((uint64_t)a << kPackedVertexBits | b) : ((uint64_t)b << kPackedVertexBits | a);
-}
+struct TopoPart {
+    const uint32_t* idx;
+    CornerMap cm;
+    uint32_t* cedge; // edge of each first corner
+    uint32_t* opp;   // by rank: rank of the edge's other corner
+    uint64_t nk;
+    uint32_t vofs, fofs; // soup offsets of the part's vertices and faces
+};
+
+struct Topo {
+    TopoPart part[2];
+    TopoSeg seg[2];
+    const TopoSeg* tab; // batches: the segments, in bucket order (null: seg)
+    uint32_t nseg;
+    unsigned long long* words;
+    uint32_t* fill; // words of each bucket, kTopoFillStride apart
+};
 
 // the corner whose insertion rank is r: a face's ranks are a permutation of
 // its corner positions, so r lies in its own face (the inverse of corner_rank)
@@ -859,204 +892,306 @@ __device__ __forceinline__ uint64_t rank_corner(const CornerMap& cm, uint32_t r,
     return b + (j == n - 1 ? 0 : j + 1);
 }
 
-__global__ void k_fill2_u64(unsigned long long* p0, uint64_t n0, unsigned long long* p1, uint64_t n1, unsigned long long v)
+// the segment that holds bucket (or scatter tile) x: the last whose first one
+// is not past it, 64 probes a step
+template <bool TILE>
+__device__ __forceinline__ TopoSeg topo_seg(const Topo& T, uint32_t x)
 {
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n0 + n1; i += (uint64_t)gridDim.x * blockDim.x) {
-        if (i < n0) p0[i] = v;
-        else p1[i - n0] = v;
+    if (!T.tab) return T.nseg > 1 && (TILE ? T.seg[1].tile0 : T.seg[1].bucket0) <= x ? T.seg[1] : T.seg[0];
+    uint32_t lo = 0, n = T.nseg;
+    while (n > 1) {
+        const uint32_t step = (n + 63) / 64, i = (threadIdx.x & 63) * step;
+        const bool le = i < n && (TILE ? T.tab[lo + i].tile0 : T.tab[lo + i].bucket0) <= x;
+        const uint32_t c = (uint32_t)__popcll(__ballot(le)) - 1;
+        lo += c * step;
+        n = n - c * step < step ? n - c * step : step;
+    }
+    return T.tab[__builtin_amdgcn_readfirstlane(lo)];
+}
+
+// corner c (of its part) as a word; its bucket within the segment in *bucket
+__device__ __forceinline__ unsigned long long topo_word(const TopoPart& P, const TopoSeg& g, uint64_t c, uint32_t* bucket)
+{
+    uint32_t f, b, n, i;
+    P.cm(c, f, b, n, i);
+    const uint32_t a = P.idx[c] - g.vb, d = P.idx[b + (i + 1 == n ? 0 : i + 1)] - g.vb;
+    const uint32_t rank = corner_rank(b, i, n, g.m) - (uint32_t)g.c0;
+    const uint64_t lo = a < d ? a : d, hi = a < d ? d : a;
+    const int gb = 2 * (g.vbits - 3);
+    const uint64_t gm = (1ull << gb) - 1;
+    uint64_t h = ((lo >> 3) << (g.vbits - 3) | (hi >> 3)) & gm; // two rounds of a bijection of gb-bit words
+    h = (h * 0x9e3779b97f4a7c15ull) & gm;
+    h ^= h >> (gb / 2);
+    h = (h * 0xd6e8feb86659fd93ull) & gm;
+    h ^= h >> (gb / 2);
+    *bucket = (uint32_t)(h >> (gb - g.bb));
+    const uint64_t rest = (h & ((1ull << (gb - g.bb)) - 1)) << 6 | (lo & 7) << 3 | (hi & 7);
+    return rest << (g.kbits + 1) | (uint64_t)rank << 1 | (a < d ? 1u : 0u);
+}
+
+// word p of bucket b: buckets fill at the same pace, and with all of them
+// starting on a 32 KB boundary the words written at one time would meet in the
+// same memory channels, so each bucket is rotated by a number of lines of its own
+__device__ __forceinline__ unsigned long long* topo_at(const Topo& T, const TopoSeg& g, uint32_t b, uint32_t p)
+{
+    return T.words + g.w0 + ((uint64_t)b << kTopoCapLog) + ((p + b * (163u * 16u)) & (kTopoCap - 1));
+}
+
+// One tile of a segment's corners into its buckets: places within the tile by
+// LDS atomics, one global reservation per bucket the tile reaches, and the
+// tile's words put in bucket order in LDS, so that a group of lanes writes each
+// bucket's run to consecutive addresses (one word a lane and bucket instead
+// reached 64 pages a wave: 8 words/ns on a 1.3 M triangle mesh).  The order
+// within a bucket does not matter.  A word past a full bucket is dropped and
+// flagged (the host runs the dispatch again with the hash tables); its corner
+// counts as a border meanwhile.
+template <int ITEMS, int BITS>
+__global__ void __launch_bounds__(kTopoScatterBlock) k_topo_scatter(Topo T, Counters* C)
+{
+    __shared__ unsigned long long stage[kTopoScatterBlock * ITEMS];
+    __shared__ uint32_t cnt[1 << BITS];   // words of the tile in each bucket, then their place in the bucket
+    __shared__ uint16_t start[1 << BITS]; // their place in the tile
+    __shared__ uint32_t wsum[kTopoScatterBlock / 64];
+    const TopoSeg g = topo_seg<true>(T, blockIdx.x);
+    const TopoPart& P = T.part[g.m];
+    const uint32_t nb = 1u << g.bb;
+    constexpr uint32_t kTile = kTopoScatterBlock * ITEMS;
+    for (uint32_t q = threadIdx.x; q < nb; q += kTopoScatterBlock) cnt[q] = 0u;
+    __syncthreads();
+    const uint32_t q0 = (blockIdx.x - g.tile0) * kTile, t0 = q0 + threadIdx.x;
+    unsigned long long w[ITEMS];
+    uint32_t bk[ITEMS], pos[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const uint32_t q = t0 + j * kTopoScatterBlock;
+        bk[j] = 0;
+        w[j] = q < g.k ? topo_word(P, g, g.c0 + q, &bk[j]) : 0ull;
+    }
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+        pos[j] = t0 + j * kTopoScatterBlock < g.k ? atomicAdd(&cnt[bk[j]], 1u) : 0u;
+    __syncthreads();
+    // exclusive scan of the counts: thread t takes `per` consecutive buckets
+    const uint32_t per = nb > kTopoScatterBlock ? nb / kTopoScatterBlock : 1, b0 = threadIdx.x * per;
+    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    uint32_t own = 0;
+    if (b0 < nb)
+        for (uint32_t q = 0; q < per; ++q) own += cnt[b0 + q];
+    uint32_t x = own;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= (uint32_t)o) x += y;
+    }
+    if (lane == 63) wsum[wid] = x;
+    __syncthreads();
+    x -= own;
+    for (uint32_t q = 0; q < wid; ++q) x += wsum[q];
+    if (b0 < nb)
+        for (uint32_t q = 0; q < per; ++q) {
+            const uint32_t c = cnt[b0 + q];
+            start[b0 + q] = (uint16_t)x; // at most kTile <= 2^14
+            x += c;
+            if (c) cnt[b0 + q] = atomicAdd(&T.fill[(uint64_t)(g.bucket0 + b0 + q) * kTopoFillStride], c);
+        }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+        if (t0 + j * kTopoScatterBlock < g.k) stage[start[bk[j]] + pos[j]] = w[j];
+    __syncthreads();
+    const uint32_t ntile = g.k - q0 < kTile ? g.k - q0 : kTile;
+    uint32_t width = 8; // lanes a run: about its mean length
+    while (width < 64 && width * nb < kTile) width <<= 1;
+    const uint32_t l = threadIdx.x & (width - 1), groups = kTopoScatterBlock / width;
+    for (uint32_t b = threadIdx.x / width; b < nb; b += groups) {
+        const uint32_t s0 = start[b], s1 = b + 1 < nb ? start[b + 1] : ntile, to = cnt[b];
+        for (uint32_t i = s0 + l; i < s1; i += width) {
+            const uint32_t p = to + (i - s0);
+            const unsigned long long v = stage[i];
+            if (p < kTopoCap) {
+                *topo_at(T, g, b, p) = v;
+            } else {
+                P.opp[g.c0 + ((v >> 1) & ((1ull << g.kbits) - 1))] = kNoCorner;
+                C->ov_topo = 1u;
+            }
+        }
     }
 }
 
-__global__ void k_edge_insert_packed(TopoMesh M0, TopoMesh M1, uint64_t start)
+// One bucket in LDS: the first (lowest) rank of every edge by an open-addressed
+// table, then its second corner, then every corner's partner.  A segment of
+// one bucket makes its words here.  A third corner on an edge, or a second one
+// in the first one's direction, is a non-manifold soup.
+__global__ void __launch_bounds__(kTopoBlock) k_topo_buckets(Topo T, Counters* C)
 {
-    const uint64_t K = M0.nk + M1.nk;
-    for (uint64_t q = start + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; q < K; q += (uint64_t)gridDim.x * blockDim.x) {
-        const int m = q >= M0.nk;
-        const TopoMesh& M = m ? M1 : M0;
-        const uint64_t c = m ? q - M0.nk : q;
-        uint32_t f, b, n, i;
-        M.cm(c, f, b, n, i);
-        const uint32_t a = M.idx[c], d = M.idx[b + (i + 1 == n ? 0 : i + 1)];
-        const uint64_t ek = packed_edge(a, d);
-        const uint32_t rank = corner_rank(b, i, n, m);
-        const unsigned long long w = (ek << kPackedRankBits) | rank;
-        uint64_t h = hash64(ek) & M.mask;
-        for (uint64_t probe = 0; probe <= M.mask; ++probe) {
-            const unsigned long long prev = atomicCAS(&M.keys[h], kEmpty64, w);
+    __shared__ unsigned long long slot[kTopoCap];
+    __shared__ uint32_t second[kTopoCap];
+    constexpr int kPer = kTopoCap / kTopoBlock;
+    const TopoSeg g = topo_seg<false>(T, blockIdx.x);
+    const TopoPart& P = T.part[g.m];
+    const uint32_t bkt = blockIdx.x - g.bucket0;
+    uint32_t n = g.bb ? T.fill[(uint64_t)blockIdx.x * kTopoFillStride] : g.k;
+    if (n > kTopoCap) n = kTopoCap;
+    if (n == 0) return; // whole block
+    unsigned long long w[kPer];
+    uint32_t at[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const uint32_t q = j * kTopoBlock + threadIdx.x;
+        uint32_t b;
+        w[j] = kEmpty64;
+        if (q < n)
+            w[j] = g.bb ? *topo_at(T, g, bkt, q) : topo_word(P, g, g.c0 + q, &b);
+    }
+    for (uint32_t q = threadIdx.x; q < kTopoCap; q += kTopoBlock) {
+        slot[q] = kEmpty64;
+        second[q] = kNoCorner;
+    }
+    __syncthreads();
+    const int ks = g.kbits + 1;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        if (w[j] == kEmpty64) continue;
+        const unsigned long long key = w[j] >> ks;
+        uint32_t h = (uint32_t)((key * 0x9e3779b97f4a7c15ull) >> (64 - kTopoCapLog));
+        for (uint32_t probe = 0; probe < kTopoCap; ++probe) { // at most kTopoCap keys: a free or equal slot exists
+            const unsigned long long prev = atomicCAS(&slot[h], kEmpty64, w[j]);
             if (prev == kEmpty64) break;
-            if ((prev >> kPackedRankBits) == ek) {
-                if ((prev & kPackedRankMask) > rank) atomicMin(&M.keys[h], w);
+            if (prev >> ks == key) {
+                if (prev > w[j]) atomicMin(&slot[h], w[j]);
                 break;
             }
-            h = (h + 1) & M.mask;
+            h = (h + 1) & (kTopoCap - 1);
         }
-        M.cedge[c] = (uint32_t)h;
+        at[j] = h;
+    }
+    __syncthreads();
+    const unsigned long long rm = (1ull << g.kbits) - 1;
+    uint32_t* opp = P.opp + g.c0;
+    bool bad = false;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        if (w[j] == kEmpty64) continue;
+        const unsigned long long f = slot[at[j]];
+        if (f == w[j]) continue;
+        bad |= ((f ^ w[j]) & 1ull) == 0; // used twice in one direction
+        bad |= atomicExch(&second[at[j]], (uint32_t)((w[j] >> 1) & rm)) != kNoCorner; // a third corner
+        opp[(w[j] >> 1) & rm] = (uint32_t)g.c0 + (uint32_t)((f >> 1) & rm);
+    }
+    if (bad) atomicOr(&C->nonmanifold, 1u);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        if (w[j] == kEmpty64 || slot[at[j]] != w[j]) continue;
+        const uint32_t s = second[at[j]];
+        opp[(w[j] >> 1) & rm] = s == kNoCorner ? kNoCorner : (uint32_t)g.c0 + s;
     }
 }
 
-// flag[moff + rank] = 1 at an edge's first use (moff = K0 for the cut mesh)
-__global__ void k_edge_flag_packed(TopoMesh M0, TopoMesh M1, uint64_t start, uint32_t* __restrict__ flag, Counters* C)
+// tiles of kTopoTile ranks: the source part's, then the cut part's (tiles do
+// not straddle the parts)
+__device__ __forceinline__ bool topo_tile(const Topo& T, uint32_t t, uint32_t tiles0, int* m, uint64_t* r0, uint64_t* r1)
 {
-    const uint64_t K = M0.nk + M1.nk;
-    for (uint64_t q = start + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; q < K; q += (uint64_t)gridDim.x * blockDim.x) {
-        const int m = q >= M0.nk;
-        const TopoMesh& M = m ? M1 : M0;
-        const uint64_t c = m ? q - M0.nk : q;
-        uint32_t f, b, n, i;
-        M.cm(c, f, b, n, i);
-        const uint32_t a = M.idx[c];
-        const uint32_t rank = corner_rank(b, i, n, m);
-        const uint32_t r0 = (uint32_t)(M.keys[M.cedge[c]] & kPackedRankMask);
-        M.cedge[c] = r0; // the assign pass reads the edge's first rank here, not through the table
-        flag[(m ? M0.nk : 0) + rank] = (r0 == rank) ? 1u : 0u;
-        if (r0 != rank && M.idx[rank_corner(M.cm, r0, m)] == a) atomicOr(&C->nonmanifold, 1u); // used twice in one direction
-    }
+    *m = t >= tiles0;
+    *r0 = (uint64_t)(*m ? t - tiles0 : t) * kTopoTile;
+    *r1 = *r0 + kTopoTile < T.part[*m].nk ? *r0 + kTopoTile : T.part[*m].nk;
+    return *r0 < *r1;
 }
 
-// edge counts from the scan: both meshes scanned together, or (resident
-// source) the cut mesh alone
-__global__ void k_store_edge_counts_packed(const uint32_t* __restrict__ eid, const uint32_t* __restrict__ flag, uint64_t K0,
-                                           const uint32_t* __restrict__ total, int cut_only, Counters* C)
+// first uses of each tile
+__global__ void __launch_bounds__(kBlock) k_topo_count(Topo T, uint32_t tiles0, uint32_t* __restrict__ tsum)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        if (cut_only) {
-            C->n_edges_cut = *total;
-        } else {
-            const uint32_t ns = K0 ? eid[K0 - 1] + flag[K0 - 1] : 0u;
-            C->n_edges_src = ns;
-            C->n_edges_cut = *total - ns;
+    int m;
+    uint64_t r0, r1;
+    topo_tile(T, blockIdx.x, tiles0, &m, &r0, &r1);
+    const uint32_t* opp = T.part[m].opp;
+    uint32_t s = 0;
+#pragma unroll
+    for (int j = 0; j < (int)(kTopoTile / kBlock); ++j) {
+        const uint64_t r = r0 + j * kBlock + threadIdx.x;
+        if (r < r1) s += opp[r] > (uint32_t)r ? 1u : 0u; // kNoCorner is past every rank
+    }
+    uint32_t tot;
+    block_exclusive_scan(s, &tot);
+    if (threadIdx.x == 0) tsum[blockIdx.x] = tot;
+}
+
+// The edge table of one tile, in order: rank r is an edge's first use when it
+// has no partner or a later one.  tsum: the tiles' counts (each block sums
+// those before its own), or with scanned their exclusive scan and total.
+__global__ void __launch_bounds__(kBlock) k_topo_apply(Topo T, uint32_t tiles0, uint32_t tiles, const uint32_t* __restrict__ tsum,
+                                                       int scanned, const uint32_t* __restrict__ total, int cut_only,
+                                                       Counters* C, uint32_t* __restrict__ ev0, uint32_t* __restrict__ ev1,
+                                                       int32_t* __restrict__ ef0, int32_t* __restrict__ ef1)
+{
+    __shared__ uint32_t wtot[kBlock / 64];
+    const uint32_t t = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    uint32_t base;
+    if (scanned) {
+        base = tsum[t];
+        if (t == 0 && threadIdx.x == 0) {
+            if (!cut_only) C->n_edges_src = tsum[tiles0]; // the cut part has a tile
+            C->n_edges_cut = *total - (cut_only ? 0u : tsum[tiles0]);
         }
-    }
-}
-
-__global__ void k_edge_assign_packed(TopoMesh M0, TopoMesh M1, uint64_t start, const uint32_t* __restrict__ eid,
-                                     int cut_only, Counters* C, uint32_t* __restrict__ ev0, uint32_t* __restrict__ ev1,
-                                     int32_t* __restrict__ ef0, int32_t* __restrict__ ef1)
-{
-    const uint64_t K = M0.nk + M1.nk;
-    const uint32_t eb1 = cut_only ? (uint32_t)C->n_edges_src : 0u;
-    for (uint64_t q = start + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; q < K; q += (uint64_t)gridDim.x * blockDim.x) {
-        const int m = q >= M0.nk;
-        const TopoMesh& M = m ? M1 : M0;
-        const uint64_t c = m ? q - M0.nk : q;
-        uint32_t f, b, n, i;
-        M.cm(c, f, b, n, i);
-        const uint32_t a = M.idx[c], d = M.idx[b + (i + 1 == n ? 0 : i + 1)];
-        const uint32_t rank = corner_rank(b, i, n, m);
-        const uint32_t r0 = M.cedge[c]; // the edge's first rank (flag pass)
-        const uint32_t e = (m ? eb1 : 0u) + eid[(m ? M0.nk : 0) + r0];
-        M.cedge[c] = e;
-        if (r0 == rank) {
-            ev0[e] = M.vofs + a;
-            ev1[e] = M.vofs + d;
-            ef0[e] = (int32_t)(M.fofs + f);
-        } else if (atomicExch(&ef1[e], (int32_t)(M.fofs + f)) != -1) {
-            atomicOr(&C->nonmanifold, 4u);
+    } else {
+        uint32_t s = 0, s0 = 0, s1 = 0;
+        for (uint32_t q = threadIdx.x; q < (t ? t : tiles); q += kBlock) {
+            const uint32_t v = tsum[q];
+            if (q < t) s += v;
+            else (q < tiles0 ? s0 : s1) += v;
         }
-    }
-}
-
-// Batches: the packed edge table with one region per (pair, mesh).  Every
-// corner's edge lies within its pair, so the words of pair p's edges live in a
-// region of 2 K_p slots at 2 c_p of its part's table (c_p: the pair's first
-// corner in the part, K_p its corner count) and hold pair-local vertex ids and
-// insertion ranks (21 and 22 bits; the host takes this path only when every
-// pair fits).  A pair's corners are consecutive, so the waves of a launch
-// touch the regions of a few pairs at a time and stay in cache, where one
-// table hashed over the whole batch misses on every probe.  Flags, scans and
-// edge ids are the part-wide ones of the two-table path: the numbering does
-// not change.
-struct BatchTopo {
-    const uint32_t* idx;        // face vertex ids of the part (ids of the concatenated part)
-    CornerMap cm;
-    unsigned long long* keys;   // 2 nk slots
-    uint32_t* cedge;
-    uint64_t nk;
-    const uint32_t* fpair;      // soup face -> pair
-    const BatchPair* bp;
-    const uint32_t* off;        // the part's face -> first corner (nf + 1 entries)
-    uint32_t fofs;              // soup id of the part's first face (0 or Fs)
-    int m;                      // 0 source part, 1 cut part
-};
-
-// the region of face f's pair: first vertex id, first corner and corner count
-__device__ __forceinline__ void batch_region(const BatchTopo& T, uint32_t f, uint32_t& vb, uint64_t& cb, uint64_t& kp)
-{
-    const BatchPair b = T.bp[T.fpair[T.fofs + f]];
-    const uint32_t f0 = T.m ? b.fc0 : b.fs0, nfp = T.m ? b.nfc : b.nfs;
-    vb = T.m ? b.vc0 : b.vs0;
-    cb = T.off[f0];
-    kp = T.off[f0 + nfp] - cb;
-}
-
-__global__ void k_edge_insert_batch(BatchTopo T)
-{
-    for (uint64_t c = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; c < T.nk; c += (uint64_t)gridDim.x * blockDim.x) {
-        uint32_t f, b, n, i;
-        T.cm(c, f, b, n, i);
-        uint32_t vb;
-        uint64_t cb, kp;
-        batch_region(T, f, vb, cb, kp);
-        const uint32_t a = T.idx[c] - vb, d = T.idx[b + (i + 1 == n ? 0 : i + 1)] - vb;
-        const uint64_t ek = packed_edge(a, d);
-        const uint32_t rank = corner_rank(b, i, n, T.m) - (uint32_t)cb;
-        const unsigned long long w = (ek << kPackedRankBits) | rank;
-        const uint64_t base = 2 * cb, size = 2 * kp;
-        uint64_t h = base + __umul64hi(hash64(ek), size);
-        for (uint64_t probe = 0; probe < size; ++probe) {
-            const unsigned long long prev = atomicCAS(&T.keys[h], kEmpty64, w);
-            if (prev == kEmpty64) break;
-            if ((prev >> kPackedRankBits) == ek) {
-                if ((prev & kPackedRankMask) > rank) atomicMin(&T.keys[h], w);
-                break;
+        block_exclusive_scan(s, &base);
+        if (t == 0) { // whole block: the counts
+            uint32_t n0, n1;
+            block_exclusive_scan(s0, &n0);
+            block_exclusive_scan(s1, &n1);
+            if (threadIdx.x == 0) {
+                if (!cut_only) C->n_edges_src = n0;
+                C->n_edges_cut = n1;
             }
-            h = (h + 1 == base + size) ? base : h + 1;
         }
-        T.cedge[c] = (uint32_t)h;
     }
-}
-
-// flag[rank] = 1 at an edge's first use (part-local corner ranks)
-__global__ void k_edge_flag_batch(BatchTopo T, uint32_t* __restrict__ flag, Counters* C)
-{
-    for (uint64_t c = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; c < T.nk; c += (uint64_t)gridDim.x * blockDim.x) {
-        uint32_t f, b, n, i;
-        T.cm(c, f, b, n, i);
-        uint32_t vb;
-        uint64_t cb, kp;
-        batch_region(T, f, vb, cb, kp);
-        const uint32_t a = T.idx[c];
-        const uint32_t rank = corner_rank(b, i, n, T.m);
-        const uint32_t r0 = (uint32_t)cb + (uint32_t)(T.keys[T.cedge[c]] & kPackedRankMask);
-        T.cedge[c] = r0; // the assign pass reads the edge's first rank here, not through the table
-        flag[rank] = (r0 == rank) ? 1u : 0u;
-        if (r0 != rank && T.idx[rank_corner(T.cm, r0, T.m)] == a) atomicOr(&C->nonmanifold, 1u); // used twice in one direction
+    if (cut_only) base += (uint32_t)C->n_edges_src; // after the resident source's edges
+    int m;
+    uint64_t r0, r1;
+    topo_tile(T, t, tiles0, &m, &r0, &r1);
+    const TopoPart& P = T.part[m];
+    constexpr int kRows = kTopoTile / kBlock;
+    // wave w takes 64 kRows consecutive ranks, 64 a row
+    const uint64_t wr = r0 + (uint64_t)wid * 64 * kRows + lane;
+    uint32_t o[kRows], before[kRows], run = 0;
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+        const uint64_t r = wr + 64 * j;
+        o[j] = r < r1 ? P.opp[r] : 0u;
     }
-}
-
-__global__ void k_edge_assign_batch(BatchTopo T, const uint32_t* __restrict__ eid_by_rank, Counters* C, uint32_t vofs,
-                                    uint32_t* __restrict__ ev0, uint32_t* __restrict__ ev1, int32_t* __restrict__ ef0,
-                                    int32_t* __restrict__ ef1)
-{
-    const uint32_t ebase = T.m ? (uint32_t)C->n_edges_src : 0u;
-    for (uint64_t c = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; c < T.nk; c += (uint64_t)gridDim.x * blockDim.x) {
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+        const uint64_t r = wr + 64 * j;
+        const uint64_t first = __ballot(r < r1 && o[j] > (uint32_t)r);
+        before[j] = run + (uint32_t)__popcll(first & ((1ull << lane) - 1ull));
+        run += (uint32_t)__popcll(first);
+    }
+    if (lane == 0) wtot[wid] = run;
+    __syncthreads();
+    for (uint32_t q = 0; q < wid; ++q) base += wtot[q];
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+        const uint64_t r = wr + 64 * j;
+        if (r >= r1 || o[j] <= (uint32_t)r) continue;
+        const uint64_t c = rank_corner(P.cm, (uint32_t)r, m);
         uint32_t f, b, n, i;
-        T.cm(c, f, b, n, i);
-        uint32_t vb;
-        uint64_t cb, kp;
-        batch_region(T, f, vb, cb, kp);
-        const uint32_t a = T.idx[c], d = T.idx[b + (i + 1 == n ? 0 : i + 1)];
-        const uint32_t rank = corner_rank(b, i, n, T.m);
-        const uint32_t r0 = T.cedge[c]; // the edge's first rank (flag pass)
-        const uint32_t e = ebase + eid_by_rank[r0];
-        T.cedge[c] = e;
-        if (r0 == rank) {
-            ev0[e] = vofs + a;
-            ev1[e] = vofs + d;
-            ef0[e] = (int32_t)(T.fofs + f);
-        } else if (atomicExch(&ef1[e], (int32_t)(T.fofs + f)) != -1) {
-            atomicOr(&C->nonmanifold, 4u);
+        P.cm(c, f, b, n, i);
+        const uint32_t e = base + before[j];
+        P.cedge[c] = e;
+        ev0[e] = P.vofs + P.idx[c];
+        ev1[e] = P.vofs + P.idx[b + (i + 1 == n ? 0 : i + 1)];
+        ef0[e] = (int32_t)(P.fofs + f);
+        int32_t f1 = -1;
+        if (o[j] != kNoCorner) {
+            P.cm(o[j], f, b, n, i);
+            f1 = (int32_t)(P.fofs + f);
         }
+        ef1[e] = f1;
     }
 }
 
@@ -1083,7 +1218,7 @@ __global__ void k_cc_init(uint32_t* __restrict__ parent, uint64_t n)
 __global__ void k_cc_hook(const uint32_t* __restrict__ ev0, const uint32_t* __restrict__ ev1, Counters* C,
                           int cut_only, uint32_t* parent)
 {
-    if (C->cc_done) return;
+    if (C->cc_done || C->bad_input) return; // a rejected face list names no vertices
     const uint64_t ne = C->n_edges_src + C->n_edges_cut;
     bool hooked = false;
     for (uint64_t e = (cut_only ? C->n_edges_src : 0) + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < ne;
@@ -2358,6 +2493,29 @@ __device__ __forceinline__ bool pair_exists(const unsigned long long* phash, uin
     return hash_find(phash, pmask, ((uint64_t)s << 32) | c) >= 0;
 }
 
+// the soup edge of corner k of a face (corners [b, b + n) of mesh m, soup face
+// self) and its other face (-1: border).  A corner that is its edge's second
+// use finds the edge at its partner's corner (k_topo_apply).
+__device__ __forceinline__ uint32_t corner_edge(const Soup& S, int m, uint32_t b, uint32_t k, uint32_t n, uint32_t self,
+                                                int32_t* other)
+{
+    if (!S.opp[m]) { // the edge of every corner is given
+        const uint32_t e = S.cedge[m][b + k];
+        const int32_t f0 = S.ef0[e], f1 = S.ef1[e];
+        *other = f0 == (int32_t)self ? f1 : f0;
+        return e;
+    }
+    const uint32_t r = corner_rank(b, k, n, m), o = S.opp[m][r];
+    const CornerMap cm{S.off[m], S.cface[m]};
+    *other = -1;
+    if (o != kNoCorner) {
+        uint32_t f, ob, on, oi;
+        cm(o, f, ob, on, oi);
+        *other = (int32_t)((m ? S.nf[0] : 0u) + f);
+    }
+    return S.cedge[m][o < r ? rank_corner(cm, o, m) : (uint64_t)(b + k)];
+}
+
 __device__ __forceinline__ bool edge_face_cull(const Soup& S, uint32_t e, uint32_t g)
 {
     const double* p0 = S.ps_v + 3 * (uint64_t)S.ev1[e]; // vertex(e, 0) = target(h0)
@@ -2413,9 +2571,8 @@ __global__ void __launch_bounds__(kStageBlock) k_tests(Soup S, const unsigned lo
             const uint32_t g = side ? s : Fs + c;    // the other face (ps id)
             const uint32_t b = S.off[side][f], nn = S.off[side][f + 1] - b;
             for (uint32_t k = j0; k < nn; k += 3) {
-                const uint32_t e = S.cedge[side][b + k];
-                const int32_t f0 = S.ef0[e], f1 = S.ef1[e];
-                const int32_t fo = (f0 == (int32_t)self) ? f1 : f0;
+                int32_t fo; // the edge's other face
+                const uint32_t e = corner_edge(S, side, b, k, nn, self, &fo);
                 // the lowest-numbered face of e paired with g emits the test
                 if (fo >= 0 && (uint32_t)fo < self) {
                     const bool paired = side ? pair_exists(phash, pmask, s, (uint32_t)fo - Fs)
@@ -3143,24 +3300,24 @@ __global__ void __launch_bounds__(1024) k_batch_layout(Params* P, const unsigned
 }
 
 // polygon-soup edge ranges of every pair, once the edges are numbered: the
-// edges first used by a pair's corners are numbered in one run, starting at
-// the count of edges first used before its first corner
+// edges first used by a pair's corners are numbered in one run, and the pair's
+// first corner (in insertion order) starts it, being no edge's second use
 __global__ void k_batch_edge_bases(BatchPair* bp, uint32_t npairs, const uint32_t* __restrict__ off_s,
                                    const uint32_t* __restrict__ off_c, uint32_t nfs, uint32_t nfc,
-                                   const uint32_t* __restrict__ eid_s, const uint32_t* __restrict__ eid_c,
+                                   const uint32_t* __restrict__ cedge_s, const uint32_t* __restrict__ cedge_c,
                                    const Counters* __restrict__ C)
 {
     const uint32_t Es = (uint32_t)C->n_edges_src, Ec = (uint32_t)C->n_edges_cut;
+    // a cut face's first rank is its second corner (corner_rank)
+    auto src_edge = [&](uint32_t f) { return f < nfs ? cedge_s[off_s[f]] : Es; };
+    auto cut_edge = [&](uint32_t f) { return f < nfc ? cedge_c[off_c[f] + 1] - Es : Ec; };
     for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < npairs; p += gridDim.x * blockDim.x) {
         const BatchPair b = bp[p];
-        const uint32_t s0 = b.fs0 < nfs ? eid_s[off_s[b.fs0]] : Es;
-        const uint32_t s1 = b.fs0 + b.nfs < nfs ? eid_s[off_s[b.fs0 + b.nfs]] : Es;
-        const uint32_t c0 = b.fc0 < nfc ? eid_c[off_c[b.fc0]] : Ec;
-        const uint32_t c1 = b.fc0 + b.nfc < nfc ? eid_c[off_c[b.fc0 + b.nfc]] : Ec;
+        const uint32_t s0 = src_edge(b.fs0), c0 = cut_edge(b.fc0);
         bp[p].es0 = s0;
-        bp[p].nes = s1 - s0;
+        bp[p].nes = src_edge(b.fs0 + b.nfs) - s0;
         bp[p].ec0 = c0;
-        bp[p].nec = c1 - c0;
+        bp[p].nec = cut_edge(b.fc0 + b.nfc) - c0;
     }
 }
 

@@ -46,6 +46,7 @@ struct Counters {
     unsigned int gp, bad_src, bad_cut, unsupported, nonmanifold, bad_input, pair_fail, partial;
     unsigned int sum_next; // batches: work-queue head of the serial sums
     unsigned int ov_trip;  // the triplet scratch overflowed
+    unsigned int ov_topo;  // a bucket of the edge numbering overflowed: the hash tables number the edges
     unsigned int trav_q[8]; // persistent traversal: head of each work queue (blocks taken)
     unsigned int ncc[2];    // connected components of each mesh's vertex graph (all pairs of a batch)
     unsigned int cc_changed, cc_done; // component check: a hook this round; no hook in the last round
@@ -91,7 +92,9 @@ struct Soup {
     uint32_t nv[2], nf[2];
     const double* ps_v;      // shifted coordinates, xyz per ps vertex
     const double* box;       // per ps face: min xyz, max xyz (cut faces enlarged)
-    const uint32_t* cedge[2];// per corner (mesh corner order): ps edge id
+    const uint32_t* cedge[2];// per corner (mesh corner order): ps edge id (with opp: of its edge's first corner only)
+    const uint32_t* opp[2];  // per insertion rank: rank of the edge's other corner (null: cedge holds every corner's)
+    const uint32_t* cface[2];// per corner: its face (null: triangles)
     const uint32_t* ev0;     // per ps edge: h0 = v0 -> v1
     const uint32_t* ev1;
     const int32_t* ef0;      // face of h0, h1 (-1 none)

@@ -135,7 +135,9 @@ struct Resident {
     const uint32_t* didx = nullptr;
     const uint32_t* dsz = nullptr;
     const uint32_t* off = nullptr;   // face offsets
-    const uint32_t* cedge = nullptr; // corner -> edge
+    const uint32_t* cedge = nullptr; // corner -> edge (of first corners, with opp)
+    const uint32_t* opp = nullptr;   // by rank: the edge's other corner
+    const uint32_t* cface = nullptr; // corner -> face (polygon meshes)
     const uint32_t *ev0 = nullptr, *ev1 = nullptr;
     const int32_t *ef0 = nullptr, *ef1 = nullptr; // source edges [0, ne)
     const float* rawbox = nullptr;   // float leaf boxes of the source faces
@@ -160,7 +162,15 @@ struct mcgpu_context_t {
     // kernel so that finish() waits once instead of copying after the wait
     DevState* hstate = nullptr;
     bool state_copied = false;
-    Buf hkeys[2], hfirst[2], eflag[2], eid[2], cedge[2], cface[2], etotal;
+    Buf hkeys[2], hfirst[2], eflag[2], eid[2], cedge[2], cface[2], etotal; // edge hash tables (topo_tables)
+    Buf opp, twords, tsum, tseg;     // edge numbering by buckets: partners, words, tile counts, a batch's segments
+    TopoSeg topo_seg[2] = {};
+    std::vector<TopoSeg> hseg;       // a batch's segments
+    uint32_t nseg = 0, topo_buckets = 0, topo_tiles = 0;
+    int topo_items = 4;
+    uint64_t topo_words = 0;
+    bool topo_hash = false;          // the hash tables number this dispatch's edges (no buckets for it, or one overflowed)
+    bool topo_given = false;         // the caller's edge numbering (mcgpu_dispatch_narrow)
     Buf ev0, ev1, ef0, ef1;
     Buf mcode, mface, mcode2, mface2; // Morton keys and leaf order of both meshes
     Buf nodes[2], rawbox;
@@ -207,7 +217,7 @@ struct mcgpu_context_t {
     bool batch = false;
     uint32_t npairs = 0;
     int batch_mb = 7;                    // Morton bits per axis within a pair
-    bool batch_packed = false;           // every pair's vertex ids and corner ranks fit the packed edge word
+    bool batch_corners = false;          // the host knows every pair's corner counts (hseg)
     bool shifted_bp = false;             // this dispatch's broad phase runs in shifted coordinates (Counters::loose)
     bool allow_loose = false;            // a single pair's own broad phase: a loose raw tolerance reruns it shifted
     bool cc_check = false;               // count each mesh's connected components (check_input_mesh)
@@ -369,10 +379,14 @@ Soup make_soup(mcgpu_context ctx)
         S.nv[m] = ctx->nv[m];
         S.nf[m] = ctx->nf[m];
         S.cedge[m] = P_<uint32_t>(ctx->cedge[m]);
+        S.cface[m] = ctx->dsz[m] ? P_<uint32_t>(ctx->cface[m]) : nullptr;
+        S.opp[m] = ctx->topo_hash || ctx->topo_given ? nullptr : P_<uint32_t>(ctx->opp) + (m ? ctx->ncorner[0] : 0);
     }
     if (ctx->res) { // the resident source's face offsets and corner edges
         S.off[0] = ctx->res->off;
         S.cedge[0] = ctx->res->cedge;
+        S.cface[0] = ctx->res->cface;
+        S.opp[0] = ctx->res->opp;
     }
     S.ps_v = P_<double>(ctx->ps_v);
     S.box = P_<double>(ctx->box);
@@ -394,6 +408,79 @@ void stage_event(mcgpu_context ctx, int e, hipStream_t st)
 {
     if (ctx->stage_timing) (void)hipEventRecord(ctx->ev[e], st);
 }
+
+// The buckets of the edge numbering: one segment per mesh (per mesh of every
+// pair in a batch), of 2^bb buckets of at most kTopoFill words on average, or
+// one of up to kTopoCap.  False when a segment needs more than 2^kTopoMaxBits
+// buckets or its words more than 64 bits, or when the host does not know a
+// batch's corner counts: the hash tables number the edges then.
+bool topo_plan(mcgpu_context ctx)
+{
+    TopoSeg* seg = ctx->topo_seg;
+    if (ctx->batch) {
+        if (!ctx->batch_corners) return false;
+        seg = ctx->hseg.data();
+        ctx->nseg = (uint32_t)ctx->hseg.size();
+    } else {
+        const int m0 = ctx->res ? 1 : 0;
+        ctx->nseg = 2 - m0;
+        for (int m = m0; m < 2; ++m) {
+            if (ctx->ncorner[m] > 0xffffffffull) return false;
+            seg[m - m0] = TopoSeg{};
+            seg[m - m0].k = (uint32_t)ctx->ncorner[m];
+            seg[m - m0].vbits = (uint8_t)std::max(8, bits_for(ctx->nv[m]));
+            seg[m - m0].m = (uint8_t)m;
+        }
+    }
+    uint32_t kmax = 0;
+    for (uint32_t i = 0; i < ctx->nseg; ++i) kmax = std::max(kmax, seg[i].k);
+    // corners a scatter block takes, a thread: the runs a block writes are tile /
+    // buckets words long, and the blocks in flight fall with the tile; the
+    // template's bucket limit (8, 10, 12 bits) holds for each range
+    ctx->topo_items = kmax <= (kTopoFill << 8) ? 4 : kmax <= (kTopoFill << 10) ? 8 : 16;
+    const uint32_t tile = kTopoScatterBlock * ctx->topo_items;
+    uint64_t words = 0, buckets = 0, tiles = 0;
+    for (uint32_t i = 0; i < ctx->nseg; ++i) {
+        TopoSeg& g = seg[i];
+        int bb = 0;
+        if (g.k > kTopoCap)
+            while (((uint64_t)kTopoFill << bb) < g.k) ++bb;
+        g.bb = (uint8_t)bb;
+        g.kbits = (uint8_t)bits_for((uint64_t)g.k + 1);
+        if (bb > kTopoMaxBits || bb > 2 * (g.vbits - 3) || 2 * g.vbits - bb + g.kbits + 1 > 64) return false;
+        g.bucket0 = (uint32_t)buckets;
+        g.tile0 = (uint32_t)tiles;
+        g.w0 = words;
+        buckets += 1ull << bb;
+        if (bb) {
+            tiles += ((uint64_t)g.k + tile - 1) / tile;
+            words += (uint64_t)kTopoCap << bb;
+        }
+    }
+    if (buckets > 0x7fffffffull || tiles > 0x7fffffffull) return false;
+    ctx->topo_buckets = (uint32_t)buckets;
+    ctx->topo_tiles = (uint32_t)tiles;
+    ctx->topo_words = words;
+    return true;
+}
+
+// the hash tables of the edge numbering: a power of two of slots per mesh
+mcgpu_result alloc_edge_tables(mcgpu_context ctx)
+{
+    uint32_t* u;
+    unsigned long long* ull;
+    for (int m = ctx->res ? 1 : 0; m < 2; ++m) {
+        const uint64_t nk = ctx->ncorner[m], hs = next_pow2(2 * nk + 2);
+        CK(ensure(ctx->hkeys[m], hs, &ull));
+        CK(ensure(ctx->hfirst[m], hs, &ull));
+        CK(ensure(ctx->eflag[m], nk, &u));
+        CK(ensure(ctx->eid[m], nk, &u));
+    }
+    CK(ensure(ctx->scan_tmp_c, scan_tmp_elems(std::max(ctx->ncorner[0], ctx->ncorner[1]) + 8) + 1024, &u));
+    return MCGPU_SUCCESS;
+}
+
+uint32_t topo_rank_tiles(uint64_t corners) { return (uint32_t)((corners + kTopoTile - 1) / kTopoTile); }
 
 mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
 {
@@ -417,19 +504,12 @@ mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
     CK(ensure(ctx->ef1, K, &i32));
     CK(ensure(ctx->etotal, 2, &u));
     uint64_t scan_need = scan_tmp_elems(K + 8);
-    // the single pair's packed table and the two-table path hash over a power
-    // of two; a packed batch takes 2 slots per corner (one region per pair)
-    // and has no first-use table
-    const bool packed_batch = ctx->batch && ctx->batch_packed;
+    ctx->topo_given = false;
+    ctx->topo_hash = !topo_plan(ctx);
     for (int m = 0; m < 2; ++m) {
         const uint64_t nk = ctx->ncorner[m], nf = ctx->nf[m];
-        const uint64_t hs = packed_batch ? 2 * nk + 8 : next_pow2(2 * nk + 2);
         CK(ensure(ctx->off[m], nf + 1, &u));
-        CK(ensure(ctx->hkeys[m], hs, &ull));
-        if (!packed_batch) CK(ensure(ctx->hfirst[m], hs, &ull));
         CK(ensure(ctx->cface[m], nk, &u));
-        CK(ensure(ctx->eflag[m], nk, &u));
-        CK(ensure(ctx->eid[m], nk, &u));
         CK(ensure(ctx->cedge[m], nk, &u));
         int D = 0;
         while ((1ull << D) < nf) ++D;
@@ -442,7 +522,8 @@ mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
     CK(ensure(ctx->mcode2, F, &u));
     CK(ensure(ctx->mface2, F, &u));
     scan_need = std::max<uint64_t>(scan_need, scan_tmp_elems(F + 8));
-    CK(ensure(ctx->cand, F + 8, &u));
+    // the candidate-face flags and, behind them, the buckets' word counts (cleared together)
+    CK(ensure(ctx->cand, F + 8 + (ctx->topo_hash ? 0 : (uint64_t)kTopoFillStride * ctx->topo_buckets), &u));
     CK(ensure(ctx->cand_list, F + 8, &u));
     Plane* pl;
     CK(ensure(ctx->planes, F, &pl));
@@ -462,12 +543,17 @@ mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
         CK(ensure(ctx->sckpt, 6 * lcap, &dp));
         CK(ensure(ctx->sflags, 16, &u));
     }
-    // the packed edge numbering scans both meshes' first-use flags as one array
-    const uint64_t K2 = ctx->ncorner[0] + ctx->ncorner[1];
-    CK(ensure(ctx->eflag[0], K2 + 8, &u));
-    CK(ensure(ctx->eid[0], K2 + 8, &u));
     if (ctx->cc_check) CK(ensure(ctx->cc_parent, (uint64_t)ctx->nv[0] + ctx->nv[1] + 8, &u));
-    CK(ensure(ctx->scan_tmp_c, scan_tmp_elems(K2 + 8) + 1024, &u));
+    if (ctx->topo_hash) {
+        const mcgpu_result r = alloc_edge_tables(ctx);
+        if (r != MCGPU_SUCCESS) return r;
+    } else {
+        CK(ensure(ctx->opp, K + 8, &u));
+        CK(ensure(ctx->twords, ctx->topo_words, &ull));
+        CK(ensure(ctx->tsum, (uint64_t)topo_rank_tiles(ctx->ncorner[0]) + topo_rank_tiles(ctx->ncorner[1]) + 8, &u));
+        TopoSeg* sg;
+        if (ctx->batch) CK(ensure(ctx->tseg, ctx->nseg, &sg));
+    }
     return MCGPU_SUCCESS;
 }
 
@@ -539,16 +625,6 @@ SumBufs sum_bufs(mcgpu_context ctx)
     B.fail = P_<uint32_t>(ctx->sflags);
     B.nb64 = P_<uint32_t>(ctx->sflags) + 8;
     return B;
-}
-
-// one packed word per edge (frontend_kernels.hpp, TopoMesh) when every vertex
-// id fits 21 bits and every corner rank 22 bits; batches keep the two tables
-bool topology_packed(mcgpu_context ctx)
-{
-    if (ctx->batch) return false;
-    for (int m = ctx->res ? 1 : 0; m < 2; ++m)
-        if (ctx->nv[m] >= (1u << kPackedVertexBits) || ctx->ncorner[m] >= (1ull << kPackedRankBits)) return false;
-    return true;
 }
 
 // the part of the pipeline that runs again for a perturbed cut mesh (whose
@@ -1008,7 +1084,7 @@ void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
     stage_event(ctx, EV_C0, s3);
     uint32_t* etotal = P_<uint32_t>(ctx->etotal);
     const uint64_t K = ctx->ncorner[0] + ctx->ncorner[1];
-    fill_u32(ctx->cand.p, 0u, F, s3);
+    fill_u32(ctx->cand.p, 0u, F + 8 + (ctx->topo_hash ? 0 : (uint64_t)kTopoFillStride * ctx->topo_buckets), s3);
     ev_record(ctx, EV_C_FILL, s3);
     const uint32_t res_ne = ctx->res ? ctx->res->ne : 0u;
     if (ctx->res) { // the resident source's edges occupy [0, ne) of the edge table
@@ -1017,7 +1093,6 @@ void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
         (void)hipMemcpyAsync(ctx->ef0.p, ctx->res->ef0, 4ull * res_ne, hipMemcpyDeviceToDevice, s3);
         (void)hipMemcpyAsync(ctx->ef1.p, ctx->res->ef1, 4ull * res_ne, hipMemcpyDeviceToDevice, s3);
     }
-    fill_u32(P_<uint32_t>(ctx->ef1) + res_ne, 0xffffffffu, K - res_ne, s3);
     CornerMap cmap[2];
     for (int m = 0; m < 2; ++m) {
         cmap[m].off = P_<uint32_t>(ctx->off[m]);
@@ -1027,42 +1102,35 @@ void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
     }
     // the scans of this stream use their own scratch: stream B's sort uses scan_tmp
     uint32_t* ctmp = P_<uint32_t>(ctx->scan_tmp_c);
-    if (topology_packed(ctx)) {
-        TopoMesh TM[2];
+    if (!ctx->topo_hash) {
+        Topo T{};
         for (int m = 0; m < 2; ++m)
-            TM[m] = TopoMesh{ctx->didx[m], cmap[m], P_<unsigned long long>(ctx->hkeys[m]),
-                             next_pow2(2 * ctx->ncorner[m] + 2) - 1, P_<uint32_t>(ctx->cedge[m]), ctx->ncorner[m],
-                             m ? ctx->nv[0] : 0u, m ? ctx->nf[0] : 0u};
-        const int cut_only = ctx->res ? 1 : 0;
-        const uint64_t K0 = ctx->ncorner[0], start = cut_only ? K0 : 0;
-        uint32_t* flag = P_<uint32_t>(ctx->eflag[0]);
-        uint32_t* eid = P_<uint32_t>(ctx->eid[0]);
-        const uint64_t t0 = cut_only ? 0 : TM[0].mask + 1, t1 = TM[1].mask + 1;
-        k_fill2_u64<<<grid_for(t0 + t1), kBlock, 0, s3>>>(TM[0].keys, t0, TM[1].keys, t1, kEmpty64);
-        k_edge_insert_packed<<<grid_for(K - start), kBlock, 0, s3>>>(TM[0], TM[1], start);
-        k_edge_flag_packed<<<grid_for(K - start), kBlock, 0, s3>>>(TM[0], TM[1], start, flag, C);
-        scan_exclusive(flag + start, eid + start, K - start, ctmp, etotal, s3);
-        k_store_edge_counts_packed<<<1, 1, 0, s3>>>(eid, flag, K0, etotal, cut_only, C);
-        k_edge_assign_packed<<<grid_for(K - start), kBlock, 0, s3>>>(TM[0], TM[1], start, eid, cut_only, C,
-                                                                     P_<uint32_t>(ctx->ev0), P_<uint32_t>(ctx->ev1),
-                                                                     P_<int32_t>(ctx->ef0), P_<int32_t>(ctx->ef1));
-    } else if (ctx->batch && ctx->batch_packed) {
-        BatchTopo T[2];
-        for (int m = 0; m < 2; ++m) {
-            T[m] = BatchTopo{ctx->didx[m], cmap[m], P_<unsigned long long>(ctx->hkeys[m]), P_<uint32_t>(ctx->cedge[m]),
-                             ctx->ncorner[m], P_<uint32_t>(ctx->fpair), P_<BatchPair>(ctx->bpairs),
-                             P_<uint32_t>(ctx->off[m]), m ? ctx->nf[0] : 0u, m};
-            fill_u64(T[m].keys, kEmpty64, 2 * ctx->ncorner[m], s3);
-            k_edge_insert_batch<<<grid_for(ctx->ncorner[m]), kBlock, 0, s3>>>(T[m]);
-            k_edge_flag_batch<<<grid_for(ctx->ncorner[m]), kBlock, 0, s3>>>(T[m], P_<uint32_t>(ctx->eflag[m]), C);
-            scan_exclusive(P_<uint32_t>(ctx->eflag[m]), P_<uint32_t>(ctx->eid[m]), ctx->ncorner[m], ctmp, etotal + m, s3);
-            k_store_edge_count<<<1, 1, 0, s3>>>(etotal + m, C, m);
+            T.part[m] = TopoPart{ctx->didx[m], cmap[m], P_<uint32_t>(ctx->cedge[m]),
+                                 P_<uint32_t>(ctx->opp) + (m ? ctx->ncorner[0] : 0), ctx->ncorner[m], m ? ctx->nv[0] : 0u,
+                                 m ? ctx->nf[0] : 0u};
+        for (int i = 0; i < 2; ++i) T.seg[i] = ctx->topo_seg[i];
+        T.nseg = ctx->nseg;
+        T.tab = ctx->batch ? P_<TopoSeg>(ctx->tseg) : nullptr;
+        T.words = P_<unsigned long long>(ctx->twords);
+        T.fill = P_<uint32_t>(ctx->cand) + F + 8;
+        if (ctx->topo_tiles) {
+            const dim3 g(ctx->topo_tiles), b(kTopoScatterBlock);
+            if (ctx->topo_items == 4) k_topo_scatter<4, 8><<<g, b, 0, s3>>>(T, C);
+            else if (ctx->topo_items == 8) k_topo_scatter<8, 10><<<g, b, 0, s3>>>(T, C);
+            else k_topo_scatter<16, 12><<<g, b, 0, s3>>>(T, C);
         }
-        for (int m = 0; m < 2; ++m)
-            k_edge_assign_batch<<<grid_for(ctx->ncorner[m]), kBlock, 0, s3>>>(
-                T[m], P_<uint32_t>(ctx->eid[m]), C, m ? ctx->nv[0] : 0u, P_<uint32_t>(ctx->ev0), P_<uint32_t>(ctx->ev1),
-                P_<int32_t>(ctx->ef0), P_<int32_t>(ctx->ef1));
+        k_topo_buckets<<<ctx->topo_buckets, kTopoBlock, 0, s3>>>(T, C);
+        const int cut_only = ctx->res ? 1 : 0;
+        const uint32_t tiles0 = cut_only ? 0 : topo_rank_tiles(ctx->ncorner[0]);
+        const uint32_t tiles = tiles0 + topo_rank_tiles(ctx->ncorner[1]);
+        uint32_t* tsum = P_<uint32_t>(ctx->tsum);
+        k_topo_count<<<tiles, kBlock, 0, s3>>>(T, tiles0, tsum);
+        const int scanned = tiles > kTopoDirectTiles;
+        if (scanned) k_scan_tiles<<<1, kScanBlock, 0, s3>>>(tsum, tiles, etotal);
+        k_topo_apply<<<tiles, kBlock, 0, s3>>>(T, tiles0, tiles, tsum, scanned, etotal, cut_only, C, P_<uint32_t>(ctx->ev0),
+                                               P_<uint32_t>(ctx->ev1), P_<int32_t>(ctx->ef0), P_<int32_t>(ctx->ef1));
     } else {
+    fill_u32(P_<uint32_t>(ctx->ef1) + res_ne, 0xffffffffu, K - res_ne, s3);
     for (int m = ctx->res ? 1 : 0; m < 2; ++m) {
         const uint64_t nk = ctx->ncorner[m];
         const uint64_t hs = next_pow2(2 * nk + 2);
@@ -1088,7 +1156,7 @@ void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
     if (ctx->batch)
         k_batch_edge_bases<<<grid_for(ctx->npairs), kBlock, 0, s3>>>(
             P_<BatchPair>(ctx->bpairs), ctx->npairs, P_<uint32_t>(ctx->off[0]), P_<uint32_t>(ctx->off[1]), ctx->nf[0],
-            ctx->nf[1], P_<uint32_t>(ctx->eid[0]), P_<uint32_t>(ctx->eid[1]), C);
+            ctx->nf[1], P_<uint32_t>(ctx->cedge[0]), P_<uint32_t>(ctx->cedge[1]), C);
     ev_record(ctx, EV_C_TOPO, s3);
 
 }
@@ -1305,6 +1373,11 @@ mcgpu_result finish(mcgpu_context ctx, mcgpu_frontend_info* info, bool* overflow
         *overflow = true;
         return MCGPU_SUCCESS;
     }
+    if (C.ov_topo) { // run again with the edges numbered through the hash tables
+        ctx->topo_hash = true;
+        *overflow = true;
+        return alloc_edge_tables(ctx);
+    }
     if (C.ov_pairs || C.ov_tests || C.ov_esc || C.ov_reg || C.ov_big || C.ov_trip) {
         *overflow = true;
         // a refusal leaves the context's capacities as they were
@@ -1415,7 +1488,7 @@ std::vector<Buf*> context_bufs(mcgpu_context ctx)
     return {&ctx->in_v[0], &ctx->in_v[1], &ctx->in_idx[0], &ctx->in_idx[1], &ctx->in_sz[0], &ctx->in_sz[1],
                   &ctx->off[0], &ctx->off[1], &ctx->state, &ctx->ps_v, &ctx->box, &ctx->hkeys[0],
                   &ctx->hkeys[1], &ctx->hfirst[0], &ctx->hfirst[1], &ctx->cface[0], &ctx->cface[1], &ctx->eflag[0],
-                  &ctx->eflag[1], &ctx->eid[0], &ctx->eid[1], &ctx->cedge[0], &ctx->cedge[1], &ctx->etotal, &ctx->ev0,
+                  &ctx->eflag[1], &ctx->eid[0], &ctx->eid[1], &ctx->cedge[0], &ctx->cedge[1], &ctx->etotal, &ctx->opp, &ctx->twords, &ctx->tsum, &ctx->tseg, &ctx->ev0,
                   &ctx->ev1, &ctx->ef0, &ctx->ef1, &ctx->mcode, &ctx->mface, &ctx->mcode2, &ctx->mface2, &ctx->nodes[0], &ctx->nodes[1],
                   &ctx->rawbox, &ctx->raw_pairs, &ctx->pairs, &ctx->phash, &ctx->cand, &ctx->cand_list,
                   &ctx->planes, &ctx->big_list, &ctx->big_off, &ctx->big_scratch, &ctx->te, &ctx->tg, &ctx->tqs, &ctx->trs,
@@ -1441,8 +1514,9 @@ std::vector<uint64_t> graph_key(mcgpu_context ctx)
     std::vector<uint64_t> k;
     auto put = [&k](uint64_t x) { k.push_back(x); };
     auto ptr = [&k](const void* p) { k.push_back((uint64_t)(uintptr_t)p); };
-    put(ctx->batch), put(ctx->npairs), put(ctx->batch_mb), put(ctx->batch_packed), put(ctx->cc_check), put(ctx->sort_bits),
-        put(ctx->shifted_bp),
+    put(ctx->batch), put(ctx->npairs), put(ctx->batch_mb), put(ctx->cc_check), put(ctx->sort_bits),
+        put(ctx->shifted_bp), put(ctx->topo_hash), put(ctx->topo_buckets), put(ctx->topo_tiles), put(ctx->topo_items),
+        put(ctx->nseg),
         put(ctx->gbits), put(ctx->kbits);
     for (int m = 0; m < 2; ++m) {
         put(ctx->nv[m]), put(ctx->nf[m]), put(ctx->ncorner[m]), put(ctx->depth[m]);
@@ -2003,27 +2077,29 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
         ctx->hstarts[3ull * np + p] = b.fc0;
         for (int j = 0; j < 6; ++j) len[6ull * p + j] = j < 3 ? b.nvs : b.nvc;
     }
-    // the packed edge numbering with one table region per pair, when every
-    // pair's vertex ids and corner ranks fit its word (corner counts are
-    // known on the host for triangle meshes and host face sizes)
-    ctx->batch_packed = true;
-    for (int m = 0; m < 2 && ctx->batch_packed; ++m) {
-        const bool tri = mesh[m]->face_sizes == nullptr;
-        if (!tri && desc->input_on_device) {
-            ctx->batch_packed = false;
-            break;
-        }
+    // the edge numbering's segments: both meshes of every pair (corner counts
+    // are known on the host for triangle meshes and host face sizes)
+    ctx->batch_corners = (!mesh[0]->face_sizes && !mesh[1]->face_sizes) || !desc->input_on_device;
+    ctx->hseg.clear();
+    for (int m = 0; m < 2 && ctx->batch_corners; ++m) {
+        uint64_t c0 = 0;
         for (uint32_t p = 0; p < np; ++p) {
             uint64_t k = 0;
-            if (tri) {
-                k = 3ull * (fo[m][p + 1] - fo[m][p]);
-            } else {
+            if (!mesh[m]->face_sizes) k = 3ull * (fo[m][p + 1] - fo[m][p]);
+            else
                 for (uint32_t f = fo[m][p]; f < fo[m][p + 1]; ++f) k += mesh[m]->face_sizes[f];
-            }
-            if (vo[m][p + 1] - vo[m][p] >= (1u << kPackedVertexBits) || k >= (1ull << kPackedRankBits)) {
-                ctx->batch_packed = false;
+            if (k > 0xffffffffull) {
+                ctx->batch_corners = false;
                 break;
             }
+            TopoSeg g{};
+            g.c0 = c0;
+            g.k = (uint32_t)k;
+            g.vb = vo[m][p];
+            g.vbits = (uint8_t)std::max(8, bits_for(vo[m][p + 1] - vo[m][p]));
+            g.m = (uint8_t)m;
+            ctx->hseg.push_back(g);
+            c0 += k;
         }
     }
     // serial-sum chains, longest first
@@ -2059,6 +2135,8 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
         CK(hipMemcpyAsync(ctx->bpairs.p, ctx->hpairs.data(), sizeof(BatchPair) * np, hipMemcpyHostToDevice, ctx->s));
         CK(hipMemcpyAsync(ctx->bstarts.p, ctx->hstarts.data(), 16ull * np, hipMemcpyHostToDevice, ctx->s));
         CK(hipMemcpyAsync(ctx->border.p, ctx->horder.data(), 24ull * np, hipMemcpyHostToDevice, ctx->s));
+        if (!ctx->topo_hash)
+            CK(hipMemcpyAsync(ctx->tseg.p, ctx->hseg.data(), sizeof(TopoSeg) * ctx->nseg, hipMemcpyHostToDevice, ctx->s));
     }
     if (ctx->cap_pairs < 4 * F) ctx->cap_pairs = std::max<uint64_t>(1 << 14, 4 * F);
     if (ctx->cap_tests < 2 * ctx->cap_pairs) ctx->cap_tests = 2 * ctx->cap_pairs;
@@ -2729,8 +2807,8 @@ uint64_t ctx_bytes(mcgpu_context c)
 {
     uint64_t t = 0;
     const Buf* all[] = {&c->in_v[1], &c->in_idx[1], &c->in_sz[1], &c->off[1], &c->state, &c->ps_v, &c->box,
-                        &c->hkeys[1], &c->hfirst[1], &c->cface[1], &c->eflag[0], &c->eid[0], &c->eflag[1],
-                        &c->eid[1], &c->cedge[1],
+                        &c->hkeys[1], &c->hfirst[1], &c->cface[1], &c->eflag[1], &c->eid[1], &c->cedge[1],
+                        &c->opp, &c->twords, &c->tsum,
                         &c->etotal, &c->ev0, &c->ev1, &c->ef0, &c->ef1, &c->mcode, &c->mface, &c->mcode2,
                         &c->mface2, &c->nodes[1], &c->rawbox, &c->raw_pairs, &c->pairs, &c->phash, &c->cand,
                         &c->cand_list, &c->planes, &c->big_list, &c->big_off, &c->big_scratch, &c->te, &c->tg, &c->esc,
@@ -2901,6 +2979,8 @@ MCGPU_API mcgpu_result mcgpu_server_create(int device, const mcgpu_mesh* src, co
     R.dsz = m->dsz[0];
     R.off = P_<uint32_t>(m->off[0]);
     R.cedge = P_<uint32_t>(m->cedge[0]);
+    R.opp = m->topo_hash ? nullptr : P_<uint32_t>(m->opp);
+    R.cface = m->dsz[0] ? P_<uint32_t>(m->cface[0]) : nullptr;
     R.ev0 = P_<uint32_t>(m->ev0);
     R.ev1 = P_<uint32_t>(m->ev1);
     R.ef0 = P_<int32_t>(m->ef0);
@@ -3326,6 +3406,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_narrow(mcgpu_context ctx, const mcgpu_mesh
     ctx->kbits = ctx->gbits + bits_for(std::max<uint64_t>(K, NE) + 1);
     if (ctx->kbits > 64) return MCGPU_ERROR_UNSUPPORTED;
     if ((r = alloc_mesh_buffers(ctx)) != MCGPU_SUCCESS) return r;
+    ctx->topo_given = topology != nullptr;
     if (topology) {
         uint32_t* u;
         int32_t* i32;
