@@ -6,6 +6,7 @@
 #pragma once
 #include "kernels.hpp"
 #include "sort.hpp"
+#include "sumseg.hpp"
 
 namespace mcgpu {
 
@@ -52,36 +53,43 @@ namespace mcgpu {
 
 constexpr int kSumRing = 16;
 
-// left-to-right sum of v[0], v[3], ..., v[3 (n - 1)] by one wavefront (the
-// whole wave returns it)
-__device__ __forceinline__ double serial_sum(const double* __restrict__ v, uint32_t n, const double* __restrict__ zero)
+// acc + v[0] + v[STRIDE] + ... + v[STRIDE (n - 1)], left to right, by one
+// wavefront (the whole wave returns it); rows (optional): the value after every
+// 16 of them
+template <int STRIDE, bool ROWS>
+__device__ __forceinline__ double serial_chain(const double* __restrict__ v, uint32_t n, const double* __restrict__ zero,
+                                               double acc, double* __restrict__ rows)
 {
     const uint32_t c = threadIdx.x & 15;
     const uint32_t nfull = n / 64;
     const uint32_t last = nfull ? nfull - 1 : 0;
-    double one = 1.0, acc = 0.0;
+    double one = 1.0;
     if (nfull > 0) {
         double X[kSumRing][4];
 #pragma unroll
         for (int r = 0; r < kSumRing; ++r) {
-            const double* vb = v + 192ull * ((uint32_t)r < last ? (uint32_t)r : last); // uniform block base
+            const double* vb = v + (uint64_t)(64 * STRIDE) * ((uint32_t)r < last ? (uint32_t)r : last); // uniform block base
 #pragma unroll
-            for (int q = 0; q < 4; ++q) X[r][q] = vb[3 * (16 * q + c)];
+            for (int q = 0; q < 4; ++q) X[r][q] = vb[STRIDE * (16 * q + c)];
         }
         for (uint32_t b0 = 0; b0 < nfull; b0 += kSumRing) {
 #pragma unroll
             for (int r = 0; r < kSumRing; ++r) {
                 if (b0 + r < nfull) {
-                    MCGPU_SUM_ROW(acc, X[r][0], one);
-                    MCGPU_SUM_ROW(acc, X[r][1], one);
-                    MCGPU_SUM_ROW(acc, X[r][2], one);
-                    MCGPU_SUM_ROW(acc, X[r][3], one);
+                    double y[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        MCGPU_SUM_ROW(acc, X[r][q], one);
+                        y[q] = acc;
+                    }
+                    if (ROWS) // one store a block: every lane of a quad one of its rows
+                        rows[4 * (b0 + r) + (c & 3)] = c & 2 ? (c & 1 ? y[3] : y[2]) : (c & 1 ? y[1] : y[0]);
                 }
                 // refill this ring slot kSumRing blocks ahead (clamped to the last block)
                 const uint32_t nb = b0 + kSumRing + r;
-                const double* vb = v + 192ull * (nb < last ? nb : last);
+                const double* vb = v + (uint64_t)(64 * STRIDE) * (nb < last ? nb : last);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) X[r][q] = vb[3 * (16 * q + c)];
+                for (int q = 0; q < 4; ++q) X[r][q] = vb[STRIDE * (16 * q + c)];
             }
         }
     }
@@ -90,351 +98,293 @@ __device__ __forceinline__ double serial_sum(const double* __restrict__ v, uint3
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const uint32_t i = nfull * 64 + 16 * q + c;
-            T[q] = *(i < n ? v + 3ull * i : zero);
+            T[q] = *(i < n ? v + (uint64_t)STRIDE * i : zero);
         }
-        MCGPU_SUM_ROW(acc, T[0], one);
-        MCGPU_SUM_ROW(acc, T[1], one);
-        MCGPU_SUM_ROW(acc, T[2], one);
-        MCGPU_SUM_ROW(acc, T[3], one);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            MCGPU_SUM_ROW(acc, T[q], one);
+            if (ROWS) rows[4 * nfull + q] = acc;
+        }
     }
     return acc;
 }
 
-__global__ void __launch_bounds__(64) k_mesh_sums(const double* __restrict__ v0, uint32_t n0,
-                                                  const double* __restrict__ v1, uint32_t n1,
-                                                  const double* __restrict__ zero, Params* P,
-                                                  const uint32_t* __restrict__ only_failed)
+__device__ __forceinline__ double serial_sum(const double* __restrict__ v, uint32_t n, const double* __restrict__ zero)
 {
-    __builtin_amdgcn_s_setprio(3);
-    const int m = blockIdx.x / 3, j = blockIdx.x % 3;
-    if (m == 0 && !v0) return; // a resident source: its sums are set already
-    if (only_failed && __builtin_amdgcn_readfirstlane(only_failed[blockIdx.x]) == 0u) return;
-    const double acc = serial_sum((m ? v1 : v0) + j, m ? n1 : n0, zero);
-    if (threadIdx.x == 0) P->sum[m][j] = acc;
+    return serial_chain<3, false>(v, n, zero, 0.0, nullptr);
 }
 
 // ---------------------------------------------------------------------------
-// The same sums from a chain about five times shorter.  A step s = RN(s' + x)
-// whose result stays in the binade of s' (|s| and |s'| in [2^e, 2^(e+1)), same
-// sign) rounds to the multiples of u = 2^(e-52), of which s' already is one:
-// s = s' + RN_u(x), whatever s' is, unless RN_u(x) is a tie.  A run of such
-// steps adds sum RN_u(x) to its start value exactly, one rounding-free add.
-// Binade changes and ties stay single steps of the chain.
+// The same sums from a short chain (sumseg.hpp says why it is exact).
+// k_sum_blocks adds every tile in any order, for the predictions.  k_sum_items
+// walks 64 values a thread (a chunk) into segments and single steps and writes
+// them with their adds, a tile's without gaps.  k_sum_chain, one block a chain
+// on the reserved CUs, runs the DPP chain over all adds, from LDS.
+// k_sum_verify checks every item on its real start, a thread a chunk, and
+// k_sum_rest takes the values one by one from the first chunk that found a
+// start its segment does not move with (as a rule there is none).
 //
-// k_sum_blocks and k_sum_items predict the binade of every partial sum from
-// an approximate prefix (any summation order) and write each 32-value thread
-// range as items: raw values, and for every same-binade run its exact sum
-// (integer multiples of u) with the interval [lo, hi] of start values for
-// which every partial sum of the run stays in [2^e + u, 2^(e+1)].  k_sum_chain adds the items left to right with the serial sum's DPP
-// chain and checkpoints every 64 items; k_sum_verify replays every 16 items
-// from the checkpoint before them and checks each run's actual start value
-// against its interval.  A start inside it proves the run exact (the prediction only
-// chooses the runs); a failure sends that coordinate to the serial sum
-// (k_mesh_sums with the failure flags).  On the icosphere-7 pair the longest
-// chain holds 35k items for 164k vertices.
-constexpr int kSumThreads = 128, kSumPer = 32;
-constexpr uint32_t kSumTile = kSumThreads * kSumPer; // values per block and per item region
+// What bounds it: the walk (64 dependent steps of about 75 instructions on one
+// wave a SIMD) and the chain (2.44 ns an add); beside the tree build and the
+// edge numbering a dependent load takes microseconds, so the chain's block
+// makes few and the checks are spread over the device.  On two subdivision-7
+// icospheres 164k values leave 7k items and 17k adds.  Composing the items of
+// eight chunks in turn left 5k adds and cost what it saved (0.35 us a step, 1.4
+// us where lanes diverge).  The stage takes 0.16 ms there (0.21 ms with one item
+// a same-binade run), 0.36 ms instead of 1.2 ms on 655k values, and 0.3 ms on a
+// 1 M vertex terrain of whole coordinates, whose sums meet powers of two and
+// were added serially in 6.4 ms beside the other streams.  Chains of up to kSumSerial values are added
+// serially at once: the walks cost that much in launches.
+constexpr int kSumThreads = 64, kSumPer = 64;
+constexpr uint32_t kSumTile = kSumThreads * kSumPer; // values per block
 constexpr int kSumLds = kSumPer + 1;                 // LDS stride of a thread's values (no bank conflicts)
+constexpr int kSumKeep = 16;                         // adds of a thread kept in LDS
+constexpr int kSumChain = 256;
+constexpr uint32_t kSumLdsAdds = 16384;              // adds of a chain in LDS at a time
+constexpr uint32_t kSumSerial = 4096;
 
 struct SumBufs {
     const double* v[2]; // vertex arrays (xyz), null when that mesh's sums are preset
     uint32_t n[2];      // vertex counts
-    uint32_t nblk;      // blocks per chain (of the larger mesh)
+    uint32_t nblk;      // tiles per chain (of the larger mesh)
     double* bsum;       // [6][nblk]
-    double* items;      // [6][nblk * kSumTile]
-    double* lo;
-    double* hi;
-    uint32_t* nitem;    // [6][nblk]: items of each block region, padded to 64
-    uint32_t* list;     // [6][lcap]: 64-item blocks in chain order
-    uint32_t lcap;
-    double* ckpt;       // [6][lcap]: chain value after each 64 items
-    uint32_t* fail;     // [6]
-    uint32_t* nb64;     // [6]: 64-item blocks of each chain
+    SumItem* items;     // [6][nblk * kSumTile]: kSumPer places a chunk
+    uint32_t* chunk;    // [6][nblk * kSumThreads]: items << 16 | first add in the tile
+    uint32_t* nadd;     // [6][nblk]: adds of each tile (padded to 16), then its first add in the chain
+    double* adds;       // [6][kSumMaxAdds * nblk * kSumTile]: the tiles' adds
+    double* past;       // the same places, for the adds LDS has none for
+    double* rows;       // [6][kSumMaxAdds * nblk * kSumTile / 16]: the chain after every 16 adds
+    uint32_t* fail;     // [6]: first chunk whose start its segment does not move with
 };
 
 __device__ __forceinline__ bool sum_chain_active(const SumBufs& B, int ch) { return B.v[ch / 3] != nullptr && B.n[ch / 3] > 0; }
-
-__global__ void __launch_bounds__(kSumThreads) k_sum_blocks(SumBufs B)
+// whether a chain goes through items
+__device__ __forceinline__ bool sum_chain_items(const SumBufs& B, int ch)
 {
-    __shared__ double red[kSumThreads / 64];
+    return sum_chain_active(B, ch) && B.n[ch / 3] > kSumSerial;
+}
+
+__global__ void __launch_bounds__(256) k_sum_blocks(SumBufs B)
+{
+    __shared__ double red[4];
     const int ch = blockIdx.y, m = ch / 3, j = ch % 3;
-    if (blockIdx.x == 0 && threadIdx.x == 0) B.fail[ch] = 0u;
-    if (!sum_chain_active(B, ch)) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) B.fail[ch] = 0xffffffffu;
+    if (!sum_chain_items(B, ch)) return;
     const uint32_t n = B.n[m], b = blockIdx.x;
     if ((uint64_t)b * kSumTile >= n) return;
     const double* v = B.v[m] + j;
     const uint64_t i0 = (uint64_t)b * kSumTile;
-    double t = 0.0;
-#pragma unroll 8
-    for (uint32_t k = threadIdx.x; k < kSumTile; k += kSumThreads)
-        if (i0 + k < n) t += v[3 * (i0 + k)];
+    double t = 0.0, X[kSumTile / 256];
+#pragma unroll
+    for (uint32_t q = 0; q < kSumTile / 256; ++q) {
+        const uint64_t i = i0 + q * 256 + threadIdx.x;
+        X[q] = v[3 * (i < n ? i : i0)];
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < kSumTile / 256; ++q) t += i0 + q * 256 + threadIdx.x < n ? X[q] : 0.0;
     for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double a = 0.0;
-        for (int w = 0; w < kSumThreads / 64; ++w) a += red[w];
-        B.bsum[(uint64_t)ch * B.nblk + b] = a;
-    }
-}
-
-// (sign, exponent) of a predicted partial sum; kSumTiny for zero, |a| < 2^-900
-// or |a| >= 2^1001 (keeps 2^(e+3) and 2^(52-e) finite)
-constexpr int kSumTiny = 1 << 20;
-__device__ __forceinline__ int sum_binade(double a)
-{
-    const uint64_t bits = (uint64_t)__double_as_longlong(a);
-    const int ex = (int)((bits >> 52) & 0x7ff);
-    if (ex < 1023 - 900 || ex > 1023 + 1000) return kSumTiny;
-    return (ex << 1) | (int)(bits >> 63);
-}
-
-struct SumRun {
-    long long q, qmin, qmax; // running sum of RN_u(x) / u and its extremes (0 included)
-    int key;                 // binade; kSumTiny when no run is open
-    bool bad;
-};
-
-// one thread's items for its values x[0..cnt) (LDS), starting from the
-// approximate prefix a: emission through emit(item, lo, hi)
-template <class Emit>
-__device__ __forceinline__ void sum_items_walk(const double* x, uint32_t cnt, double a, Emit emit)
-{
-    SumRun R{0, 0, 0, kSumTiny, false};
-    int prev = sum_binade(a);
-    const double inf = __longlong_as_double(0x7ff0000000000000ll);
-    auto close = [&]() {
-        if (R.key == kSumTiny) return;
-        const int e = (R.key >> 1) - 1023;
-        const double u = __longlong_as_double((long long)(e - 52 + 1023) << 52);
-        // in units of u: every partial sum v + Q within [2^e + u, 2^(e+1)]
-        // (mirrored for a negative binade).  The exact step value is within u/2
-        // of v + Q, and there the nearest double is v + Q: inside the binade the
-        // doubles are the multiples of u, and just above 2^(e+1) they are 2u
-        // apart.  Exact in integers, rounded inward to doubles.
-        const long long L = (R.key & 1) ? -(1ll << 53) : (1ll << 52) + 1;
-        const long long H = (R.key & 1) ? -((1ll << 52) + 1) : (1ll << 53);
-        const long long lo_u = L - R.qmin, hi_u = H - R.qmax;
-        double lod = (double)lo_u, hid = (double)hi_u;
-        if ((long long)lod < lo_u) lod = nextafter(lod, 1.0e300);
-        if ((long long)hid > hi_u) hid = nextafter(hid, -1.0e300);
-        double lo = lod * u, hi = hid * u;
-        if (R.bad) { // empty: the verification fails
-            lo = inf;
-            hi = -inf;
-        }
-        emit((double)R.q * u, lo, hi);
-        R.key = kSumTiny;
-    };
-    for (uint32_t i = 0; i < cnt; ++i) {
-        const double xi = x[i];
-        a = a + xi;
-        const int key = sum_binade(a);
-        bool stateless = key == prev && key != kSumTiny;
-        double c = 0.0;
-        if (stateless) {
-            const int e = (key >> 1) - 1023;
-            const double inv_u = __longlong_as_double((long long)(52 - e + 1023) << 52);
-            const double ax = xi < 0 ? -xi : xi;
-            if (!(ax < __longlong_as_double((long long)(e + 3 + 1023) << 52))) {
-                stateless = false;
-            } else {
-                const double q = xi * inv_u;
-                c = rint(q);
-                if (q - floor(q) == 0.5) stateless = false; // a tie: the parity of s' decides
-            }
-        }
-        if (stateless) {
-            if (R.key != key) {
-                close();
-                R = SumRun{0, 0, 0, key, false};
-            }
-            R.q += (long long)c;
-            R.qmin = R.q < R.qmin ? R.q : R.qmin;
-            R.qmax = R.q > R.qmax ? R.q : R.qmax;
-            if (R.q > (1ll << 53) || R.q < -(1ll << 53)) R.bad = true;
-        } else {
-            close();
-            emit(xi, -inf, inf);
-        }
-        prev = key;
-    }
-    close();
+    if (threadIdx.x == 0) B.bsum[(uint64_t)ch * B.nblk + b] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 __global__ void __launch_bounds__(kSumThreads) k_sum_items(SumBufs B)
 {
     __shared__ double xs[kSumThreads * kSumLds];
-    __shared__ double wpre[kSumThreads / 64];
-    __shared__ uint32_t wcnt[kSumThreads / 64];
-    __shared__ double a0s;
+    __shared__ double kept[kSumKeep][kSumThreads];
     const int ch = blockIdx.y, m = ch / 3, j = ch % 3;
-    if (!sum_chain_active(B, ch)) return;
+    if (!sum_chain_items(B, ch)) return;
     const uint32_t n = B.n[m], b = blockIdx.x;
-    if ((uint64_t)b * kSumTile >= n) {
-        if (threadIdx.x == 0) B.nitem[(uint64_t)ch * B.nblk + b] = 0u;
-        return;
-    }
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if ((uint64_t)b * kSumTile >= n) return;
+    const uint32_t t = threadIdx.x;
     const double* v = B.v[m] + j;
     const uint64_t i0 = (uint64_t)b * kSumTile;
     const uint32_t nb = (n - i0) < kSumTile ? (uint32_t)(n - i0) : kSumTile;
     // the block's values into LDS (coalesced), value k of thread t at t * kSumLds + k
-#pragma unroll 8
-    for (uint32_t k = threadIdx.x; k < kSumTile; k += kSumThreads)
-        xs[(k / kSumPer) * kSumLds + k % kSumPer] = k < nb ? v[3 * (i0 + k)] : 0.0;
-    if (threadIdx.x == 0) {
-        double a = 0.0;
-        for (uint32_t q = 0; q < b; ++q) a += B.bsum[(uint64_t)ch * B.nblk + q];
-        a0s = a;
+    for (int q0 = 0; q0 < kSumPer; q0 += 16) {
+        double X[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) { // a clamped index, not a branch: sixteen loads in flight
+            const uint32_t k = (q0 + q) * kSumThreads + t;
+            X[q] = v[3 * (i0 + (k < nb ? k : nb - 1))];
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const uint32_t k = (q0 + q) * kSumThreads + t;
+            xs[(k / kSumPer) * kSumLds + k % kSumPer] = k < nb ? X[q] : 0.0;
+        }
     }
+    double a0 = 0.0; // the tiles before this one
+    for (uint32_t q = t; q < b; q += kSumThreads) a0 += B.bsum[(uint64_t)ch * B.nblk + q];
+    for (int o = 32; o > 0; o >>= 1) a0 += __shfl_xor(a0, o, 64);
     __syncthreads();
-    const double* x = xs + threadIdx.x * kSumLds;
-    const uint32_t t0 = threadIdx.x * kSumPer;
-    const uint32_t cnt = t0 < nb ? (nb - t0 < (uint32_t)kSumPer ? nb - t0 : (uint32_t)kSumPer) : 0u;
-    double t = 0.0;
-    for (uint32_t k = 0; k < cnt; ++k) t += x[k];
-    // approximate prefix at this thread's first value
-    double y = t;
+    const double* x = xs + t * kSumLds;
+    double own = 0.0;
+#pragma unroll 8
+    for (int k = 0; k < kSumPer; ++k) own += x[k];
+    double y = own; // predicted sum before this thread's values
     for (int o = 1; o < 64; o <<= 1) {
         const double z = __shfl_up(y, o, 64);
-        if (lane >= o) y += z;
+        if (t >= (uint32_t)o) y += z;
     }
-    if (lane == 63) wpre[wid] = y;
-    __syncthreads();
-    double a = a0s + (y - t);
-    for (int w = 0; w < wid; ++w) a += wpre[w];
-    uint32_t nit = 0;
-    if (cnt) sum_items_walk(x, cnt, a, [&](double, double, double) { ++nit; });
-    // this thread's offset in the block region
-    uint32_t r = nit;
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t z = __shfl_up(r, o, 64);
-        if (lane >= o) r += z;
-    }
-    if (lane == 63) wcnt[wid] = r;
-    __syncthreads();
-    uint32_t off = r - nit, tot = 0;
-    for (int w = 0; w < kSumThreads / 64; ++w) {
-        if (w < wid) off += wcnt[w];
-        tot += wcnt[w];
-    }
-    const uint64_t base = ((uint64_t)ch * B.nblk + b) * kSumTile;
-    double* it = B.items + base;
-    double* lo = B.lo + base;
-    double* hi = B.hi + base;
-    if (cnt) {
-        uint32_t k = off;
-        sum_items_walk(x, cnt, a, [&](double val, double l, double h) {
-            it[k] = val;
-            lo[k] = l;
-            hi[k] = h;
-            ++k;
-        });
-    }
-    // +0.0 to the next multiple of 64 (adding +0.0 changes no partial sum)
-    const uint32_t padded = (tot + 63u) & ~63u;
-    const double inf = __longlong_as_double(0x7ff0000000000000ll);
-    for (uint32_t k = tot + threadIdx.x; k < padded; k += kSumThreads) {
-        it[k] = 0.0;
-        lo[k] = -inf;
-        hi[k] = inf;
-    }
-    if (threadIdx.x == 0) B.nitem[(uint64_t)ch * B.nblk + b] = padded;
-}
-
-// one wave per chain (on the reserved CUs): the DPP chain over the item
-// regions in order, a checkpoint after every 16 items.  A scalar cursor
-// (region, 64-item block) walks the regions ahead of the chain, so every
-// refill address is a uniform base with no dependent load; the block list is
-// written for the verification.
-__global__ void __launch_bounds__(64) k_sum_chain(SumBufs B, Params* P)
-{
-    extern __shared__ uint32_t cnt64[]; // 64-item blocks of each region
-    __builtin_amdgcn_s_setprio(3);
-    const int ch = blockIdx.x, m = ch / 3, j = ch % 3;
-    if (!sum_chain_active(B, ch)) return;
-    const uint32_t lane = threadIdx.x, c = lane & 15;
-    const uint32_t* nit = B.nitem + (uint64_t)ch * B.nblk;
-    uint32_t* list = B.list + (uint64_t)ch * B.lcap;
-    uint32_t nb = 0;
-    for (uint32_t b = 0; b < B.nblk; ++b) {
-        const uint32_t k = nit[b] / 64u;
-        if (lane == 0) cnt64[b] = k;
-        for (uint32_t q = lane; q < k; q += 64) list[nb + q] = b * (kSumTile / 64) + q;
-        nb += k;
-    }
-    __syncthreads();
-    nb = __builtin_amdgcn_readfirstlane(nb);
-    if (lane == 0) B.nb64[ch] = nb;
-    const double* items = B.items + (uint64_t)ch * B.nblk * kSumTile;
-    double* ckpt = B.ckpt + (uint64_t)ch * B.lcap;
-    // load cursor: region rb (cur 64-item blocks), block jb within it; it
-    // reads a region's count only when it enters the region and stays on the
-    // last block at the end
-    uint32_t rb = 0, jb = 0, last_blk = 0, cur = __builtin_amdgcn_readfirstlane(cnt64[0]);
-    auto next_blk = [&]() -> uint32_t {
-        while (jb >= cur && rb < B.nblk) {
-            ++rb;
-            jb = 0;
-            cur = rb < B.nblk ? __builtin_amdgcn_readfirstlane(cnt64[rb]) : 0u;
-        }
-        if (rb < B.nblk) last_blk = rb * (kSumTile / 64) + jb++;
-        return last_blk;
-    };
-    double one = 1.0, acc = 0.0;
-    if (nb > 0) {
-        double X[kSumRing][4];
+    y = __shfl_up(y, 1, 64);
+    const uint32_t k0 = t * kSumPer, cnt = k0 < nb ? (nb - k0 < (uint32_t)kSumPer ? nb - k0 : (uint32_t)kSumPer) : 0u;
+    const uint64_t tile = ((uint64_t)ch * B.nblk + b) * kSumTile;
+    SumItem* out = B.items + tile + k0; // every item covers a value
+    double* tadds = B.adds + kSumMaxAdds * tile;
+    double* past = B.past + kSumMaxAdds * (tile + k0); // the adds LDS has no place for, until they are copied below
+    uint32_t k = 0, na = 0;
+    {
+        auto emit = [&](const SumItem& it) {
+            double a[kSumMaxAdds];
+            const int c = sum_add_list(it, a);
+            out[k++] = it;
 #pragma unroll
-        for (int r = 0; r < kSumRing; ++r) {
-            const double* vb = items + 64ull * next_blk();
-#pragma unroll
-            for (int q = 0; q < 4; ++q) X[r][q] = vb[16 * q + c];
-        }
-        for (uint32_t b0 = 0; b0 < nb; b0 += kSumRing) {
-#pragma unroll
-            for (int r = 0; r < kSumRing; ++r) {
-                if (b0 + r < nb) {
-                    MCGPU_SUM_ROW(acc, X[r][0], one);
-                    MCGPU_SUM_ROW(acc, X[r][1], one);
-                    MCGPU_SUM_ROW(acc, X[r][2], one);
-                    MCGPU_SUM_ROW(acc, X[r][3], one);
-                    if (lane == 0) ckpt[b0 + r] = acc;
+            for (int q = 0; q < kSumMaxAdds; ++q)
+                if (q < c) {
+                    if (na + q < (uint32_t)kSumKeep) kept[na + q][t] = a[q];
+                    else past[na + q] = a[q];
                 }
-                const double* vb = items + 64ull * next_blk();
-#pragma unroll
-                for (int q = 0; q < 4; ++q) X[r][q] = vb[16 * q + c];
-            }
-        }
+            na += c;
+        };
+        SumWalk W;
+        sum_restart(W, t ? a0 + y : a0);
+        for (uint32_t i = 0; i < cnt; ++i) sum_step(W, x[i], emit);
+        sum_close(W, emit);
     }
-    if (lane == 0) P->sum[m][j] = acc;
+    uint32_t off = na; // exclusive scan over the tile
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t z = __shfl_up(off, o, 64);
+        if (t >= (uint32_t)o) off += z;
+    }
+    const uint32_t tot = __shfl(off, 63, 64), padded = (tot + 15u) & ~15u; // rows do not straddle tiles
+    if (t == 0) B.nadd[(uint64_t)ch * B.nblk + b] = padded;
+    if (t < padded - tot) tadds[tot + t] = 0.0; // adding +0.0 changes no partial sum
+    off -= na;
+    B.chunk[((uint64_t)ch * B.nblk + b) * kSumThreads + t] = k << 16 | off; // at most 64 items, 320 * 64 adds
+    for (uint32_t q = 0; q < na && q < (uint32_t)kSumKeep; ++q) tadds[off + q] = kept[q][t];
+    for (uint32_t q = kSumKeep; q < na; ++q) tadds[off + q] = past[q]; // the lane's own stores
 }
 
-// one thread per 16 items: replay from the checkpoint before their 64-item
-// block (at most 48 unchecked adds), then check each run's start value in
-// the 16 against its interval, and the block's last row against the next
-// checkpoint
-__global__ void __launch_bounds__(256) k_sum_verify(SumBufs B)
+__global__ void __launch_bounds__(kSumChain) k_sum_chain(SumBufs B, const double* __restrict__ zero, Params* P)
+{
+    constexpr int kWaves = kSumChain / 64;
+    __shared__ double ladds[kSumLdsAdds], lrows[kSumLdsAdds / 16];
+    __shared__ uint32_t wsum[kWaves];
+    const int ch = blockIdx.x, m = ch / 3, j = ch % 3;
+    if (!sum_chain_active(B, ch)) return; // a resident source: its sums are set already
+    const uint32_t n = B.n[m], t = threadIdx.x, lane = t & 63, wid = t >> 6;
+    if (!sum_chain_items(B, ch)) {
+        if (wid == 0) {
+            __builtin_amdgcn_s_setprio(3);
+            const double acc = serial_sum(B.v[m] + j, n, zero);
+            if (lane == 0) P->sum[m][j] = acc;
+        }
+        return;
+    }
+    const uint32_t tiles = (n + kSumTile - 1) / kSumTile;
+    uint32_t* nadd = B.nadd + (uint64_t)ch * B.nblk;
+    const uint64_t base = kSumMaxAdds * (uint64_t)ch * B.nblk * kSumTile;
+    double* rows = B.rows + base / 16;
+    // the tiles' first adds: thread t takes `per` consecutive tiles
+    const uint32_t per = (tiles + kSumChain - 1) / kSumChain;
+    const uint32_t b0 = t * per < tiles ? t * per : tiles, b1 = b0 + per < tiles ? b0 + per : tiles;
+    uint32_t na = 0;
+    for (uint32_t b = b0; b < b1; ++b) na += nadd[b];
+    uint32_t x = na;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= (uint32_t)o) x += y;
+    }
+    if (lane == 63) wsum[wid] = x;
+    __syncthreads();
+    uint32_t run = x - na, tot = 0;
+    for (uint32_t q = 0; q < kWaves; ++q) {
+        if (q < wid) run += wsum[q];
+        tot += wsum[q];
+    }
+    for (uint32_t b = b0; b < b1; ++b) {
+        const uint32_t c = nadd[b];
+        nadd[b] = run;
+        run += c;
+    }
+    __syncthreads();
+    double acc = 0.0;
+    for (uint32_t r0 = 0; r0 < tot; r0 += kSumLdsAdds) {
+        const uint32_t r1 = tot - r0 < kSumLdsAdds ? tot : r0 + kSumLdsAdds;
+        for (uint32_t b = wid; b < tiles; b += kWaves) { // the tiles' adds in [r0, r1), a wave a tile
+            const uint32_t o = nadd[b], e = b + 1 < tiles ? nadd[b + 1] : tot;
+            if (e <= r0 || o >= r1) continue;
+            const double* src = B.adds + base + (uint64_t)kSumMaxAdds * b * kSumTile;
+            const uint32_t q0 = o < r0 ? r0 : o, q1 = e < r1 ? e : r1;
+#pragma unroll 4
+            for (uint32_t q = q0 + lane; q < q1; q += 64) ladds[q - r0] = src[q - o];
+        }
+        __syncthreads();
+        if (wid == 0) {
+            __builtin_amdgcn_s_setprio(3);
+            acc = serial_chain<1, true>(ladds, r1 - r0, zero, acc, lrows);
+            __builtin_amdgcn_s_setprio(0);
+        }
+        __syncthreads();
+        for (uint32_t q = t; q < (r1 - r0) / 16; q += kSumChain) rows[r0 / 16 + q] = lrows[q];
+    }
+    if (t == 0) P->sum[m][j] = acc;
+}
+
+// the chain's value before chunk c: the row before its first add, and the adds since
+__device__ __forceinline__ double sum_chunk_start(const SumBufs& B, int ch, uint32_t c)
+{
+    const uint32_t b = c / kSumThreads, off = B.chunk[(uint64_t)ch * B.nblk * kSumThreads + c] & 0xffffu, o16 = off & ~15u;
+    const uint64_t base = kSumMaxAdds * (uint64_t)ch * B.nblk * kSumTile;
+    const uint32_t row = (B.nadd[(uint64_t)ch * B.nblk + b] + o16) / 16;
+    const double* adds = B.adds + base + (uint64_t)kSumMaxAdds * b * kSumTile + o16; // a row's worth is there
+    double X[15];
+#pragma unroll
+    for (uint32_t q = 0; q < 15; ++q) X[q] = adds[q];
+    double s = row ? B.rows[base / 16 + row - 1] : 0.0;
+#pragma unroll
+    for (uint32_t q = 0; q < 15; ++q) s = o16 + q < off ? s + X[q] : s;
+    return s;
+}
+
+__global__ void __launch_bounds__(kSumThreads) k_sum_verify(SumBufs B)
 {
     const int ch = blockIdx.y;
-    if (!sum_chain_active(B, ch)) return;
-    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= 4 * B.nb64[ch]) return;
-    const uint32_t k = r / 4, row = r % 4;
-    const uint64_t cb = (uint64_t)ch * B.lcap;
-    const uint64_t base = (uint64_t)ch * B.nblk * kSumTile + 64ull * B.list[cb + k];
-    double v = k ? B.ckpt[cb + k - 1] : 0.0;
-    for (uint32_t i = 0; i < 16 * row; ++i) v = v + B.items[base + i];
+    if (!sum_chain_items(B, ch)) return;
+    const uint32_t c = blockIdx.x * kSumThreads + threadIdx.x;
+    if ((uint64_t)c * kSumPer >= B.n[ch / 3]) return;
+    const uint64_t chunk = (uint64_t)ch * B.nblk * kSumThreads + c;
+    const SumItem* it = B.items + chunk * kSumPer;
+    const uint32_t k = B.chunk[chunk] >> 16;
+    double s = sum_chunk_start(B, ch, c);
     bool ok = true;
+    for (uint32_t q0 = 0; q0 < k; q0 += 4) {
+        SumItem I[4];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const uint64_t at = base + 16 * row + i;
-        const double l = B.lo[at], h = B.hi[at], x = B.items[at];
-        ok &= (l <= v) & (v <= h);
-        v = v + x;
+        for (uint32_t q = 0; q < 4; ++q) I[q] = it[q0 + q < k ? q0 + q : k - 1];
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            if (q0 + q >= k) break;
+            double end = s + I[q].p, d;
+            bool odd;
+            if (!sum_is_step(I[q])) ok &= sum_apply(I[q], s, &end, &d, &odd);
+            s = end;
+        }
     }
-    if (row == 3) ok &= __double_as_longlong(v) == __double_as_longlong(B.ckpt[cb + k]);
-    if (!ok) B.fail[ch] = 1u;
+    if (!ok) atomicMin(&B.fail[ch], c);
+}
+
+__global__ void __launch_bounds__(64) k_sum_rest(SumBufs B, const double* __restrict__ zero, Params* P)
+{
+    const int ch = blockIdx.x, m = ch / 3, j = ch % 3;
+    const uint32_t c = __builtin_amdgcn_readfirstlane(B.fail[ch]);
+    if (c == 0xffffffffu) return;
+    __builtin_amdgcn_s_setprio(3);
+    const uint32_t i0 = c * kSumPer;
+    const double start = sum_chunk_start(B, ch, c);
+    const double acc = serial_chain<3, false>(B.v[m] + j + 3ull * i0, B.n[m] - i0, zero, start, nullptr);
+    if (threadIdx.x == 0) P->sum[m][j] = acc;
 }
 
 // Batches: the 6 chains of every pair (pair p, mesh m, coordinate j is chain

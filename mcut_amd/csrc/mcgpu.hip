@@ -29,9 +29,9 @@ struct Buf {
     size_t cap = 0;
 };
 
-// Stages of one dispatch.  The serial coordinate sums run alone on a stream
-// whose CU mask reserves kSumCUs compute units for them; stream A carries the
-// chain that depends on the shift; stream B builds both trees and runs the
+// Stages of one dispatch.  The serial part of the coordinate sums runs alone on
+// a stream whose CU mask reserves kSumCUs compute units for it; stream A makes
+// and checks its items and carries what depends on the shift; stream B builds both trees and runs the
 // broad phase in raw coordinates alongside the sums; stream C numbers the
 // polygon-soup edges.  B and C are masked off the reserved CUs: a serial FP64
 // chain that shares its CU with memory- or atomic-heavy waves runs 4-8 times
@@ -51,7 +51,7 @@ constexpr double kBroadShare = 0.70;
 constexpr double kBatchBroadShare = 0.46;
 constexpr uint32_t kBatchSumWaves = 128; // persistent waves of the batched serial sums (on the reserved CUs)
 enum Stage {
-    ST_SUMS,      // A: serial coordinate sums and raw boxes (k_mesh_sums alone)
+    ST_SUMS,      // A: coordinate sums
     ST_PARAMS,    // A: shift parameters
     ST_SHIFT,     // A: shifted vertices, shifted face boxes
     ST_TOPOLOGY,  // C: polygon-soup edge numbering
@@ -74,8 +74,8 @@ const char* kStageNames[ST_COUNT] = {"coordinate_sums", "shift_params", "shift_b
 
 // event slots: stage boundaries on the three streams
 enum Ev { EV_A0, EV_S0, EV_A_SUMS, EV_A_PARAMS, EV_A_SHIFT, EV_A_BOXES, EV_A_JOIN, EV_A_FILTER, EV_A_PLANES, EV_A_JOIN2, EV_A_TESTS, EV_A_NARROW,
-          EV_A_END, EV_FORK, EV_B0, EV_B_SORT, EV_B_REFIT, EV_B_TRAV, EV_C0, EV_C_FILL, EV_C_TOPO, EV_SUM_ITEMS,
-          EV_SUM_CHAIN, EV_TRAV_K0, EV_TRAV_K1, EV_B_CC, EV_COUNT };
+          EV_A_END, EV_FORK, EV_B0, EV_B_SORT, EV_B_REFIT, EV_B_TRAV, EV_C0, EV_C_FILL, EV_C_TOPO, EV_SUM_ITEMS, EV_SUM_CHAIN,
+          EV_TRAV_K0, EV_TRAV_K1, EV_B_CC, EV_COUNT };
 
 // Launch shape of the traversal kernel, chosen per workload class by the
 // autotuner (mcgpu_autotune) or set by the caller (mcgpu_set_tuning).
@@ -180,8 +180,9 @@ struct mcgpu_context_t {
     Buf shkeys, shcnt;
     Buf pqs, prs, pcounts; // predicate stage: per-test signs, stage counts
     Buf scan_tmp, scan_tmp_c, hist;
-    Buf sbsum, sitems, slo, shi, snitem, slist, sckpt, sflags; // coordinate sums from run items
+    Buf sbsum, sitems, snitem, sadds, srows; // coordinate sums from segments
     uint32_t sum_nblk = 0;
+    bool sum_items = false;          // a mesh's chains are long enough to go through segments
 
     uint64_t cap_pairs = 0, cap_tests = 0, cap_esc = 0, cap_reg = 0, cap_big = 0, cap_trip = 0;
 
@@ -529,19 +530,20 @@ mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
     CK(ensure(ctx->planes, F, &pl));
     (void)p;
     CK(ensure(ctx->scan_tmp, scan_need + 1024, &u));
-    if (!ctx->batch) { // coordinate sums from run items (k_sum_blocks .. k_sum_verify), for the chains computed here
+    if (!ctx->batch) { // coordinate sums from segments (k_sum_blocks .. k_sum_rest), for the chains computed here
         const uint64_t nmax = std::max<uint64_t>(ctx->res ? 0 : ctx->nv[0], ctx->nv[1]);
         const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, (nmax + kSumTile - 1) / kSumTile);
-        const uint64_t region = 6ull * nblk * kSumTile, lcap = (uint64_t)nblk * (kSumTile / 64);
         ctx->sum_nblk = nblk;
-        CK(ensure(ctx->sbsum, 6ull * nblk, &dp));
-        CK(ensure(ctx->sitems, region, &dp));
-        CK(ensure(ctx->slo, region, &dp));
-        CK(ensure(ctx->shi, region, &dp));
-        CK(ensure(ctx->snitem, 6ull * nblk, &u));
-        CK(ensure(ctx->slist, 6 * lcap, &u));
-        CK(ensure(ctx->sckpt, 6 * lcap, &dp));
-        CK(ensure(ctx->sflags, 16, &u));
+        ctx->sum_items = nmax > kSumSerial;
+        if (ctx->sum_items) {
+            const uint64_t region = 6ull * nblk * kSumTile;
+            SumItem* si;
+            CK(ensure(ctx->sbsum, 6ull * nblk, &dp));
+            CK(ensure(ctx->sitems, region, &si));
+            CK(ensure(ctx->snitem, region / kSumPer + 6ull * nblk + 8, &u));
+            CK(ensure(ctx->sadds, 2 * kSumMaxAdds * region, &dp));
+            CK(ensure(ctx->srows, kSumMaxAdds * region / 16, &dp));
+        }
     }
     if (ctx->cc_check) CK(ensure(ctx->cc_parent, (uint64_t)ctx->nv[0] + ctx->nv[1] + 8, &u));
     if (ctx->topo_hash) {
@@ -615,15 +617,14 @@ SumBufs sum_bufs(mcgpu_context ctx)
     B.n[1] = ctx->nv[1];
     B.nblk = ctx->sum_nblk;
     B.bsum = P_<double>(ctx->sbsum);
-    B.items = P_<double>(ctx->sitems);
-    B.lo = P_<double>(ctx->slo);
-    B.hi = P_<double>(ctx->shi);
-    B.nitem = P_<uint32_t>(ctx->snitem);
-    B.list = P_<uint32_t>(ctx->slist);
-    B.lcap = ctx->sum_nblk * (kSumTile / 64);
-    B.ckpt = P_<double>(ctx->sckpt);
-    B.fail = P_<uint32_t>(ctx->sflags);
-    B.nb64 = P_<uint32_t>(ctx->sflags) + 8;
+    B.items = P_<SumItem>(ctx->sitems);
+    const uint64_t region = 6ull * ctx->sum_nblk * kSumTile;
+    B.chunk = P_<uint32_t>(ctx->snitem);
+    B.nadd = B.chunk + region / kSumPer;
+    B.fail = B.nadd + 6ull * ctx->sum_nblk;
+    B.adds = P_<double>(ctx->sadds);
+    B.past = B.adds + kSumMaxAdds * region;
+    B.rows = P_<double>(ctx->srows);
     return B;
 }
 
@@ -1203,8 +1204,8 @@ void enqueue_frontend(mcgpu_context ctx)
         k_batch_sums<<<std::min<uint32_t>(nch, kBatchSumWaves), 64, 0, ctx->ssum>>>(
             ctx->dv[0], ctx->dv[1], P_<BatchPair>(ctx->bpairs), P_<uint32_t>(ctx->border), nch, C, Pb);
     } else {
-        // run items on stream A (every CU), the chain and its check on the
-        // reserved CUs, the serial sum only for a coordinate that failed
+        // items and their check on stream A (every CU), the chain on the
+        // reserved CUs, the values one by one only where a check failed
         if (early_clear) { // the pair hash, before the sum kernels (its fill would slow the sum chain beside it)
             const uint64_t table = next_pow2(2 * ctx->cap_pairs);
             k_pair_hash_clear<<<grid_for(table, kBlock, 2048), kBlock, 0, s>>>(P_<unsigned long long>(ctx->phash), table);
@@ -1212,17 +1213,19 @@ void enqueue_frontend(mcgpu_context ctx)
         stage_event(ctx, EV_S0, s);
         const SumBufs SB = sum_bufs(ctx);
         const dim3 grid(SB.nblk, 6);
-        k_sum_blocks<<<grid, kSumThreads, 0, s>>>(SB);
-        k_sum_items<<<grid, kSumThreads, 0, s>>>(SB);
+        if (ctx->sum_items) {
+            k_sum_blocks<<<grid, 256, 0, s>>>(SB);
+            k_sum_items<<<grid, kSumThreads, 0, s>>>(SB);
+        }
         ev_record(ctx, EV_SUM_ITEMS, s);
         ev_wait(ctx, ctx->ssum, EV_SUM_ITEMS);
-
-        k_sum_chain<<<6, 64, 4 * SB.nblk, ctx->ssum>>>(SB, Pd);
+        k_sum_chain<<<6, kSumChain, 0, ctx->ssum>>>(SB, &C->zero, Pd);
         ev_record(ctx, EV_SUM_CHAIN, ctx->ssum);
         ev_wait(ctx, s, EV_SUM_CHAIN);
-        k_sum_verify<<<dim3(4 * SB.nblk * (kSumTile / 64) / 256, 6), 256, 0, s>>>(SB);
-        k_mesh_sums<<<6, 64, 0, s>>>(ctx->res ? nullptr : ctx->dv[0], ctx->nv[0], ctx->dv[1], ctx->nv[1], &C->zero, Pd,
-                                     SB.fail);
+        if (ctx->sum_items) {
+            k_sum_verify<<<grid, kSumThreads, 0, s>>>(SB);
+            k_sum_rest<<<6, 64, 0, s>>>(SB, &C->zero, Pd);
+        }
         ev_record(ctx, EV_A_SUMS, s);
     }
     if (ctx->batch) {
@@ -1497,7 +1500,7 @@ std::vector<Buf*> context_bufs(mcgpu_context ctx)
                   &ctx->re_in, &ctx->rg_in, &ctx->bpairs, &ctx->bstarts, &ctx->fpair, &ctx->vpair, &ctx->bparams,
                   &ctx->brbox, &ctx->pflags, &ctx->border, &ctx->bidx[0], &ctx->bidx[1], &ctx->rle, &ctx->rlg,
                   &ctx->rstart, &ctx->rend, &ctx->pqs, &ctx->prs, &ctx->pcounts, &ctx->sbsum,
-                  &ctx->sitems, &ctx->slo, &ctx->shi, &ctx->snitem, &ctx->slist, &ctx->sckpt, &ctx->sflags,
+                  &ctx->sitems, &ctx->snitem, &ctx->sadds, &ctx->srows,
                   &ctx->tune_c, &ctx->cc_parent, &ctx->cp_order, &ctx->cp_keys, &ctx->cp_vals, &ctx->cp_keys2, &ctx->cp_vals2,
                   &ctx->cp_flag, &ctx->cp_gid, &ctx->cp_gstart, &ctx->cp_ncand, &ctx->cp_coff, &ctx->cp_trip,
                   &ctx->cp_src, &ctx->cp_tgt, &ctx->cp_fa, &ctx->cp_fb, &ctx->cp_group, &ctx->cp_kind, &ctx->cp_acc,
@@ -2814,8 +2817,7 @@ uint64_t ctx_bytes(mcgpu_context c)
                         &c->cand_list, &c->planes, &c->big_list, &c->big_off, &c->big_scratch, &c->te, &c->tg, &c->esc,
                         &c->rkey, &c->rval, &c->rkey2, &c->rval2, &c->rp, &c->re, &c->rg, &c->rpts, &c->rcount,
                         &c->re_in, &c->rg_in, &c->shkeys, &c->shcnt, &c->scan_tmp, &c->scan_tmp_c, &c->hist,
-                        &c->sbsum, &c->sitems, &c->slo, &c->shi, &c->snitem, &c->slist, &c->sckpt,
-                        &c->sflags};
+                        &c->sbsum, &c->sitems, &c->snitem, &c->sadds, &c->srows};
     for (const Buf* b : all) t += b->cap;
     return t;
 }
