@@ -2105,6 +2105,275 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
     if (lane == 0 && lane_walks) atomicAdd(&C->n_lane_walks, lane_walks);
 }
 
+// ---------------------------------------------------------------------------
+// The same pairs breadth first over pairs of nodes, the default: all pairs of
+// nodes of two start levels are tested at once, each surviving pair's children
+// (up to 8 x 8) by one wave a step, and at the levels whose nodes hold 32
+// leaves a wave tests the leaves of a pair against each other, after dropping
+// those that miss the other node.  Every launch spreads its pairs evenly over
+// the device, where a walk of the cut tree per source block (above) ends with
+// the few blocks whose surfaces run close together (subdivision-7 icosphere
+// pair: its last waves walk alone for 85 of 110 us).  What bounds it: the
+// latency of a step's dependent loads (list entry, boxes), three launches for
+// that pair; with millions of pairs the leaf tests.
+// A list that overflows its buffer is flagged and the host runs the dispatch
+// again with the walk, which needs none.
+// ---------------------------------------------------------------------------
+constexpr int kPairLeavesLog = 5;  // leaves of a node at the last level of the lists
+constexpr int kPairStartLevel = 11; // 2^11 x 2^11 node pairs tested at the start: about 4 us of tests
+constexpr int kPairStep = 3;       // levels a side descends per step
+constexpr int kPairBlock = 512;    // 8 waves
+constexpr int kPairWaves = kPairBlock / 64;
+// Pairs a wave keeps in LDS before it appends them with one atomic: 12 ns
+// each on one address, which a launch that finds millions waits for.  A
+// terrain pair's last step (3M raw pairs) took 0.26 ms with 256, 0.13 ms with
+// 560 and 0.09 ms with 896; a subdivision-8 icosphere pair's, whose bound is
+// the waves in flight, 0.09 ms with 560 and 0.13 ms with 896.
+constexpr int kPairStage = 512;    // node pairs, upper steps: 32 KB a block
+constexpr int kPairKeep = 560;     // raw pairs, last step: with the leaves 51 KB a block, three a compute unit
+
+__device__ __forceinline__ void load_box(const float* nodes, int level, uint32_t k, float* b)
+{
+    const float* p = nodes + 6 * ((uint64_t)(1u << level) - 1 + k);
+    for (int j = 0; j < 6; ++j) b[j] = p[j];
+}
+
+// nodes of a level that hold a leaf
+__host__ __device__ inline uint32_t level_nodes(int n, int D, int level)
+{
+    const int span = D - level;
+    return (uint32_t)(((uint64_t)n + (1ull << span) - 1) >> span);
+}
+
+// LDS written by one lane and read by another of the same wave
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A wave's staged pairs: add() takes one from each lane that has a hit (the
+// whole wave calls it), flush() appends them all, close() those of every wave
+// of the block with one atomic.  Entries past the list's capacity set *over.
+template <int CAP>
+struct PairStage {
+    unsigned long long* st; // CAP entries of LDS, this wave's
+    uint32_t n;             // wave-uniform
+    unsigned long long* out;
+    uint64_t cap;
+    unsigned long long* counter;
+    unsigned int* over;
+
+    __device__ __forceinline__ void put(unsigned long long at)
+    {
+        for (uint32_t q = threadIdx.x & 63; q < n; q += 64) {
+            if (at + q < cap) out[at + q] = st[q];
+            else *over = 1u;
+        }
+    }
+    // returns the end of the list when it had to flush, else 0
+    __device__ __forceinline__ unsigned long long add(bool hit, unsigned long long e)
+    {
+        const uint64_t h = __ballot(hit);
+        if (!h) return 0;
+        const uint32_t lane = threadIdx.x & 63;
+        if (hit) st[n + __popcll(h & (lane ? (~0ull >> (64 - lane)) : 0ull))] = e;
+        n += __popcll(h);
+        if (n <= (uint32_t)CAP - 64) return 0; // room for another call
+        wave_lds_fence();
+        unsigned long long at = 0;
+        if (lane == 0) at = atomicAdd(counter, (unsigned long long)n);
+        at = __shfl(at, 0, 64);
+        put(at);
+        const unsigned long long end = at + n;
+        n = 0;
+        wave_lds_fence();
+        return end;
+    }
+    __device__ __forceinline__ void close(uint32_t* left, unsigned long long* base)
+    {
+        const uint32_t wid = threadIdx.x >> 6;
+        if ((threadIdx.x & 63) == 0) left[wid] = n;
+        __syncthreads();
+        uint32_t off = 0, tot = 0;
+        for (uint32_t q = 0; q < (uint32_t)kPairWaves; ++q) {
+            if (q < wid) off += left[q];
+            tot += left[q];
+        }
+        put(block_reserve(counter, tot, base) + off);
+    }
+};
+
+// every (source node of level s0, cut node of level c0) whose boxes overlap:
+// 256 source nodes, one a thread, against 32 cut nodes in LDS, the outcomes
+// kept as one mask (a stage in LDS cost an atomic per test with a survivor:
+// 30 us for 1,280 x 1,280 nodes
+// where this takes 14)
+__global__ void __launch_bounds__(256) k_pairs_start(Tree src, Tree cut, int s0, int c0, unsigned long long* __restrict__ out,
+                                                     uint64_t cap, unsigned long long* n, Counters* C)
+{
+    __shared__ float cb[32][8];
+    __shared__ uint32_t wsum[4];
+    __shared__ unsigned long long base;
+    const uint32_t ns = level_nodes(src.n, src.D, s0), nc = level_nodes(cut.n, cut.D, c0);
+    const uint32_t s = blockIdx.x * 256 + threadIdx.x, c1 = blockIdx.y * 32, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if (threadIdx.x < 32) {
+        float b[6];
+        load_box(cut.nodes, c0, c1 + threadIdx.x < nc ? c1 + threadIdx.x : nc - 1, b);
+        for (int j = 0; j < 6; ++j) cb[threadIdx.x][j] = b[j];
+    }
+    float sb[6];
+    load_box(src.nodes, s0, s < ns ? s : ns - 1, sb);
+    __syncthreads();
+    const uint32_t m = c1 + 32 <= nc ? 32u : nc - c1;
+    uint32_t hits = 0;
+#pragma unroll 8
+    for (uint32_t j = 0; j < 32; ++j) hits |= (uint32_t)boxes_overlap(sb, cb[j]) << j;
+    hits &= s < ns ? (m == 32 ? ~0u : (1u << m) - 1) : 0u;
+    uint32_t incl = __popc(hits);
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t v = __shfl_up(incl, o, 64);
+        incl += (int)lane >= o ? v : 0u;
+    }
+    if (lane == 63) wsum[wid] = incl;
+    __syncthreads();
+    uint32_t off = 0, tot = 0;
+    for (uint32_t q = 0; q < 4; ++q) {
+        if (q < wid) off += wsum[q];
+        tot += wsum[q];
+    }
+    unsigned long long at = block_reserve(n, tot, &base) + off + incl - __popc(hits);
+    if (at + __popc(hits) > cap) C->ov_nodes = 1u;
+    for (; hits; hits &= hits - 1, ++at)
+        if (at < cap) out[at] = (uint64_t)s << 32 | (c1 + (uint32_t)__builtin_ctz(hits));
+}
+
+// the pairs of a list (levels ls, lc) descended es and ec levels: one wave a
+// pair, a lane a pair of children
+__global__ void __launch_bounds__(kPairBlock) k_pairs_expand(Tree src, Tree cut, int ls, int lc, int es, int ec,
+                                                             const unsigned long long* __restrict__ in,
+                                                             const unsigned long long* __restrict__ nin,
+                                                             unsigned long long* __restrict__ out, uint64_t cap,
+                                                             unsigned long long* n, Counters* C)
+{
+    __shared__ unsigned long long st[kPairWaves][kPairStage];
+    __shared__ uint32_t left[kPairWaves];
+    __shared__ unsigned long long base;
+    PairStage<kPairStage> S{st[threadIdx.x >> 6], 0, out, cap, n, &C->ov_nodes};
+    const uint64_t cnt = *nin < cap ? *nin : cap;
+    const uint32_t lane = threadIdx.x & 63, i = lane & ((1u << es) - 1), j = lane >> es;
+    const bool mine = j < (1u << ec);
+    // an empty node past a tree's last leaf would meet a box without bounds
+    const uint32_t ns = level_nodes(src.n, src.D, ls + es), nc = level_nodes(cut.n, cut.D, lc + ec);
+    const uint64_t stride = (uint64_t)gridDim.x * kPairWaves;
+    for (uint64_t p = (uint64_t)blockIdx.x * kPairWaves + (threadIdx.x >> 6); p < cnt; p += 2 * stride) {
+        unsigned long long e[2];
+        uint32_t ks[2], kc[2];
+        float a[2][6], b[2][6];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) e[u] = in[p + u * stride < cnt ? p + u * stride : p];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            ks[u] = ((uint32_t)(e[u] >> 32) << es) + i;
+            kc[u] = ((uint32_t)e[u] << ec) + j;
+            load_box(src.nodes, ls + es, ks[u] < ns ? ks[u] : 0u, a[u]);
+            load_box(cut.nodes, lc + ec, mine && kc[u] < nc ? kc[u] : 0u, b[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            S.add(mine && (u == 0 || p + stride < cnt) && ks[u] < ns && kc[u] < nc && boxes_overlap(a[u], b[u]),
+                  (uint64_t)ks[u] << 32 | kc[u]);
+    }
+    S.close(left, &base);
+}
+
+// one lane's part of a pair of nodes: a leaf of its side, the other side's node
+struct LeafLoad {
+    float b[6], w[6];
+    uint32_t face;
+    bool valid;
+
+    __device__ __forceinline__ void load(const Tree& own, const Tree& other, int lown, int lother, bool on_cut,
+                                         unsigned long long e)
+    {
+        const uint32_t mk = on_cut ? (uint32_t)e : (uint32_t)(e >> 32), ok = on_cut ? (uint32_t)(e >> 32) : (uint32_t)e;
+        const int span = own.D - lown;
+        const uint32_t l = threadIdx.x & 31, leaf = (mk << span) + l;
+        valid = l < (1u << span) && leaf < (uint32_t)own.n;
+        load_box(own.nodes, own.D, valid ? leaf : 0u, b);
+        load_box(other.nodes, lother, ok, w);
+        face = own.sface[valid ? leaf : 0u];
+    }
+};
+
+// The leaves of the last list's pairs (levels ls, lc; at most 32 leaves a
+// node): lanes 0-31 take the source leaves, 32-63 the cut leaves; those that
+// meet the other node's box are packed into LDS and every two of them tested.
+__global__ void __launch_bounds__(kPairBlock) k_pairs_leaves(Tree src, Tree cut, int ls, int lc,
+                                                             const unsigned long long* __restrict__ in,
+                                                             const unsigned long long* __restrict__ nin, uint64_t cap_in,
+                                                             unsigned long long* __restrict__ pairs, uint64_t cap, Counters* C)
+{
+    __shared__ float lb[kPairWaves][2][32][8]; // box and face of the packed leaves
+    __shared__ unsigned long long st[kPairWaves][kPairKeep];
+    __shared__ uint32_t left[kPairWaves];
+    __shared__ unsigned long long base;
+    const uint64_t cnt = *nin < cap_in ? *nin : cap_in;
+    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const bool on_cut = lane >= 32;
+    const Tree& own = on_cut ? cut : src;
+    const Tree& other = on_cut ? src : cut;
+    const int lown = on_cut ? lc : ls, lother = on_cut ? ls : lc;
+    const uint32_t l = lane & 31;
+    PairStage<kPairKeep> S{st[wid], 0, pairs, cap, &C->n_raw, &C->ov_pairs};
+    const uint64_t stride = (uint64_t)gridDim.x * kPairWaves;
+    uint64_t p = (uint64_t)blockIdx.x * kPairWaves + wid;
+    if (p < cnt) {
+        // the boxes of the next pair and the entry after it load during the tests
+        LeafLoad at, next;
+        at.load(own, other, lown, lother, on_cut, in[p]);
+        unsigned long long e = in[p + stride < cnt ? p + stride : p];
+        for (; p < cnt; p += stride, at = next) {
+            next.load(own, other, lown, lother, on_cut, e);
+            e = in[p + 2 * stride < cnt ? p + 2 * stride : p];
+            const float* b = at.b;
+            const bool keep = at.valid && boxes_overlap(at.b, at.w);
+            const uint64_t m = __ballot(keep);
+            const uint32_t ms = (uint32_t)m, mc = (uint32_t)(m >> 32);
+            if (!ms || !mc) continue;
+            if (keep) {
+                float* o = lb[wid][on_cut][__popc((on_cut ? mc : ms) & ((1u << l) - 1))];
+                for (int j = 0; j < 6; ++j) o[j] = b[j];
+                o[6] = __uint_as_float(at.face);
+            }
+            wave_lds_fence();
+            const uint32_t ns = __popc(ms), nc = __popc(mc);
+            int wlog = 0; // cut leaves across the lanes, 64 >> wlog source leaves a step
+            while ((1u << wlog) < nc) ++wlog;
+            const uint32_t j = lane & ((1u << wlog) - 1), r = lane >> wlog, rows = 64u >> wlog;
+            float cbx[6];
+            const float* cp = lb[wid][1][j < nc ? j : 0];
+            for (int q = 0; q < 6; ++q) cbx[q] = cp[q];
+            const uint32_t cface = __float_as_uint(cp[6]);
+            for (uint32_t i0 = 0; i0 < ns; i0 += rows) {
+                const uint32_t i = i0 + r;
+                bool hit = false;
+                uint32_t sface = 0;
+                if (i < ns && j < nc) {
+                    const float* sp = lb[wid][0][i];
+                    hit = boxes_overlap(sp, cbx);
+                    sface = __float_as_uint(sp[6]);
+                }
+                // past 2^32 raw pairs the host refuses the dispatch whatever the exact count
+                if (S.add(hit, (uint64_t)sface << 32 | cface) > kMaxListEntries) p = cnt - 1;
+            }
+            wave_lds_fence(); // lb is rewritten for the next pair
+        }
+    }
+    S.close(left, &base);
+}
+
 // ===========================================================================
 // 6. candidate faces and their planes (kernel.cpp:2184-2356)
 // ===========================================================================

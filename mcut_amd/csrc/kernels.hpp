@@ -36,6 +36,7 @@ struct Counters {
     unsigned long long n_edges_src, n_edges_cut;
     unsigned long long n_raw;                              // raw-space (superset) candidate pairs
     unsigned long long n_fallback, n_lane_walks; // traversal statistics: node splits, per-lane walks
+    unsigned long long n_nodes[8]; // node pairs of each step of the broad phase
     unsigned long long n_f32, n_f64;            // tests whose two signs the FP32 / FP64 filter settled
     unsigned long long pmask; // pair hash slots - 1 (set once the raw pairs are known)
     unsigned long long n_trip; // triplet-scratch entries reserved by the polygons of more than five vertices
@@ -46,6 +47,7 @@ struct Counters {
     unsigned int gp, bad_src, bad_cut, unsupported, nonmanifold, bad_input, pair_fail, partial;
     unsigned int sum_next; // batches: work-queue head of the serial sums
     unsigned int ov_trip;  // the triplet scratch overflowed
+    unsigned int ov_nodes; // a list of node pairs overflowed: the tree is walked instead
     unsigned int ov_topo;  // a bucket of the edge numbering overflowed: the hash tables number the edges
     unsigned int trav_q[8]; // persistent traversal: head of each work queue (blocks taken)
     unsigned int ncc[2];    // connected components of each mesh's vertex graph (all pairs of a batch)

@@ -85,6 +85,7 @@ struct TravConfig {
     int queues = kTravQueues; // 0: one wave per block; 1: the same in per-XCD runs of `chunk`; 8: persistent
                               // waves over XCD work queues
     int chunk = kTravRun;     // blocks a persistent wave takes per queue pop; with queues 1 the run length
+    bool walk = false;        // walk the cut tree with this shape (else lists of node pairs, which have none)
 };
 constexpr int kTravWavesPerCU = 16; // persistent grid: four waves per SIMD (the kernel's occupancy)
 
@@ -174,6 +175,9 @@ struct mcgpu_context_t {
     Buf ev0, ev1, ef0, ef1;
     Buf mcode, mface, mcode2, mface2; // Morton keys and leaf order of both meshes
     Buf nodes[2], rawbox;
+    Buf node_pairs[2];
+    uint64_t cap_nodes = 0;
+    bool walk = false;               // this dispatch walks the cut tree: its node-pair lists outgrew their buffers
     Buf raw_pairs, pairs, phash, cand, cand_list, planes, big_list, big_off, big_scratch;
     Buf te, tg, tqs, trs, ttype, tpip, esc;
     Buf rkey, rval, rkey2, rval2, rp, re, rg, rpts, rcount, re_in, rg_in;
@@ -559,6 +563,29 @@ mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
     return MCGPU_SUCCESS;
 }
 
+// the broad phase's lists of node pairs: a pair for every four faces (an
+// icosphere pair's longest list holds one for fifty), at least 2^16
+mcgpu_result alloc_node_pairs(mcgpu_context ctx)
+{
+    unsigned long long* ull;
+    const uint64_t want = std::max<uint64_t>(1 << 16, ((uint64_t)ctx->nf[0] + ctx->nf[1]) / 4);
+    if (ctx->cap_nodes < want) ctx->cap_nodes = want;
+    for (Buf& b : ctx->node_pairs) CK(ensure(b, ctx->cap_nodes, &ull));
+    return MCGPU_SUCCESS;
+}
+
+// A list overflowed: this dispatch walks the tree, and later ones get longer
+// lists (up to kMaxNodePairs; past that they overflow and walk again).
+constexpr uint64_t kMaxNodePairs = 1ull << 24;
+void node_pairs_overflowed(mcgpu_context ctx, const Counters& C)
+{
+    ctx->walk = true;
+    uint64_t need = 0;
+    for (unsigned long long n : C.n_nodes) need = std::max<uint64_t>(need, n);
+    if (ctx->cap_nodes < kMaxNodePairs)
+        ctx->cap_nodes = std::min(kMaxNodePairs, std::max(2 * ctx->cap_nodes, need + need / 4));
+}
+
 mcgpu_result alloc_list_buffers(mcgpu_context ctx)
 {
     uint32_t* u;
@@ -567,6 +594,7 @@ mcgpu_result alloc_list_buffers(mcgpu_context ctx)
     CK(ensure(ctx->raw_pairs, ctx->cap_pairs, &ull));
     CK(ensure(ctx->pairs, ctx->cap_pairs, &ull));
     CK(ensure(ctx->phash, next_pow2(2 * ctx->cap_pairs), &ull));
+    if (const mcgpu_result r = alloc_node_pairs(ctx); r != MCGPU_SUCCESS) return r;
     CK(ensure(ctx->te, ctx->cap_tests, &u));
     CK(ensure(ctx->tg, ctx->cap_tests, &u));
     if (ctx->keep_tests) {
@@ -898,6 +926,8 @@ struct BroadView {
     int src_depth;
     TravConfig trav; // traversal launch shape
     int cus;         // compute units of the stream the traversal runs on
+    unsigned long long* node_pairs[2]; // lists of node pairs (null: the tree is walked)
+    uint64_t cap_nodes;
 };
 
 template <int LL, int ST>
@@ -941,10 +971,48 @@ void launch_traversal(const TravConfig& t, int cus, const Tree& src, const Tree&
     }
 }
 
+// The broad phase over lists of node pairs (k_pairs_*), on stream st.  a, b
+// (optional): the events of its first kernel's start and last kernel's end.
+template <typename K, typename... A>
+void launch_timed(K k, dim3 grid, dim3 block, hipStream_t st, hipEvent_t a, hipEvent_t b, A... args)
+{
+    if (a || b) hipExtLaunchKernelGGL(k, grid, block, 0, st, a, b, 0, args...);
+    else k<<<grid, block, 0, st>>>(args...);
+}
+
+void launch_node_pairs(const BroadView& B, const Tree& src, const Tree& cut, Counters* C, hipStream_t st, hipEvent_t a,
+                       hipEvent_t b)
+{
+    const int ts = std::max(0, src.D - kPairLeavesLog), tc = std::max(0, cut.D - kPairLeavesLog);
+    int ls = std::min(ts, kPairStartLevel), lc = std::min(tc, kPairStartLevel), step = 0;
+    const dim3 g0((level_nodes(src.n, src.D, ls) + 255) / 256, (level_nodes(cut.n, cut.D, lc) + 31) / 32);
+    launch_timed(k_pairs_start, g0, dim3(256), st, a, (hipEvent_t) nullptr, src, cut, ls, lc, B.node_pairs[0], B.cap_nodes,
+                 &C->n_nodes[0], C);
+    for (; ls < ts || lc < tc; ++step) {
+        const int es = std::min(kPairStep, ts - ls), ec = std::min(kPairStep, tc - lc);
+        k_pairs_expand<<<512, kPairBlock, 0, st>>>(src, cut, ls, lc, es, ec, B.node_pairs[step & 1], &C->n_nodes[step],
+                                                   B.node_pairs[(step & 1) ^ 1], B.cap_nodes, &C->n_nodes[step + 1], C);
+        ls += es;
+        lc += ec;
+    }
+    launch_timed(k_pairs_leaves, dim3(1024), dim3(kPairBlock), st, (hipEvent_t) nullptr, b, src, cut, ls, lc,
+                 B.node_pairs[step & 1], &C->n_nodes[step], B.cap_nodes, B.raw_pairs, B.cap_pairs, C);
+}
+
+// the steps of launch_node_pairs fit Counters::n_nodes for any tree of 32-bit leaves
+static_assert((32 - kPairLeavesLog - kPairStartLevel + kPairStep - 1) / kPairStep + 1 <= 8, "steps of the node-pair lists");
+
 bool trav_config_valid(const TravConfig& t)
 {
     return t.ll >= 3 && t.ll <= 5 && t.stride >= 2 && t.stride <= 4 && (t.queues == 0 || t.queues == 1 || t.queues == 8) &&
            t.chunk >= 1 && t.chunk <= 64;
+}
+
+// the pairs of two refitted trees, by node-pair lists or the walk
+void launch_broad(const BroadView& B, const Tree& src, const Tree& cut, Counters* C, hipStream_t st, hipEvent_t a, hipEvent_t b)
+{
+    if (B.node_pairs[0] && !B.trav.walk) launch_node_pairs(B, src, cut, C, st, a, b);
+    else launch_traversal(B.trav, B.cus, src, cut, B.raw_pairs, B.cap_pairs, C, st, a, b);
 }
 
 // The two trees of a broad view once its leaves are sorted (into mface2 when
@@ -1017,7 +1085,7 @@ bool enqueue_trees_traverse(const BroadView& B, hipStream_t st, Counters* C, boo
         }
     }
     if (b_refit) (void)hipEventRecord(b_refit, st);
-    launch_traversal(B.trav, B.cus, T[0], T[1], B.raw_pairs, B.cap_pairs, C, st, k_start, k_stop);
+    launch_broad(B, T[0], T[1], C, st, k_start, k_stop);
     return alt;
 }
 
@@ -1061,6 +1129,8 @@ BroadView broad_view(mcgpu_context ctx)
     }
     B.trav = ctx->trav;
     B.cus = cus_of(ctx, ctx->batch);
+    for (int q = 0; q < 2; ++q) B.node_pairs[q] = ctx->walk ? nullptr : P_<unsigned long long>(ctx->node_pairs[q]);
+    B.cap_nodes = ctx->cap_nodes;
     return B;
 }
 
@@ -1376,6 +1446,11 @@ mcgpu_result finish(mcgpu_context ctx, mcgpu_frontend_info* info, bool* overflow
         *overflow = true;
         return MCGPU_SUCCESS;
     }
+    if (C.ov_nodes) { // run again with the walk
+        node_pairs_overflowed(ctx, C);
+        *overflow = true;
+        return MCGPU_SUCCESS;
+    }
     if (C.ov_topo) { // run again with the edges numbered through the hash tables
         ctx->topo_hash = true;
         *overflow = true;
@@ -1493,7 +1568,7 @@ std::vector<Buf*> context_bufs(mcgpu_context ctx)
                   &ctx->hkeys[1], &ctx->hfirst[0], &ctx->hfirst[1], &ctx->cface[0], &ctx->cface[1], &ctx->eflag[0],
                   &ctx->eflag[1], &ctx->eid[0], &ctx->eid[1], &ctx->cedge[0], &ctx->cedge[1], &ctx->etotal, &ctx->opp, &ctx->twords, &ctx->tsum, &ctx->tseg, &ctx->ev0,
                   &ctx->ev1, &ctx->ef0, &ctx->ef1, &ctx->mcode, &ctx->mface, &ctx->mcode2, &ctx->mface2, &ctx->nodes[0], &ctx->nodes[1],
-                  &ctx->rawbox, &ctx->raw_pairs, &ctx->pairs, &ctx->phash, &ctx->cand, &ctx->cand_list,
+                  &ctx->rawbox, &ctx->node_pairs[0], &ctx->node_pairs[1], &ctx->raw_pairs, &ctx->pairs, &ctx->phash, &ctx->cand, &ctx->cand_list,
                   &ctx->planes, &ctx->big_list, &ctx->big_off, &ctx->big_scratch, &ctx->te, &ctx->tg, &ctx->tqs, &ctx->trs,
                   &ctx->ttype, &ctx->tpip, &ctx->esc, &ctx->rkey, &ctx->rval, &ctx->rkey2, &ctx->rval2, &ctx->rp,
                   &ctx->re, &ctx->rg, &ctx->rpts, &ctx->rcount, &ctx->shkeys, &ctx->shcnt, &ctx->scan_tmp, &ctx->scan_tmp_c, &ctx->hist,
@@ -1518,7 +1593,7 @@ std::vector<uint64_t> graph_key(mcgpu_context ctx)
     auto put = [&k](uint64_t x) { k.push_back(x); };
     auto ptr = [&k](const void* p) { k.push_back((uint64_t)(uintptr_t)p); };
     put(ctx->batch), put(ctx->npairs), put(ctx->batch_mb), put(ctx->cc_check), put(ctx->sort_bits),
-        put(ctx->shifted_bp), put(ctx->topo_hash), put(ctx->topo_buckets), put(ctx->topo_tiles), put(ctx->topo_items),
+        put(ctx->shifted_bp), put(ctx->walk), put(ctx->trav.walk), put(ctx->cap_nodes), put(ctx->topo_hash), put(ctx->topo_buckets), put(ctx->topo_tiles), put(ctx->topo_items),
         put(ctx->nseg),
         put(ctx->gbits), put(ctx->kbits);
     for (int m = 0; m < 2; ++m) {
@@ -1767,7 +1842,7 @@ static mcgpu_result time_traversal(mcgpu_context ctx, const TravConfig& t, int r
     *same = true;
     for (int i = 0; i < reps && r == MCGPU_SUCCESS; ++i) {
         fill_u32(C, 0u, sizeof(Counters) / 4, st);
-        launch_traversal(t, B.cus, T[0], T[1], B.raw_pairs, B.cap_pairs, C, st, e[0], e[1]);
+        launch_broad(B, T[0], T[1], C, st, e[0], e[1]);
         Counters h;
         float x = 0.f;
         if (hipStreamSynchronize(st) != hipSuccess || hipGetLastError() != hipSuccess ||
@@ -1776,7 +1851,7 @@ static mcgpu_result time_traversal(mcgpu_context ctx, const TravConfig& t, int r
             r = MCGPU_ERROR_DEVICE;
             break;
         }
-        if (h.n_raw != ctx->C.n_raw || h.ov_pairs) *same = false;
+        if (h.n_raw != ctx->C.n_raw || h.ov_pairs || h.ov_nodes) *same = false;
         v.push_back(x);
     }
     (void)hipEventDestroy(e[0]);
@@ -1787,9 +1862,10 @@ static mcgpu_result time_traversal(mcgpu_context ctx, const TravConfig& t, int r
     return MCGPU_SUCCESS;
 }
 
-// The autotuner for the last dispatch's workload class: every traversal
-// launch shape of the candidate lists (leaves per block, levels per step,
-// queue mode) is timed alone on the dispatch's own trees (a median of three)
+// The autotuner for the last dispatch's workload class: the default (lists of
+// node pairs, or the walk where a list outgrew its buffer) and every launch
+// shape of the walk in the candidate lists (leaves per block, levels per step,
+// queue mode) are timed alone on the dispatch's own trees (a median of three)
 // and must find the same raw pairs; the fastest wins.  The whole dispatch is
 // then re-run with the default and with the chosen shape (best of two device
 // times each) for the report.  The choice is kept for the class (single pair
@@ -1804,6 +1880,12 @@ static mcgpu_result autotune(mcgpu_context ctx, mcgpu_tuning* out)
     TravConfig bt = def;
     uint32_t n = 0;
     mcgpu_result r;
+    {
+        bool same = true;
+        if ((r = time_traversal(ctx, def, 3, &def_trav, &same)) != MCGPU_SUCCESS) return r;
+        if (!same) return MCGPU_ERROR_DEVICE;
+        best = def_trav;
+    }
     for (int ll : kTuneLL)
         for (int st : kTuneStride)
             for (const auto& q : kTuneQueue) {
@@ -1812,12 +1894,12 @@ static mcgpu_result autotune(mcgpu_context ctx, mcgpu_tuning* out)
                 t.stride = st;
                 t.queues = q[0];
                 t.chunk = q[1];
+                t.walk = true;
                 float ms = 0.f;
                 bool same = true;
                 if ((r = time_traversal(ctx, t, 3, &ms, &same)) != MCGPU_SUCCESS) return r;
                 if (!same) return MCGPU_ERROR_DEVICE; // every shape finds the same pairs
                 ++n;
-                if (t.ll == def.ll && t.stride == def.stride && t.queues == def.queues && t.chunk == def.chunk) def_trav = ms;
                 if (ms < best) {
                     best = ms;
                     bt = t;
@@ -1937,6 +2019,7 @@ static mcgpu_result frontend_prepare(mcgpu_context ctx, const mcgpu_mesh* src, c
     ctx->broad_only = false;
     ctx->batch = false;
     ctx->shifted_bp = false;
+    ctx->walk = false;
     ctx->allow_loose = true;
     ctx->cc_check = (desc->flags & MCGPU_DISPATCH_CHECK_COMPONENTS) != 0;
     ctx->sort_bits = 22;
@@ -2051,6 +2134,8 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
     ctx->have = false;
     ctx->broad_only = false;
     ctx->batch = true;
+    ctx->shifted_bp = false;
+    ctx->walk = false;
     ctx->allow_loose = false;
     ctx->cc_check = (desc->flags & MCGPU_DISPATCH_CHECK_COMPONENTS) != 0;
     ctx->npairs = np;
@@ -2220,6 +2305,7 @@ MCGPU_API mcgpu_result mcgpu_broad_phase(mcgpu_context ctx, const double* src_bo
     ctx->cc_check = false;
     ctx->sort_bits = 22;
     ctx->trav = ctx->forced ? ctx->forced_trav : TravConfig{};
+    ctx->walk = false;
     ctx->nf[0] = num_src;
     ctx->nf[1] = num_cut;
     ctx->nv[0] = ctx->nv[1] = 0;
@@ -2254,6 +2340,7 @@ MCGPU_API mcgpu_result mcgpu_broad_phase(mcgpu_context ctx, const double* src_bo
         CK(ensure(ctx->raw_pairs, ctx->cap_pairs, &ull));
         CK(ensure(ctx->pairs, ctx->cap_pairs, &ull));
         CK(ensure(ctx->phash, next_pow2(2 * ctx->cap_pairs), &ull));
+        if (const mcgpu_result r = alloc_node_pairs(ctx); r != MCGPU_SUCCESS) return r;
         Counters* C = &st->C;
         (void)hipEventRecord(ctx->ev[EV_A0], s);
         fill_u32(C, 0u, sizeof(Counters) / 4, s);
@@ -2279,6 +2366,10 @@ MCGPU_API mcgpu_result mcgpu_broad_phase(mcgpu_context ctx, const double* src_bo
         CK(hipStreamSynchronize(s));
         CK(hipGetLastError());
         CK(hipMemcpy(&ctx->C, C, sizeof(Counters), hipMemcpyDeviceToHost));
+        if (ctx->C.ov_nodes) {
+            node_pairs_overflowed(ctx, ctx->C);
+            continue;
+        }
         if (ctx->C.ov_pairs) {
             ctx->cap_pairs = std::max<uint64_t>(2 * ctx->cap_pairs, ctx->C.n_raw + ctx->C.n_raw / 4);
             continue;
@@ -2766,6 +2857,7 @@ MCGPU_API mcgpu_result mcgpu_set_tuning(mcgpu_context ctx, const mcgpu_tuning* t
     c.stride = (int)t->tree_stride;
     c.queues = (int)t->queues;
     c.chunk = (int)t->chunk;
+    c.walk = true;
     if ((1u << ll) != t->wave_leaves || !trav_config_valid(c) || t->broad_share_pct != 0)
         return MCGPU_ERROR_INVALID_VALUE;
     ctx->forced = true;
@@ -2813,7 +2905,7 @@ uint64_t ctx_bytes(mcgpu_context c)
                         &c->hkeys[1], &c->hfirst[1], &c->cface[1], &c->eflag[1], &c->eid[1], &c->cedge[1],
                         &c->opp, &c->twords, &c->tsum,
                         &c->etotal, &c->ev0, &c->ev1, &c->ef0, &c->ef1, &c->mcode, &c->mface, &c->mcode2,
-                        &c->mface2, &c->nodes[1], &c->rawbox, &c->raw_pairs, &c->pairs, &c->phash, &c->cand,
+                        &c->mface2, &c->nodes[1], &c->rawbox, &c->node_pairs[0], &c->node_pairs[1], &c->raw_pairs, &c->pairs, &c->phash, &c->cand,
                         &c->cand_list, &c->planes, &c->big_list, &c->big_off, &c->big_scratch, &c->te, &c->tg, &c->esc,
                         &c->rkey, &c->rval, &c->rkey2, &c->rval2, &c->rp, &c->re, &c->rg, &c->rpts, &c->rcount,
                         &c->re_in, &c->rg_in, &c->shkeys, &c->shcnt, &c->scan_tmp, &c->scan_tmp_c, &c->hist,
@@ -2878,6 +2970,7 @@ mcgpu_result slot_bind(mcgpu_server srv, mcgpu_context ctx, const mcgpu_mesh* cu
     ctx->have = false;
     ctx->broad_only = false;
     ctx->batch = false;
+    ctx->walk = false;
     ctx->cc_check = (srv->desc.flags & MCGPU_DISPATCH_CHECK_COMPONENTS) != 0;
     ctx->sort_bits = 22;
     ctx->flags = srv->desc.flags;
@@ -3381,6 +3474,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_narrow(mcgpu_context ctx, const mcgpu_mesh
     ctx->broad_only = false;
     ctx->batch = false;
     ctx->shifted_bp = false;
+    ctx->walk = false;
     ctx->allow_loose = false; // the caller's pairs: no broad phase runs here
     ctx->cc_check = false;
     ctx->sort_bits = 22;
