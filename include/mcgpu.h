@@ -228,7 +228,7 @@ MCGPU_API mcgpu_result mcgpu_broad_phase(mcgpu_context ctx, const double* src_bo
  * it is mcgpu_broad_phase for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  It calls no hipMalloc / hipFree: every array it needs lives in
- * a static device array of MCGPU_NOALLOC_SCRATCH_BYTES (50.1 MiB), which each
+ * a static device array of MCGPU_NOALLOC_SCRATCH_BYTES (34.1 MiB), which each
  * device that runs it holds until the process ends.  Limits: at most
  * MCGPU_NOALLOC_MAX_FACES faces per mesh (larger inputs return
  * MCGPU_ERROR_INVALID_VALUE before any device work) and at most
@@ -243,7 +243,7 @@ MCGPU_API mcgpu_result mcgpu_broad_phase(mcgpu_context ctx, const double* src_bo
  * array, so calls that overlap in time on one device race. */
 #define MCGPU_NOALLOC_MAX_FACES 65536u
 #define MCGPU_NOALLOC_MAX_PAIRS (1u << 20)
-#define MCGPU_NOALLOC_SCRATCH_BYTES 52566528ull
+#define MCGPU_NOALLOC_SCRATCH_BYTES 35789312ull
 MCGPU_API mcgpu_result mcgpu_broad_phase_noalloc(int device, const double* src_boxes, uint32_t num_src,
                                                  const double* cut_boxes, uint32_t num_cut, uint64_t* pairs,
                                                  uint64_t capacity, uint64_t* num_pairs, void* stream);

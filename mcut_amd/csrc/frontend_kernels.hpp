@@ -2380,9 +2380,10 @@ __global__ void __launch_bounds__(kPairBlock) k_pairs_leaves(Tree src, Tree cut,
 
 // The exact broad-phase test on the shifted boxes (bvh.cpp:661-781 with the
 // boxes of bvh.cpp:242-313) applied to the raw-space superset.  A surviving
-// pair is appended to the candidate-pair list and the pair hash used for test
-// dedup, and each of its faces is flagged once and appended to the candidate
-// face list.
+// pair is appended to the candidate-pair list, and each of its faces is flagged
+// once and appended to the candidate face list.  Pairs that the caller gave
+// (phash not null) also enter the pair hash in which k_tests looks them up;
+// the other dispatches need no lookup (PairRule).
 // The pair hash is sized from the raw pair count: twice the pairs it can
 // receive, rounded up to a power of two, within the allocated table.
 __device__ __forceinline__ uint64_t pair_hash_slots(const Counters* C, uint64_t cap, uint64_t table)
@@ -2391,14 +2392,6 @@ __device__ __forceinline__ uint64_t pair_hash_slots(const Counters* C, uint64_t 
     uint64_t m = 1024;
     while (m < 2 * n) m <<= 1;
     return m < table ? m : table;
-}
-
-// the whole table, for a dispatch whose stream A is idle before the join: the
-// filter then sizes the hash itself (pair_hash_slots) and skips the init
-__global__ void k_pair_hash_clear(unsigned long long* __restrict__ phash, uint64_t table)
-{
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < table; i += (uint64_t)gridDim.x * blockDim.x)
-        phash[i] = kEmpty64;
 }
 
 __global__ void k_pair_hash_init(unsigned long long* __restrict__ phash, uint64_t cap, uint64_t table, Counters* C)
@@ -2423,17 +2416,14 @@ __global__ void __launch_bounds__(kStageBlock) k_filter_pairs(const double* __re
                                                          unsigned long long* __restrict__ pairs,
                                                          unsigned long long* __restrict__ phash,
                                                          uint32_t* __restrict__ cand, uint32_t* __restrict__ cand_list,
-                                                         uint64_t table, Counters* C)
+                                                         Counters* C)
 {
     __shared__ unsigned long long st_pair[kFilterTile];
     __shared__ uint32_t st_face[2 * kFilterTile];
     __shared__ uint32_t st_np, st_nf;
     __shared__ unsigned long long st_base;
     const uint64_t n = C->n_raw < cap ? C->n_raw : cap;
-    // table > 0: the table was cleared whole before the join, and the hash's
-    // size follows the raw pair count here
-    const uint64_t pmask = table ? pair_hash_slots(C, cap, table) - 1 : C->pmask;
-    if (table && blockIdx.x == 0 && threadIdx.x == 0) C->pmask = pmask;
+    const uint64_t pmask = C->pmask;
     for (uint64_t t0 = (uint64_t)blockIdx.x * kFilterTile; t0 < n; t0 += (uint64_t)gridDim.x * kFilterTile) {
         if (threadIdx.x == 0) st_np = st_nf = 0;
         __syncthreads();
@@ -2450,7 +2440,7 @@ __global__ void __launch_bounds__(kStageBlock) k_filter_pairs(const double* __re
             }
             if (!boxes_overlap(a, b)) continue;
             st_pair[wave_reserve(&st_np)] = k; // one per item: the stage cannot overflow
-            hash_insert(phash, pmask, k);
+            if (phash) hash_insert(phash, pmask, k);
             for (int side = 0; side < 2; ++side)
                 if (cand[f[side]] == 0u && atomicExch(&cand[f[side]], 1u) == 0u)
                     st_face[wave_reserve(&st_nf)] = f[side]; // at most two per item
@@ -2707,6 +2697,18 @@ __global__ void __launch_bounds__(64) k_big_polygons(Soup S, const uint32_t* __r
 // only when e's box (endpoints, never enlarged) overlaps g's box.
 // ===========================================================================
 
+// How a face that is not its edge's lowest learns whether the lowest, fo, is
+// paired with g as well:
+// - the broad phase's own pairs: every face's box holds its edges' boxes, so
+//   when e passes the cull against g, all its faces are paired with g, and only
+//   the lowest need look at e at all (a lookup in a hash of all pairs took half
+//   of this kernel, and filling it most of the filter: the tests 1.04
+//   and the filter 0.40 ms for 2.7M pairs of a terrain pair, 0.59 and 0.18 without);
+// - the pairs kept from an earlier dispatch, with the cut vertices moved since:
+//   the boxes are still those of that dispatch, and overlap for the pairs;
+// - pairs that the caller gave: the hash of them.
+enum PairRule { kPairsOwn = 0, kPairsMoved = 1, kPairsGiven = 2 };
+
 __device__ __forceinline__ bool pair_exists(const unsigned long long* phash, uint64_t pmask, uint32_t s, uint32_t c)
 {
     return hash_find(phash, pmask, ((uint64_t)s << 32) | c) >= 0;
@@ -2735,10 +2737,8 @@ __device__ __forceinline__ uint32_t corner_edge(const Soup& S, int m, uint32_t b
     return S.cedge[m][o < r ? rank_corner(cm, o, m) : (uint64_t)(b + k)];
 }
 
-__device__ __forceinline__ bool edge_face_cull(const Soup& S, uint32_t e, uint32_t g)
+__device__ __forceinline__ bool edge_box_overlaps(const double* p0, const double* p1, const double* fb)
 {
-    const double* p0 = S.ps_v + 3 * (uint64_t)S.ev1[e]; // vertex(e, 0) = target(h0)
-    const double* p1 = S.ps_v + 3 * (uint64_t)S.ev0[e];
     double eb[6];
     for (int j = 0; j < 3; ++j) {
         double lo = 1.7976931348623157e308, hi = -1.7976931348623157e308;
@@ -2749,20 +2749,22 @@ __device__ __forceinline__ bool edge_face_cull(const Soup& S, uint32_t e, uint32
         eb[j] = lo;
         eb[3 + j] = hi;
     }
-    double fb[6];
-    for (int j = 0; j < 6; ++j) fb[j] = S.box[6 * (uint64_t)g + j];
     return boxes_overlap(eb, fb);
 }
 
-// six work items per pair: (side, corner slot); a polygon's corners beyond
-// the third are taken by the same slot in steps of three.  A block takes a
-// tile of kTestTile items and stages the tests it emits in LDS.
-constexpr int kTestItems = 1;
-constexpr int kTestTile = kStageBlock * kTestItems;
-constexpr int kTestStage = 2048;
+// Two work items per pair, one a side: the edges of one face against the box
+// of the other.  A triangle's three vertices are loaded once and its edges
+// culled first, from registers; only an edge that passes has its other face
+// and its number looked up (an item per edge, which looked both up first and
+// loaded its vertices through the edge: 0.59 ms for the
+// 2.7M pairs of a terrain pair, 0.29 this way).  What bounds it: the
+// gathers (vertices, boxes, edge numbers).  A block takes a tile of kTestTile
+// items and stages the tests it emits in LDS.
+constexpr int kTestTile = kStageBlock;
+constexpr int kTestStage = 3 * kTestTile; // a triangle's three edges each
 
 __global__ void __launch_bounds__(kStageBlock) k_tests(Soup S, const unsigned long long* __restrict__ pairs, uint64_t cap_pairs,
-                                                  const unsigned long long* __restrict__ phash,
+                                                  int rule, const unsigned long long* __restrict__ phash,
                                                   uint32_t* __restrict__ te, uint32_t* __restrict__ tg, uint64_t cap_tests,
                                                   Counters* C)
 {
@@ -2772,33 +2774,34 @@ __global__ void __launch_bounds__(kStageBlock) k_tests(Soup S, const unsigned lo
     const uint64_t n = C->n_pairs < cap_pairs ? C->n_pairs : cap_pairs;
     const uint64_t pmask = C->pmask;
     const uint32_t Fs = S.nf[0];
-    const uint64_t items = 6 * n;
+    const uint64_t items = 2 * n;
     for (uint64_t t0 = (uint64_t)blockIdx.x * kTestTile; t0 < items; t0 += (uint64_t)gridDim.x * kTestTile) {
         if (threadIdx.x == 0) st_n = 0;
         __syncthreads();
-        for (int rr = 0; rr < kTestItems; ++rr) {
-            const uint64_t w = t0 + (uint64_t)rr * kStageBlock + threadIdx.x;
-            if (w >= items) continue;
-            const uint64_t i = w / 6;
-            const uint32_t slot = (uint32_t)(w - 6 * i);
-            const int side = slot >= 3;
-            const uint32_t j0 = side ? slot - 3 : slot;
-            const uint64_t key = pairs[i];
+        const uint64_t w = t0 + threadIdx.x;
+        if (w < items) {
+            const int side = (int)(w & 1);
+            const uint64_t key = pairs[w >> 1];
             const uint32_t s = (uint32_t)(key >> 32), c = (uint32_t)key;
             const uint32_t f = side ? c : s;         // face whose edges are tested
             const uint32_t self = side ? Fs + c : s; // its ps id
             const uint32_t g = side ? s : Fs + c;    // the other face (ps id)
             const uint32_t b = S.off[side][f], nn = S.off[side][f + 1] - b;
-            for (uint32_t k = j0; k < nn; k += 3) {
-                int32_t fo; // the edge's other face
-                const uint32_t e = corner_edge(S, side, b, k, nn, self, &fo);
-                // the lowest-numbered face of e paired with g emits the test
+            const uint32_t* idx = S.idx[side] + b;
+            const uint32_t vofs = side ? S.nv[0] : 0u;
+            double fb[6];
+            for (int j = 0; j < 6; ++j) fb[j] = S.box[6 * (uint64_t)g + j];
+            // edge k passed the cull: emitted by its lowest-numbered face paired with g
+            auto emit = [&](uint32_t e, int32_t fo) {
                 if (fo >= 0 && (uint32_t)fo < self) {
-                    const bool paired = side ? pair_exists(phash, pmask, s, (uint32_t)fo - Fs)
-                                             : pair_exists(phash, pmask, (uint32_t)fo, c);
-                    if (paired) continue;
+                    bool paired = true;
+                    if (rule == kPairsMoved)
+                        paired = boxes_overlap(S.box + 6 * (uint64_t)fo, S.box + 6 * (uint64_t)g);
+                    else if (rule == kPairsGiven)
+                        paired = side ? pair_exists(phash, pmask, s, (uint32_t)fo - Fs)
+                                      : pair_exists(phash, pmask, (uint32_t)fo, c);
+                    if (paired) return;
                 }
-                if (!edge_face_cull(S, e, g)) continue;
                 const uint32_t at = wave_reserve(&st_n);
                 if (at < (uint32_t)kTestStage) {
                     st_e[at] = e;
@@ -2811,6 +2814,42 @@ __global__ void __launch_bounds__(kStageBlock) k_tests(Soup S, const unsigned lo
                     } else {
                         atomicOr(&C->ov_tests, 1u);
                     }
+                }
+            };
+            if (!S.opp[side]) { // the edge of every corner is given, its vertices with it
+                for (uint32_t k = 0; k < nn; ++k) {
+                    int32_t fo;
+                    const uint32_t e = corner_edge(S, side, b, k, nn, self, &fo);
+                    double p0[3], p1[3];
+                    load3(S.ps_v + 3 * (uint64_t)S.ev1[e], p0); // vertex(e, 0) = target(h0)
+                    load3(S.ps_v + 3 * (uint64_t)S.ev0[e], p1);
+                    if (edge_box_overlaps(p0, p1, fb)) emit(e, fo);
+                }
+            } else if (nn == 3) {
+                double p[3][3];
+                for (int k = 0; k < 3; ++k) load3(S.ps_v + 3 * (uint64_t)(vofs + idx[k]), p[k]);
+                bool pass[3];
+                for (int k = 0; k < 3; ++k) pass[k] = edge_box_overlaps(p[k], p[k == 2 ? 0 : k + 1], fb);
+                for (uint32_t k = 0; k < 3; ++k)
+                    if (pass[k]) {
+                        int32_t fo;
+                        const uint32_t e = corner_edge(S, side, b, k, 3, self, &fo);
+                        emit(e, fo);
+                    }
+            } else {
+                double first[3], p0[3], p1[3];
+                load3(S.ps_v + 3 * (uint64_t)(vofs + idx[0]), first);
+                for (int j = 0; j < 3; ++j) p0[j] = first[j];
+                for (uint32_t k = 0; k < nn; ++k) {
+                    if (k + 1 < nn) load3(S.ps_v + 3 * (uint64_t)(vofs + idx[k + 1]), p1);
+                    else
+                        for (int j = 0; j < 3; ++j) p1[j] = first[j];
+                    if (edge_box_overlaps(p0, p1, fb)) {
+                        int32_t fo;
+                        const uint32_t e = corner_edge(S, side, b, k, nn, self, &fo);
+                        emit(e, fo);
+                    }
+                    for (int j = 0; j < 3; ++j) p0[j] = p1[j];
                 }
             }
         }

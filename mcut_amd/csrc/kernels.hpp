@@ -38,7 +38,7 @@ struct Counters {
     unsigned long long n_fallback, n_lane_walks; // traversal statistics: node splits, per-lane walks
     unsigned long long n_nodes[8]; // node pairs of each step of the broad phase
     unsigned long long n_f32, n_f64;            // tests whose two signs the FP32 / FP64 filter settled
-    unsigned long long pmask; // pair hash slots - 1 (set once the raw pairs are known)
+    unsigned long long pmask; // pair hash slots - 1 (pairs given by the caller)
     unsigned long long n_trip; // triplet-scratch entries reserved by the polygons of more than five vertices
     double zero;              // +0.0 (the per-dispatch reset clears it): padding the serial sums load
     unsigned int ov_pairs, ov_tests, ov_esc, ov_reg, ov_big;

@@ -58,7 +58,7 @@ enum Stage {
     ST_BVH_SORT,  // B: raw face boxes, Morton codes, leaf sort
     ST_REFIT,     // B: implicit-tree boxes
     ST_TRAVERSE,  // B: raw-space broad phase (superset of the pairs)
-    ST_FILTER,    // A: exact shifted-box test, pair hash, candidate faces
+    ST_FILTER,    // A: exact shifted-box test, candidate faces
     ST_PLANES,    // A: candidate-face planes
     ST_TESTS,     // A: edge-face tests
     ST_NARROW,    // A: narrow phase
@@ -177,6 +177,7 @@ struct mcgpu_context_t {
     Buf nodes[2], rawbox;
     Buf node_pairs[2];
     uint64_t cap_nodes = 0;
+    bool pairs_given = false;        // the caller gave this dispatch's pairs (mcgpu_dispatch_narrow)
     bool walk = false;               // this dispatch walks the cut tree: its node-pair lists outgrew their buffers
     Buf raw_pairs, pairs, phash, cand, cand_list, planes, big_list, big_off, big_scratch;
     Buf te, tg, tqs, trs, ttype, tpip, esc;
@@ -593,7 +594,7 @@ mcgpu_result alloc_list_buffers(mcgpu_context ctx)
     double* dp;
     CK(ensure(ctx->raw_pairs, ctx->cap_pairs, &ull));
     CK(ensure(ctx->pairs, ctx->cap_pairs, &ull));
-    CK(ensure(ctx->phash, next_pow2(2 * ctx->cap_pairs), &ull));
+    if (ctx->pairs_given) CK(ensure(ctx->phash, next_pow2(2 * ctx->cap_pairs), &ull));
     if (const mcgpu_result r = alloc_node_pairs(ctx); r != MCGPU_SUCCESS) return r;
     CK(ensure(ctx->te, ctx->cap_tests, &u));
     CK(ensure(ctx->tg, ctx->cap_tests, &u));
@@ -708,7 +709,7 @@ void ev_wait(mcgpu_context ctx, hipStream_t st, int e)
     ctx->prog.push_back(GraphOp{GraphOp::WAIT, st, e, nullptr});
 }
 
-void enqueue_narrow(mcgpu_context ctx, const Soup& S, bool join_topology)
+void enqueue_narrow(mcgpu_context ctx, const Soup& S, bool join_topology, PairRule rule)
 {
     hipStream_t s = ctx->s;
     const uint64_t F = (uint64_t)ctx->nf[0] + ctx->nf[1];
@@ -723,7 +724,7 @@ void enqueue_narrow(mcgpu_context ctx, const Soup& S, bool join_topology)
     stage_event(ctx, EV_A_PLANES, s);
     if (join_topology) ev_wait(ctx, s, EV_C_TOPO);
     stage_event(ctx, EV_A_JOIN2, s);
-    k_tests<<<grid_for(6 * ctx->cap_pairs, kTestTile, 2048), kStageBlock, 0, s>>>(S, P_<unsigned long long>(ctx->pairs), ctx->cap_pairs,
+    k_tests<<<grid_for(2 * ctx->cap_pairs, kTestTile, 2048), kStageBlock, 0, s>>>(S, P_<unsigned long long>(ctx->pairs), ctx->cap_pairs, (int)rule,
                                                         P_<unsigned long long>(ctx->phash), P_<uint32_t>(ctx->te),
                                                         P_<uint32_t>(ctx->tg), ctx->cap_tests, C);
     stage_event(ctx, EV_A_TESTS, s);
@@ -1260,10 +1261,6 @@ void enqueue_frontend(mcgpu_context ctx)
 
     // ---- stream A, enqueued first: the serial sums start at once ----
     ev_record(ctx, EV_FORK, s);
-    // a single dispatch on its own four streams clears the whole pair hash
-    // early; batches (huge tables) and serving slots (one stream) size it
-    // after the traversal
-    const bool early_clear = ctx->own_streams && !ctx->batch;
     const bool absolute = (ctx->flags & MCGPU_DISPATCH_ENFORCE_GENERAL_POSITION_ABSOLUTE) != 0;
     Params* Pb = P_<Params>(ctx->bparams);
     const auto* brbox = (const unsigned long long(*)[2][6])ctx->brbox.p;
@@ -1276,10 +1273,6 @@ void enqueue_frontend(mcgpu_context ctx)
     } else {
         // items and their check on stream A (every CU), the chain on the
         // reserved CUs, the values one by one only where a check failed
-        if (early_clear) { // the pair hash, before the sum kernels (its fill would slow the sum chain beside it)
-            const uint64_t table = next_pow2(2 * ctx->cap_pairs);
-            k_pair_hash_clear<<<grid_for(table, kBlock, 2048), kBlock, 0, s>>>(P_<unsigned long long>(ctx->phash), table);
-        }
         stage_event(ctx, EV_S0, s);
         const SumBufs SB = sum_bufs(ctx);
         const dim3 grid(SB.nblk, 6);
@@ -1373,19 +1366,13 @@ void enqueue_frontend(mcgpu_context ctx)
     ev_wait(ctx, s, EV_B_TRAV);
     ev_wait(ctx, s, EV_C_FILL);
     stage_event(ctx, EV_A_JOIN, s);
-    const uint64_t table = next_pow2(2 * ctx->cap_pairs);
-    if (!early_clear)
-        k_pair_hash_init<<<grid_for(table, kBlock, 1024), kBlock, 0, s>>>(P_<unsigned long long>(ctx->phash),
-                                                                          ctx->cap_pairs, table, C);
     k_filter_pairs<<<grid_for(ctx->cap_pairs, kFilterTile, 2048), kStageBlock, 0, s>>>(P_<double>(ctx->box), P_<unsigned long long>(ctx->raw_pairs),
                                                                ctx->cap_pairs, Fs,
                                                                ctx->batch ? P_<uint32_t>(ctx->fpair) : nullptr,
-                                                               P_<unsigned long long>(ctx->pairs),
-                                                               P_<unsigned long long>(ctx->phash), P_<uint32_t>(ctx->cand),
-                                                               P_<uint32_t>(ctx->cand_list), early_clear ? table : 0,
-                                                               C);
+                                                               P_<unsigned long long>(ctx->pairs), nullptr,
+                                                               P_<uint32_t>(ctx->cand), P_<uint32_t>(ctx->cand_list), C);
     stage_event(ctx, EV_A_FILTER, s);
-    enqueue_narrow(ctx, S, true);
+    enqueue_narrow(ctx, S, true, kPairsOwn);
 }
 
 // The state's copy to pinned host memory, on stream A behind the dispatch
@@ -2020,6 +2007,7 @@ static mcgpu_result frontend_prepare(mcgpu_context ctx, const mcgpu_mesh* src, c
     ctx->batch = false;
     ctx->shifted_bp = false;
     ctx->walk = false;
+    ctx->pairs_given = false;
     ctx->allow_loose = true;
     ctx->cc_check = (desc->flags & MCGPU_DISPATCH_CHECK_COMPONENTS) != 0;
     ctx->sort_bits = 22;
@@ -2136,6 +2124,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
     ctx->batch = true;
     ctx->shifted_bp = false;
     ctx->walk = false;
+    ctx->pairs_given = false;
     ctx->allow_loose = false;
     ctx->cc_check = (desc->flags & MCGPU_DISPATCH_CHECK_COMPONENTS) != 0;
     ctx->npairs = np;
@@ -2306,6 +2295,7 @@ MCGPU_API mcgpu_result mcgpu_broad_phase(mcgpu_context ctx, const double* src_bo
     ctx->sort_bits = 22;
     ctx->trav = ctx->forced ? ctx->forced_trav : TravConfig{};
     ctx->walk = false;
+    ctx->pairs_given = false;
     ctx->nf[0] = num_src;
     ctx->nf[1] = num_cut;
     ctx->nv[0] = ctx->nv[1] = 0;
@@ -2339,7 +2329,6 @@ MCGPU_API mcgpu_result mcgpu_broad_phase(mcgpu_context ctx, const double* src_bo
     for (int attempt = 0; attempt < 6; ++attempt) {
         CK(ensure(ctx->raw_pairs, ctx->cap_pairs, &ull));
         CK(ensure(ctx->pairs, ctx->cap_pairs, &ull));
-        CK(ensure(ctx->phash, next_pow2(2 * ctx->cap_pairs), &ull));
         if (const mcgpu_result r = alloc_node_pairs(ctx); r != MCGPU_SUCCESS) return r;
         Counters* C = &st->C;
         (void)hipEventRecord(ctx->ev[EV_A0], s);
@@ -2355,13 +2344,10 @@ MCGPU_API mcgpu_result mcgpu_broad_phase(mcgpu_context ctx, const double* src_bo
                                                                   m ? (1u << 21) : 0u);
         }
         enqueue_bvh_traverse(ctx, s, C, false);
-        const uint64_t table = next_pow2(2 * ctx->cap_pairs);
-        k_pair_hash_init<<<grid_for(table, kBlock, 1024), kBlock, 0, s>>>(P_<unsigned long long>(ctx->phash), ctx->cap_pairs,
-                                                                          table, C);
         fill_u32(ctx->cand.p, 0u, F, s);
         k_filter_pairs<<<grid_for(ctx->cap_pairs, kFilterTile, 2048), kStageBlock, 0, s>>>(
             dp, P_<unsigned long long>(ctx->raw_pairs), ctx->cap_pairs, num_src, nullptr, P_<unsigned long long>(ctx->pairs),
-            P_<unsigned long long>(ctx->phash), P_<uint32_t>(ctx->cand), P_<uint32_t>(ctx->cand_list), 0, C);
+            nullptr, P_<uint32_t>(ctx->cand), P_<uint32_t>(ctx->cand_list), C);
         (void)hipEventRecord(ctx->ev[EV_A_END], s);
         CK(hipStreamSynchronize(s));
         CK(hipGetLastError());
@@ -2411,7 +2397,7 @@ MCGPU_API mcgpu_result mcgpu_redispatch_perturbed(mcgpu_context ctx, const doubl
         stage_event(ctx, EV_A_SHIFT, s);
         stage_event(ctx, EV_A_JOIN, s);
         stage_event(ctx, EV_A_FILTER, s);
-        enqueue_narrow(ctx, make_soup(ctx), false);
+        enqueue_narrow(ctx, make_soup(ctx), false, ctx->pairs_given ? kPairsGiven : kPairsMoved);
         bool overflow = false;
         if ((r = finish(ctx, info, &overflow)) != MCGPU_SUCCESS) return r;
         if (!overflow) return MCGPU_SUCCESS;
@@ -2971,6 +2957,7 @@ mcgpu_result slot_bind(mcgpu_server srv, mcgpu_context ctx, const mcgpu_mesh* cu
     ctx->broad_only = false;
     ctx->batch = false;
     ctx->walk = false;
+    ctx->pairs_given = false;
     ctx->cc_check = (srv->desc.flags & MCGPU_DISPATCH_CHECK_COMPONENTS) != 0;
     ctx->sort_bits = 22;
     ctx->flags = srv->desc.flags;
@@ -3294,23 +3281,21 @@ MCGPU_API mcgpu_result mcgpu_server_get_registry(mcgpu_server srv, uint32_t requ
 // the array (from module load until the process ends); its address is looked
 // up once per device with that device current and kept in g_scratch_ptr.
 // Every call on a device shares that device's array, and each call clears
-// what must start empty (counters, candidate-face flags, pair hash, the
+// what must start empty (counters, candidate-face flags, the
 // sort's group totals): calls that overlap on one device race.
 namespace {
 
 constexpr uint64_t kNaFaces = MCGPU_NOALLOC_MAX_FACES;         // per mesh
 constexpr uint64_t kNaF = 2 * kNaFaces;                        // both meshes
 constexpr uint64_t kNaPairs = MCGPU_NOALLOC_MAX_PAIRS;         // raw-space pairs
-constexpr uint64_t kNaTable = 2 * kNaPairs;                    // pair hash slots (a power of two)
 constexpr int kNaDepth = 16;                                   // leaf level of a tree of kNaFaces leaves
 static_assert((1ull << kNaDepth) == kNaFaces, "tree depth of the largest mesh");
-static_assert((kNaTable & (kNaTable - 1)) == 0, "pair hash size is a power of two");
 
 constexpr uint64_t na_align(uint64_t x) { return (x + 255) & ~255ull; }
 
 struct NaLayout {
     uint64_t state, box, rawbox, mcode, mface, mcode2, mface2, cand, cand_list, hist, scan, nodes0, nodes1, raw, pairs,
-        phash, total;
+        total;
 };
 
 constexpr NaLayout na_layout()
@@ -3338,7 +3323,6 @@ constexpr NaLayout na_layout()
     L.nodes1 = take(4 * 6 * ((2ull << kNaDepth) - 1));
     L.raw = take(8 * kNaPairs);
     L.pairs = take(8 * kNaPairs);
-    L.phash = take(8 * kNaTable);
     L.total = at;
     return L;
 }
@@ -3397,7 +3381,6 @@ MCGPU_API mcgpu_result mcgpu_broad_phase_noalloc(int device, const double* src_b
     uint32_t* cand = (uint32_t*)(base + kNa.cand);
     unsigned long long* raw = (unsigned long long*)(base + kNa.raw);
     unsigned long long* found = (unsigned long long*)(base + kNa.pairs);
-    unsigned long long* phash = (unsigned long long*)(base + kNa.phash);
 
     fill_u32(C, 0u, sizeof(Counters) / 4, s);
     if (hipMemcpyAsync(box, src_boxes, 48ull * num_src, hipMemcpyDeviceToDevice, s) != hipSuccess ||
@@ -3430,10 +3413,9 @@ MCGPU_API mcgpu_result mcgpu_broad_phase_noalloc(int device, const double* src_b
     B.cap_pairs = kNaPairs;
     B.sort_bits = 22;
     enqueue_trees_traverse(B, s, C, false, nullptr, nullptr);
-    k_pair_hash_init<<<grid_for(kNaTable, kBlock, 1024), kBlock, 0, s>>>(phash, kNaPairs, kNaTable, C);
     fill_u32(cand, 0u, F, s);
     k_filter_pairs<<<grid_for(kNaPairs, kFilterTile, 2048), kStageBlock, 0, s>>>(
-        box, raw, kNaPairs, num_src, nullptr, found, phash, cand, (uint32_t*)(base + kNa.cand_list), 0, C);
+        box, raw, kNaPairs, num_src, nullptr, found, nullptr, cand, (uint32_t*)(base + kNa.cand_list), C);
     Counters h;
     if (hipMemcpyAsync(&h, C, sizeof(Counters), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess || hipGetLastError() != hipSuccess)
@@ -3475,6 +3457,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_narrow(mcgpu_context ctx, const mcgpu_mesh
     ctx->batch = false;
     ctx->shifted_bp = false;
     ctx->walk = false;
+    ctx->pairs_given = true;
     ctx->allow_loose = false; // the caller's pairs: no broad phase runs here
     ctx->cc_check = false;
     ctx->sort_bits = 22;
@@ -3560,9 +3543,9 @@ MCGPU_API mcgpu_result mcgpu_dispatch_narrow(mcgpu_context ctx, const mcgpu_mesh
         k_filter_pairs<<<grid_for(ctx->cap_pairs, kFilterTile, 2048), kStageBlock, 0, s>>>(
             P_<double>(ctx->box), P_<unsigned long long>(ctx->raw_pairs), ctx->cap_pairs, Fs, nullptr,
             P_<unsigned long long>(ctx->pairs), P_<unsigned long long>(ctx->phash), P_<uint32_t>(ctx->cand),
-            P_<uint32_t>(ctx->cand_list), 0, C);
+            P_<uint32_t>(ctx->cand_list), C);
         stage_event(ctx, EV_A_FILTER, s);
-        enqueue_narrow(ctx, make_soup(ctx), false);
+        enqueue_narrow(ctx, make_soup(ctx), false, kPairsGiven);
         bool overflow = false;
         if ((r = finish(ctx, info, &overflow)) != MCGPU_SUCCESS) return r;
         if (!overflow) return MCGPU_SUCCESS;
