@@ -766,8 +766,8 @@ __global__ void k_edge_assign(const uint32_t* __restrict__ idx, CornerMap cm, ui
 }
 
 // The edge numbering without a table in memory.  Every corner's word (its
-// undirected edge, insertion rank and direction) is scattered into the bucket
-// its edge hashes to; a block then resolves one bucket in LDS and writes, for
+// undirected edge, insertion rank and direction) is scattered into a bucket
+// chosen by its edge; a block then resolves one bucket in LDS and writes, for
 // every corner, the rank of the edge's other corner (opp; kNoCorner on a
 // border); the first uses (no partner, or a later one) are counted per tile of
 // ranks, and the last pass numbers them by the prefix of those counts and
@@ -783,22 +783,27 @@ __global__ void k_edge_assign(const uint32_t* __restrict__ idx, CornerMap cm, ui
 // from 0.26 to 0.15 ms beside the other streams, on two of 1.3 M triangles from
 // 1.9 to 1.4 ms, on 320 uneven pairs (31 M corners) from 4.9 to 1.9 ms.
 //
-// Two levels of locality: vertex ids are grouped by 8 before they are hashed,
-// so the edges of a neighbourhood share a bucket and the block's stores to opp
-// meet in the same lines; and a segment (one mesh of one pair) has its own
-// buckets, so a batch's stores stay within the pair's.
+// A segment (one mesh of one pair) has its own buckets, so a batch's stores
+// stay within the pair's.  A bucket is a range of vertices (topo_range): meshes
+// are mostly numbered along their surface, a tile of corners then reaches few
+// buckets, and a bucket's stores to opp meet in the same lines (a subdivision-8
+// icosphere's tile reaches a fifth of the buckets, a grid's a hundredth).  Where
+// a range would hold too many words (k_topo_ranges counts them first), and in
+// small meshes, the edge's key is hashed instead, vertex ids grouped by 8 so
+// that the edges of a neighbourhood share a bucket.
 //
-// Words: the edge key is mixed by a bijection, whose top bits are the bucket,
-// so a word need not hold them: 2 vbits - bb key bits, kbits rank bits and the
-// direction fit 64 bits for any mesh the bucket limit admits (kTopoMaxBits).
+// Words: with ranges the vertex that chose the bucket by its low bits and the
+// other one; hashed, the key is mixed by a bijection, whose top bits are the
+// bucket, so a word need not hold them.  2 vbits - bb key bits (one more with
+// ranges), kbits rank bits and the direction fit 64 bits, or the mesh goes
+// without ranges, or to the hash tables (topo_plan).
 constexpr uint32_t kNoCorner = 0xffffffffu;
 constexpr int kTopoCapLog = 12;                    // words a bucket holds
 constexpr uint32_t kTopoCap = 1u << kTopoCapLog;
-constexpr uint32_t kTopoFillStride = 32;           // one counter per 128-byte line
 constexpr uint32_t kTopoFill = kTopoCap / 2;       // mean words of a bucket, at most: 4096 lies 6 sigma above
-constexpr int kTopoMaxBits = 12;                   // buckets a segment may have: 2^12 counters and a tile fill the LDS
+constexpr int kTopoMaxBits = 12;                   // buckets a segment may have: 16 KB of counters a scatter block
 constexpr int kTopoBlock = 512;
-constexpr int kTopoScatterBlock = 1024;
+constexpr int kTopoScatterBlock = 256, kTopoItems = 16; // corners of a scatter tile
 constexpr uint32_t kTopoTile = 4096;               // ranks per counting tile
 constexpr uint32_t kTopoDirectTiles = 2048;        // up to here a block sums the tiles before its own
 
@@ -811,6 +816,9 @@ struct TopoSeg {
     uint32_t bucket0;      // first bucket
     uint32_t tile0;        // first scatter tile (a segment of one bucket has none)
     uint8_t bb, vbits, kbits, m;
+    uint32_t inv; // buckets of vertex ranges: floor(2^(32 + bb) / vertices); 0: hashed buckets only
+    uint32_t nv;  // vertices
+    uint32_t id;  // its number (Topo::hashed)
 };
 
 struct TopoPart {
@@ -828,7 +836,10 @@ struct Topo {
     const TopoSeg* tab; // batches: the segments, in bucket order (null: seg)
     uint32_t nseg;
     unsigned long long* words;
-    uint32_t* fill; // words of each bucket, kTopoFillStride apart
+    uint32_t* fill;   // words of each bucket
+    uint32_t* rfill;  // words it would hold by vertex ranges
+    uint32_t* hashed; // per segment: a range holds too many; then: one of them does
+    int ranges;       // every segment of several buckets has ranges
 };
 
 // the corner whose insertion rank is r: a face's ranks are a permutation of
@@ -859,111 +870,160 @@ __device__ __forceinline__ TopoSeg topo_seg(const Topo& T, uint32_t x)
     return T.tab[__builtin_amdgcn_readfirstlane(lo)];
 }
 
-// corner c (of its part) as a word; its bucket within the segment in *bucket
-__device__ __forceinline__ unsigned long long topo_word(const TopoPart& P, const TopoSeg& g, uint64_t c, uint32_t* bucket)
+// corner q of a segment: its edge's vertices (of the mesh; a -> d) and its rank
+__device__ __forceinline__ void topo_corner(const TopoPart& P, const TopoSeg& g, uint32_t q, uint32_t* a, uint32_t* d,
+                                            uint32_t* rank)
 {
-    uint32_t f, b, n, i;
-    P.cm(c, f, b, n, i);
-    const uint32_t a = P.idx[c] - g.vb, d = P.idx[b + (i + 1 == n ? 0 : i + 1)] - g.vb;
-    const uint32_t rank = corner_rank(b, i, n, g.m) - (uint32_t)g.c0;
-    const uint64_t lo = a < d ? a : d, hi = a < d ? d : a;
-    const int gb = 2 * (g.vbits - 3);
-    const uint64_t gm = (1ull << gb) - 1;
-    uint64_t h = ((lo >> 3) << (g.vbits - 3) | (hi >> 3)) & gm; // two rounds of a bijection of gb-bit words
-    h = (h * 0x9e3779b97f4a7c15ull) & gm;
-    h ^= h >> (gb / 2);
-    h = (h * 0xd6e8feb86659fd93ull) & gm;
-    h ^= h >> (gb / 2);
-    *bucket = (uint32_t)(h >> (gb - g.bb));
-    const uint64_t rest = (h & ((1ull << (gb - g.bb)) - 1)) << 6 | (lo & 7) << 3 | (hi & 7);
+    uint32_t i, n = 3;
+    if (!P.cm.cface) {
+        i = q % 3;
+    } else {
+        uint32_t f, b;
+        P.cm(g.c0 + q, f, b, n, i);
+    }
+    const uint32_t b = q - i, nx = b + (i + 1 == n ? 0 : i + 1);
+    *a = P.idx[g.c0 + q] - g.vb;
+    *d = P.idx[g.c0 + nx] - g.vb;
+    *rank = corner_rank(b, i, n, g.m);
+}
+
+// An edge's bucket by vertex ranges: that of one of its ends, the lower for
+// every other edge so that vertices numbered before their neighbours (coarse
+// ones of a subdivision) do not fill theirs.
+__device__ __forceinline__ uint32_t topo_range(const TopoSeg& g, uint32_t a, uint32_t d, uint32_t* own, uint32_t* oth)
+{
+    const uint32_t lo = a < d ? a : d, hi = a < d ? d : a;
+    *own = (lo ^ hi) & 1 ? hi : lo;
+    *oth = (lo ^ hi) & 1 ? lo : hi;
+    return (uint32_t)(((uint64_t)*own * g.inv) >> 32);
+}
+
+// corner q of a segment as a word; its bucket in *bucket
+__device__ __forceinline__ unsigned long long topo_word(const TopoPart& P, const TopoSeg& g, uint32_t q, bool hashed,
+                                                        uint32_t* bucket)
+{
+    uint32_t a, d, rank;
+    topo_corner(P, g, q, &a, &d, &rank);
+    uint64_t rest;
+    if (!hashed) {
+        // a range spans at most 2^(vbits - bb) + 1 vertices: these low bits tell them apart
+        uint32_t own, oth;
+        *bucket = topo_range(g, a, d, &own, &oth);
+        rest = (uint64_t)(own & ((2u << (g.vbits - g.bb)) - 1)) << g.vbits | oth;
+    } else {
+        const uint64_t lo = a < d ? a : d, hi = a < d ? d : a;
+        const int gb = 2 * (g.vbits - 3);
+        const uint64_t gm = (1ull << gb) - 1;
+        uint64_t h = ((lo >> 3) << (g.vbits - 3) | (hi >> 3)) & gm; // two rounds of a bijection of gb-bit words
+        h = (h * 0x9e3779b97f4a7c15ull) & gm;
+        h ^= h >> (gb / 2);
+        h = (h * 0xd6e8feb86659fd93ull) & gm;
+        h ^= h >> (gb / 2);
+        *bucket = (uint32_t)(h >> (gb - g.bb));
+        rest = (h & ((1ull << (gb - g.bb)) - 1)) << 6 | (lo & 7) << 3 | (hi & 7);
+    }
     return rest << (g.kbits + 1) | (uint64_t)rank << 1 | (a < d ? 1u : 0u);
 }
 
-// word p of bucket b: buckets fill at the same pace, and with all of them
-// starting on a 32 KB boundary the words written at one time would meet in the
-// same memory channels, so each bucket is rotated by a number of lines of its own
+// word p of bucket b: buckets are read and filled at the same pace, and with all
+// of them starting on a 32 KB boundary the words in use at one time would meet
+// in the same memory channels, so each bucket is rotated by lines of its own
 __device__ __forceinline__ unsigned long long* topo_at(const Topo& T, const TopoSeg& g, uint32_t b, uint32_t p)
 {
     return T.words + g.w0 + ((uint64_t)b << kTopoCapLog) + ((p + b * (163u * 16u)) & (kTopoCap - 1));
 }
 
-// One tile of a segment's corners into its buckets: places within the tile by
-// LDS atomics, one global reservation per bucket the tile reaches, and the
-// tile's words put in bucket order in LDS, so that a group of lanes writes each
-// bucket's run to consecutive addresses (one word a lane and bucket instead
-// reached 64 pages a wave: 8 words/ns on a 1.3 M triangle mesh).  The order
-// within a bucket does not matter.  A word past a full bucket is dropped and
-// flagged (the host runs the dispatch again with the hash tables); its corner
-// counts as a border meanwhile.
-template <int ITEMS, int BITS>
-__global__ void __launch_bounds__(kTopoScatterBlock) k_topo_scatter(Topo T, Counters* C)
+// Words each vertex range would hold; a segment with one past a bucket's
+// capacity (a vertex of thousands of faces) uses the hashed buckets.
+template <int BITS>
+__global__ void __launch_bounds__(kTopoScatterBlock) k_topo_ranges(Topo T)
 {
-    __shared__ unsigned long long stage[kTopoScatterBlock * ITEMS];
-    __shared__ uint32_t cnt[1 << BITS];   // words of the tile in each bucket, then their place in the bucket
-    __shared__ uint16_t start[1 << BITS]; // their place in the tile
-    __shared__ uint32_t wsum[kTopoScatterBlock / 64];
+    __shared__ uint32_t cnt[1 << BITS];
     const TopoSeg g = topo_seg<true>(T, blockIdx.x);
+    if (!g.inv) return; // whole block
     const TopoPart& P = T.part[g.m];
     const uint32_t nb = 1u << g.bb;
-    constexpr uint32_t kTile = kTopoScatterBlock * ITEMS;
     for (uint32_t q = threadIdx.x; q < nb; q += kTopoScatterBlock) cnt[q] = 0u;
     __syncthreads();
-    const uint32_t q0 = (blockIdx.x - g.tile0) * kTile, t0 = q0 + threadIdx.x;
-    unsigned long long w[ITEMS];
-    uint32_t bk[ITEMS], pos[ITEMS];
+    const uint32_t t0 = (blockIdx.x - g.tile0) * (kTopoScatterBlock * kTopoItems) + threadIdx.x;
+    uint32_t bk[kTopoItems];
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
+    for (int j = 0; j < kTopoItems; ++j) {
         const uint32_t q = t0 + j * kTopoScatterBlock;
-        bk[j] = 0;
-        w[j] = q < g.k ? topo_word(P, g, g.c0 + q, &bk[j]) : 0ull;
+        uint32_t a, d, rank, own, oth;
+        topo_corner(P, g, q < g.k ? q : 0u, &a, &d, &rank);
+        bk[j] = topo_range(g, a, d, &own, &oth);
     }
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j)
-        pos[j] = t0 + j * kTopoScatterBlock < g.k ? atomicAdd(&cnt[bk[j]], 1u) : 0u;
+    for (int j = 0; j < kTopoItems; ++j)
+        if (t0 + j * kTopoScatterBlock < g.k) atomicAdd(&cnt[bk[j]], 1u);
     __syncthreads();
-    // exclusive scan of the counts: thread t takes `per` consecutive buckets
-    const uint32_t per = nb > kTopoScatterBlock ? nb / kTopoScatterBlock : 1, b0 = threadIdx.x * per;
-    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    uint32_t own = 0;
-    if (b0 < nb)
-        for (uint32_t q = 0; q < per; ++q) own += cnt[b0 + q];
-    uint32_t x = own;
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = __shfl_up(x, o, 64);
-        if (lane >= (uint32_t)o) x += y;
+    for (uint32_t q = threadIdx.x; q < nb; q += kTopoScatterBlock) {
+        const uint32_t c = cnt[q];
+        if (c && atomicAdd(&T.rfill[g.bucket0 + q], c) + c > kTopoCap) T.hashed[g.id] = T.hashed[T.nseg] = 1u;
     }
-    if (lane == 63) wsum[wid] = x;
-    __syncthreads();
-    x -= own;
-    for (uint32_t q = 0; q < wid; ++q) x += wsum[q];
-    if (b0 < nb)
-        for (uint32_t q = 0; q < per; ++q) {
-            const uint32_t c = cnt[b0 + q];
-            start[b0 + q] = (uint16_t)x; // at most kTile <= 2^14
-            x += c;
-            if (c) cnt[b0 + q] = atomicAdd(&T.fill[(uint64_t)(g.bucket0 + b0 + q) * kTopoFillStride], c);
+}
+
+// One tile of a segment's corners into its buckets: places within the tile by
+// LDS atomics, then one global reservation per bucket the tile reaches.  The
+// order within a bucket does not matter.  A word past a full bucket is dropped
+// and flagged (the host runs the dispatch again with the hash tables); its
+// corner counts as a border meanwhile.
+//
+// Small blocks: one of 1,024 threads and 152 KB of LDS (16,384 corners, 42 us
+// with hashed buckets, half of it the words' 64-bit products, a third the
+// stores of 4,096 runs of four words) found room only where a whole compute
+// unit fell idle, beside streams whose blocks are small: 0.35-0.41 ms for two
+// meshes of 1.3 M triangles, 0.54 ms for a terrain pair, against 0.10 and
+// 0.15 ms (and 0.05-0.07 for the ranges' counts).
+template <bool HASHED, int BITS>
+__global__ void __launch_bounds__(kTopoScatterBlock) k_topo_scatter(Topo T, uint32_t tiles, Counters* C)
+{
+    __shared__ uint32_t cnt[1 << BITS]; // words of the tile in each bucket, then their place in the bucket
+    if (HASHED && T.ranges && !T.hashed[T.nseg]) return; // no segment is hashed
+    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const TopoSeg g = topo_seg<true>(T, tile);
+        if (HASHED != (!g.inv || T.hashed[g.id])) continue; // whole block
+        const TopoPart& P = T.part[g.m];
+        const uint32_t nb = 1u << g.bb;
+        for (uint32_t q = threadIdx.x; q < nb; q += kTopoScatterBlock) cnt[q] = 0u;
+        __syncthreads();
+        const uint32_t t0 = (tile - g.tile0) * (kTopoScatterBlock * kTopoItems) + threadIdx.x;
+        unsigned long long w[kTopoItems];
+        uint32_t at[kTopoItems]; // bucket, and the place within the tile's words there (at most the tile, 2^12)
+#pragma unroll
+        for (int j = 0; j < kTopoItems; ++j) {
+            const uint32_t q = t0 + j * kTopoScatterBlock;
+            w[j] = topo_word(P, g, q < g.k ? q : 0u, HASHED, &at[j]);
         }
-    __syncthreads();
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j)
-        if (t0 + j * kTopoScatterBlock < g.k) stage[start[bk[j]] + pos[j]] = w[j];
-    __syncthreads();
-    const uint32_t ntile = g.k - q0 < kTile ? g.k - q0 : kTile;
-    uint32_t width = 8; // lanes a run: about its mean length
-    while (width < 64 && width * nb < kTile) width <<= 1;
-    const uint32_t l = threadIdx.x & (width - 1), groups = kTopoScatterBlock / width;
-    for (uint32_t b = threadIdx.x / width; b < nb; b += groups) {
-        const uint32_t s0 = start[b], s1 = b + 1 < nb ? start[b + 1] : ntile, to = cnt[b];
-        for (uint32_t i = s0 + l; i < s1; i += width) {
-            const uint32_t p = to + (i - s0);
-            const unsigned long long v = stage[i];
+        for (int j = 0; j < kTopoItems; ++j)
+            if (t0 + j * kTopoScatterBlock < g.k) at[j] |= atomicAdd(&cnt[at[j]], 1u) << BITS;
+        __syncthreads();
+        for (uint32_t q0 = threadIdx.x; q0 < nb; q0 += 4 * kTopoScatterBlock) {
+            uint32_t c[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) c[q] = q0 + q * kTopoScatterBlock < nb ? cnt[q0 + q * kTopoScatterBlock] : 0u;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (c[q]) c[q] = atomicAdd(&T.fill[g.bucket0 + q0 + q * kTopoScatterBlock], c[q]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (q0 + q * kTopoScatterBlock < nb) cnt[q0 + q * kTopoScatterBlock] = c[q];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kTopoItems; ++j) {
+            if (t0 + j * kTopoScatterBlock >= g.k) continue;
+            const uint32_t b = at[j] & ((1u << BITS) - 1), p = cnt[b] + (at[j] >> BITS);
             if (p < kTopoCap) {
-                *topo_at(T, g, b, p) = v;
+                *topo_at(T, g, b, p) = w[j];
             } else {
-                P.opp[g.c0 + ((v >> 1) & ((1ull << g.kbits) - 1))] = kNoCorner;
+                P.opp[g.c0 + ((w[j] >> 1) & ((1ull << g.kbits) - 1))] = kNoCorner;
                 C->ov_topo = 1u;
             }
         }
+        __syncthreads(); // cnt is the next tile's
     }
 }
 
@@ -979,7 +1039,7 @@ __global__ void __launch_bounds__(kTopoBlock) k_topo_buckets(Topo T, Counters* C
     const TopoSeg g = topo_seg<false>(T, blockIdx.x);
     const TopoPart& P = T.part[g.m];
     const uint32_t bkt = blockIdx.x - g.bucket0;
-    uint32_t n = g.bb ? T.fill[(uint64_t)blockIdx.x * kTopoFillStride] : g.k;
+    uint32_t n = g.bb ? T.fill[blockIdx.x] : g.k;
     if (n > kTopoCap) n = kTopoCap;
     if (n == 0) return; // whole block
     unsigned long long w[kPer];
@@ -990,7 +1050,7 @@ __global__ void __launch_bounds__(kTopoBlock) k_topo_buckets(Topo T, Counters* C
         uint32_t b;
         w[j] = kEmpty64;
         if (q < n)
-            w[j] = g.bb ? *topo_at(T, g, bkt, q) : topo_word(P, g, g.c0 + q, &b);
+            w[j] = g.bb ? *topo_at(T, g, bkt, q) : topo_word(P, g, q, true, &b);
     }
     for (uint32_t q = threadIdx.x; q < kTopoCap; q += kTopoBlock) {
         slot[q] = kEmpty64;

@@ -168,7 +168,8 @@ struct mcgpu_context_t {
     TopoSeg topo_seg[2] = {};
     std::vector<TopoSeg> hseg;       // a batch's segments
     uint32_t nseg = 0, topo_buckets = 0, topo_tiles = 0;
-    int topo_items = 4;
+    int topo_bits = 8;
+    bool topo_ranges = false;        // every mesh of several buckets may use vertex ranges
     uint64_t topo_words = 0;
     bool topo_hash = false;          // the hash tables number this dispatch's edges (no buckets for it, or one overflowed)
     bool topo_given = false;         // the caller's edge numbering (mcgpu_dispatch_narrow)
@@ -434,18 +435,20 @@ bool topo_plan(mcgpu_context ctx)
             if (ctx->ncorner[m] > 0xffffffffull) return false;
             seg[m - m0] = TopoSeg{};
             seg[m - m0].k = (uint32_t)ctx->ncorner[m];
+            seg[m - m0].nv = ctx->nv[m];
             seg[m - m0].vbits = (uint8_t)std::max(8, bits_for(ctx->nv[m]));
             seg[m - m0].m = (uint8_t)m;
         }
     }
     uint32_t kmax = 0;
     for (uint32_t i = 0; i < ctx->nseg; ++i) kmax = std::max(kmax, seg[i].k);
-    // corners a scatter block takes, a thread: the runs a block writes are tile /
-    // buckets words long, and the blocks in flight fall with the tile; the
-    // template's bucket limit (8, 10, 12 bits) holds for each range
-    ctx->topo_items = kmax <= (kTopoFill << 8) ? 4 : kmax <= (kTopoFill << 10) ? 8 : 16;
-    const uint32_t tile = kTopoScatterBlock * ctx->topo_items;
+    // counters of a scatter block: 1, 4 or 16 KB of LDS.  Meshes of at most 256
+    // buckets keep to the hash: their words stay in the caches, and counting the
+    // ranges first would cost what they save.
+    ctx->topo_bits = kmax <= (kTopoFill << 8) ? 8 : kmax <= (kTopoFill << 10) ? 10 : kTopoMaxBits;
+    constexpr uint32_t tile = kTopoScatterBlock * kTopoItems;
     uint64_t words = 0, buckets = 0, tiles = 0;
+    ctx->topo_ranges = true;
     for (uint32_t i = 0; i < ctx->nseg; ++i) {
         TopoSeg& g = seg[i];
         int bb = 0;
@@ -457,6 +460,12 @@ bool topo_plan(mcgpu_context ctx)
         g.bucket0 = (uint32_t)buckets;
         g.tile0 = (uint32_t)tiles;
         g.w0 = words;
+        g.id = i;
+        // buckets of vertex ranges: fewer than vertices, and a word has a bit more
+        g.inv = 0;
+        if (ctx->topo_bits > 8 && bb && (g.nv >> bb) && 2 * g.vbits - bb + g.kbits + 2 <= 64)
+            g.inv = (uint32_t)(((uint64_t)1 << (32 + bb)) / g.nv);
+        if (bb && !g.inv) ctx->topo_ranges = false;
         buckets += 1ull << bb;
         if (bb) {
             tiles += ((uint64_t)g.k + tile - 1) / tile;
@@ -485,6 +494,9 @@ mcgpu_result alloc_edge_tables(mcgpu_context ctx)
     CK(ensure(ctx->scan_tmp_c, scan_tmp_elems(std::max(ctx->ncorner[0], ctx->ncorner[1]) + 8) + 1024, &u));
     return MCGPU_SUCCESS;
 }
+
+// the edge numbering's counters behind the candidate-face flags: two a bucket, one a segment, one
+uint64_t topo_counters(mcgpu_context ctx) { return ctx->topo_hash ? 0 : 2ull * ctx->topo_buckets + ctx->nseg + 1; }
 
 uint32_t topo_rank_tiles(uint64_t corners) { return (uint32_t)((corners + kTopoTile - 1) / kTopoTile); }
 
@@ -529,7 +541,7 @@ mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
     CK(ensure(ctx->mface2, F, &u));
     scan_need = std::max<uint64_t>(scan_need, scan_tmp_elems(F + 8));
     // the candidate-face flags and, behind them, the buckets' word counts (cleared together)
-    CK(ensure(ctx->cand, F + 8 + (ctx->topo_hash ? 0 : (uint64_t)kTopoFillStride * ctx->topo_buckets), &u));
+    CK(ensure(ctx->cand, F + 8 + topo_counters(ctx), &u));
     CK(ensure(ctx->cand_list, F + 8, &u));
     Plane* pl;
     CK(ensure(ctx->planes, F, &pl));
@@ -1156,7 +1168,7 @@ void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
     stage_event(ctx, EV_C0, s3);
     uint32_t* etotal = P_<uint32_t>(ctx->etotal);
     const uint64_t K = ctx->ncorner[0] + ctx->ncorner[1];
-    fill_u32(ctx->cand.p, 0u, F + 8 + (ctx->topo_hash ? 0 : (uint64_t)kTopoFillStride * ctx->topo_buckets), s3);
+    fill_u32(ctx->cand.p, 0u, F + 8 + topo_counters(ctx), s3);
     ev_record(ctx, EV_C_FILL, s3);
     const uint32_t res_ne = ctx->res ? ctx->res->ne : 0u;
     if (ctx->res) { // the resident source's edges occupy [0, ne) of the edge table
@@ -1185,11 +1197,25 @@ void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
         T.tab = ctx->batch ? P_<TopoSeg>(ctx->tseg) : nullptr;
         T.words = P_<unsigned long long>(ctx->twords);
         T.fill = P_<uint32_t>(ctx->cand) + F + 8;
+        T.rfill = T.fill + ctx->topo_buckets;
+        T.hashed = T.rfill + ctx->topo_buckets;
+        T.ranges = ctx->topo_ranges;
         if (ctx->topo_tiles) {
-            const dim3 g(ctx->topo_tiles), b(kTopoScatterBlock);
-            if (ctx->topo_items == 4) k_topo_scatter<4, 8><<<g, b, 0, s3>>>(T, C);
-            else if (ctx->topo_items == 8) k_topo_scatter<8, 10><<<g, b, 0, s3>>>(T, C);
-            else k_topo_scatter<16, 12><<<g, b, 0, s3>>>(T, C);
+            const uint32_t n = ctx->topo_tiles;
+            const dim3 g(n), b(kTopoScatterBlock);
+            // a few blocks look whether a segment is hashed: most dispatches have none
+            const dim3 gh(ctx->topo_ranges ? std::min<uint32_t>(n, 2 * ctx->ncu) : n);
+            if (ctx->topo_bits == 8) {
+                k_topo_scatter<true, 8><<<gh, b, 0, s3>>>(T, n, C);
+            } else if (ctx->topo_bits == 10) {
+                k_topo_ranges<10><<<g, b, 0, s3>>>(T);
+                k_topo_scatter<false, 10><<<g, b, 0, s3>>>(T, n, C);
+                k_topo_scatter<true, 10><<<gh, b, 0, s3>>>(T, n, C);
+            } else {
+                k_topo_ranges<kTopoMaxBits><<<g, b, 0, s3>>>(T);
+                k_topo_scatter<false, kTopoMaxBits><<<g, b, 0, s3>>>(T, n, C);
+                k_topo_scatter<true, kTopoMaxBits><<<gh, b, 0, s3>>>(T, n, C);
+            }
         }
         k_topo_buckets<<<ctx->topo_buckets, kTopoBlock, 0, s3>>>(T, C);
         const int cut_only = ctx->res ? 1 : 0;
@@ -1580,7 +1606,7 @@ std::vector<uint64_t> graph_key(mcgpu_context ctx)
     auto put = [&k](uint64_t x) { k.push_back(x); };
     auto ptr = [&k](const void* p) { k.push_back((uint64_t)(uintptr_t)p); };
     put(ctx->batch), put(ctx->npairs), put(ctx->batch_mb), put(ctx->cc_check), put(ctx->sort_bits),
-        put(ctx->shifted_bp), put(ctx->walk), put(ctx->trav.walk), put(ctx->cap_nodes), put(ctx->topo_hash), put(ctx->topo_buckets), put(ctx->topo_tiles), put(ctx->topo_items),
+        put(ctx->shifted_bp), put(ctx->walk), put(ctx->trav.walk), put(ctx->cap_nodes), put(ctx->topo_hash), put(ctx->topo_buckets), put(ctx->topo_tiles), put(ctx->topo_bits),
         put(ctx->nseg),
         put(ctx->gbits), put(ctx->kbits);
     for (int m = 0; m < 2; ++m) {
@@ -2173,6 +2199,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
             g.c0 = c0;
             g.k = (uint32_t)k;
             g.vb = vo[m][p];
+            g.nv = vo[m][p + 1] - vo[m][p];
             g.vbits = (uint8_t)std::max(8, bits_for(vo[m][p + 1] - vo[m][p]));
             g.m = (uint8_t)m;
             ctx->hseg.push_back(g);

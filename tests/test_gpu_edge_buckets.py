@@ -89,3 +89,38 @@ def test_overflowing_bucket_falls_back_to_the_tables(ctx):
     R, O = compare(ctx, src, cut)
     compare(ctx, *meshes.icosphere_pair(4))  # the next dispatch numbers its edges by buckets again
     compare(ctx, cut, src)
+
+
+def fans(rings, hub):
+    """A closed double fan over each ring of vertices: two hubs a ring, every
+    other vertex on four faces."""
+    V, F = [], []
+    base = 0
+    for r in rings:
+        t = np.linspace(0, 2 * np.pi, r, endpoint=False)
+        ring = np.stack([np.cos(t), np.sin(t), 0 * t], 1) + [0, 0, 3.0 * len(V)]
+        ends = np.array([[0, 0, -1.0], [0, 0, 1.0]]) + [0, 0, 3.0 * len(V)]
+        i = np.arange(r)
+        if hub == "first":
+            V.append(np.vstack([ends, ring]))
+            lo, hi, o = base, base + 1, base + 2
+        else:
+            V.append(np.vstack([ring, ends]))
+            lo, hi, o = base + r, base + r + 1, base
+        F.append(np.stack([o + i, o + (i + 1) % r, 0 * i + hi], 1))
+        F.append(np.stack([o + (i + 1) % r, o + i, 0 * i + lo], 1))
+        base += r + 2
+    return np.vstack(V), np.concatenate(F).astype(np.uint32).ravel(), None
+
+
+@pytest.mark.parametrize("hub", ["first", "last"])
+@pytest.mark.parametrize("rings", [[100000], [3000] * 40, [700] * 200])
+def test_vertices_of_many_faces(ctx, rings, hub):
+    # past 2^19 corners the buckets are vertex ranges unless one holds too much:
+    # a hub of 100,000 or 3,000 faces does (hashed buckets), of 700 does not
+    src = fans(rings, hub)
+    cut = blade(1.0)
+    compare(ctx, src, cut, detail=False)
+    R = ctx.dispatch(src, cut)
+    v0, v1, f0, f1 = R.edges()
+    assert v0.size == 3 * sum(rings) + 33 and int((f1 < 0).sum()) == 12
