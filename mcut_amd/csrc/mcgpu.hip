@@ -39,16 +39,17 @@ struct Buf {
 // build's small launches queue behind the edge numbering's large hash grids
 // and the sort stretches from 0.12 to 0.25 ms.  B takes kBroadShare of the
 // CUs left after the sums (174 of 248 on the 256-CU part): it is the longest
-// of the three paths, and the edge numbering finishes well inside it.  A joins B before the exact pair filter and
-// C before the edge-face tests.  A batch runs on a second pair of streams
-// kBatchBroadShare : rest (mcgpu_set_batch_split before the first batch):
-// its edge numbering runs over every pair's corners and is its longest path
-// (a 4096-pair batch: 80.2 ms at 0.46, 81.7 ms at 0.40, 85.8 ms at 0.52,
-// 86.1 ms at 0.58).  The pair is made on a context's first batch, so a
-// context that never batches holds four hardware queues.
+// of the three paths up to a subdivision-7 icosphere pair (0.464 ms with 0.70,
+// 0.486 with 0.65; on two meshes of 1.3 M triangles 1.47 and 1.50).  A joins B
+// before the exact pair filter and C before the edge-face tests.  A batch runs
+// on the same streams: with a pair of its own (for another split,
+// mcgpu_set_batch_split before the first batch) the context holds six hardware
+// queues, some of which then share one of the device's four pipes, and a large
+// grid being placed holds up the kernels of the other queue (96 small pairs:
+// 0.54 ms, with six queues 0.89).
 constexpr int kSumCUs = 8;
 constexpr double kBroadShare = 0.70;
-constexpr double kBatchBroadShare = 0.46;
+constexpr double kBatchBroadShare = kBroadShare;
 constexpr uint32_t kBatchSumWaves = 128; // persistent waves of the batched serial sums (on the reserved CUs)
 enum Stage {
     ST_SUMS,      // A: coordinate sums
@@ -1749,6 +1750,17 @@ MCGPU_API const char* mcgpu_result_string(mcgpu_result r)
     return "unknown";
 }
 
+// Stream A: a mask of every CU, which gives it a hardware queue of its own like
+// the other three.  On a queue of the runtime's pool its kernels waited while
+// a large grid of stream C was being placed (a one-thread kernel for 0.33 ms
+// on two 1.3 M triangle meshes, the whole dispatch 1.69 ms against 1.47).
+static hipError_t create_full_stream(int ncu, hipStream_t* s)
+{
+    std::vector<uint32_t> m((ncu + 31) / 32, 0u);
+    for (int i = 0; i < ncu; ++i) m[i / 32] |= 1u << (i % 32);
+    return hipExtStreamCreateWithCUMask(s, (uint32_t)m.size(), m.data());
+}
+
 // Streams B and C of a dispatch: disjoint CU sets outside the first kSumCUs,
 // B taking `share` of them; a device too small to partition gets no masks.
 static hipError_t create_split_streams(int ncu, double share, hipStream_t* b, hipStream_t* c)
@@ -1794,8 +1806,14 @@ static mcgpu_tuning tuning_report(const TravConfig& t, int pct)
 // default.  Batches get their stream pair on the context's first batch.
 static mcgpu_result apply_tuning(mcgpu_context ctx)
 {
-    if (ctx->batch && ctx->own_streams && !ctx->s2b)
-        CK(create_split_streams(ctx->ncu, ctx->batch_share_pct / 100.0, &ctx->s2b, &ctx->s3b));
+    if (ctx->batch && ctx->own_streams && !ctx->s2b) {
+        if (ctx->batch_share_pct == (int)(kBroadShare * 100.0 + 0.5)) { // the single pairs' streams have this split
+            ctx->s2b = ctx->s2;
+            ctx->s3b = ctx->s3;
+        } else {
+            CK(create_split_streams(ctx->ncu, ctx->batch_share_pct / 100.0, &ctx->s2b, &ctx->s3b));
+        }
+    }
     TravConfig t;
     const TuneEntry* hit = nullptr;
     if (ctx->forced) {
@@ -1968,7 +1986,7 @@ MCGPU_API mcgpu_result mcgpu_create_context(int device, mcgpu_context* out)
     ctx->device = device;
     hipDeviceProp_t prop;
     if (hipSetDevice(device) != hipSuccess || hipGetDeviceProperties(&prop, device) != hipSuccess ||
-        hipStreamCreateWithFlags(&ctx->s, hipStreamNonBlocking) != hipSuccess) {
+        create_full_stream(prop.multiProcessorCount, &ctx->s) != hipSuccess) {
         delete ctx;
         return MCGPU_ERROR_DEVICE;
     }
@@ -2009,6 +2027,7 @@ MCGPU_API mcgpu_result mcgpu_release_context(mcgpu_context ctx)
     for (int i = 0; i < EV_COUNT; ++i) (void)hipEventDestroy(ctx->ev[i]);
     if (ctx->ev_user) (void)hipEventDestroy(ctx->ev_user);
     if (ctx->own_streams) {
+        if (ctx->s2b == ctx->s2) ctx->s2b = ctx->s3b = nullptr;
         for (hipStream_t st : {ctx->ssum, ctx->s3, ctx->s2, ctx->s3b, ctx->s2b})
             if (st) (void)hipStreamDestroy(st);
     }
