@@ -2269,9 +2269,10 @@ struct PairStage {
 // 256 source nodes, one a thread, against 32 cut nodes in LDS, the outcomes
 // kept as one mask (a stage in LDS cost an atomic per test with a survivor:
 // 30 us for 1,280 x 1,280 nodes
-// where this takes 14)
+// where this takes 14).  With the face boxes in place of nodes (one level) it
+// tests all faces of two meshes.
 __global__ void __launch_bounds__(256) k_pairs_start(Tree src, Tree cut, int s0, int c0, unsigned long long* __restrict__ out,
-                                                     uint64_t cap, unsigned long long* n, Counters* C)
+                                                     uint64_t cap, unsigned long long* n, unsigned int* over)
 {
     __shared__ float cb[32][8];
     __shared__ uint32_t wsum[4];
@@ -2304,7 +2305,7 @@ __global__ void __launch_bounds__(256) k_pairs_start(Tree src, Tree cut, int s0,
         tot += wsum[q];
     }
     unsigned long long at = block_reserve(n, tot, &base) + off + incl - __popc(hits);
-    if (at + __popc(hits) > cap) C->ov_nodes = 1u;
+    if (at + __popc(hits) > cap) *over = 1u;
     for (; hits; hits &= hits - 1, ++at)
         if (at < cap) out[at] = (uint64_t)s << 32 | (c1 + (uint32_t)__builtin_ctz(hits));
 }

@@ -180,6 +180,8 @@ struct mcgpu_context_t {
     Buf node_pairs[2];
     uint64_t cap_nodes = 0;
     bool pairs_given = false;        // the caller gave this dispatch's pairs (mcgpu_dispatch_narrow)
+    bool one_stream = false;         // this dispatch runs on stream A alone
+    bool want_trees = false;         // trees also for meshes that tests_all_pairs would take
     bool walk = false;               // this dispatch walks the cut tree: its node-pair lists outgrew their buffers
     Buf raw_pairs, pairs, phash, cand, cand_list, planes, big_list, big_off, big_scratch;
     Buf te, tg, tqs, trs, ttype, tpip, esc;
@@ -704,6 +706,10 @@ void graph_cut(mcgpu_context ctx, hipStream_t st)
 
 void ev_record(mcgpu_context ctx, int e, hipStream_t st)
 {
+    if (ctx->one_stream && e != EV_A0 && e != EV_A_END) { // no other stream waits
+        stage_event(ctx, e, st);
+        return;
+    }
     if (!ctx->recording) {
         (void)hipEventRecord(ctx->ev[e], st);
         return;
@@ -714,6 +720,7 @@ void ev_record(mcgpu_context ctx, int e, hipStream_t st)
 
 void ev_wait(mcgpu_context ctx, hipStream_t st, int e)
 {
+    if (ctx->one_stream) return;
     if (!ctx->recording) {
         (void)hipStreamWaitEvent(st, ctx->ev[e], 0);
         return;
@@ -1001,7 +1008,7 @@ void launch_node_pairs(const BroadView& B, const Tree& src, const Tree& cut, Cou
     int ls = std::min(ts, kPairStartLevel), lc = std::min(tc, kPairStartLevel), step = 0;
     const dim3 g0((level_nodes(src.n, src.D, ls) + 255) / 256, (level_nodes(cut.n, cut.D, lc) + 31) / 32);
     launch_timed(k_pairs_start, g0, dim3(256), st, a, (hipEvent_t) nullptr, src, cut, ls, lc, B.node_pairs[0], B.cap_nodes,
-                 &C->n_nodes[0], C);
+                 &C->n_nodes[0], &C->ov_nodes);
     for (; ls < ts || lc < tc; ++step) {
         const int es = std::min(kPairStep, ts - ls), ec = std::min(kPairStep, tc - lc);
         k_pairs_expand<<<512, kPairBlock, 0, st>>>(src, cut, ls, lc, es, ec, B.node_pairs[step & 1], &C->n_nodes[step],
@@ -1011,6 +1018,39 @@ void launch_node_pairs(const BroadView& B, const Tree& src, const Tree& cut, Cou
     }
     launch_timed(k_pairs_leaves, dim3(1024), dim3(kPairBlock), st, (hipEvent_t) nullptr, b, src, cut, ls, lc,
                  B.node_pairs[step & 1], &C->n_nodes[step], B.cap_nodes, B.raw_pairs, B.cap_pairs, C);
+}
+
+// Two meshes of few faces: every pair of face boxes tested, without trees.
+// Two launches where the trees take 11 to 16, each of which costs the host
+// 4-5 us and its successor 5-10 us; 53M tests take 27 us, 65k 8-12.
+constexpr uint64_t kAllPairs = 1ull << 26;
+bool tests_all_pairs(mcgpu_context ctx)
+{
+    return ctx->own_streams && !ctx->batch && !ctx->forced && !ctx->trav.walk && !ctx->want_trees &&
+           (uint64_t)ctx->nf[0] * ctx->nf[1] <= kAllPairs;
+}
+
+// One stream for a pair whose kernels are all shorter than a launch and than
+// the 5-10 us that a wait across streams takes (960 against 192 faces: 0.25 ms
+// with four streams, 0.21 with one; 2^14 to 2^16 faces: no gain).
+constexpr uint64_t kOneStream = 1ull << 13; // faces
+bool uses_one_stream(mcgpu_context ctx)
+{
+    return tests_all_pairs(ctx) && !ctx->sum_items && (uint64_t)ctx->nf[0] + ctx->nf[1] <= kOneStream;
+}
+
+void launch_all_pairs(mcgpu_context ctx, hipStream_t st, Counters* C)
+{
+    const bool t = ctx->stage_timing, kt = t || ctx->kernel_timing;
+    stage_event(ctx, EV_B_SORT, st);
+    stage_event(ctx, EV_B_REFIT, st);
+    Tree T[2];
+    for (int m = 0; m < 2; ++m)
+        T[m] = Tree{nullptr, P_<float>(ctx->rawbox) + (m ? 6ull * ctx->nf[0] : 0), (int)ctx->nf[m], 0};
+    const dim3 g((ctx->nf[0] + 255) / 256, (ctx->nf[1] + 31) / 32);
+    launch_timed(k_pairs_start, g, dim3(256), st, kt ? ctx->ev[EV_TRAV_K0] : nullptr, kt ? ctx->ev[EV_TRAV_K1] : nullptr, T[0],
+                 T[1], 0, 0, P_<unsigned long long>(ctx->raw_pairs), ctx->cap_pairs, &C->n_raw, &C->ov_pairs);
+    ev_record(ctx, EV_B_TRAV, st);
 }
 
 // the steps of launch_node_pairs fit Counters::n_nodes for any tree of 32-bit leaves
@@ -1280,7 +1320,8 @@ void enqueue_cc_rounds(mcgpu_context ctx, hipStream_t st)
 
 void enqueue_frontend(mcgpu_context ctx)
 {
-    hipStream_t s = ctx->s, s2 = ctx->batch ? ctx->s2b : ctx->s2, s3 = ctx->batch ? ctx->s3b : ctx->s3;
+    hipStream_t s = ctx->s, s2 = ctx->batch ? ctx->s2b : ctx->s2, s3 = ctx->batch ? ctx->s3b : ctx->s3, ssum = ctx->ssum;
+    if (ctx->one_stream) s2 = s3 = ssum = s;
     const uint32_t Fs = ctx->nf[0];
     const uint64_t F = (uint64_t)Fs + ctx->nf[1], V = (uint64_t)ctx->nv[0] + ctx->nv[1];
     Counters* C = &P_<DevState>(ctx->state)->C;
@@ -1292,10 +1333,10 @@ void enqueue_frontend(mcgpu_context ctx)
     Params* Pb = P_<Params>(ctx->bparams);
     const auto* brbox = (const unsigned long long(*)[2][6])ctx->brbox.p;
     if (ctx->batch) {
-        ev_wait(ctx, ctx->ssum, EV_FORK);
-        stage_event(ctx, EV_S0, ctx->ssum);
+        ev_wait(ctx, ssum, EV_FORK);
+        stage_event(ctx, EV_S0, ssum);
         const uint32_t nch = 6 * ctx->npairs;
-        k_batch_sums<<<std::min<uint32_t>(nch, kBatchSumWaves), 64, 0, ctx->ssum>>>(
+        k_batch_sums<<<std::min<uint32_t>(nch, kBatchSumWaves), 64, 0, ssum>>>(
             ctx->dv[0], ctx->dv[1], P_<BatchPair>(ctx->bpairs), P_<uint32_t>(ctx->border), nch, C, Pb);
     } else {
         // items and their check on stream A (every CU), the chain on the
@@ -1308,9 +1349,9 @@ void enqueue_frontend(mcgpu_context ctx)
             k_sum_items<<<grid, kSumThreads, 0, s>>>(SB);
         }
         ev_record(ctx, EV_SUM_ITEMS, s);
-        ev_wait(ctx, ctx->ssum, EV_SUM_ITEMS);
-        k_sum_chain<<<6, kSumChain, 0, ctx->ssum>>>(SB, &C->zero, Pd);
-        ev_record(ctx, EV_SUM_CHAIN, ctx->ssum);
+        ev_wait(ctx, ssum, EV_SUM_ITEMS);
+        k_sum_chain<<<6, kSumChain, 0, ssum>>>(SB, &C->zero, Pd);
+        ev_record(ctx, EV_SUM_CHAIN, ssum);
         ev_wait(ctx, s, EV_SUM_CHAIN);
         if (ctx->sum_items) {
             k_sum_verify<<<grid, kSumThreads, 0, s>>>(SB);
@@ -1319,7 +1360,7 @@ void enqueue_frontend(mcgpu_context ctx)
         ev_record(ctx, EV_A_SUMS, s);
     }
     if (ctx->batch) {
-        ev_record(ctx, EV_A_SUMS, ctx->ssum);
+        ev_record(ctx, EV_A_SUMS, ssum);
         ev_wait(ctx, s, EV_A_SUMS);
     }
     if (ctx->batch) {
@@ -1372,7 +1413,8 @@ void enqueue_frontend(mcgpu_context ctx)
         k_morton_raw<<<grid_for(F - start), kBlock, 0, s2>>>(M[0], M[1], start, P_<uint32_t>(ctx->mcode),
                                                              P_<uint32_t>(ctx->mface), rawbox, Pd, C, zero, nzero);
     }
-    enqueue_bvh_traverse(ctx, s2, C, !ctx->batch); // k_morton_raw cleared the sort's group totals
+    if (tests_all_pairs(ctx)) launch_all_pairs(ctx, s2, C);
+    else enqueue_bvh_traverse(ctx, s2, C, !ctx->batch); // k_morton_raw cleared the sort's group totals
 
     // ---- stream C: polygon-soup edge numbering, and the tables the filter fills ----
     ev_wait(ctx, s3, EV_FORK);
@@ -1607,7 +1649,7 @@ std::vector<uint64_t> graph_key(mcgpu_context ctx)
     auto put = [&k](uint64_t x) { k.push_back(x); };
     auto ptr = [&k](const void* p) { k.push_back((uint64_t)(uintptr_t)p); };
     put(ctx->batch), put(ctx->npairs), put(ctx->batch_mb), put(ctx->cc_check), put(ctx->sort_bits),
-        put(ctx->shifted_bp), put(ctx->walk), put(ctx->trav.walk), put(ctx->cap_nodes), put(ctx->topo_hash), put(ctx->topo_buckets), put(ctx->topo_tiles), put(ctx->topo_bits),
+        put(ctx->shifted_bp), put(ctx->walk), put(ctx->trav.walk), put(ctx->want_trees), put(ctx->one_stream), put(ctx->forced), put(ctx->cap_nodes), put(ctx->topo_hash), put(ctx->topo_buckets), put(ctx->topo_tiles), put(ctx->topo_bits),
         put(ctx->nseg),
         put(ctx->gbits), put(ctx->kbits);
     for (int m = 0; m < 2; ++m) {
@@ -1638,6 +1680,7 @@ void graph_drop(mcgpu_context ctx)
 // dispatch's shape differs from the one it was recorded for.
 mcgpu_result enqueue_dispatch(mcgpu_context ctx)
 {
+    ctx->one_stream = uses_one_stream(ctx);
     ctx->state_copied = false;
     if (!ctx->graphs || ctx->stage_timing || ctx->kernel_timing || !ctx->own_streams) {
         if (ctx->batch) enqueue_validate_batch(ctx);
@@ -1911,6 +1954,15 @@ static mcgpu_result autotune(mcgpu_context ctx, mcgpu_tuning* out)
     TravConfig bt = def;
     uint32_t n = 0;
     mcgpu_result r;
+    if (tests_all_pairs(ctx)) { // trees for the walks: the dispatch made none
+        float ms;
+        ctx->want_trees = true;
+        if ((r = rerun_dispatch(ctx, &ms)) != MCGPU_SUCCESS && ctx->walk) { // a list of node pairs overflowed
+            if ((r = alloc_node_pairs(ctx)) == MCGPU_SUCCESS) r = rerun_dispatch(ctx, &ms);
+        }
+        ctx->want_trees = false;
+        if (r != MCGPU_SUCCESS) return r;
+    }
     {
         bool same = true;
         if ((r = time_traversal(ctx, def, 3, &def_trav, &same)) != MCGPU_SUCCESS) return r;
@@ -1945,7 +1997,14 @@ static mcgpu_result autotune(mcgpu_context ctx, mcgpu_tuning* out)
         return e;
     };
     float def_disp = 0.f, disp = 0.f;
-    if ((r = timed(def, &def_disp)) != MCGPU_SUCCESS || (r = timed(bt, &disp)) != MCGPU_SUCCESS) return r;
+    if ((r = timed(def, &def_disp)) != MCGPU_SUCCESS) return r;
+    const bool all = tests_all_pairs(ctx); // the default makes no trees
+    if ((r = timed(bt, &disp)) != MCGPU_SUCCESS) return r;
+    if (all && def_disp < disp) {
+        bt = ctx->trav = def;
+        best = def_trav;
+        disp = def_disp;
+    }
     TuneEntry e;
     e.batch = ctx->batch;
     e.bs = bits_for((uint64_t)ctx->nf[0] + 1);
@@ -3089,6 +3148,7 @@ MCGPU_API mcgpu_result mcgpu_server_create(int device, const mcgpu_mesh* src, co
             dummy.face_indices = di;
         }
         mcgpu_frontend_info info;
+        m->want_trees = true;
         r = mcgpu_dispatch_frontend(m, src, &dummy, &d, &info);
         if (dv) (void)hipFree(dv);
         if (di) (void)hipFree(di);
