@@ -2594,62 +2594,89 @@ __global__ void k_planes(Soup S, const uint32_t* __restrict__ cand_list, Plane* 
     }
 }
 
-// Candidate polygons of more than five vertices, one wave each.  The wave
+// Candidate polygons of more than five vertices, one block each.  The block
 // lists the polygon's C(n, 3) triplets with non-zero orient2d in the
-// reference's (i < j < k) lexicographic order, 64 third vertices a step with
-// ballot-ranked appends, in a region of the triplet scratch that k_planes
-// reserved (big_polygon_units: the n projected vertices as 16-byte records,
-// the triplets, then the two position lists of the partitions), and takes the
-// element that the reference's std::sort puts first (trip_first in
-// tripsort.hpp: the left-most chain of the introsort's partitions), each
-// partition computed a wave at a time in the form of pairs that
-// tests/support/tripsort_check.cpp holds to std::__unguarded_partition.  A
-// region past the scratch's capacity is left undone and flagged; the host
-// grows the scratch and runs the dispatch again.
+// reference's (i < j < k) lexicographic order, a triplet a thread with ranked
+// appends, and takes the element that the reference's std::sort puts first
+// (trip_first in tripsort.hpp: the left-most chain of the introsort's
+// partitions), each partition computed a block at a time in the form of pairs
+// that tests/support/tripsort_check.cpp holds to std::__unguarded_partition.
+// Up to kTripLds triplets lie in LDS; more in a region of the triplet scratch
+// that k_planes reserved (big_polygon_units: the n projected vertices as
+// 16-byte records, the triplets, then the two position lists of the
+// partitions).  A region past the scratch's capacity is left undone and
+// flagged; the host grows the scratch and runs the dispatch again.
+// What bounds it: the chain of rounds, each with a barrier.  One wave a
+// polygon, a row of third vertices a step and all of it in the scratch, took
+// 184 us for two 24-gons; this takes 57.
+constexpr int kTripBlock = 256;
+constexpr int kTripWaves = kTripBlock / 64;
+constexpr int kTripLds = 2048; // triplets kept in LDS: polygons of up to 24 vertices
+
+// this thread's place among the block's flagged ones, and their number; cnt:
+// two rows of LDS, used in turn (one barrier a call)
+struct TripRank {
+    uint32_t (*cnt)[kTripWaves];
+    int row;
+
+    __device__ __forceinline__ uint32_t operator()(bool flag, uint32_t* total)
+    {
+        const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+        const unsigned long long m = __ballot(flag);
+        if (lane == 0) cnt[row][wid] = (uint32_t)__popcll(m);
+        __syncthreads();
+        uint32_t at = (uint32_t)__popcll(m & ((1ull << lane) - 1ull)), t = 0;
+        for (uint32_t q = 0; q < (uint32_t)kTripWaves; ++q) {
+            const uint32_t c = cnt[row][q];
+            if (q < wid) at += c;
+            t += c;
+        }
+        row ^= 1;
+        *total = t;
+        return at;
+    }
+};
+
 // The unguarded partition of T[1, l) around the pivot T[0] (std::__unguarded_partition
-// after the median-of-three move), by the whole wave.  Let L be the positions in
+// after the median-of-three move), by the whole block.  Let L be the positions in
 // [1, l) whose element is not greater than the pivot, ascending, and R those
 // in [0, l) whose element is not less than it, descending (the pivot itself
 // last).  The sequential partition swaps L[k] with R[k] for k = 0, 1, ... while
 // L[k] < R[k]; at the first k = K that fails it returns L[0] if K = 0 and
 // otherwise the smaller of L[K] (l if L has no K-th entry) and R[K - 1]
 // (a later left scan stops at the element swapped into R[K - 1] at the latest).
+// L ascends and R descends, so K is the number of k with L[k] < R[k].
 // Positions of different pairs before K are distinct, so the swaps run in
-// parallel.  Lp and Rp hold the lists (at most l entries each).  Every lane
+// parallel.  Lp and Rp hold the lists (at most l entries each).  Every thread
 // returns the cut.
-__device__ inline long wave_trip_partition(Trip* T, long l, unsigned long long* Lp, unsigned long long* Rp)
+template <typename Pos>
+__device__ inline long block_trip_partition(Trip* T, long l, Pos* Lp, Pos* Rp, TripRank& rank)
 {
-    const int lane = (int)(threadIdx.x & 63);
-    const unsigned long long below = (1ull << lane) - 1ull;
     const Trip P = T[0];
     long nL = 0, nR = 0;
-    for (long p0 = 1; p0 < l; p0 += 64) {
-        const long p = p0 + lane;
-        const bool s = p < l && !trip_less(T[p], P);
-        const unsigned long long m = __ballot(s);
-        if (s) Lp[nL + __popcll(m & below)] = (unsigned long long)p;
-        nL += __popcll(m);
+    for (long p0 = 0; p0 < l; p0 += kTripBlock) {
+        const long p = p0 + threadIdx.x, r = l - 1 - p;
+        uint32_t n;
+        const bool s = p >= 1 && p < l && !trip_less(T[p], P);
+        uint32_t at = rank(s, &n);
+        if (s) Lp[nL + at] = (Pos)p;
+        nL += n;
+        const bool e = r >= 0 && !trip_less(P, T[r]);
+        at = rank(e, &n);
+        if (e) Rp[nR + at] = (Pos)r;
+        nR += n;
     }
-    for (long p0 = l - 1; p0 >= 0; p0 -= 64) {
-        const long p = p0 - lane;
-        const bool s = p >= 0 && !trip_less(P, T[p]);
-        const unsigned long long m = __ballot(s);
-        if (s) Rp[nR + __popcll(m & below)] = (unsigned long long)p;
-        nR += __popcll(m);
-    }
-    __syncthreads(); // the lists, written lane by lane, are read across the wave
+    __syncthreads(); // the lists, written thread by thread, are read across the block
     const long np = nL < nR ? nL : nR;
-    long K = np;
-    for (long k0 = 0; k0 < np; k0 += 64) {
-        const long k = k0 + lane;
-        const bool fail = k < np && !(Lp[k] < Rp[k]);
-        const unsigned long long m = __ballot(fail);
-        if (m) {
-            K = k0 + __ffsll((long long)m) - 1;
-            break;
-        }
+    long K = 0;
+    for (long k0 = 0; k0 < np; k0 += kTripBlock) {
+        const long k = k0 + threadIdx.x;
+        const bool both = k < np && Lp[k] < Rp[k];
+        if (both) trip_swap(T + Lp[k], T + Rp[k]);
+        const int n = __syncthreads_count(both);
+        K += n;
+        if (n < kTripBlock) break;
     }
-    for (long k = lane; k < K; k += 64) trip_swap(T + Lp[k], T + Rp[k]);
     long cut;
     if (K == 0) {
         cut = (long)Lp[0];
@@ -2658,28 +2685,28 @@ __device__ inline long wave_trip_partition(Trip* T, long l, unsigned long long* 
         const long rK = (long)Rp[K - 1];
         cut = lK < rK ? lK : rK;
     }
-    __syncthreads(); // the swaps land before the next partition reads the range
+    __syncthreads(); // the swaps land, and the lists are read, before the next partition
     return cut;
 }
 
-// trip_first over T[0, m) by the whole wave: lane 0 moves the median to the
+// trip_first over T[0, m) by the whole block: thread 0 moves the median to the
 // front and, when the depth budget runs out, heap sorts the range; the
-// partitions are the wave's
-__device__ inline Trip wave_trip_first(Trip* T, long m, unsigned long long* Lp, unsigned long long* Rp)
+// partitions are the block's
+template <typename Pos>
+__device__ inline Trip block_trip_first(Trip* T, long m, Pos* Lp, Pos* Rp, TripRank& rank)
 {
-    const int lane = (int)(threadIdx.x & 63);
     long l = m;
     int depth = trip_depth_budget(m);
     while (l > 16) {
         if (depth == 0) {
-            if (lane == 0) trip_heap_sort(T, T + l);
+            if (threadIdx.x == 0) trip_heap_sort(T, T + l);
             __syncthreads();
             return T[0];
         }
         --depth;
-        if (lane == 0) trip_median_to_first(T, T + l);
+        if (threadIdx.x == 0) trip_median_to_first(T, T + l);
         __syncthreads();
-        l = wave_trip_partition(T, l, Lp, Rp);
+        l = block_trip_partition(T, l, Lp, Rp, rank);
     }
     Trip best = T[0];
     for (long p = 1; p < l; ++p)
@@ -2687,13 +2714,50 @@ __device__ inline Trip wave_trip_first(Trip* T, long m, unsigned long long* Lp, 
     return best;
 }
 
-__global__ void __launch_bounds__(64) k_big_polygons(Soup S, const uint32_t* __restrict__ big_list,
+// the non-degenerate triplets of the n projected vertices X into T, in
+// lexicographic order; returns their number
+__device__ inline long block_trips(const double* X, int n, Trip* T, TripRank& rank)
+{
+    const uint64_t c3 = (uint64_t)n * (n - 1) * (n - 2) / 6;
+    int a = 0, b = 1, c = 2 + (int)threadIdx.x;
+    long m = 0;
+    for (uint64_t t0 = 0; t0 < c3; t0 += kTripBlock) {
+        const bool in = t0 + threadIdx.x < c3;
+        while (in && c >= n) { // carry: the places past this row's end continue in the next
+            const int over = c - n;
+            if (++b >= n - 1) {
+                ++a;
+                b = a + 1;
+            }
+            c = b + 1 + over;
+        }
+        const double r = in ? orient2d_adaptive(X + 2 * a, X + 2 * b, X + 2 * c) : 0.0;
+        const bool keep = r != 0.0;
+        uint32_t k;
+        const uint32_t at = rank(keep, &k);
+        if (keep) {
+            Trip t;
+            t.a = fabs(r);
+            t.ijk = (uint64_t)a | ((uint64_t)b << 16) | ((uint64_t)c << 32);
+            T[m + at] = t;
+        }
+        m += k;
+        c += kTripBlock;
+    }
+    __syncthreads();
+    return m;
+}
+
+__global__ void __launch_bounds__(kTripBlock) k_big_polygons(Soup S, const uint32_t* __restrict__ big_list,
                                                      const unsigned long long* __restrict__ big_off,
                                                      const Counters* __restrict__ C, uint64_t cap_big, uint64_t cap_trip,
                                                      Plane* __restrict__ planes, Trip* __restrict__ scratch, Counters* Cw)
 {
-    const int lane = (int)threadIdx.x;
-    const unsigned long long below = (1ull << lane) - 1ull;
+    __shared__ Trip lt[kTripLds];
+    __shared__ uint16_t ll[kTripLds], lr[kTripLds];
+    __shared__ double lx[2 * 24];
+    __shared__ uint32_t cnt[2][kTripWaves];
+    TripRank rank{cnt, 0};
     const uint64_t nb = C->n_big < cap_big ? C->n_big : cap_big;
     for (uint64_t w = blockIdx.x; w < nb; w += gridDim.x) {
         const uint32_t g = big_list[w];
@@ -2701,50 +2765,42 @@ __global__ void __launch_bounds__(64) k_big_polygons(Soup S, const uint32_t* __r
         const uint64_t n = fv.n;
         const uint64_t off = big_off[w];
         if (off + big_polygon_units(n) > cap_trip) {
-            if (lane == 0) atomicOr(&Cw->ov_trip, 1u);
+            if (threadIdx.x == 0) atomicOr(&Cw->ov_trip, 1u);
             continue;
         }
         Plane pl = planes[g];
         double M[6];
         projection_matrix(pl.n, pl.k, M);
+        const uint64_t c3 = n * (n - 1) * (n - 2) / 6;
+        const bool lds = c3 <= (uint64_t)kTripLds;
         double* X = reinterpret_cast<double*>(scratch + off); // projected vertex i: X[2i], X[2i + 1]
-        for (uint32_t i = lane; i < fv.n; i += 64) {
-            double p[3];
+        for (uint32_t i = threadIdx.x; i < fv.n; i += kTripBlock) {
+            double p[3], x[2];
             fv((int)i, p);
-            project2(M, p, X + 2 * i);
+            project2(M, p, x);
+            if (lds) lx[2 * i] = x[0], lx[2 * i + 1] = x[1];
+            else X[2 * i] = x[0], X[2 * i + 1] = x[1];
         }
         __syncthreads();
-        const uint64_t c3 = n * (n - 1) * (n - 2) / 6;
-        Trip* T = scratch + off + n;
-        unsigned long long* Lp = reinterpret_cast<unsigned long long*>(scratch + off + n + c3);
-        unsigned long long* Rp = Lp + c3;
-        long m = 0;
-        for (int a = 0; a < (int)n; ++a)
-            for (int b = a + 1; b < (int)n; ++b)
-                for (int c0 = b + 1; c0 < (int)n; c0 += 64) {
-                    const int c = c0 + lane;
-                    double r = 0.0;
-                    if (c < (int)n) r = orient2d_adaptive(X + 2 * a, X + 2 * b, X + 2 * c);
-                    const bool keep = r != 0.0;
-                    const unsigned long long mk = __ballot(keep);
-                    if (keep) {
-                        Trip t;
-                        t.a = fabs(r);
-                        t.ijk = (uint64_t)a | ((uint64_t)b << 16) | ((uint64_t)c << 32);
-                        T[m + __popcll(mk & below)] = t;
-                    }
-                    m += __popcll(mk);
-                }
-        __syncthreads();
+        long m;
+        Trip best;
+        if (lds) {
+            m = block_trips(lx, (int)n, lt, rank);
+            if (m) best = block_trip_first(lt, m, ll, lr, rank);
+        } else {
+            Trip* T = scratch + off + n;
+            unsigned long long* Lp = reinterpret_cast<unsigned long long*>(scratch + off + n + c3);
+            m = block_trips(X, (int)n, T, rank);
+            if (m) best = block_trip_first(T, m, Lp, Lp + c3, rank);
+        }
         if (m == 0) {
             pl.tri[0] = kCollinear;
         } else {
-            const Trip best = wave_trip_first(T, m, Lp, Rp);
             pl.tri[0] = (uint16_t)(best.ijk & 0xffff);
             pl.tri[1] = (uint16_t)((best.ijk >> 16) & 0xffff);
             pl.tri[2] = (uint16_t)((best.ijk >> 32) & 0xffff);
         }
-        if (lane == 0) planes[g] = pl;
+        if (threadIdx.x == 0) planes[g] = pl;
         __syncthreads();
     }
 }

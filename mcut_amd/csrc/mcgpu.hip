@@ -738,7 +738,7 @@ void enqueue_narrow(mcgpu_context ctx, const Soup& S, bool join_topology, PairRu
                                              P_<uint32_t>(ctx->big_list), P_<unsigned long long>(ctx->big_off),
                                              ctx->cap_big, C);
     if (ctx->dsz[0] || ctx->dsz[1]) // faces of more than 5 vertices: none in two triangle meshes
-        k_big_polygons<<<(unsigned)std::min<uint64_t>(std::max<uint64_t>(ctx->cap_big, 1), 1024), 64, 0, s>>>(
+        k_big_polygons<<<(unsigned)std::min<uint64_t>(std::max<uint64_t>(ctx->cap_big, 1), 1024), kTripBlock, 0, s>>>(
             S, P_<uint32_t>(ctx->big_list), P_<unsigned long long>(ctx->big_off), C, ctx->cap_big, ctx->cap_trip,
             P_<Plane>(ctx->planes), P_<Trip>(ctx->big_scratch), C);
     stage_event(ctx, EV_A_PLANES, s);
