@@ -116,7 +116,7 @@ __device__ __forceinline__ double serial_sum(const double* __restrict__ v, uint3
 
 // ---------------------------------------------------------------------------
 // The same sums from a short chain (sumseg.hpp says why it is exact).
-// k_sum_blocks adds every tile in any order, for the predictions.  k_sum_items
+// k_head adds every tile in any order (sum_block), for the predictions.  k_sum_items
 // walks 64 values a thread (a chunk) into segments and single steps and writes
 // them with their adds, a tile's without gaps.  k_sum_chain, one block a chain
 // on the reserved CUs, runs the DPP chain over all adds, from LDS.
@@ -164,13 +164,13 @@ __device__ __forceinline__ bool sum_chain_items(const SumBufs& B, int ch)
     return sum_chain_active(B, ch) && B.n[ch / 3] > kSumSerial;
 }
 
-__global__ void __launch_bounds__(256) k_sum_blocks(SumBufs B)
+// tile b of chain ch, by a block of 256 threads (k_head); red: 4 doubles of LDS
+__device__ __forceinline__ void sum_block(const SumBufs& B, uint32_t b, int ch, double* red)
 {
-    __shared__ double red[4];
-    const int ch = blockIdx.y, m = ch / 3, j = ch % 3;
-    if (blockIdx.x == 0 && threadIdx.x == 0) B.fail[ch] = 0xffffffffu;
+    const int m = ch / 3, j = ch % 3;
+    if (b == 0 && threadIdx.x == 0) B.fail[ch] = 0xffffffffu;
     if (!sum_chain_items(B, ch)) return;
-    const uint32_t n = B.n[m], b = blockIdx.x;
+    const uint32_t n = B.n[m];
     if ((uint64_t)b * kSumTile >= n) return;
     const double* v = B.v[m] + j;
     const uint64_t i0 = (uint64_t)b * kSumTile;
@@ -266,19 +266,58 @@ __global__ void __launch_bounds__(kSumThreads) k_sum_items(SumBufs B)
     for (uint32_t q = kSumKeep; q < na; ++q) tadds[off + q] = past[q]; // the lane's own stores
 }
 
-__global__ void __launch_bounds__(kSumChain) k_sum_chain(SumBufs B, const double* __restrict__ zero, Params* P)
+// what the shift follows from, besides the sums and raw boxes
+struct ShiftArgs {
+    uint32_t n0, n1;
+    double gp_constant;
+    int absolute;
+};
+__device__ inline void shift_params_of(Params* P, const unsigned long long (*rbox)[6], uint32_t n0, uint32_t n1,
+                                       double gp_constant, int eps_absolute);
+__device__ inline void shift_params(Params* P, const Counters* C, const ShiftArgs& A)
+{
+    shift_params_of(P, C->rbox, A.n0, A.n1, A.gp_constant, A.absolute);
+    P->has_pert = 0;
+    P->pert[0] = P->pert[1] = P->pert[2] = 0.0;
+}
+
+// The chains of meshes without items, and then the shift by the block that
+// ends last: the sums pass between blocks by device-scope atomics, each
+// waited for before the next, so no cache has to be written back.
+__device__ inline void sum_done(double sum, bool store, int m, int j, Params* P, Counters* C, const ShiftArgs& A)
+{
+    if (threadIdx.x != 0) return;
+    auto* bits = reinterpret_cast<unsigned long long*>(&P->sum[0][0]);
+    if (store) {
+        const unsigned long long old = atomicExch(bits + 3 * m + j, (unsigned long long)__double_as_longlong(sum));
+        asm volatile("" : : "v"(old) : "memory"); // its result is here: it is done
+    }
+    if (atomicAdd(&C->sums_done, 1u) != 5u) return;
+    double all[6];
+    for (int q = 0; q < 6; ++q) all[q] = __longlong_as_double((long long)atomicAdd(bits + q, 0ull));
+    for (int q = 0; q < 6; ++q) P->sum[q / 3][q % 3] = all[q];
+    shift_params(P, C, A);
+}
+
+// finish: no chain has items, so the shift follows here
+__global__ void __launch_bounds__(kSumChain) k_sum_chain(SumBufs B, const double* __restrict__ zero, Params* P, Counters* C,
+                                                         ShiftArgs A, int finish)
 {
     constexpr int kWaves = kSumChain / 64;
     __shared__ double ladds[kSumLdsAdds], lrows[kSumLdsAdds / 16];
     __shared__ uint32_t wsum[kWaves];
     const int ch = blockIdx.x, m = ch / 3, j = ch % 3;
-    if (!sum_chain_active(B, ch)) return; // a resident source: its sums are set already
+    if (!sum_chain_active(B, ch)) { // a resident source: its sums are set already
+        if (finish) sum_done(0.0, false, m, j, P, C, A);
+        return;
+    }
     const uint32_t n = B.n[m], t = threadIdx.x, lane = t & 63, wid = t >> 6;
     if (!sum_chain_items(B, ch)) {
         if (wid == 0) {
             __builtin_amdgcn_s_setprio(3);
             const double acc = serial_sum(B.v[m] + j, n, zero);
-            if (lane == 0) P->sum[m][j] = acc;
+            if (finish) sum_done(acc, true, m, j, P, C, A);
+            else if (lane == 0) P->sum[m][j] = acc;
         }
         return;
     }
@@ -375,16 +414,21 @@ __global__ void __launch_bounds__(kSumThreads) k_sum_verify(SumBufs B)
     if (!ok) atomicMin(&B.fail[ch], c);
 }
 
-__global__ void __launch_bounds__(64) k_sum_rest(SumBufs B, const double* __restrict__ zero, Params* P)
+// the rest of the chains that failed a check, a wave each, and the shift
+__global__ void __launch_bounds__(384) k_sum_rest(SumBufs B, const double* __restrict__ zero, Params* P, const Counters* C,
+                                                  ShiftArgs A)
 {
-    const int ch = blockIdx.x, m = ch / 3, j = ch % 3;
+    const int ch = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = ch / 3, j = ch % 3;
     const uint32_t c = __builtin_amdgcn_readfirstlane(B.fail[ch]);
-    if (c == 0xffffffffu) return;
-    __builtin_amdgcn_s_setprio(3);
-    const uint32_t i0 = c * kSumPer;
-    const double start = sum_chunk_start(B, ch, c);
-    const double acc = serial_chain<3, false>(B.v[m] + j + 3ull * i0, B.n[m] - i0, zero, start, nullptr);
-    if (threadIdx.x == 0) P->sum[m][j] = acc;
+    if (c != 0xffffffffu) {
+        __builtin_amdgcn_s_setprio(3);
+        const uint32_t i0 = c * kSumPer;
+        const double start = sum_chunk_start(B, ch, c);
+        const double acc = serial_chain<3, false>(B.v[m] + j + 3ull * i0, B.n[m] - i0, zero, start, nullptr);
+        if ((threadIdx.x & 63) == 0) P->sum[m][j] = acc;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) shift_params(P, C, A);
 }
 
 // Batches: the 6 chains of every pair (pair p, mesh m, coordinate j is chain
@@ -444,17 +488,6 @@ __device__ inline void shift_params_of(Params* P, const unsigned long long (*rbo
     P->gp_constant = gp_constant;
     P->eps_absolute = eps_absolute;
     P->eps = (eps_absolute ? 1.0 : P->diag) * gp_constant; // preproc.cpp:2667-2676
-}
-
-__global__ void k_shift_params(Params* P, const Counters* __restrict__ C, uint32_t n0, uint32_t n1, double gp_constant,
-                               int eps_absolute, int has_pert, double p0, double p1, double p2)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    shift_params_of(P, C->rbox, n0, n1, gp_constant, eps_absolute);
-    P->has_pert = has_pert;
-    P->pert[0] = p0;
-    P->pert[1] = p1;
-    P->pert[2] = p2;
 }
 
 // batches: one thread per pair
@@ -532,13 +565,19 @@ __device__ inline bool tolerance_of(const unsigned long long (*rbox)[6], uint32_
 
 // allow_loose: the dispatch can rerun with its broad phase in shifted
 // coordinates (a single pair whose source is not resident)
-__global__ void k_tolerance(Params* P, Counters* C, uint32_t nv0, uint32_t nv1, double gp_constant, int absolute,
-                            int allow_loose)
+struct TolArgs {
+    uint32_t nv0, nv1;
+    double gp_constant;
+    int absolute, allow_loose;
+};
+
+// for a dispatch whose leaves k_morton_raw does not make (it finds the bound itself)
+__global__ void k_tolerance(Params* P, Counters* C, TolArgs A)
 {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     bool loose = false;
-    if (!tolerance_of(C->rbox, nv0, nv1, gp_constant, absolute, P->tol, &loose)) C->unsupported |= 2u;
-    else if (loose && allow_loose) C->loose = 1u;
+    if (!tolerance_of(C->rbox, A.nv0, A.nv1, A.gp_constant, A.absolute, P->tol, &loose)) C->unsupported |= 2u;
+    else if (loose && A.allow_loose) C->loose = 1u;
 }
 
 // batches: one thread per pair; any pair without a finite bound rejects the batch
@@ -576,21 +615,13 @@ __global__ void k_shift_vertices(const double* __restrict__ vs, uint32_t ns, con
     }
 }
 
-// serving: the resident source's sums, raw box and edge count into this
-// dispatch's parameters and counters (after the counter reset)
+// serving: the resident source's sums, raw box and edge count, for this
+// dispatch's parameters and counters (k_reset_counters)
 struct ResidentGpuView {
     double sum[3];
     unsigned long long rbox[6];
     unsigned long long ne;
 };
-
-__global__ void k_resident_source(Counters* C, Params* P, const ResidentGpuView* r)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    for (int j = 0; j < 3; ++j) P->sum[0][j] = r->sum[j];
-    for (int j = 0; j < 6; ++j) C->rbox[0][j] = r->rbox[j];
-    C->n_edges_src = r->ne;
-}
 
 // batches: every pair's vertices with its own shift (no perturbation)
 __global__ void k_batch_shift_vertices(const double* __restrict__ vs, uint32_t ns, const double* __restrict__ vc,
@@ -635,19 +666,59 @@ __global__ void k_offsets_tail(uint32_t* __restrict__ off, uint32_t nf, const ui
     if (threadIdx.x == 0 && blockIdx.x == 0) off[nf] = *total;
 }
 
-__global__ void k_validate(const uint32_t* __restrict__ idx, const uint32_t* __restrict__ off,
-                           const uint32_t* __restrict__ sizes, uint32_t nf, uint32_t nv, Counters* C)
+// the face offsets of meshes of few faces, a block each (four launches of the
+// scan otherwise)
+struct OffsetMesh {
+    const uint32_t* sizes; // null: nothing to do
+    uint32_t* off;
+    uint32_t nf;
+};
+__global__ void __launch_bounds__(1024) k_small_offsets(OffsetMesh m0, OffsetMesh m1)
 {
-    for (uint64_t f = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; f < nf; f += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t b = off[f], n = sizes ? sizes[f] : 3u;
-        bool bad = n < 3;
-        for (uint32_t i = 0; i < n && !bad; ++i) {
-            const uint32_t a = idx[b + i];
-            bad = a >= nv;
-            for (uint32_t k = 0; k < i && !bad; ++k) bad = idx[b + k] == a; // duplicate vertex in a face
+    __shared__ uint32_t wsum[16];
+    const OffsetMesh M = blockIdx.x ? m1 : m0;
+    if (!M.sizes) return; // whole block
+    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    uint32_t base = 0;
+    for (uint32_t f0 = 0; f0 < M.nf; f0 += 4096) {
+        uint32_t v[4], own = 0;
+        const uint32_t f = f0 + 4 * threadIdx.x;
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) v[q] = f + q < M.nf ? M.sizes[f + q] : 0u;
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) own += v[q];
+        uint32_t x = own;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o, 64);
+            if (lane >= (uint32_t)o) x += y;
         }
-        if (bad) atomicOr(&C->bad_input, 1u);
+        if (lane == 63) wsum[wid] = x;
+        __syncthreads();
+        x += base - own;
+        for (uint32_t q = 0; q < 16; ++q) {
+            if (q < wid) x += wsum[q];
+            base += wsum[q];
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            if (f + q < M.nf) M.off[f + q] = x;
+            x += v[q];
+        }
+        __syncthreads();
     }
+    if (threadIdx.x == 0) M.off[M.nf] = base;
+}
+
+// a face list's bounds and repeated vertices
+__device__ __forceinline__ bool face_bad(const uint32_t* __restrict__ idx, uint32_t n, uint32_t nv)
+{
+    bool bad = n < 3;
+    for (uint32_t i = 0; i < n && !bad; ++i) {
+        const uint32_t a = idx[i];
+        bad = a >= nv;
+        for (uint32_t k = 0; k < i && !bad; ++k) bad = idx[k] == a; // duplicate vertex in a face
+    }
+    return bad;
 }
 
 // ===========================================================================
@@ -1313,6 +1384,52 @@ __global__ void k_face_boxes(Soup S, const Params* __restrict__ P, const Counter
     }
 }
 
+// The shifted vertices and, from the raw ones, the shifted face boxes of a
+// dispatch that moves no vertex besides (a launch for the two: the boxes would
+// gather the shifted vertices as they gather the raw ones).
+__global__ void __launch_bounds__(256) k_shift_boxes(Soup S, const double* __restrict__ vs, const double* __restrict__ vc,
+                                                     const Params* __restrict__ P, const Counters* __restrict__ C,
+                                                     uint32_t face_blocks, double* __restrict__ ps_v, double* __restrict__ box)
+{
+    const double com[3] = {P->com[0], P->com[1], P->com[2]};
+    const double t[3] = {P->t[0], P->t[1], P->t[2]};
+    if (blockIdx.x >= face_blocks) {
+        const uint64_t total = (uint64_t)(S.nv[0] + S.nv[1]) * 3, split = (uint64_t)S.nv[0] * 3;
+        const uint64_t stride = (uint64_t)(gridDim.x - face_blocks) * 256;
+        for (uint64_t i = (uint64_t)(blockIdx.x - face_blocks) * 256 + threadIdx.x; i < total; i += stride) {
+            const double x = i >= split ? vc[i - split] : vs[i];
+            const int j = (int)(i % 3);
+            ps_v[i] = ((x - com[j]) + t[j]) + 0.0;
+        }
+        return;
+    }
+    const uint32_t F = S.nf[0] + S.nf[1];
+    const double eps = P->eps;
+    const bool aborted = dispatch_aborted(C);
+    for (uint64_t g = (uint64_t)blockIdx.x * 256 + threadIdx.x; g < F; g += (uint64_t)face_blocks * 256) {
+        const FaceView fv = face_view(S, (uint32_t)g);
+        const bool cut = g >= S.nf[0];
+        const double* v = cut ? vc : vs;
+        double lo[3] = {1.7976931348623157e308, 1.7976931348623157e308, 1.7976931348623157e308};
+        double hi[3] = {-1.7976931348623157e308, -1.7976931348623157e308, -1.7976931348623157e308};
+        for (uint32_t i = 0; i < (aborted ? 0u : fv.n); ++i) {
+            const double* q = v + 3 * (uint64_t)fv.idx[fv.base + i];
+            for (int j = 0; j < 3; ++j) {
+                const double p = ((q[j] - com[j]) + t[j]) + 0.0;
+                hi[j] = (hi[j] < p) ? p : hi[j];
+                lo[j] = (p < lo[j]) ? p : lo[j];
+            }
+        }
+        if (cut && eps > 0.0)
+            for (int j = 0; j < 3; ++j) {
+                hi[j] = hi[j] + eps;
+                lo[j] = lo[j] - eps;
+            }
+        double* o = box + 6 * g;
+        o[0] = lo[0], o[1] = lo[1], o[2] = lo[2], o[3] = hi[0], o[4] = hi[1], o[5] = hi[2];
+    }
+}
+
 __device__ __forceinline__ uint32_t expand_bits10(uint32_t v)
 {
     v = (v * 0x00010001u) & 0xFF0000FFu;
@@ -1322,64 +1439,48 @@ __device__ __forceinline__ uint32_t expand_bits10(uint32_t v)
     return v;
 }
 
-// raw (unshifted) bounding box of a mesh: ord keys lo[3], hi[3]; one atomic
-// per block and coordinate after an LDS reduction
-__global__ void __launch_bounds__(256) k_raw_bbox(const double* __restrict__ v, uint32_t n, unsigned long long* __restrict__ box)
-{
-    __shared__ double red[4][6];
-    double lo[3] = {1.7976931348623157e308, 1.7976931348623157e308, 1.7976931348623157e308};
-    double hi[3] = {-1.7976931348623157e308, -1.7976931348623157e308, -1.7976931348623157e308};
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        for (int j = 0; j < 3; ++j) {
-            const double x = v[3 * i + j];
-            lo[j] = x < lo[j] ? x : lo[j];
-            hi[j] = x > hi[j] ? x : hi[j];
-        }
-    for (int o = 32; o > 0; o >>= 1)
-        for (int j = 0; j < 3; ++j) {
-            const double a = __shfl_xor(lo[j], o, 64), b = __shfl_xor(hi[j], o, 64);
-            lo[j] = a < lo[j] ? a : lo[j];
-            hi[j] = b > hi[j] ? b : hi[j];
-        }
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0)
-        for (int j = 0; j < 3; ++j) {
-            red[w][j] = lo[j];
-            red[w][3 + j] = hi[j];
-        }
-    __syncthreads();
-    if (threadIdx.x < 3) {
-        const int j = threadIdx.x;
-        double a = red[0][j], b = red[0][3 + j];
-        for (int q = 1; q < (int)(blockDim.x >> 6); ++q) {
-            a = red[q][j] < a ? red[q][j] : a;
-            b = red[q][3 + j] > b ? red[q][3 + j] : b;
-        }
-        atomicMin(&box[j], ord_key(a));
-        atomicMax(&box[3 + j], ord_key(b));
-    }
-}
-
-// Validation of two triangle meshes in three launches instead of nine (every
-// launch before the fork delays the broad phase): the counters reset with the
-// raw-box minima preset in one block, both raw boxes in one reduction (each
-// thread keeps one box per mesh, so a block may straddle the meshes), and both
-// meshes' faces checked with their offset tables written in one pass.
-__global__ void __launch_bounds__(256) k_reset_counters(Counters* C, int first_mesh)
+// The counters, with the raw-box minima preset, and a resident source's part.
+__global__ void __launch_bounds__(256) k_reset_counters(Counters* C, Params* P, const ResidentGpuView* res)
 {
     uint32_t* w = reinterpret_cast<uint32_t*>(C);
     for (uint32_t i = threadIdx.x; i < (uint32_t)(sizeof(Counters) / 4); i += blockDim.x) w[i] = 0u;
     __syncthreads();
     if (threadIdx.x < 6) {
         const int m = (int)threadIdx.x / 3, j = (int)threadIdx.x % 3;
-        if (m >= first_mesh) C->rbox[m][j] = ~0ull;
+        C->rbox[m][j] = res && m == 0 ? res->rbox[j] : ~0ull;
+        if (res && m == 0) C->rbox[0][3 + j] = res->rbox[3 + j];
+        if (res && m == 0) P->sum[0][j] = res->sum[j];
     }
+    if (res && threadIdx.x == 0) C->n_edges_src = res->ne;
 }
 
-__global__ void __launch_bounds__(256) k_raw_bbox2(const double* __restrict__ v0, uint32_t n0, const double* __restrict__ v1,
-                                                   uint32_t n1, Counters* C)
+// What a dispatch does before its streams part, in one launch (every launch
+// delays the broad phase, and each costs the host 4-5 us): blocks of raw
+// boxes, of face checks, of fills, of copies and of tile sums.
+struct HeadMesh {
+    const double* v;
+    const uint32_t* idx;
+    const uint32_t* sizes; // null: triangles, whose offsets are written here
+    uint32_t* off;
+    uint32_t* cface;       // polygons: face of each corner
+    uint32_t nv, nf;
+};
+struct Head {
+    HeadMesh mesh[2];      // a resident source: no vertices and faces
+    uint32_t* zero;        // the candidate-face flags and the edge numbering's counters
+    uint64_t nzero;
+    const uint32_t* from[4]; // a resident source's edges
+    uint32_t* to[4];
+    uint32_t ncopy;
+    SumBufs sums;
+    uint32_t box, face, fill, copy; // blocks of each kind; the rest: 6 sums.nblk tile sums
+};
+
+// both raw boxes, one atomic per block and coordinate after an LDS reduction
+// (each thread keeps a box per mesh: a block may straddle the meshes)
+__device__ inline void head_boxes(const Head& H, uint32_t blk, double (*red)[2][6], Counters* C)
 {
-    __shared__ double red[4][2][6];
+    const uint32_t n0 = H.mesh[0].nv, n1 = H.mesh[1].nv;
     double lo[2][3], hi[2][3];
     for (int m = 0; m < 2; ++m)
         for (int j = 0; j < 3; ++j) {
@@ -1387,9 +1488,9 @@ __global__ void __launch_bounds__(256) k_raw_bbox2(const double* __restrict__ v0
             hi[m][j] = -1.7976931348623157e308;
         }
     const uint64_t n = (uint64_t)n0 + n1;
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t i = blk * 256ull + threadIdx.x; i < n; i += H.box * 256ull) {
         const int m = i >= n0;
-        const double* p = m ? v1 + 3 * (i - n0) : v0 + 3 * i;
+        const double* p = m ? H.mesh[1].v + 3 * (i - n0) : H.mesh[0].v + 3 * i;
         for (int j = 0; j < 3; ++j) {
             const double x = p[j];
             lo[m][j] = x < lo[m][j] ? x : lo[m][j];
@@ -1415,7 +1516,7 @@ __global__ void __launch_bounds__(256) k_raw_bbox2(const double* __restrict__ v0
         const int m = (int)threadIdx.x / 3, j = (int)threadIdx.x % 3;
         if (m ? n1 : n0) {
             double a = red[0][m][j], b = red[0][m][3 + j];
-            for (int q = 1; q < (int)(blockDim.x >> 6); ++q) {
+            for (int q = 1; q < 4; ++q) {
                 a = red[q][m][j] < a ? red[q][m][j] : a;
                 b = red[q][m][3 + j] > b ? red[q][m][3 + j] : b;
             }
@@ -1425,25 +1526,50 @@ __global__ void __launch_bounds__(256) k_raw_bbox2(const double* __restrict__ v0
     }
 }
 
-// faces of both triangle meshes (nf0 = 0 skips the source): off[f] = 3 f,
 // every vertex index below its mesh's count, no vertex twice in a face
-__global__ void k_validate_tri2(const uint32_t* __restrict__ idx0, uint32_t* __restrict__ off0, uint32_t nf0, uint32_t nv0,
-                                const uint32_t* __restrict__ idx1, uint32_t* __restrict__ off1, uint32_t nf1, uint32_t nv1,
-                                Counters* C)
+__device__ inline void head_faces(const Head& H, uint32_t blk, Counters* C)
 {
-    const uint64_t n = (uint64_t)nf0 + nf1;
-    for (uint64_t g = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; g < n; g += (uint64_t)gridDim.x * blockDim.x) {
-        const int m = g >= nf0;
-        const uint32_t f = (uint32_t)(m ? g - nf0 : g);
-        uint32_t* off = m ? off1 : off0;
-        const uint32_t nf = m ? nf1 : nf0;
-        off[f] = 3 * f;
-        if (f + 1 == nf) off[nf] = 3 * nf;
-        const uint32_t* idx = m ? idx1 : idx0;
-        const uint32_t nv = m ? nv1 : nv0;
-        const uint32_t a = idx[3 * (uint64_t)f], b = idx[3 * (uint64_t)f + 1], c = idx[3 * (uint64_t)f + 2];
-        if (a >= nv || b >= nv || c >= nv || a == b || b == c || a == c) atomicOr(&C->bad_input, 1u);
+    const uint32_t n0 = H.mesh[0].nf;
+    const uint64_t n = (uint64_t)n0 + H.mesh[1].nf;
+    for (uint64_t g = blk * 256ull + threadIdx.x; g < n; g += H.face * 256ull) {
+        const HeadMesh& M = H.mesh[g >= n0];
+        const uint32_t f = (uint32_t)(g >= n0 ? g - n0 : g);
+        bool bad;
+        if (!M.sizes) {
+            M.off[f] = 3 * f;
+            if (f + 1 == M.nf) M.off[M.nf] = 3 * M.nf;
+            const uint32_t* i = M.idx + 3 * (uint64_t)f;
+            const uint32_t a = i[0], b = i[1], c = i[2];
+            bad = a >= M.nv || b >= M.nv || c >= M.nv || a == b || b == c || a == c;
+        } else {
+            const uint32_t b = M.off[f], k = M.sizes[f];
+            bad = face_bad(M.idx + b, k, M.nv);
+            for (uint32_t c = 0; c < k; ++c) M.cface[b + c] = f;
+        }
+        if (bad) atomicOr(&C->bad_input, 1u);
     }
+}
+
+__global__ void __launch_bounds__(256) k_head(Head H, Counters* C)
+{
+    __shared__ double red[4][2][6];
+    uint32_t b = blockIdx.x;
+    if (b < H.box) return head_boxes(H, b, red, C);
+    b -= H.box;
+    if (b < H.face) return head_faces(H, b, C);
+    b -= H.face;
+    if (b < H.fill) {
+        for (uint64_t i = b * 256ull + threadIdx.x; i < H.nzero; i += H.fill * 256ull) H.zero[i] = 0u;
+        return;
+    }
+    b -= H.fill;
+    if (b < H.copy) {
+        for (uint64_t i = b * 256ull + threadIdx.x; i < H.ncopy; i += H.copy * 256ull)
+            for (int q = 0; q < 4; ++q) H.to[q][i] = H.from[q][i];
+        return;
+    }
+    b -= H.copy;
+    sum_block(H.sums, b / 6, (int)(b % 6), &red[0][0][0]);
 }
 
 // 21-bit Morton codes (128 cells per axis) of raw face-box centres with the
@@ -1470,14 +1596,30 @@ struct MortonMesh {
 
 // leaves of both meshes in one launch: faces [start, nf0 + nf1) of the soup
 // (start = nf0 when the source's leaves are already made)
-__global__ void k_morton_raw(MortonMesh M0, MortonMesh M1, uint32_t start, uint32_t* __restrict__ code,
-                             uint32_t* __restrict__ face, float* __restrict__ rawbox, const Params* __restrict__ P,
-                             const Counters* __restrict__ C, uint32_t* __restrict__ zero, uint64_t nzero)
+// Every block finds the tolerance of the raw boxes (a launch of its own would
+// delay this one); block 0 records it.  drop: low code bits left out.
+__global__ void k_morton_raw(MortonMesh M0, MortonMesh M1, uint32_t start, int drop, uint32_t* __restrict__ code,
+                             uint32_t* __restrict__ face, float* __restrict__ rawbox, TolArgs A, Params* P, Counters* C,
+                             uint32_t* __restrict__ zero, uint64_t nzero)
 {
+    __shared__ double tol[3];
+    __shared__ int none;
+    if (threadIdx.x == 0) {
+        bool loose = false;
+        const bool finite = tolerance_of(C->rbox, A.nv0, A.nv1, A.gp_constant, A.absolute, tol, &loose);
+        loose = loose && finite && A.allow_loose; // the rerun in shifted coordinates finds the pairs
+        none = !finite || loose;
+        if (blockIdx.x == 0) {
+            for (int j = 0; j < 3; ++j) P->tol[j] = tol[j];
+            if (!finite) atomicOr(&C->unsupported, 2u);
+            if (loose) C->loose = 1u;
+        }
+    }
+    __syncthreads();
     // the leaf sort's group totals (radix_ghist), cleared here rather than by a launch of their own
     for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nzero; i += (uint64_t)gridDim.x * blockDim.x)
         zero[i] = 0u;
-    const bool aborted = dispatch_aborted(C) || C->loose; // loose: the rerun in shifted coordinates finds the pairs
+    const bool aborted = C->bad_input != 0 || none;
     const uint32_t F = M0.nf + M1.nf;
     for (uint64_t g = start + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; g < F; g += (uint64_t)gridDim.x * blockDim.x) {
         const bool cutm = g >= M0.nf;
@@ -1486,7 +1628,7 @@ __global__ void k_morton_raw(MortonMesh M0, MortonMesh M1, uint32_t start, uint3
         face[g] = f;
         float* o = rawbox + 6 * g;
         if (aborted) { // empty box: the broad phase finds nothing
-            code[g] = M.mesh_bit;
+            code[g] = M.mesh_bit >> drop;
             o[0] = o[1] = o[2] = 3.402823466e38f;
             o[3] = o[4] = o[5] = -3.402823466e38f;
             continue;
@@ -1509,7 +1651,7 @@ __global__ void k_morton_raw(MortonMesh M0, MortonMesh M1, uint32_t start, uint3
             x = fminf(fmaxf(x * 128.0f, 0.0f), 127.0f);
             c[j] = expand_bits10((uint32_t)x);
         }
-        code[g] = (c[0] * 4 + c[1] * 2 + c[2]) | M.mesh_bit;
+        code[g] = ((c[0] * 4 + c[1] * 2 + c[2]) | M.mesh_bit) >> drop;
         // single precision, rounded outward, relative to the source mesh's raw
         // lower corner (a resident source keeps its tree in that frame): far
         // from the origin float32 would otherwise merge whole meshes into one
@@ -1518,7 +1660,7 @@ __global__ void k_morton_raw(MortonMesh M0, MortonMesh M1, uint32_t start, uint3
         // covers them, so the float box still contains the exact box and the
         // superset property carries over.
         for (int j = 0; j < 3; ++j) {
-            const double t = M.widen ? P->tol[j] : 0.0;
+            const double t = M.widen ? tol[j] : 0.0;
             const double org = ord_value(M0.rbox[j]);
             const double dlo = mn[j] - org, dhi = mx[j] - org;
             o[j] = __double2float_rd((dlo - t) - (fabs(dlo) + t) * 3.552713678800501e-15);
@@ -1535,7 +1677,7 @@ __global__ void k_morton_raw(MortonMesh M0, MortonMesh M1, uint32_t start, uint3
 // raw union box (s() is monotone, so it bounds every shifted box up to
 // rounding); codes only order the leaves, and the clamp absorbs the rest.
 __global__ void k_morton_shifted(const double* __restrict__ box, uint32_t nf0, uint32_t nf1, const Params* __restrict__ P,
-                                 const Counters* __restrict__ C, uint32_t* __restrict__ code, uint32_t* __restrict__ face,
+                                 const Counters* __restrict__ C, int drop, uint32_t* __restrict__ code, uint32_t* __restrict__ face,
                                  float* __restrict__ rawbox, uint32_t* __restrict__ zero, uint64_t nzero)
 {
     for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nzero; i += (uint64_t)gridDim.x * blockDim.x)
@@ -1556,7 +1698,7 @@ __global__ void k_morton_shifted(const double* __restrict__ box, uint32_t nf0, u
         float* o = rawbox + 6 * g;
         const uint32_t mesh_bit = cutm ? (1u << 21) : 0u;
         if (aborted) {
-            code[g] = mesh_bit;
+            code[g] = mesh_bit >> drop;
             o[0] = o[1] = o[2] = 3.402823466e38f;
             o[3] = o[4] = o[5] = -3.402823466e38f;
             continue;
@@ -1570,7 +1712,7 @@ __global__ void k_morton_shifted(const double* __restrict__ box, uint32_t nf0, u
             o[j] = __double2float_rd(b[j]);
             o[3 + j] = __double2float_ru(b[3 + j]);
         }
-        code[g] = (c[0] * 4 + c[1] * 2 + c[2]) | mesh_bit;
+        code[g] = ((c[0] * 4 + c[1] * 2 + c[2]) | mesh_bit) >> drop;
     }
 }
 
@@ -3569,7 +3711,7 @@ __global__ void k_segment_ids(const uint32_t* __restrict__ starts, uint32_t nseg
 }
 
 // Face lists of a batch mesh part: checks every pair's faces against its own
-// vertex count (as k_validate does for one mesh) and writes the indices as
+// vertex count (as k_head does for one pair) and writes the indices as
 // ids of the concatenated part.
 __global__ void k_batch_globalize(const uint32_t* __restrict__ idx, const uint32_t* __restrict__ off,
                                   const uint32_t* __restrict__ sizes, uint32_t nf, int m, uint32_t fofs,

@@ -47,6 +47,7 @@ struct Counters {
     unsigned int gp, bad_src, bad_cut, unsupported, nonmanifold, bad_input, pair_fail, partial;
     unsigned int sum_next; // batches: work-queue head of the serial sums
     unsigned int ov_trip;  // the triplet scratch overflowed
+    unsigned int sums_done; // chains of the coordinate sums that have ended (k_sum_chain)
     unsigned int ov_nodes; // a list of node pairs overflowed: the tree is walked instead
     unsigned int ov_topo;  // a bucket of the edge numbering overflowed: the hash tables number the edges
     unsigned int trav_q[8]; // persistent traversal: head of each work queue (blocks taken)

@@ -75,7 +75,7 @@ const char* kStageNames[ST_COUNT] = {"coordinate_sums", "shift_params", "shift_b
 
 // event slots: stage boundaries on the three streams
 enum Ev { EV_A0, EV_S0, EV_A_SUMS, EV_A_PARAMS, EV_A_SHIFT, EV_A_BOXES, EV_A_JOIN, EV_A_FILTER, EV_A_PLANES, EV_A_JOIN2, EV_A_TESTS, EV_A_NARROW,
-          EV_A_END, EV_FORK, EV_B0, EV_B_SORT, EV_B_REFIT, EV_B_TRAV, EV_C0, EV_C_FILL, EV_C_TOPO, EV_SUM_ITEMS, EV_SUM_CHAIN,
+          EV_A_END, EV_FORK, EV_B0, EV_B_SORT, EV_B_REFIT, EV_B_TRAV, EV_C0, EV_C_TOPO, EV_SUM_ITEMS, EV_SUM_CHAIN,
           EV_TRAV_K0, EV_TRAV_K1, EV_B_CC, EV_COUNT };
 
 // Launch shape of the traversal kernel, chosen per workload class by the
@@ -811,6 +811,14 @@ void enqueue_narrow(mcgpu_context ctx, const Soup& S, bool join_topology, PairRu
 // lists write empty boxes when the input was rejected, so no later kernel
 // indexes a vertex through a bad face list, and the host reports the
 // rejection after the dispatch.
+TolArgs tol_args(mcgpu_context ctx)
+{
+    const bool absolute = (ctx->flags & MCGPU_DISPATCH_ENFORCE_GENERAL_POSITION_ABSOLUTE) != 0;
+    return TolArgs{ctx->nv[0], ctx->nv[1], ctx->gp_constant, absolute ? 1 : 0, (ctx->allow_loose && !ctx->res) ? 1 : 0};
+}
+
+constexpr uint32_t kSmallOffsets = 1u << 16; // faces whose offsets one block scans
+
 void enqueue_validate(mcgpu_context ctx)
 {
     ctx->state_copied = false; // a state copy belongs to the dispatch it follows
@@ -820,36 +828,49 @@ void enqueue_validate(mcgpu_context ctx)
     Counters* C = &P_<DevState>(ctx->state)->C;
     uint32_t* etotal = P_<uint32_t>(ctx->etotal);
     ev_record(ctx, EV_A0, s);
-    if (!ctx->dsz[0] && !ctx->dsz[1]) { // two triangle meshes: three launches (k_reset_counters)
-        const int m0 = ctx->res ? 1 : 0;
-        k_reset_counters<<<1, kBlock, 0, s>>>(C, m0);
-        if (ctx->res) k_resident_source<<<1, 1, 0, s>>>(C, &P_<DevState>(ctx->state)->P, ctx->res->dres);
-        const uint32_t n0 = m0 ? 0u : ctx->nv[0], f0 = m0 ? 0u : ctx->nf[0];
-        k_raw_bbox2<<<grid_for((uint64_t)n0 + ctx->nv[1], kBlock, 64), kBlock, 0, s>>>(m0 ? nullptr : ctx->dv[0], n0,
-                                                                                         ctx->dv[1], ctx->nv[1], C);
-        k_validate_tri2<<<grid_for((uint64_t)f0 + ctx->nf[1]), kBlock, 0, s>>>(
-            ctx->didx[0], P_<uint32_t>(ctx->off[0]), f0, ctx->nv[0], ctx->didx[1], P_<uint32_t>(ctx->off[1]), ctx->nf[1],
-            ctx->nv[1], C);
-    } else {
-    fill_u32(C, 0u, sizeof(Counters) / 4, s);
-    if (ctx->res) k_resident_source<<<1, 1, 0, s>>>(C, &P_<DevState>(ctx->state)->P, ctx->res->dres);
-    for (int m = 0; m < 2; ++m) {
-        if (ctx->res && m == 0) continue; // resident source: validated, boxed and summed once
-        fill_u64(C->rbox[m], ~0ull, 3, s);
-        k_raw_bbox<<<grid_for(ctx->nv[m], kBlock, 64), kBlock, 0, s>>>(ctx->dv[m], ctx->nv[m], C->rbox[m]);
+    k_reset_counters<<<1, kBlock, 0, s>>>(C, &P_<DevState>(ctx->state)->P, ctx->res ? ctx->res->dres : nullptr);
+    // polygon meshes' face offsets
+    OffsetMesh om[2]{};
+    for (int m = ctx->res ? 1 : 0; m < 2; ++m) {
+        if (!ctx->dsz[m]) continue;
         uint32_t* off = P_<uint32_t>(ctx->off[m]);
-        if (ctx->dsz[m]) {
+        if (ctx->nf[m] <= kSmallOffsets) {
+            om[m] = OffsetMesh{ctx->dsz[m], off, ctx->nf[m]};
+        } else {
             scan_exclusive(ctx->dsz[m], off, ctx->nf[m], P_<uint32_t>(ctx->scan_tmp), etotal + m, s);
             k_offsets_tail<<<1, 1, 0, s>>>(off, ctx->nf[m], etotal + m);
-        } else {
-            k_triangle_offsets<<<grid_for((uint64_t)ctx->nf[m] + 1), kBlock, 0, s>>>(off, ctx->nf[m]);
         }
-        k_validate<<<grid_for(ctx->nf[m]), kBlock, 0, s>>>(ctx->didx[m], off, ctx->dsz[m], ctx->nf[m], ctx->nv[m], C);
     }
+    if (om[0].sizes || om[1].sizes) k_small_offsets<<<2, 1024, 0, s>>>(om[0], om[1]);
+    Head H{};
+    uint64_t nv = 0, nf = 0;
+    for (int m = 0; m < 2; ++m) {
+        if (ctx->res && m == 0) continue; // resident source: validated, boxed and summed once
+        H.mesh[m] = HeadMesh{ctx->dv[m], ctx->didx[m], ctx->dsz[m], P_<uint32_t>(ctx->off[m]),
+                             ctx->dsz[m] ? P_<uint32_t>(ctx->cface[m]) : nullptr, ctx->nv[m], ctx->nf[m]};
+        nv += ctx->nv[m];
+        nf += ctx->nf[m];
     }
-    const bool absolute = (ctx->flags & MCGPU_DISPATCH_ENFORCE_GENERAL_POSITION_ABSOLUTE) != 0;
-    k_tolerance<<<1, 1, 0, s>>>(&P_<DevState>(ctx->state)->P, C, ctx->nv[0], ctx->nv[1], ctx->gp_constant,
-                                absolute ? 1 : 0, (ctx->allow_loose && !ctx->res) ? 1 : 0);
+    H.zero = P_<uint32_t>(ctx->cand);
+    H.nzero = (uint64_t)ctx->nf[0] + ctx->nf[1] + 8 + topo_counters(ctx);
+    if (ctx->res) { // the resident source's edges occupy [0, ne) of the edge table
+        const void* from[4] = {ctx->res->ev0, ctx->res->ev1, ctx->res->ef0, ctx->res->ef1};
+        void* to[4] = {ctx->ev0.p, ctx->ev1.p, ctx->ef0.p, ctx->ef1.p};
+        for (int q = 0; q < 4; ++q) {
+            H.from[q] = (const uint32_t*)from[q];
+            H.to[q] = (uint32_t*)to[q];
+        }
+        H.ncopy = ctx->res->ne;
+    }
+    H.sums = sum_bufs(ctx);
+    H.box = (uint32_t)grid_for(nv, 4 * kBlock, 256);
+    H.face = (uint32_t)grid_for(nf, kBlock, 1024);
+    H.fill = (uint32_t)grid_for(H.nzero, 8 * kBlock, 128);
+    H.copy = H.ncopy ? (uint32_t)grid_for(H.ncopy, 4 * kBlock, 128) : 0;
+    const uint32_t tiles = ctx->sum_items && !ctx->pairs_given ? 6 * H.sums.nblk : 0;
+    k_head<<<H.box + H.face + H.fill + H.copy + tiles, kBlock, 0, s>>>(H, C);
+    if (ctx->pairs_given || ctx->shifted_bp) // k_morton_raw finds it otherwise
+        k_tolerance<<<1, 1, 0, s>>>(&P_<DevState>(ctx->state)->P, C, tol_args(ctx));
 }
 
 // Batches: the same reset and validation, per pair: segment ids of every
@@ -874,6 +895,7 @@ void enqueue_validate_batch(mcgpu_context ctx)
     ev_record(ctx, EV_A0, s);
     fill_u32(C, 0u, sizeof(Counters) / 4, s);
     fill_u32(ctx->pflags.p, 0u, np, s);
+    fill_u32(ctx->cand.p, 0u, (uint64_t)ctx->nf[0] + ctx->nf[1] + 8 + topo_counters(ctx), s);
     k_segment_ids<<<grid_for(ctx->nv[0]), kBlock, 0, s>>>(st, np, ctx->nv[0], vp);
     k_segment_ids<<<grid_for(ctx->nv[1]), kBlock, 0, s>>>(st + np, np, ctx->nv[1], vp + ctx->nv[0]);
     k_segment_ids<<<grid_for(ctx->nf[0]), kBlock, 0, s>>>(st + 2 * np, np, ctx->nf[0], fp);
@@ -1199,9 +1221,17 @@ void enqueue_bvh_traverse(mcgpu_context ctx, hipStream_t st, Counters* C, bool g
     ev_record(ctx, EV_B_TRAV, st);
 }
 
-// Polygon-soup edge numbering on stream s3, and the candidate-face flags the
-// pair filter fills: records EV_C_FILL once the flags are clear and
-// EV_C_TOPO at the end.
+// Leaf key bits of a single pair: a sort pass (two launches) less for up to
+// 2^15 leaves, whose order within 32 cells an axis costs the trees nothing
+// that shows.
+constexpr int kMortonBits = 22;
+int leaf_bits(mcgpu_context ctx)
+{
+    const uint64_t leaves = (uint64_t)(ctx->res ? 0 : ctx->nf[0]) + ctx->nf[1];
+    return leaves <= (1u << 15) ? 16 : kMortonBits;
+}
+
+// Polygon-soup edge numbering on stream s3: records EV_C_TOPO at the end.
 void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
 {
     const uint64_t F = (uint64_t)ctx->nf[0] + ctx->nf[1];
@@ -1209,20 +1239,12 @@ void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
     stage_event(ctx, EV_C0, s3);
     uint32_t* etotal = P_<uint32_t>(ctx->etotal);
     const uint64_t K = ctx->ncorner[0] + ctx->ncorner[1];
-    fill_u32(ctx->cand.p, 0u, F + 8 + topo_counters(ctx), s3);
-    ev_record(ctx, EV_C_FILL, s3);
     const uint32_t res_ne = ctx->res ? ctx->res->ne : 0u;
-    if (ctx->res) { // the resident source's edges occupy [0, ne) of the edge table
-        (void)hipMemcpyAsync(ctx->ev0.p, ctx->res->ev0, 4ull * res_ne, hipMemcpyDeviceToDevice, s3);
-        (void)hipMemcpyAsync(ctx->ev1.p, ctx->res->ev1, 4ull * res_ne, hipMemcpyDeviceToDevice, s3);
-        (void)hipMemcpyAsync(ctx->ef0.p, ctx->res->ef0, 4ull * res_ne, hipMemcpyDeviceToDevice, s3);
-        (void)hipMemcpyAsync(ctx->ef1.p, ctx->res->ef1, 4ull * res_ne, hipMemcpyDeviceToDevice, s3);
-    }
     CornerMap cmap[2];
     for (int m = 0; m < 2; ++m) {
         cmap[m].off = P_<uint32_t>(ctx->off[m]);
         cmap[m].cface = ctx->dsz[m] ? P_<uint32_t>(ctx->cface[m]) : nullptr;
-        if (ctx->dsz[m] && !(ctx->res && m == 0))
+        if (ctx->batch && ctx->dsz[m]) // else: written by the head
             k_corner_faces<<<grid_for(ctx->nf[m]), kBlock, 0, s3>>>(cmap[m].off, ctx->nf[m], P_<uint32_t>(ctx->cface[m]));
     }
     // the scans of this stream use their own scratch: stream B's sort uses scan_tmp
@@ -1320,6 +1342,7 @@ void enqueue_cc_rounds(mcgpu_context ctx, hipStream_t st)
 
 void enqueue_frontend(mcgpu_context ctx)
 {
+    if (!ctx->batch) ctx->sort_bits = leaf_bits(ctx);
     hipStream_t s = ctx->s, s2 = ctx->batch ? ctx->s2b : ctx->s2, s3 = ctx->batch ? ctx->s3b : ctx->s3, ssum = ctx->ssum;
     if (ctx->one_stream) s2 = s3 = ssum = s;
     const uint32_t Fs = ctx->nf[0];
@@ -1344,18 +1367,16 @@ void enqueue_frontend(mcgpu_context ctx)
         stage_event(ctx, EV_S0, s);
         const SumBufs SB = sum_bufs(ctx);
         const dim3 grid(SB.nblk, 6);
-        if (ctx->sum_items) {
-            k_sum_blocks<<<grid, 256, 0, s>>>(SB);
-            k_sum_items<<<grid, kSumThreads, 0, s>>>(SB);
-        }
+        const ShiftArgs SA{ctx->nv[0], ctx->nv[1], ctx->gp_constant, absolute ? 1 : 0};
+        if (ctx->sum_items) k_sum_items<<<grid, kSumThreads, 0, s>>>(SB);
         ev_record(ctx, EV_SUM_ITEMS, s);
         ev_wait(ctx, ssum, EV_SUM_ITEMS);
-        k_sum_chain<<<6, kSumChain, 0, ssum>>>(SB, &C->zero, Pd);
+        k_sum_chain<<<6, kSumChain, 0, ssum>>>(SB, &C->zero, Pd, C, SA, ctx->sum_items ? 0 : 1);
         ev_record(ctx, EV_SUM_CHAIN, ssum);
         ev_wait(ctx, s, EV_SUM_CHAIN);
         if (ctx->sum_items) {
             k_sum_verify<<<grid, kSumThreads, 0, s>>>(SB);
-            k_sum_rest<<<6, 64, 0, s>>>(SB, &C->zero, Pd);
+            k_sum_rest<<<1, 384, 0, s>>>(SB, &C->zero, Pd, C, SA);
         }
         ev_record(ctx, EV_A_SUMS, s);
     }
@@ -1370,13 +1391,16 @@ void enqueue_frontend(mcgpu_context ctx)
         k_batch_shift_vertices<<<grid_for(3 * V), kBlock, 0, s>>>(ctx->dv[0], ctx->nv[0], ctx->dv[1], ctx->nv[1],
                                                                   P_<uint32_t>(ctx->vpair), Pb, P_<double>(ctx->ps_v));
     } else {
-        k_shift_params<<<1, 1, 0, s>>>(Pd, C, ctx->nv[0], ctx->nv[1], ctx->gp_constant, absolute ? 1 : 0, 0, 0.0, 0.0, 0.0);
-        stage_event(ctx, EV_A_PARAMS, s);
-        k_shift_vertices<<<grid_for(3 * V), kBlock, 0, s>>>(ctx->dv[0], ctx->nv[0], ctx->dv[1], ctx->nv[1], Pd,
-                                                            P_<double>(ctx->ps_v), 0);
+        stage_event(ctx, EV_A_PARAMS, s); // the last of the sum kernels made them
     }
     const Soup S = make_soup(ctx);
-    k_face_boxes<<<grid_for(F), kBlock, 0, s>>>(S, ctx->batch ? Pb : Pd, C, P_<double>(ctx->box), 0);
+    if (ctx->batch) {
+        k_face_boxes<<<grid_for(F), kBlock, 0, s>>>(S, Pb, C, P_<double>(ctx->box), 0);
+    } else {
+        const uint32_t fb = (uint32_t)grid_for(F);
+        k_shift_boxes<<<fb + (uint32_t)grid_for(3 * V, 4 * kBlock, 1024), kBlock, 0, s>>>(
+            S, ctx->dv[0], ctx->dv[1], Pd, C, fb, P_<double>(ctx->ps_v), P_<double>(ctx->box));
+    }
     stage_event(ctx, EV_A_SHIFT, s);
     if (ctx->shifted_bp) ev_record(ctx, EV_A_BOXES, s);
 
@@ -1390,8 +1414,8 @@ void enqueue_frontend(mcgpu_context ctx)
         uint32_t* zero = radix_ghist(RadixTemp{P_<uint32_t>(ctx->hist), P_<uint32_t>(ctx->scan_tmp)}, F, ctx->sort_bits,
                                      &nzero);
         k_morton_shifted<<<grid_for(F), kBlock, 0, s2>>>(P_<double>(ctx->box), ctx->nf[0], ctx->nf[1], Pd, C,
-                                                         P_<uint32_t>(ctx->mcode), P_<uint32_t>(ctx->mface), rawbox,
-                                                         zero, nzero);
+                                                         kMortonBits - ctx->sort_bits, P_<uint32_t>(ctx->mcode),
+                                                         P_<uint32_t>(ctx->mface), rawbox, zero, nzero);
     } else if (ctx->batch) {
         for (int m = 0; m < 2; ++m) {
             const uint32_t nf = ctx->nf[m];
@@ -1410,8 +1434,9 @@ void enqueue_frontend(mcgpu_context ctx)
         uint64_t nzero = 0;
         uint32_t* zero = radix_ghist(RadixTemp{P_<uint32_t>(ctx->hist), P_<uint32_t>(ctx->scan_tmp)}, F - start,
                                      ctx->sort_bits, &nzero);
-        k_morton_raw<<<grid_for(F - start), kBlock, 0, s2>>>(M[0], M[1], start, P_<uint32_t>(ctx->mcode),
-                                                             P_<uint32_t>(ctx->mface), rawbox, Pd, C, zero, nzero);
+        k_morton_raw<<<grid_for(F - start), kBlock, 0, s2>>>(M[0], M[1], start, kMortonBits - ctx->sort_bits,
+                                                             P_<uint32_t>(ctx->mcode), P_<uint32_t>(ctx->mface), rawbox,
+                                                             tol_args(ctx), Pd, C, zero, nzero);
     }
     if (tests_all_pairs(ctx)) launch_all_pairs(ctx, s2, C);
     else enqueue_bvh_traverse(ctx, s2, C, !ctx->batch); // k_morton_raw cleared the sort's group totals
@@ -1433,7 +1458,6 @@ void enqueue_frontend(mcgpu_context ctx)
 
     // ---- stream A: join the broad phase, exact filter, narrow phase ----
     ev_wait(ctx, s, EV_B_TRAV);
-    ev_wait(ctx, s, EV_C_FILL);
     stage_event(ctx, EV_A_JOIN, s);
     k_filter_pairs<<<grid_for(ctx->cap_pairs, kFilterTile, 2048), kStageBlock, 0, s>>>(P_<double>(ctx->box), P_<unsigned long long>(ctx->raw_pairs),
                                                                ctx->cap_pairs, Fs,
@@ -1648,7 +1672,7 @@ std::vector<uint64_t> graph_key(mcgpu_context ctx)
     std::vector<uint64_t> k;
     auto put = [&k](uint64_t x) { k.push_back(x); };
     auto ptr = [&k](const void* p) { k.push_back((uint64_t)(uintptr_t)p); };
-    put(ctx->batch), put(ctx->npairs), put(ctx->batch_mb), put(ctx->cc_check), put(ctx->sort_bits),
+    put(ctx->batch), put(ctx->npairs), put(ctx->batch_mb), put(ctx->cc_check), put(ctx->batch ? ctx->sort_bits : leaf_bits(ctx)),
         put(ctx->shifted_bp), put(ctx->walk), put(ctx->trav.walk), put(ctx->want_trees), put(ctx->one_stream), put(ctx->forced), put(ctx->cap_nodes), put(ctx->topo_hash), put(ctx->topo_buckets), put(ctx->topo_tiles), put(ctx->topo_bits),
         put(ctx->nseg),
         put(ctx->gbits), put(ctx->kbits);
@@ -2114,7 +2138,6 @@ static mcgpu_result frontend_prepare(mcgpu_context ctx, const mcgpu_mesh* src, c
     ctx->pairs_given = false;
     ctx->allow_loose = true;
     ctx->cc_check = (desc->flags & MCGPU_DISPATCH_CHECK_COMPONENTS) != 0;
-    ctx->sort_bits = 22;
     ctx->flags = desc->flags;
     ctx->gp_constant = desc->gp_constant;
     ctx->enforcement_count = desc->enforcement_count;
@@ -3064,7 +3087,6 @@ mcgpu_result slot_bind(mcgpu_server srv, mcgpu_context ctx, const mcgpu_mesh* cu
     ctx->walk = false;
     ctx->pairs_given = false;
     ctx->cc_check = (srv->desc.flags & MCGPU_DISPATCH_CHECK_COMPONENTS) != 0;
-    ctx->sort_bits = 22;
     ctx->flags = srv->desc.flags;
     ctx->gp_constant = srv->desc.gp_constant;
     ctx->enforcement_count = 0;
