@@ -257,4 +257,29 @@ __device__ __forceinline__ unsigned long long block_reserve(unsigned long long* 
     return base;
 }
 
+// Several small copies by one launch, between device memory and a pinned
+// stage: a copy of pageable memory costs 10-20 us a call, and as many calls as
+// there are arrays.  A row of blocks a segment; both ends at least 4-byte
+// aligned (buffers, and places of 16 bytes in the stage).
+constexpr int kCopySegs = 8;
+struct CopySegs {
+    const void* from[kCopySegs];
+    void* to[kCopySegs];
+    unsigned long long bytes[kCopySegs];
+};
+__global__ void __launch_bounds__(256) k_copy_segs(CopySegs S)
+{
+    const int q = blockIdx.y;
+    const uint64_t n = S.bytes[q], i0 = blockIdx.x * 256ull + threadIdx.x, stride = gridDim.x * 256ull;
+    const auto* f = static_cast<const uint32_t*>(S.from[q]);
+    auto* t = static_cast<uint32_t*>(S.to[q]);
+    const bool wide = ((reinterpret_cast<uintptr_t>(f) | reinterpret_cast<uintptr_t>(t)) & 15) == 0;
+    if (wide)
+        for (uint64_t i = i0; i < n / 16; i += stride)
+            reinterpret_cast<uint4*>(t)[i] = reinterpret_cast<const uint4*>(f)[i];
+    for (uint64_t i = (wide ? n / 16 * 4 : 0) + i0; i < n / 4; i += stride) t[i] = f[i];
+    if (i0 < n % 4) // the last bytes of an array of bytes
+        static_cast<uint8_t*>(S.to[q])[n - n % 4 + i0] = static_cast<const uint8_t*>(S.from[q])[n - n % 4 + i0];
+}
+
 } // namespace mcgpu

@@ -162,6 +162,12 @@ struct mcgpu_context_t {
     Buf off[2], state, ps_v, box; // state: DevState (counters and shift parameters)
     // pinned host copy of the state, enqueued right behind a dispatch's last
     // kernel so that finish() waits once instead of copying after the wait
+    // pinned stages of small copies in and out (kStageBytes each, made on first use)
+    char *stage_in = nullptr, *stage_out = nullptr;
+    uint64_t stage_used = 0;   // bytes of stage_in taken since it was last free
+    CopySegs stage_segs{};     // copies out of it not yet launched
+    int stage_count = 0;
+    std::mutex stage_mutex;    // results may be fetched by several threads
     DevState* hstate = nullptr;
     bool state_copied = false;
     Buf hkeys[2], hfirst[2], eflag[2], eid[2], cedge[2], cface[2], etotal; // edge hash tables (topo_tables)
@@ -919,6 +925,49 @@ void enqueue_validate_batch(mcgpu_context ctx)
 
 // per-pair results of a batch, after finish(): status bits and registry
 // ranges read back, statuses decided as for one pair
+// Device to host, ordered behind stream A's work and complete on return: up to
+// kStageBytes through the pinned stage by one launch, more by a copy each.
+struct Fetch {
+    void* to;
+    const void* from;
+    uint64_t bytes;
+};
+mcgpu_result fetch(mcgpu_context ctx, std::initializer_list<Fetch> list)
+{
+    CopySegs S{};
+    const Fetch* of[kCopySegs];
+    int n = 0;
+    uint64_t at = 0, most = 0, place[kCopySegs];
+    bool small = true;
+    for (const Fetch& f : list) {
+        if (!f.to || !f.bytes) continue;
+        of[n] = &f;
+        place[n++] = at;
+        at += (f.bytes + 15) & ~15ull;
+        most = std::max(most, f.bytes);
+    }
+    small = at <= (1u << 20);
+    if (!n) return MCGPU_SUCCESS;
+    CK(hipSetDevice(ctx->device));
+    if (!small) {
+        for (int q = 0; q < n; ++q) CK(hipMemcpyAsync(of[q]->to, of[q]->from, of[q]->bytes, hipMemcpyDeviceToHost, ctx->s));
+        CK(hipStreamSynchronize(ctx->s));
+        return MCGPU_SUCCESS;
+    }
+    std::lock_guard<std::mutex> lock(ctx->stage_mutex);
+    if (!ctx->stage_out) CK(hipHostMalloc((void**)&ctx->stage_out, 1u << 20, hipHostMallocDefault));
+    for (int q = 0; q < n; ++q) {
+        S.from[q] = of[q]->from;
+        S.to[q] = ctx->stage_out + place[q];
+        S.bytes[q] = of[q]->bytes;
+    }
+    k_copy_segs<<<dim3((unsigned)grid_for(most / 4 + 1, 4 * 256, 256), n), 256, 0, ctx->s>>>(S);
+    CK(hipGetLastError());
+    CK(hipStreamSynchronize(ctx->s));
+    for (int q = 0; q < n; ++q) std::memcpy(of[q]->to, ctx->stage_out + place[q], of[q]->bytes);
+    return MCGPU_SUCCESS;
+}
+
 mcgpu_result finish_batch(mcgpu_context ctx, mcgpu_frontend_info* info)
 {
     const uint32_t np = ctx->npairs;
@@ -927,10 +976,11 @@ mcgpu_result finish_batch(mcgpu_context ctx, mcgpu_frontend_info* info)
     ctx->hrend.resize(np);
     ctx->hstatus.resize(np);
     ctx->hpartial.resize(np);
-    CK(hipMemcpy(ctx->hflags.data(), ctx->pflags.p, 4ull * np, hipMemcpyDeviceToHost));
-    CK(hipMemcpy(ctx->hrstart.data(), ctx->rstart.p, 4ull * np, hipMemcpyDeviceToHost));
-    CK(hipMemcpy(ctx->hrend.data(), ctx->rend.p, 4ull * np, hipMemcpyDeviceToHost));
-    CK(hipMemcpy(ctx->hpairs.data(), ctx->bpairs.p, sizeof(BatchPair) * np, hipMemcpyDeviceToHost));
+    const mcgpu_result r = fetch(ctx, {{ctx->hflags.data(), ctx->pflags.p, 4ull * np},
+                                       {ctx->hrstart.data(), ctx->rstart.p, 4ull * np},
+                                       {ctx->hrend.data(), ctx->rend.p, 4ull * np},
+                                       {ctx->hpairs.data(), ctx->bpairs.p, sizeof(BatchPair) * np}});
+    if (r != MCGPU_SUCCESS) return r;
     int32_t first = MCGPU_STATUS_SUCCESS;
     for (uint32_t p = 0; p < np; ++p) {
         const uint32_t f = ctx->hflags[p];
@@ -1750,6 +1800,52 @@ mcgpu_result enqueue_dispatch(mcgpu_context ctx)
     return enqueue_state_copy(ctx);
 }
 
+// Host to device, on stream A: small arrays through the pinned stage, by one
+// launch for all (upload_flush, before their first use); others directly.
+constexpr uint64_t kStageBytes = 1u << 20;
+
+mcgpu_result upload_flush(mcgpu_context ctx)
+{
+    if (!ctx->stage_count) return MCGPU_SUCCESS;
+    uint64_t most = 0;
+    for (int q = 0; q < ctx->stage_count; ++q) most = std::max<uint64_t>(most, ctx->stage_segs.bytes[q]);
+    k_copy_segs<<<dim3((unsigned)grid_for(most / 4 + 1, 4 * 256, 256), ctx->stage_count), 256, 0, ctx->s>>>(ctx->stage_segs);
+    ctx->stage_count = 0;
+    CK(hipGetLastError());
+    return MCGPU_SUCCESS;
+}
+
+mcgpu_result upload(mcgpu_context ctx, void* to, const void* from, uint64_t bytes)
+{
+    if (!bytes) return MCGPU_SUCCESS;
+    const uint64_t padded = (bytes + 15) & ~15ull;
+    if (padded > kStageBytes - ctx->stage_used || ctx->stage_count == kCopySegs) {
+        CK(hipMemcpyAsync(to, from, bytes, hipMemcpyHostToDevice, ctx->s));
+        return MCGPU_SUCCESS;
+    }
+    if (!ctx->stage_in) CK(hipHostMalloc((void**)&ctx->stage_in, kStageBytes, hipHostMallocDefault));
+    char* p = ctx->stage_in + ctx->stage_used;
+    std::memcpy(p, from, bytes);
+    ctx->stage_segs.from[ctx->stage_count] = p;
+    ctx->stage_segs.to[ctx->stage_count] = to;
+    ctx->stage_segs.bytes[ctx->stage_count] = bytes;
+    ++ctx->stage_count;
+    ctx->stage_used += padded;
+    return MCGPU_SUCCESS;
+}
+
+// the start of an entry point that uploads: nothing left behind by one that
+// failed, and the stage free once stream A has read what it held
+mcgpu_result upload_begin(mcgpu_context ctx)
+{
+    ctx->stage_count = 0;
+    if (ctx->stage_used) {
+        CK(hipStreamSynchronize(ctx->s));
+        ctx->stage_used = 0;
+    }
+    return MCGPU_SUCCESS;
+}
+
 mcgpu_result upload_mesh(mcgpu_context ctx, int m, const mcgpu_mesh* mesh, bool on_device)
 {
     ctx->nv[m] = mesh->num_vertices;
@@ -1782,15 +1878,16 @@ mcgpu_result upload_mesh(mcgpu_context ctx, int m, const mcgpu_mesh* mesh, bool 
     uint32_t* ix;
     CK(ensure(ctx->in_v[m], 3ull * mesh->num_vertices, &v));
     CK(ensure(ctx->in_idx[m], k, &ix));
-    CK(hipMemcpyAsync(v, mesh->vertices, 24ull * mesh->num_vertices, hipMemcpyHostToDevice, ctx->s));
-    CK(hipMemcpyAsync(ix, mesh->face_indices, 4ull * k, hipMemcpyHostToDevice, ctx->s));
+    mcgpu_result r;
+    if ((r = upload(ctx, v, mesh->vertices, 24ull * mesh->num_vertices)) != MCGPU_SUCCESS) return r;
+    if ((r = upload(ctx, ix, mesh->face_indices, 4ull * k)) != MCGPU_SUCCESS) return r;
     ctx->dv[m] = v;
     ctx->didx[m] = ix;
     ctx->dsz[m] = nullptr;
     if (mesh->face_sizes) {
         uint32_t* sz;
         CK(ensure(ctx->in_sz[m], mesh->num_faces, &sz));
-        CK(hipMemcpyAsync(sz, mesh->face_sizes, 4ull * mesh->num_faces, hipMemcpyHostToDevice, ctx->s));
+        if ((r = upload(ctx, sz, mesh->face_sizes, 4ull * mesh->num_faces)) != MCGPU_SUCCESS) return r;
         ctx->dsz[m] = sz;
     }
     return MCGPU_SUCCESS;
@@ -2106,7 +2203,8 @@ MCGPU_API mcgpu_result mcgpu_release_context(mcgpu_context ctx)
         if (op.exec) (void)hipGraphExecDestroy(op.exec);
     for (Buf* b : context_bufs(ctx))
         if (b->p) (void)hipFree(b->p);
-    if (ctx->hstate) (void)hipHostFree(ctx->hstate);
+    for (void* p : {(void*)ctx->hstate, (void*)ctx->stage_in, (void*)ctx->stage_out})
+        if (p) (void)hipHostFree(p);
     for (int i = 0; i < EV_COUNT; ++i) (void)hipEventDestroy(ctx->ev[i]);
     if (ctx->ev_user) (void)hipEventDestroy(ctx->ev_user);
     if (ctx->own_streams) {
@@ -2142,8 +2240,10 @@ static mcgpu_result frontend_prepare(mcgpu_context ctx, const mcgpu_mesh* src, c
     ctx->gp_constant = desc->gp_constant;
     ctx->enforcement_count = desc->enforcement_count;
     ctx->keep_tests = desc->keep_tests ? 1 : 0;
+    if ((r = upload_begin(ctx)) != MCGPU_SUCCESS) return r;
     if ((r = upload_mesh(ctx, 0, src, desc->input_on_device != 0)) != MCGPU_SUCCESS) return r;
     if ((r = upload_mesh(ctx, 1, cut, desc->input_on_device != 0)) != MCGPU_SUCCESS) return r;
+    if ((r = upload_flush(ctx)) != MCGPU_SUCCESS) return r;
     const uint64_t F = (uint64_t)ctx->nf[0] + ctx->nf[1];
     ctx->gbits = bits_for(F + 1);
     ctx->kbits = ctx->gbits + bits_for(ctx->ncorner[0] + ctx->ncorner[1] + 1);
@@ -2262,6 +2362,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
     ctx->enforcement_count = desc->enforcement_count;
     ctx->keep_tests = 0;
     for (int m = 0; m < 2; ++m) {
+        if (m == 0 && (r = upload_begin(ctx)) != MCGPU_SUCCESS) return r;
         if ((r = upload_mesh(ctx, m, mesh[m], desc->input_on_device != 0)) != MCGPU_SUCCESS) return r;
         ctx->bin_idx[m] = ctx->didx[m];
     }
@@ -2337,11 +2438,13 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
             CK(ensure(ctx->bidx[m], ctx->ncorner[m], &u));
             ctx->didx[m] = P_<uint32_t>(ctx->bidx[m]);
         }
-        CK(hipMemcpyAsync(ctx->bpairs.p, ctx->hpairs.data(), sizeof(BatchPair) * np, hipMemcpyHostToDevice, ctx->s));
-        CK(hipMemcpyAsync(ctx->bstarts.p, ctx->hstarts.data(), 16ull * np, hipMemcpyHostToDevice, ctx->s));
-        CK(hipMemcpyAsync(ctx->border.p, ctx->horder.data(), 24ull * np, hipMemcpyHostToDevice, ctx->s));
-        if (!ctx->topo_hash)
-            CK(hipMemcpyAsync(ctx->tseg.p, ctx->hseg.data(), sizeof(TopoSeg) * ctx->nseg, hipMemcpyHostToDevice, ctx->s));
+        if ((r = upload_flush(ctx)) != MCGPU_SUCCESS) return r; // the meshes
+        if ((r = upload(ctx, ctx->bpairs.p, ctx->hpairs.data(), sizeof(BatchPair) * np)) != MCGPU_SUCCESS) return r;
+        if ((r = upload(ctx, ctx->bstarts.p, ctx->hstarts.data(), 16ull * np)) != MCGPU_SUCCESS) return r;
+        if ((r = upload(ctx, ctx->border.p, ctx->horder.data(), 24ull * np)) != MCGPU_SUCCESS) return r;
+        if (!ctx->topo_hash && (r = upload(ctx, ctx->tseg.p, ctx->hseg.data(), sizeof(TopoSeg) * ctx->nseg)) != MCGPU_SUCCESS)
+            return r;
+        if ((r = upload_flush(ctx)) != MCGPU_SUCCESS) return r;
     }
     if (ctx->cap_pairs < 4 * F) ctx->cap_pairs = std::max<uint64_t>(1 << 14, 4 * F);
     if (ctx->cap_tests < 2 * ctx->cap_pairs) ctx->cap_tests = 2 * ctx->cap_pairs;
@@ -2389,14 +2492,38 @@ MCGPU_API mcgpu_result mcgpu_get_batch_partial_cuts(mcgpu_context ctx, uint32_t*
     return MCGPU_SUCCESS;
 }
 
+// The candidate pairs in ascending order: by source face with a counting sort
+// where the pairs are not few among the faces (7,600 pairs of 20,480 faces:
+// 0.03 ms instead of 0.3), then each face's own.
+static mcgpu_result sorted_pairs(mcgpu_context ctx, std::vector<unsigned long long>& out)
+{
+    const uint64_t n = ctx->C.n_pairs;
+    out.resize(n);
+    const mcgpu_result r = fetch(ctx, {{out.data(), ctx->pairs.p, 8 * n}});
+    if (r != MCGPU_SUCCESS) return r;
+    const uint64_t nf = ctx->nf[0];
+    if (n < 64 || nf > 8 * n) {
+        std::sort(out.begin(), out.end());
+        return MCGPU_SUCCESS;
+    }
+    std::vector<uint64_t> at(nf + 1, 0);
+    for (unsigned long long k : out) ++at[(k >> 32) + 1];
+    for (uint64_t f = 0; f < nf; ++f) at[f + 1] += at[f];
+    std::vector<unsigned long long> h(n);
+    for (unsigned long long k : out) h[at[k >> 32]++] = k;
+    for (uint64_t f = 0, b = 0; f < nf; b = at[f++]) // at[f]: now the end of face f's pairs
+        if (at[f] - b > 1) std::sort(h.begin() + b, h.begin() + at[f]);
+    out.swap(h);
+    return MCGPU_SUCCESS;
+}
+
 MCGPU_API mcgpu_result mcgpu_get_batch_candidate_pairs(mcgpu_context ctx, uint32_t* triples, uint64_t capacity)
 {
     if (!ctx || !triples) return MCGPU_ERROR_INVALID_VALUE;
     if (!ctx->have || !ctx->batch) return MCGPU_ERROR_NO_RESULT;
     const uint64_t n = ctx->C.n_pairs;
-    std::vector<unsigned long long> h(n);
-    if (n) CK(hipMemcpy(h.data(), ctx->pairs.p, 8 * n, hipMemcpyDeviceToHost));
-    std::sort(h.begin(), h.end()); // source faces ascend with the pair
+    std::vector<unsigned long long> h;
+    if (const mcgpu_result r = sorted_pairs(ctx, h); r != MCGPU_SUCCESS) return r; // source faces ascend with the pair
     const uint64_t m = std::min<uint64_t>(n, capacity);
     uint32_t p = 0;
     for (uint64_t i = 0; i < m; ++i) {
@@ -2477,9 +2604,8 @@ MCGPU_API mcgpu_result mcgpu_broad_phase(mcgpu_context ctx, const double* src_bo
             dp, P_<unsigned long long>(ctx->raw_pairs), ctx->cap_pairs, num_src, nullptr, P_<unsigned long long>(ctx->pairs),
             nullptr, P_<uint32_t>(ctx->cand), P_<uint32_t>(ctx->cand_list), C);
         (void)hipEventRecord(ctx->ev[EV_A_END], s);
-        CK(hipStreamSynchronize(s));
         CK(hipGetLastError());
-        CK(hipMemcpy(&ctx->C, C, sizeof(Counters), hipMemcpyDeviceToHost));
+        if (const mcgpu_result r = fetch(ctx, {{&ctx->C, C, sizeof(Counters)}}); r != MCGPU_SUCCESS) return r;
         if (ctx->C.ov_nodes) {
             node_pairs_overflowed(ctx, ctx->C);
             continue;
@@ -2630,12 +2756,7 @@ MCGPU_API mcgpu_result mcgpu_get_registry(mcgpu_context ctx, uint32_t* edges, ui
     const uint64_t n = std::min<uint64_t>(ctx->C.n_reg, capacity);
     const Buf& be = ctx->batch ? ctx->rle : ctx->re; // batches: pair-local ids, pairs in order
     const Buf& bg = ctx->batch ? ctx->rlg : ctx->rg;
-    // ordered on the context's own stream (a server slot's stream synchronises with the null stream)
-    if (edges) CK(hipMemcpyAsync(edges, be.p, 4 * n, hipMemcpyDeviceToHost, ctx->s));
-    if (faces) CK(hipMemcpyAsync(faces, bg.p, 4 * n, hipMemcpyDeviceToHost, ctx->s));
-    if (points) CK(hipMemcpyAsync(points, ctx->rpts.p, 24 * n, hipMemcpyDeviceToHost, ctx->s));
-    CK(hipStreamSynchronize(ctx->s));
-    return MCGPU_SUCCESS;
+    return fetch(ctx, {{edges, be.p, 4 * n}, {faces, bg.p, 4 * n}, {points, ctx->rpts.p, 24 * n}});
 }
 
 MCGPU_API mcgpu_result mcgpu_registry_device(mcgpu_context ctx, const uint32_t** edges, const uint32_t** faces,
@@ -2655,9 +2776,8 @@ MCGPU_API mcgpu_result mcgpu_get_candidate_pairs(mcgpu_context ctx, uint32_t* pa
     if (!ctx || !pairs) return MCGPU_ERROR_INVALID_VALUE;
     if (!ctx->have) return MCGPU_ERROR_NO_RESULT;
     const uint64_t n = ctx->C.n_pairs;
-    std::vector<unsigned long long> h(n);
-    if (n) CK(hipMemcpy(h.data(), ctx->pairs.p, 8 * n, hipMemcpyDeviceToHost));
-    std::sort(h.begin(), h.end()); // listing order only; the set is the device's
+    std::vector<unsigned long long> h;
+    if (const mcgpu_result r = sorted_pairs(ctx, h); r != MCGPU_SUCCESS) return r; // listing order only; the set is the device's
     const uint64_t m = std::min<uint64_t>(n, capacity);
     for (uint64_t i = 0; i < m; ++i) {
         pairs[2 * i] = (uint32_t)(h[i] >> 32);
@@ -2876,7 +2996,7 @@ MCGPU_API mcgpu_result mcgpu_cutpath_edges(mcgpu_context ctx, const uint32_t* or
     if (err == hipSuccess) err = hipGetLastError();
     float ms = 0.f;
     if (err == hipSuccess) err = hipEventElapsedTime(&ms, e0, e1);
-    if (err == hipSuccess) err = hipMemcpy(&ctx->cp_counts, cc, sizeof(CutCounts), hipMemcpyDeviceToHost);
+    if (err == hipSuccess && fetch(ctx, {{&ctx->cp_counts, cc, sizeof(CutCounts)}}) != MCGPU_SUCCESS) err = ctx->last_error;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     CK(err);
@@ -2900,14 +3020,15 @@ MCGPU_API mcgpu_result mcgpu_get_cutpath_edges(mcgpu_context ctx, uint32_t* src,
     if (!ctx->cp_have) return MCGPU_ERROR_NO_RESULT;
     const uint64_t n = std::min<uint64_t>(ctx->cp_counts.edges, capacity);
     if (n == 0) return MCGPU_SUCCESS;
-    if (src) CK(hipMemcpy(src, ctx->cp_osrc.p, 4 * n, hipMemcpyDeviceToHost));
-    if (tgt) CK(hipMemcpy(tgt, ctx->cp_otgt.p, 4 * n, hipMemcpyDeviceToHost));
-    if (groups) CK(hipMemcpy(groups, ctx->cp_ogroup.p, 4 * n, hipMemcpyDeviceToHost));
-    if (kinds) CK(hipMemcpy(kinds, ctx->cp_okind.p, n, hipMemcpyDeviceToHost));
+    std::vector<uint32_t> a(faces ? n : 0), b(faces ? n : 0);
+    const mcgpu_result r = fetch(ctx, {{src, ctx->cp_osrc.p, 4 * n},
+                                       {tgt, ctx->cp_otgt.p, 4 * n},
+                                       {groups, ctx->cp_ogroup.p, 4 * n},
+                                       {kinds, ctx->cp_okind.p, n},
+                                       {a.data(), ctx->cp_ofa.p, 4ull * a.size()},
+                                       {b.data(), ctx->cp_ofb.p, 4ull * b.size()}});
+    if (r != MCGPU_SUCCESS) return r;
     if (faces) {
-        std::vector<uint32_t> a(n), b(n);
-        CK(hipMemcpy(a.data(), ctx->cp_ofa.p, 4 * n, hipMemcpyDeviceToHost));
-        CK(hipMemcpy(b.data(), ctx->cp_ofb.p, 4 * n, hipMemcpyDeviceToHost));
         for (uint64_t i = 0; i < n; ++i) {
             faces[2 * i] = a[i];
             faces[2 * i + 1] = b[i];
@@ -3098,7 +3219,9 @@ mcgpu_result slot_bind(mcgpu_server srv, mcgpu_context ctx, const mcgpu_mesh* cu
     ctx->didx[0] = r.didx;
     ctx->dsz[0] = r.dsz;
     mcgpu_result rr;
+    if ((rr = upload_begin(ctx)) != MCGPU_SUCCESS) return rr;
     if ((rr = upload_mesh(ctx, 1, cut, on_device)) != MCGPU_SUCCESS) return rr;
+    if ((rr = upload_flush(ctx)) != MCGPU_SUCCESS) return rr;
     const uint64_t F = (uint64_t)ctx->nf[0] + ctx->nf[1];
     ctx->gbits = bits_for(F + 1);
     ctx->kbits = ctx->gbits + bits_for(ctx->ncorner[0] + ctx->ncorner[1] + 1);
@@ -3593,8 +3716,10 @@ MCGPU_API mcgpu_result mcgpu_dispatch_narrow(mcgpu_context ctx, const mcgpu_mesh
     ctx->gp_constant = desc->gp_constant > 0.0 ? desc->gp_constant : 1e-4;
     ctx->enforcement_count = desc->enforcement_count;
     ctx->keep_tests = desc->keep_tests ? 1 : 0;
+    if ((r = upload_begin(ctx)) != MCGPU_SUCCESS) return r;
     if ((r = upload_mesh(ctx, 0, src, false)) != MCGPU_SUCCESS) return r;
     if ((r = upload_mesh(ctx, 1, cut, false)) != MCGPU_SUCCESS) return r;
+    if ((r = upload_flush(ctx)) != MCGPU_SUCCESS) return r;
     const uint32_t Fs = ctx->nf[0];
     const uint64_t F = (uint64_t)Fs + ctx->nf[1];
     const uint64_t K = ctx->ncorner[0] + ctx->ncorner[1];
