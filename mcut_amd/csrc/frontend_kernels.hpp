@@ -1102,8 +1102,13 @@ __global__ void __launch_bounds__(kTopoScatterBlock) k_topo_scatter(Topo T, uint
 // table, then its second corner, then every corner's partner.  A segment of
 // one bucket makes its words here.  A third corner on an edge, or a second one
 // in the first one's direction, is a non-manifold soup.
-__global__ void __launch_bounds__(kTopoBlock) k_topo_buckets(Topo T, Counters* C)
+// tsum (few rank tiles; else null): the first uses of each, which k_topo_count
+// finds otherwise, a launch later.
+constexpr uint32_t kTopoFewTiles = 64;
+__global__ void __launch_bounds__(kTopoBlock) k_topo_buckets(Topo T, uint32_t tiles0, uint32_t* tsum, Counters* C)
 {
+    __shared__ uint32_t firsts[kTopoFewTiles];
+    if (tsum && threadIdx.x < kTopoFewTiles) firsts[threadIdx.x] = 0u;
     __shared__ unsigned long long slot[kTopoCap];
     __shared__ uint32_t second[kTopoCap];
     constexpr int kPer = kTopoCap / kTopoBlock;
@@ -1164,7 +1169,13 @@ __global__ void __launch_bounds__(kTopoBlock) k_topo_buckets(Topo T, Counters* C
     for (int j = 0; j < kPer; ++j) {
         if (w[j] == kEmpty64 || slot[at[j]] != w[j]) continue;
         const uint32_t s = second[at[j]];
-        opp[(w[j] >> 1) & rm] = s == kNoCorner ? kNoCorner : (uint32_t)g.c0 + s;
+        const uint32_t r = (uint32_t)((w[j] >> 1) & rm);
+        opp[r] = s == kNoCorner ? kNoCorner : (uint32_t)g.c0 + s;
+        if (tsum) atomicAdd(&firsts[(g.m ? tiles0 : 0u) + ((uint32_t)g.c0 + r) / kTopoTile], 1u);
+    }
+    if (tsum) {
+        __syncthreads();
+        if (threadIdx.x < kTopoFewTiles && firsts[threadIdx.x]) atomicAdd(&tsum[threadIdx.x], firsts[threadIdx.x]);
     }
 }
 
@@ -1783,9 +1794,12 @@ __global__ void k_batch_morton_raw(const double* __restrict__ v, const uint32_t*
 
 // Broad phase over caller-given face boxes (min xyz, max xyz, doubles): the
 // union box of one mesh's face boxes, as order keys ...
-__global__ void __launch_bounds__(256) k_box_bounds(const double* __restrict__ box, uint32_t nf,
-                                                    unsigned long long* __restrict__ rbox)
+// both meshes' boxes (mesh blockIdx.y), the source's first
+__global__ void __launch_bounds__(256) k_box_bounds(const double* __restrict__ box, uint32_t nf0, uint32_t nf1, Counters* C)
 {
+    const uint32_t nf = blockIdx.y ? nf1 : nf0;
+    unsigned long long* rbox = C->rbox[blockIdx.y];
+    box += blockIdx.y ? 6ull * nf0 : 0;
     __shared__ double red[4][6];
     double lo[3] = {1.7976931348623157e308, 1.7976931348623157e308, 1.7976931348623157e308};
     double hi[3] = {-1.7976931348623157e308, -1.7976931348623157e308, -1.7976931348623157e308};
@@ -1822,10 +1836,19 @@ __global__ void __launch_bounds__(256) k_box_bounds(const double* __restrict__ b
 
 // ... and the leaf keys and single-precision leaf boxes (rounded outward) of
 // those face boxes, as k_morton_raw makes them from vertices
-__global__ void k_morton_boxes(const double* __restrict__ box, uint32_t nf, const unsigned long long* __restrict__ rbox,
+__global__ void k_morton_boxes(const double* __restrict__ box, uint32_t nf0, uint32_t nf1, const Counters* __restrict__ C,
                                uint32_t* __restrict__ code, uint32_t* __restrict__ face, float* __restrict__ fbox,
-                               uint32_t mesh_bit)
+                               uint32_t* __restrict__ cand, uint32_t* __restrict__ zero, uint64_t nzero)
 {
+    const uint32_t nf = blockIdx.y ? nf1 : nf0, mesh_bit = blockIdx.y ? 1u << 21 : 0u;
+    const unsigned long long* rbox = C->rbox[blockIdx.y];
+    if (blockIdx.y == 0) // the leaf sort's group totals (radix_ghist)
+        for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nzero; i += (uint64_t)gridDim.x * blockDim.x)
+            zero[i] = 0u;
+    if (blockIdx.y) {
+        box += 6ull * nf0, code += nf0, face += nf0, cand += nf0;
+        fbox += 6ull * nf0;
+    }
     double lo[3], ext[3];
     for (int j = 0; j < 3; ++j) {
         lo[j] = ord_value(rbox[j]);
@@ -1841,6 +1864,7 @@ __global__ void k_morton_boxes(const double* __restrict__ box, uint32_t nf, cons
             c[j] = expand_bits10((uint32_t)x);
         }
         code[f] = (c[0] * 4 + c[1] * 2 + c[2]) | mesh_bit;
+        cand[f] = 0u;
         face[f] = (uint32_t)f;
         float* o = fbox + 6 * f;
         for (int j = 0; j < 3; ++j) {
@@ -2322,7 +2346,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
 // again with the walk, which needs none.
 // ---------------------------------------------------------------------------
 constexpr int kPairLeavesLog = 5;  // leaves of a node at the last level of the lists
-constexpr int kPairStartLevel = 11; // 2^11 x 2^11 node pairs tested at the start: about 4 us of tests
+constexpr uint64_t kPairStart = 1ull << 22; // node pairs tested at the start: about 4 us of tests
 constexpr int kPairStep = 3;       // levels a side descends per step
 constexpr int kPairBlock = 512;    // 8 waves
 constexpr int kPairWaves = kPairBlock / 64;
@@ -3132,6 +3156,14 @@ __global__ void __launch_bounds__(kStageBlock) k_tests(Soup S, const unsigned lo
 // 8. narrow phase (kernel.cpp:2456-2658)
 // ===========================================================================
 
+// a dispatch of given pairs: no shift, the pairs' number
+__global__ void __launch_bounds__(256) k_given_pairs(Params* P, Counters* C, unsigned long long n)
+{
+    uint32_t* w = reinterpret_cast<uint32_t*>(P);
+    for (uint32_t i = threadIdx.x; i < (uint32_t)(sizeof(Params) / 4); i += blockDim.x) w[i] = 0u;
+    if (threadIdx.x == 0) C->n_raw = n;
+}
+
 struct TestOut {
     int8_t* qs;
     int8_t* rs;
@@ -3601,22 +3633,29 @@ __global__ void k_reg_merge(Soup S, const unsigned long long* __restrict__ skey,
         const unsigned long long k = skey[i];
         uint64_t rank = i - t * kRegTile;
         for (uint64_t u0 = 0; u0 < ntiles; u0 += kRegMergeILP) {
-            uint32_t lo[kRegMergeILP], hi[kRegMergeILP];
+            // entries below k in eight tiles at once: 13 halvings cover 4096,
+            // every load unconditional (a load behind a branch is waited for at
+            // once), so that the eight are in flight together
+            const unsigned long long* tile[kRegMergeILP];
+            uint32_t lo[kRegMergeILP], len[kRegMergeILP];
 #pragma unroll
             for (int q = 0; q < kRegMergeILP; ++q) {
-                const uint64_t u = u0 + q;
-                const uint64_t base = u * kRegTile;
+                const uint64_t u = u0 + q, base = u * kRegTile;
+                const bool other = u < ntiles && u != t;
+                tile[q] = skey + (other ? base : 0);
                 lo[q] = 0;
-                hi[q] = (u < ntiles && u != t) ? (uint32_t)((n - base) < (uint64_t)kRegTile ? (n - base) : kRegTile) : 0u;
+                len[q] = other ? (uint32_t)((n - base) < (uint64_t)kRegTile ? (n - base) : kRegTile) : 0u;
             }
-            for (int step = 0; step < 13; ++step) { // 13 halvings cover 4096 entries
+            for (int step = 0; step < 13; ++step) {
+                unsigned long long v[kRegMergeILP];
+#pragma unroll
+                for (int q = 0; q < kRegMergeILP; ++q) v[q] = tile[q][len[q] ? lo[q] + (len[q] >> 1) : 0];
 #pragma unroll
                 for (int q = 0; q < kRegMergeILP; ++q) {
-                    if (lo[q] < hi[q]) {
-                        const uint32_t mid = (lo[q] + hi[q]) >> 1;
-                        if (skey[(u0 + q) * kRegTile + mid] < k) lo[q] = mid + 1;
-                        else hi[q] = mid;
-                    }
+                    const uint32_t half = len[q] >> 1;
+                    const bool right = len[q] && v[q] < k;
+                    lo[q] += right ? half + 1 : 0;
+                    len[q] = right ? len[q] - half - 1 : half;
                 }
             }
 #pragma unroll
@@ -3685,10 +3724,14 @@ __global__ void k_status_check(Soup S, const unsigned long long* __restrict__ n_
     uint64_t slots = status_slots(*n_dev);
     if (slots > max_slots) slots = max_slots;
     for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < slots; i += (uint64_t)gridDim.x * blockDim.x)
-        if (hkeys[i] != kEmpty64 && hcnt[i] < 2) {
+    {
+        const unsigned long long k = hkeys[i];
+        const uint32_t c = hcnt[i];
+        if (k != kEmpty64 && c < 2) {
             atomicOr(&C->pair_fail, 1u);
-            pair_flag(S, (uint32_t)(hkeys[i] >> 32), PF_PAIR_FAIL); // the key's source face
+            pair_flag(S, (uint32_t)(k >> 32), PF_PAIR_FAIL); // the key's source face
         }
+    }
 }
 
 // ===========================================================================

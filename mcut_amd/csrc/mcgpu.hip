@@ -504,8 +504,9 @@ mcgpu_result alloc_edge_tables(mcgpu_context ctx)
     return MCGPU_SUCCESS;
 }
 
-// the edge numbering's counters behind the candidate-face flags: two a bucket, one a segment, one
-uint64_t topo_counters(mcgpu_context ctx) { return ctx->topo_hash ? 0 : 2ull * ctx->topo_buckets + ctx->nseg + 1; }
+// the edge numbering's counters behind the candidate-face flags: two a bucket, one a segment, one,
+// and those of few rank tiles
+uint64_t topo_counters(mcgpu_context ctx) { return ctx->topo_hash ? 0 : 2ull * ctx->topo_buckets + ctx->nseg + 1 + kTopoFewTiles; }
 
 uint32_t topo_rank_tiles(uint64_t corners) { return (uint32_t)((corners + kTopoTile - 1) / kTopoTile); }
 
@@ -1077,7 +1078,10 @@ void launch_node_pairs(const BroadView& B, const Tree& src, const Tree& cut, Cou
                        hipEvent_t b)
 {
     const int ts = std::max(0, src.D - kPairLeavesLog), tc = std::max(0, cut.D - kPairLeavesLog);
-    int ls = std::min(ts, kPairStartLevel), lc = std::min(tc, kPairStartLevel), step = 0;
+    int ls = ts, lc = tc, step = 0; // as deep as kPairStart tests allow: a step less for a small cut mesh
+    while ((uint64_t)level_nodes(src.n, src.D, ls) * level_nodes(cut.n, cut.D, lc) > kPairStart)
+        if (level_nodes(src.n, src.D, ls) >= level_nodes(cut.n, cut.D, lc)) --ls;
+        else --lc;
     const dim3 g0((level_nodes(src.n, src.D, ls) + 255) / 256, (level_nodes(cut.n, cut.D, lc) + 31) / 32);
     launch_timed(k_pairs_start, g0, dim3(256), st, a, (hipEvent_t) nullptr, src, cut, ls, lc, B.node_pairs[0], B.cap_nodes,
                  &C->n_nodes[0], &C->ov_nodes);
@@ -1125,8 +1129,10 @@ void launch_all_pairs(mcgpu_context ctx, hipStream_t st, Counters* C)
     ev_record(ctx, EV_B_TRAV, st);
 }
 
-// the steps of launch_node_pairs fit Counters::n_nodes for any tree of 32-bit leaves
-static_assert((32 - kPairLeavesLog - kPairStartLevel + kPairStep - 1) / kPairStep + 1 <= 8, "steps of the node-pair lists");
+// The steps of launch_node_pairs fit Counters::n_nodes for any trees of 32-bit
+// leaves: the start stops at the first level pair within its budget, so a side
+// starts at 2^10 nodes or more or at its last level.
+static_assert((32 - kPairLeavesLog - 10 + kPairStep - 1) / kPairStep + 1 <= 8, "steps of the node-pair lists");
 
 bool trav_config_valid(const TravConfig& t)
 {
@@ -1330,12 +1336,13 @@ void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
                 k_topo_scatter<true, kTopoMaxBits><<<gh, b, 0, s3>>>(T, n, C);
             }
         }
-        k_topo_buckets<<<ctx->topo_buckets, kTopoBlock, 0, s3>>>(T, C);
         const int cut_only = ctx->res ? 1 : 0;
         const uint32_t tiles0 = cut_only ? 0 : topo_rank_tiles(ctx->ncorner[0]);
         const uint32_t tiles = tiles0 + topo_rank_tiles(ctx->ncorner[1]);
-        uint32_t* tsum = P_<uint32_t>(ctx->tsum);
-        k_topo_count<<<tiles, kBlock, 0, s3>>>(T, tiles0, tsum);
+        const bool few = tiles <= kTopoFewTiles; // counted by the buckets, in counters that the head clears
+        uint32_t* tsum = few ? T.hashed + ctx->nseg + 1 : P_<uint32_t>(ctx->tsum);
+        k_topo_buckets<<<ctx->topo_buckets, kTopoBlock, 0, s3>>>(T, tiles0, few ? tsum : nullptr, C);
+        if (!few) k_topo_count<<<tiles, kBlock, 0, s3>>>(T, tiles0, tsum);
         const int scanned = tiles > kTopoDirectTiles;
         if (scanned) k_scan_tiles<<<1, kScanBlock, 0, s3>>>(tsum, tiles, etotal);
         k_topo_apply<<<tiles, kBlock, 0, s3>>>(T, tiles0, tiles, tsum, scanned, etotal, cut_only, C, P_<uint32_t>(ctx->ev0),
@@ -2580,26 +2587,31 @@ MCGPU_API mcgpu_result mcgpu_broad_phase(mcgpu_context ctx, const double* src_bo
         CK(ensure(ctx->nodes[m], 6 * ((2ull << D) - 1), &fp));
     }
     if (ctx->cap_pairs < 4 * F) ctx->cap_pairs = std::max<uint64_t>(1 << 14, 4 * F);
-    const hipMemcpyKind kind = input_on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
     for (int attempt = 0; attempt < 6; ++attempt) {
         CK(ensure(ctx->raw_pairs, ctx->cap_pairs, &ull));
         CK(ensure(ctx->pairs, ctx->cap_pairs, &ull));
         if (const mcgpu_result r = alloc_node_pairs(ctx); r != MCGPU_SUCCESS) return r;
         Counters* C = &st->C;
         (void)hipEventRecord(ctx->ev[EV_A0], s);
-        fill_u32(C, 0u, sizeof(Counters) / 4, s);
-        CK(hipMemcpyAsync(dp, src_boxes, 48ull * num_src, kind, s));
-        CK(hipMemcpyAsync(dp + 6ull * num_src, cut_boxes, 48ull * num_cut, kind, s));
-        for (int m = 0; m < 2; ++m) {
-            const uint64_t o = m ? num_src : 0;
-            fill_u64(C->rbox[m], ~0ull, 3, s);
-            k_box_bounds<<<grid_for(ctx->nf[m], kBlock, 64), kBlock, 0, s>>>(dp + 6 * o, ctx->nf[m], C->rbox[m]);
-            k_morton_boxes<<<grid_for(ctx->nf[m]), kBlock, 0, s>>>(dp + 6 * o, ctx->nf[m], C->rbox[m], P_<uint32_t>(ctx->mcode) + o,
-                                                                  P_<uint32_t>(ctx->mface) + o, P_<float>(ctx->rawbox) + 6 * o,
-                                                                  m ? (1u << 21) : 0u);
+        k_reset_counters<<<1, kBlock, 0, s>>>(C, &st->P, nullptr);
+        if (input_on_device) {
+            CK(hipMemcpyAsync(dp, src_boxes, 48ull * num_src, hipMemcpyDeviceToDevice, s));
+            CK(hipMemcpyAsync(dp + 6ull * num_src, cut_boxes, 48ull * num_cut, hipMemcpyDeviceToDevice, s));
+        } else if (attempt == 0) {
+            mcgpu_result r;
+            if ((r = upload_begin(ctx)) != MCGPU_SUCCESS) return r;
+            if ((r = upload(ctx, dp, src_boxes, 48ull * num_src)) != MCGPU_SUCCESS) return r;
+            if ((r = upload(ctx, dp + 6ull * num_src, cut_boxes, 48ull * num_cut)) != MCGPU_SUCCESS) return r;
+            if ((r = upload_flush(ctx)) != MCGPU_SUCCESS) return r;
         }
-        enqueue_bvh_traverse(ctx, s, C, false);
-        fill_u32(ctx->cand.p, 0u, F, s);
+        uint64_t nzero = 0;
+        uint32_t* zero = radix_ghist(RadixTemp{P_<uint32_t>(ctx->hist), P_<uint32_t>(ctx->scan_tmp)}, F, ctx->sort_bits, &nzero);
+        const uint32_t most = std::max(num_src, num_cut);
+        k_box_bounds<<<dim3(grid_for(most, kBlock, 64), 2), kBlock, 0, s>>>(dp, num_src, num_cut, C);
+        k_morton_boxes<<<dim3(grid_for(most), 2), kBlock, 0, s>>>(dp, num_src, num_cut, C, P_<uint32_t>(ctx->mcode),
+                                                                 P_<uint32_t>(ctx->mface), P_<float>(ctx->rawbox),
+                                                                 P_<uint32_t>(ctx->cand), zero, nzero);
+        enqueue_bvh_traverse(ctx, s, C, true);
         k_filter_pairs<<<grid_for(ctx->cap_pairs, kFilterTile, 2048), kStageBlock, 0, s>>>(
             dp, P_<unsigned long long>(ctx->raw_pairs), ctx->cap_pairs, num_src, nullptr, P_<unsigned long long>(ctx->pairs),
             nullptr, P_<uint32_t>(ctx->cand), P_<uint32_t>(ctx->cand_list), C);
@@ -3171,6 +3183,7 @@ mcgpu_result slot_create(int device, mcgpu_context* out)
     mcgpu_context ctx = new mcgpu_context_t();
     ctx->device = device;
     ctx->own_streams = false;
+    ctx->one_stream = true;
     // A slot's stream carries a CU mask (every CU), which gives it a hardware
     // queue of its own: plain streams share the process's few queues (four
     // by default), and in a program that had made and released other
@@ -3622,7 +3635,6 @@ MCGPU_API mcgpu_result mcgpu_broad_phase_noalloc(int device, const double* src_b
     unsigned char* base = scratch_on(device);
     if (!base) return MCGPU_ERROR_DEVICE;
     hipStream_t s = (hipStream_t)stream;
-    const uint64_t F = (uint64_t)num_src + num_cut;
     DevState* st = (DevState*)(base + kNa.state);
     Counters* C = &st->C;
     double* box = (double*)(base + kNa.box);
@@ -3633,18 +3645,13 @@ MCGPU_API mcgpu_result mcgpu_broad_phase_noalloc(int device, const double* src_b
     unsigned long long* raw = (unsigned long long*)(base + kNa.raw);
     unsigned long long* found = (unsigned long long*)(base + kNa.pairs);
 
-    fill_u32(C, 0u, sizeof(Counters) / 4, s);
+    k_reset_counters<<<1, kBlock, 0, s>>>(C, &st->P, nullptr);
     if (hipMemcpyAsync(box, src_boxes, 48ull * num_src, hipMemcpyDeviceToDevice, s) != hipSuccess ||
         hipMemcpyAsync(box + 6ull * num_src, cut_boxes, 48ull * num_cut, hipMemcpyDeviceToDevice, s) != hipSuccess)
         return MCGPU_ERROR_DEVICE;
-    const uint32_t nf[2] = {num_src, num_cut};
-    for (int m = 0; m < 2; ++m) {
-        const uint64_t o = m ? num_src : 0;
-        fill_u64(C->rbox[m], ~0ull, 3, s);
-        k_box_bounds<<<grid_for(nf[m], kBlock, 64), kBlock, 0, s>>>(box + 6 * o, nf[m], C->rbox[m]);
-        k_morton_boxes<<<grid_for(nf[m]), kBlock, 0, s>>>(box + 6 * o, nf[m], C->rbox[m], mcode + o, mface + o,
-                                                         rawbox + 6 * o, m ? (1u << 21) : 0u);
-    }
+    const uint32_t nf[2] = {num_src, num_cut}, most = std::max(num_src, num_cut);
+    k_box_bounds<<<dim3(grid_for(most, kBlock, 64), 2), kBlock, 0, s>>>(box, num_src, num_cut, C);
+    k_morton_boxes<<<dim3(grid_for(most), 2), kBlock, 0, s>>>(box, num_src, num_cut, C, mcode, mface, rawbox, cand, nullptr, 0);
     BroadView B{};
     B.mcode = mcode;
     B.mface = mface;
@@ -3664,7 +3671,6 @@ MCGPU_API mcgpu_result mcgpu_broad_phase_noalloc(int device, const double* src_b
     B.cap_pairs = kNaPairs;
     B.sort_bits = 22;
     enqueue_trees_traverse(B, s, C, false, nullptr, nullptr);
-    fill_u32(cand, 0u, F, s);
     k_filter_pairs<<<grid_for(kNaPairs, kFilterTile, 2048), kStageBlock, 0, s>>>(
         box, raw, kNaPairs, num_src, nullptr, found, nullptr, cand, (uint32_t*)(base + kNa.cand_list), C);
     Counters h;
@@ -3765,16 +3771,20 @@ MCGPU_API mcgpu_result mcgpu_dispatch_narrow(mcgpu_context ctx, const mcgpu_mesh
         enqueue_validate(ctx); // counters, face offsets, face-list validation
         DevState* st = P_<DevState>(ctx->state);
         Counters* C = &st->C;
-        fill_u32(&st->P, 0u, sizeof(Params) / 4, s); // no shift: the coordinates are the soup's own
+        k_given_pairs<<<1, 256, 0, s>>>(&st->P, C, (unsigned long long)num_pairs); // no shift: the coordinates are the soup's own
         // the soup's coordinates, face boxes and candidate pairs as given
-        CK(hipMemcpyAsync(ctx->ps_v.p, ctx->dv[0], 24ull * ctx->nv[0], hipMemcpyDeviceToDevice, s));
-        CK(hipMemcpyAsync(P_<double>(ctx->ps_v) + 3ull * ctx->nv[0], ctx->dv[1], 24ull * ctx->nv[1],
-                          hipMemcpyDeviceToDevice, s));
+        CopySegs own{};
+        for (int m = 0; m < 2; ++m) {
+            own.from[m] = ctx->dv[m];
+            own.to[m] = P_<double>(ctx->ps_v) + (m ? 3ull * ctx->nv[0] : 0);
+            own.bytes[m] = 24ull * ctx->nv[m];
+        }
+        k_copy_segs<<<dim3(256, 2), 256, 0, s>>>(own);
         CK(hipMemcpyAsync(ctx->box.p, src_boxes, 48ull * Fs, hipMemcpyHostToDevice, s));
         CK(hipMemcpyAsync(P_<double>(ctx->box) + 6ull * Fs, cut_boxes, 48ull * ctx->nf[1], hipMemcpyHostToDevice, s));
         if (num_pairs)
-            CK(hipMemcpyAsync(ctx->raw_pairs.p, keys.data(), 8ull * num_pairs, hipMemcpyHostToDevice, s));
-        fill_u64(&C->n_raw, (unsigned long long)num_pairs, 1, s);
+            if ((r = upload(ctx, ctx->raw_pairs.p, keys.data(), 8ull * num_pairs)) != MCGPU_SUCCESS) return r;
+        if ((r = upload_flush(ctx)) != MCGPU_SUCCESS) return r;
         if (topology) { // the caller's edge numbering
             for (int m = 0; m < 2; ++m)
                 CK(hipMemcpyAsync(ctx->cedge[m].p, topology->corner_edges[m], 4ull * ctx->ncorner[m],
@@ -3785,7 +3795,6 @@ MCGPU_API mcgpu_result mcgpu_dispatch_narrow(mcgpu_context ctx, const mcgpu_mesh
             CK(hipMemcpyAsync(ctx->ef1.p, topology->edge_f1, 4ull * NE, hipMemcpyHostToDevice, s));
             fill_u64(&C->n_edges_src, (unsigned long long)NE, 1, s);
             fill_u64(&C->n_edges_cut, 0ull, 1, s);
-            fill_u32(ctx->cand.p, 0u, F, s);
         } else {
             enqueue_topology(ctx, s);
         }
