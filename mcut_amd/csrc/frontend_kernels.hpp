@@ -655,12 +655,6 @@ __global__ void k_fill_u64(unsigned long long* p, unsigned long long v, uint64_t
         p[i] = v;
 }
 
-__global__ void k_triangle_offsets(uint32_t* __restrict__ off, uint32_t nf)
-{
-    for (uint64_t f = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; f <= nf; f += (uint64_t)gridDim.x * blockDim.x)
-        off[f] = (uint32_t)(3 * f);
-}
-
 __global__ void k_offsets_tail(uint32_t* __restrict__ off, uint32_t nf, const uint32_t* __restrict__ total)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) off[nf] = *total;
@@ -3740,43 +3734,85 @@ __global__ void k_status_check(Soup S, const unsigned long long* __restrict__ n_
 
 // out[base + i] = the segment of element i, starts[] being the first element
 // of each of the nseg segments (increasing)
-__global__ void k_segment_ids(const uint32_t* __restrict__ starts, uint32_t nseg, uint32_t n, uint32_t* __restrict__ out)
+// What a batch does first, in one launch: the pair of every vertex and face
+// (rows 0-3 of blocks), the fills (4) and the raw boxes' presets (5).
+struct BatchHead {
+    const uint32_t* starts; // vertex starts (source, cut), face starts (source, cut), np each
+    uint32_t np;
+    uint32_t n[4];
+    uint32_t* out[4];
+    uint32_t* pflags;
+    uint32_t* zero;
+    uint64_t nzero;
+    unsigned long long* rbox; // [np][2][6]
+};
+__global__ void k_batch_head(BatchHead H, Counters* C)
 {
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-        uint32_t lo = 0, hi = nseg; // last segment whose start is <= i
+    const uint64_t i0 = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
+    const uint32_t q = blockIdx.y;
+    if (q == 4) {
+        for (uint64_t i = i0; i < sizeof(Counters) / 4; i += stride) reinterpret_cast<uint32_t*>(C)[i] = 0u;
+        for (uint64_t i = i0; i < H.np; i += stride) H.pflags[i] = 0u;
+        for (uint64_t i = i0; i < H.nzero; i += stride) H.zero[i] = 0u;
+        return;
+    }
+    if (q == 5) {
+        for (uint64_t i = i0; i < 12ull * H.np; i += stride) H.rbox[i] = i % 6 < 3 ? ~0ull : 0ull;
+        return;
+    }
+    const uint32_t* starts = H.starts + (uint64_t)q * H.np;
+    for (uint64_t i = i0; i < H.n[q]; i += stride) {
+        uint32_t lo = 0, hi = H.np; // last segment whose start is <= i
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) >> 1;
             if (starts[mid] <= (uint32_t)i) lo = mid;
             else hi = mid;
         }
-        out[i] = lo;
+        H.out[q][i] = lo;
     }
 }
 
 // Face lists of a batch mesh part: checks every pair's faces against its own
 // vertex count (as k_head does for one pair) and writes the indices as
 // ids of the concatenated part.
-__global__ void k_batch_globalize(const uint32_t* __restrict__ idx, const uint32_t* __restrict__ off,
-                                  const uint32_t* __restrict__ sizes, uint32_t nf, int m, uint32_t fofs,
-                                  const uint32_t* __restrict__ fpair, const BatchPair* __restrict__ bp,
-                                  uint32_t* __restrict__ out, Counters* C)
+struct BatchFaces {
+    const uint32_t* idx;
+    uint32_t* off;
+    const uint32_t* sizes; // null: triangles, whose offsets are written here
+    uint32_t nf;
+    uint32_t* out;
+};
+__global__ void k_batch_globalize(BatchFaces M0, BatchFaces M1, const uint32_t* __restrict__ fpair,
+                                  const BatchPair* __restrict__ bp, Counters* C)
 {
-    for (uint64_t f = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; f < nf; f += (uint64_t)gridDim.x * blockDim.x) {
-        const BatchPair b = bp[fpair[fofs + f]];
+    const uint64_t n = (uint64_t)M0.nf + M1.nf;
+    for (uint64_t g = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; g < n; g += (uint64_t)gridDim.x * blockDim.x) {
+        const int m = g >= M0.nf;
+        const BatchFaces& M = m ? M1 : M0;
+        const uint32_t f = (uint32_t)(m ? g - M0.nf : g);
+        const BatchPair b = bp[fpair[g]];
         const uint32_t nv = m ? b.nvc : b.nvs, v0 = m ? b.vc0 : b.vs0;
-        const uint32_t o = off[f], n = sizes ? sizes[f] : 3u;
-        bool bad = n < 3;
-        for (uint32_t i = 0; i < n && !bad; ++i) {
-            const uint32_t a = idx[o + i];
-            bad = a >= nv;
-            for (uint32_t k = 0; k < i && !bad; ++k) bad = idx[o + k] == a;
-            out[o + i] = v0 + a;
+        bool bad;
+        if (!M.sizes) {
+            const uint32_t o = 3 * f;
+            M.off[f] = o;
+            if (f + 1 == M.nf) M.off[M.nf] = 3 * M.nf;
+            const uint32_t a = M.idx[o], c = M.idx[o + 1], d = M.idx[o + 2];
+            bad = a >= nv || c >= nv || d >= nv || a == c || c == d || a == d;
+            M.out[o] = v0 + a, M.out[o + 1] = v0 + c, M.out[o + 2] = v0 + d;
+        } else {
+            const uint32_t o = M.off[f], k = M.sizes[f];
+            bad = face_bad(M.idx + o, k, nv);
+            for (uint32_t i = 0; i < k; ++i) M.out[o + i] = v0 + M.idx[o + i];
         }
         if (bad) atomicOr(&C->bad_input, 1u);
     }
 }
 
 // raw box of every (pair, mesh) segment: one block each, order keys out
+// raw boxes, a tile of a mesh's vertices a block (a block a mesh took 0.20 ms of a
+// batch whose largest mesh has 100k vertices)
+constexpr uint32_t kBatchBoxTile = 4096;
 __global__ void __launch_bounds__(256) k_batch_bbox(const double* __restrict__ vs, const double* __restrict__ vc,
                                                     const BatchPair* __restrict__ bp, unsigned long long (*rbox)[2][6])
 {
@@ -3784,10 +3820,12 @@ __global__ void __launch_bounds__(256) k_batch_bbox(const double* __restrict__ v
     const uint32_t p = blockIdx.x >> 1, m = blockIdx.x & 1;
     const BatchPair b = bp[p];
     const double* v = m ? vc + 3ull * b.vc0 : vs + 3ull * b.vs0;
-    const uint32_t n = m ? b.nvc : b.nvs;
+    const uint32_t n = m ? b.nvc : b.nvs, i0 = blockIdx.y * kBatchBoxTile;
+    if (i0 >= n && i0) return; // whole block
+    const uint32_t i1 = n - i0 < kBatchBoxTile ? n : i0 + kBatchBoxTile;
     double lo[3] = {1.7976931348623157e308, 1.7976931348623157e308, 1.7976931348623157e308};
     double hi[3] = {-1.7976931348623157e308, -1.7976931348623157e308, -1.7976931348623157e308};
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
+    for (uint32_t i = i0 + threadIdx.x; i < i1; i += blockDim.x)
         for (int j = 0; j < 3; ++j) {
             const double x = v[3ull * i + j];
             lo[j] = x < lo[j] ? x : lo[j];
@@ -3813,8 +3851,8 @@ __global__ void __launch_bounds__(256) k_batch_bbox(const double* __restrict__ v
             a = red[q][j] < a ? red[q][j] : a;
             c = red[q][3 + j] > c ? red[q][3 + j] : c;
         }
-        rbox[p][m][j] = ord_key(a);
-        rbox[p][m][3 + j] = ord_key(c);
+        atomicMin(&rbox[p][m][j], ord_key(a));
+        atomicMax(&rbox[p][m][3 + j], ord_key(c));
     }
 }
 

@@ -75,7 +75,7 @@ const char* kStageNames[ST_COUNT] = {"coordinate_sums", "shift_params", "shift_b
 
 // event slots: stage boundaries on the three streams
 enum Ev { EV_A0, EV_S0, EV_A_SUMS, EV_A_PARAMS, EV_A_SHIFT, EV_A_BOXES, EV_A_JOIN, EV_A_FILTER, EV_A_PLANES, EV_A_JOIN2, EV_A_TESTS, EV_A_NARROW,
-          EV_A_END, EV_FORK, EV_B0, EV_B_SORT, EV_B_REFIT, EV_B_TRAV, EV_C0, EV_C_TOPO, EV_SUM_ITEMS, EV_SUM_CHAIN,
+          EV_A_END, EV_FORK, EV_B0, EV_B_SORT, EV_B_REFIT, EV_B_TRAV, EV_C0, EV_C_WORDS, EV_C_TOPO, EV_SUM_ITEMS, EV_SUM_CHAIN,
           EV_TRAV_K0, EV_TRAV_K1, EV_B_CC, EV_COUNT };
 
 // Launch shape of the traversal kernel, chosen per workload class by the
@@ -900,25 +900,31 @@ void enqueue_validate_batch(mcgpu_context ctx)
     auto* brbox = (unsigned long long(*)[2][6])ctx->brbox.p;
     Params* Pb = P_<Params>(ctx->bparams);
     ev_record(ctx, EV_A0, s);
-    fill_u32(C, 0u, sizeof(Counters) / 4, s);
-    fill_u32(ctx->pflags.p, 0u, np, s);
-    fill_u32(ctx->cand.p, 0u, (uint64_t)ctx->nf[0] + ctx->nf[1] + 8 + topo_counters(ctx), s);
-    k_segment_ids<<<grid_for(ctx->nv[0]), kBlock, 0, s>>>(st, np, ctx->nv[0], vp);
-    k_segment_ids<<<grid_for(ctx->nv[1]), kBlock, 0, s>>>(st + np, np, ctx->nv[1], vp + ctx->nv[0]);
-    k_segment_ids<<<grid_for(ctx->nf[0]), kBlock, 0, s>>>(st + 2 * np, np, ctx->nf[0], fp);
-    k_segment_ids<<<grid_for(ctx->nf[1]), kBlock, 0, s>>>(st + 3 * np, np, ctx->nf[1], fp + ctx->nf[0]);
+    BatchHead H{};
+    H.starts = st;
+    H.np = np;
+    H.n[0] = ctx->nv[0], H.n[1] = ctx->nv[1], H.n[2] = ctx->nf[0], H.n[3] = ctx->nf[1];
+    H.out[0] = vp, H.out[1] = vp + ctx->nv[0], H.out[2] = fp, H.out[3] = fp + ctx->nf[0];
+    H.pflags = P_<uint32_t>(ctx->pflags);
+    H.zero = P_<uint32_t>(ctx->cand);
+    H.nzero = (uint64_t)ctx->nf[0] + ctx->nf[1] + 8 + topo_counters(ctx);
+    H.rbox = &brbox[0][0][0];
+    const uint64_t most = std::max({(uint64_t)ctx->nv[0], (uint64_t)ctx->nv[1], (uint64_t)ctx->nf[0], (uint64_t)ctx->nf[1],
+                                    (uint64_t)12 * np});
+    k_batch_head<<<dim3(grid_for(most, kBlock, 2048), 6), kBlock, 0, s>>>(H, C);
+    BatchFaces BF[2];
     for (int m = 0; m < 2; ++m) {
         uint32_t* off = P_<uint32_t>(ctx->off[m]);
         if (ctx->dsz[m]) {
             scan_exclusive(ctx->dsz[m], off, ctx->nf[m], P_<uint32_t>(ctx->scan_tmp), etotal + m, s);
             k_offsets_tail<<<1, 1, 0, s>>>(off, ctx->nf[m], etotal + m);
-        } else {
-            k_triangle_offsets<<<grid_for((uint64_t)ctx->nf[m] + 1), kBlock, 0, s>>>(off, ctx->nf[m]);
         }
-        k_batch_globalize<<<grid_for(ctx->nf[m]), kBlock, 0, s>>>(ctx->bin_idx[m], off, ctx->dsz[m], ctx->nf[m], m,
-                                                                  m ? ctx->nf[0] : 0u, fp, bp, P_<uint32_t>(ctx->bidx[m]), C);
+        BF[m] = BatchFaces{ctx->bin_idx[m], off, ctx->dsz[m], ctx->nf[m], P_<uint32_t>(ctx->bidx[m])};
     }
-    k_batch_bbox<<<2 * np, 256, 0, s>>>(ctx->dv[0], ctx->dv[1], bp, brbox);
+    k_batch_globalize<<<grid_for((uint64_t)ctx->nf[0] + ctx->nf[1]), kBlock, 0, s>>>(BF[0], BF[1], fp, bp, C);
+    uint32_t nvmax = 1;
+    for (const BatchPair& q : ctx->hpairs) nvmax = std::max({nvmax, q.nvs, q.nvc});
+    k_batch_bbox<<<dim3(2 * np, (nvmax + kBatchBoxTile - 1) / kBatchBoxTile), 256, 0, s>>>(ctx->dv[0], ctx->dv[1], bp, brbox);
     const bool absolute = (ctx->flags & MCGPU_DISPATCH_ENFORCE_GENERAL_POSITION_ABSOLUTE) != 0;
     k_batch_tolerance<<<grid_for(np), kBlock, 0, s>>>(Pb, brbox, bp, np, ctx->gp_constant, absolute ? 1 : 0, C);
     k_batch_layout<<<1, 1024, 0, s>>>(Pb, brbox, np);
@@ -1287,12 +1293,99 @@ int leaf_bits(mcgpu_context ctx)
     return leaves <= (1u << 15) ? 16 : kMortonBits;
 }
 
-// Polygon-soup edge numbering on stream s3: records EV_C_TOPO at the end.
-void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
+// The edge numbering's meshes, buckets and counters.
+Topo topo_view(mcgpu_context ctx)
 {
     const uint64_t F = (uint64_t)ctx->nf[0] + ctx->nf[1];
-    Counters* C = &P_<DevState>(ctx->state)->C;
+    CornerMap cmap[2];
+    for (int m = 0; m < 2; ++m) {
+        cmap[m].off = P_<uint32_t>(ctx->off[m]);
+        cmap[m].cface = ctx->dsz[m] ? P_<uint32_t>(ctx->cface[m]) : nullptr;
+    }
+    Topo T{};
+    for (int m = 0; m < 2; ++m)
+        T.part[m] = TopoPart{ctx->didx[m], cmap[m], P_<uint32_t>(ctx->cedge[m]),
+                             P_<uint32_t>(ctx->opp) + (m ? ctx->ncorner[0] : 0), ctx->ncorner[m], m ? ctx->nv[0] : 0u,
+                             m ? ctx->nf[0] : 0u};
+    for (int i = 0; i < 2; ++i) T.seg[i] = ctx->topo_seg[i];
+    T.nseg = ctx->nseg;
+    T.tab = ctx->batch ? P_<TopoSeg>(ctx->tseg) : nullptr;
+    T.words = P_<unsigned long long>(ctx->twords);
+    T.fill = P_<uint32_t>(ctx->cand) + F + 8;
+    T.rfill = T.fill + ctx->topo_buckets;
+    T.hashed = T.rfill + ctx->topo_buckets;
+    T.ranges = ctx->topo_ranges;
+    return T;
+}
+
+void enqueue_topology_hash(mcgpu_context ctx, hipStream_t s3);
+
+// Polygon-soup edge numbering in two parts, the corners' words into their
+// buckets and the edges from those: both on stream C for one pair, the second
+// on stream A for a batch (on one pair stream A's part gained nothing:
+// 1.49 ms on two 1.3 M-triangle meshes became 1.53).
+void enqueue_topology_words(mcgpu_context ctx, hipStream_t s3)
+{
     stage_event(ctx, EV_C0, s3);
+    for (int m = 0; m < 2; ++m)
+        if (ctx->batch && ctx->dsz[m]) // else: written by the head
+            k_corner_faces<<<grid_for(ctx->nf[m]), kBlock, 0, s3>>>(P_<uint32_t>(ctx->off[m]), ctx->nf[m],
+                                                                    P_<uint32_t>(ctx->cface[m]));
+    if (ctx->topo_hash) {
+        enqueue_topology_hash(ctx, s3);
+        return;
+    }
+    Counters* C = &P_<DevState>(ctx->state)->C;
+    const Topo T = topo_view(ctx);
+    if (ctx->topo_tiles) {
+        const uint32_t n = ctx->topo_tiles;
+        const dim3 g(n), b(kTopoScatterBlock);
+        // a few blocks look whether a segment is hashed: most dispatches have none
+        const dim3 gh(ctx->topo_ranges ? std::min<uint32_t>(n, 2 * ctx->ncu) : n);
+        if (ctx->topo_bits == 8) {
+            k_topo_scatter<true, 8><<<gh, b, 0, s3>>>(T, n, C);
+        } else if (ctx->topo_bits == 10) {
+            k_topo_ranges<10><<<g, b, 0, s3>>>(T);
+            k_topo_scatter<false, 10><<<g, b, 0, s3>>>(T, n, C);
+            k_topo_scatter<true, 10><<<gh, b, 0, s3>>>(T, n, C);
+        } else {
+            k_topo_ranges<kTopoMaxBits><<<g, b, 0, s3>>>(T);
+            k_topo_scatter<false, kTopoMaxBits><<<g, b, 0, s3>>>(T, n, C);
+            k_topo_scatter<true, kTopoMaxBits><<<gh, b, 0, s3>>>(T, n, C);
+        }
+    }
+    if (ctx->batch) ev_record(ctx, EV_C_WORDS, s3);
+}
+
+// after enqueue_topology_words; records EV_C_TOPO at the end
+void enqueue_topology_edges(mcgpu_context ctx, hipStream_t s)
+{
+    if (ctx->topo_hash) return; // numbered on stream C
+    Counters* C = &P_<DevState>(ctx->state)->C;
+    const Topo T = topo_view(ctx);
+    uint32_t* etotal = P_<uint32_t>(ctx->etotal);
+    if (s != ctx->s3b && ctx->batch) ev_wait(ctx, s, EV_C_WORDS);
+    const int cut_only = ctx->res ? 1 : 0;
+    const uint32_t tiles0 = cut_only ? 0 : topo_rank_tiles(ctx->ncorner[0]);
+    const uint32_t tiles = tiles0 + topo_rank_tiles(ctx->ncorner[1]);
+    const bool few = tiles <= kTopoFewTiles; // counted by the buckets, in counters that the head clears
+    uint32_t* tsum = few ? T.hashed + ctx->nseg + 1 : P_<uint32_t>(ctx->tsum);
+    k_topo_buckets<<<ctx->topo_buckets, kTopoBlock, 0, s>>>(T, tiles0, few ? tsum : nullptr, C);
+    if (!few) k_topo_count<<<tiles, kBlock, 0, s>>>(T, tiles0, tsum);
+    const int scanned = tiles > kTopoDirectTiles;
+    if (scanned) k_scan_tiles<<<1, kScanBlock, 0, s>>>(tsum, tiles, etotal);
+    k_topo_apply<<<tiles, kBlock, 0, s>>>(T, tiles0, tiles, tsum, scanned, etotal, cut_only, C, P_<uint32_t>(ctx->ev0),
+                                           P_<uint32_t>(ctx->ev1), P_<int32_t>(ctx->ef0), P_<int32_t>(ctx->ef1));
+    if (ctx->batch)
+        k_batch_edge_bases<<<grid_for(ctx->npairs), kBlock, 0, s>>>(
+            P_<BatchPair>(ctx->bpairs), ctx->npairs, P_<uint32_t>(ctx->off[0]), P_<uint32_t>(ctx->off[1]), ctx->nf[0],
+            ctx->nf[1], P_<uint32_t>(ctx->cedge[0]), P_<uint32_t>(ctx->cedge[1]), C);
+    ev_record(ctx, EV_C_TOPO, s);
+}
+
+void enqueue_topology_hash(mcgpu_context ctx, hipStream_t s3)
+{
+    Counters* C = &P_<DevState>(ctx->state)->C;
     uint32_t* etotal = P_<uint32_t>(ctx->etotal);
     const uint64_t K = ctx->ncorner[0] + ctx->ncorner[1];
     const uint32_t res_ne = ctx->res ? ctx->res->ne : 0u;
@@ -1300,54 +1393,9 @@ void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
     for (int m = 0; m < 2; ++m) {
         cmap[m].off = P_<uint32_t>(ctx->off[m]);
         cmap[m].cface = ctx->dsz[m] ? P_<uint32_t>(ctx->cface[m]) : nullptr;
-        if (ctx->batch && ctx->dsz[m]) // else: written by the head
-            k_corner_faces<<<grid_for(ctx->nf[m]), kBlock, 0, s3>>>(cmap[m].off, ctx->nf[m], P_<uint32_t>(ctx->cface[m]));
     }
     // the scans of this stream use their own scratch: stream B's sort uses scan_tmp
     uint32_t* ctmp = P_<uint32_t>(ctx->scan_tmp_c);
-    if (!ctx->topo_hash) {
-        Topo T{};
-        for (int m = 0; m < 2; ++m)
-            T.part[m] = TopoPart{ctx->didx[m], cmap[m], P_<uint32_t>(ctx->cedge[m]),
-                                 P_<uint32_t>(ctx->opp) + (m ? ctx->ncorner[0] : 0), ctx->ncorner[m], m ? ctx->nv[0] : 0u,
-                                 m ? ctx->nf[0] : 0u};
-        for (int i = 0; i < 2; ++i) T.seg[i] = ctx->topo_seg[i];
-        T.nseg = ctx->nseg;
-        T.tab = ctx->batch ? P_<TopoSeg>(ctx->tseg) : nullptr;
-        T.words = P_<unsigned long long>(ctx->twords);
-        T.fill = P_<uint32_t>(ctx->cand) + F + 8;
-        T.rfill = T.fill + ctx->topo_buckets;
-        T.hashed = T.rfill + ctx->topo_buckets;
-        T.ranges = ctx->topo_ranges;
-        if (ctx->topo_tiles) {
-            const uint32_t n = ctx->topo_tiles;
-            const dim3 g(n), b(kTopoScatterBlock);
-            // a few blocks look whether a segment is hashed: most dispatches have none
-            const dim3 gh(ctx->topo_ranges ? std::min<uint32_t>(n, 2 * ctx->ncu) : n);
-            if (ctx->topo_bits == 8) {
-                k_topo_scatter<true, 8><<<gh, b, 0, s3>>>(T, n, C);
-            } else if (ctx->topo_bits == 10) {
-                k_topo_ranges<10><<<g, b, 0, s3>>>(T);
-                k_topo_scatter<false, 10><<<g, b, 0, s3>>>(T, n, C);
-                k_topo_scatter<true, 10><<<gh, b, 0, s3>>>(T, n, C);
-            } else {
-                k_topo_ranges<kTopoMaxBits><<<g, b, 0, s3>>>(T);
-                k_topo_scatter<false, kTopoMaxBits><<<g, b, 0, s3>>>(T, n, C);
-                k_topo_scatter<true, kTopoMaxBits><<<gh, b, 0, s3>>>(T, n, C);
-            }
-        }
-        const int cut_only = ctx->res ? 1 : 0;
-        const uint32_t tiles0 = cut_only ? 0 : topo_rank_tiles(ctx->ncorner[0]);
-        const uint32_t tiles = tiles0 + topo_rank_tiles(ctx->ncorner[1]);
-        const bool few = tiles <= kTopoFewTiles; // counted by the buckets, in counters that the head clears
-        uint32_t* tsum = few ? T.hashed + ctx->nseg + 1 : P_<uint32_t>(ctx->tsum);
-        k_topo_buckets<<<ctx->topo_buckets, kTopoBlock, 0, s3>>>(T, tiles0, few ? tsum : nullptr, C);
-        if (!few) k_topo_count<<<tiles, kBlock, 0, s3>>>(T, tiles0, tsum);
-        const int scanned = tiles > kTopoDirectTiles;
-        if (scanned) k_scan_tiles<<<1, kScanBlock, 0, s3>>>(tsum, tiles, etotal);
-        k_topo_apply<<<tiles, kBlock, 0, s3>>>(T, tiles0, tiles, tsum, scanned, etotal, cut_only, C, P_<uint32_t>(ctx->ev0),
-                                               P_<uint32_t>(ctx->ev1), P_<int32_t>(ctx->ef0), P_<int32_t>(ctx->ef1));
-    } else {
     fill_u32(P_<uint32_t>(ctx->ef1) + res_ne, 0xffffffffu, K - res_ne, s3);
     for (int m = ctx->res ? 1 : 0; m < 2; ++m) {
         const uint64_t nk = ctx->ncorner[m];
@@ -1370,13 +1418,11 @@ void enqueue_topology(mcgpu_context ctx, hipStream_t s3)
             hs - 1, P_<uint32_t>(ctx->eid[m]), C, m ? ctx->nv[0] : 0, m ? ctx->nf[0] : 0, P_<uint32_t>(ctx->cedge[m]),
             P_<uint32_t>(ctx->ev0), P_<uint32_t>(ctx->ev1), P_<int32_t>(ctx->ef0), P_<int32_t>(ctx->ef1));
     }
-    }
     if (ctx->batch)
         k_batch_edge_bases<<<grid_for(ctx->npairs), kBlock, 0, s3>>>(
             P_<BatchPair>(ctx->bpairs), ctx->npairs, P_<uint32_t>(ctx->off[0]), P_<uint32_t>(ctx->off[1]), ctx->nf[0],
             ctx->nf[1], P_<uint32_t>(ctx->cedge[0]), P_<uint32_t>(ctx->cedge[1]), C);
     ev_record(ctx, EV_C_TOPO, s3);
-
 }
 
 // Rounds of the component check (hook, jump, round end) and the root count,
@@ -1439,6 +1485,14 @@ void enqueue_frontend(mcgpu_context ctx)
     }
     if (ctx->batch) {
         ev_record(ctx, EV_A_SUMS, ssum);
+        // stream A, which has every compute unit, numbers the edges while it
+        // waits for the long chains of large meshes (96 small pairs: 0.53 ms
+        // instead of 0.49)
+        if (ctx->topo_bits > 8) {
+            ev_wait(ctx, s3, EV_FORK);
+            enqueue_topology_words(ctx, s3);
+            enqueue_topology_edges(ctx, s);
+        }
         ev_wait(ctx, s, EV_A_SUMS);
     }
     if (ctx->batch) {
@@ -1460,6 +1514,14 @@ void enqueue_frontend(mcgpu_context ctx)
     }
     stage_event(ctx, EV_A_SHIFT, s);
     if (ctx->shifted_bp) ev_record(ctx, EV_A_BOXES, s);
+
+    // ---- stream C: the edge numbering's words, enqueued before stream B's many
+    // launches where they take as long as its sort ----
+    const bool words_done = ctx->batch && ctx->topo_bits > 8, words_first = ctx->topo_bits > 10 && !ctx->batch;
+    if (words_first) {
+        ev_wait(ctx, s3, EV_FORK);
+        enqueue_topology_words(ctx, s3);
+    }
 
     // ---- stream B: raw-space trees and broad phase (in shifted coordinates,
     // after the face boxes, for a pair whose raw-space tolerance is loose) ----
@@ -1498,9 +1560,11 @@ void enqueue_frontend(mcgpu_context ctx)
     if (tests_all_pairs(ctx)) launch_all_pairs(ctx, s2, C);
     else enqueue_bvh_traverse(ctx, s2, C, !ctx->batch); // k_morton_raw cleared the sort's group totals
 
-    // ---- stream C: polygon-soup edge numbering, and the tables the filter fills ----
-    ev_wait(ctx, s3, EV_FORK);
-    enqueue_topology(ctx, s3);
+    if (!words_first && !words_done) {
+        ev_wait(ctx, s3, EV_FORK);
+        enqueue_topology_words(ctx, s3);
+    }
+    if (!words_done) enqueue_topology_edges(ctx, s3);
 
     // ---- stream B, once its traversal and stream C's edge table are done:
     // one connected component per input mesh (per pair in a batch), in the
@@ -3796,7 +3860,8 @@ MCGPU_API mcgpu_result mcgpu_dispatch_narrow(mcgpu_context ctx, const mcgpu_mesh
             fill_u64(&C->n_edges_src, (unsigned long long)NE, 1, s);
             fill_u64(&C->n_edges_cut, 0ull, 1, s);
         } else {
-            enqueue_topology(ctx, s);
+            enqueue_topology_words(ctx, s);
+            enqueue_topology_edges(ctx, s);
         }
         // pair hash and candidate faces; the exact box test keeps every given pair
         const uint64_t table = next_pow2(2 * ctx->cap_pairs);
