@@ -37,9 +37,9 @@ HBM_PEAK_GBS = 8000.0
 
 # stage -> the kernel that carries it (stages of one kernel are timed exactly
 # by the events around that kernel on its stream).  The coordinate sums are
-# five kernels (run items, chain, verification, serial fallback).
+# several kernels (tile sums, items, chain, verification, rest).
 STAGE_KERNEL = {
-    "traversal": "k_traverse_wave",
+    "traversal": "k_pairs_start + k_pairs_expand + k_pairs_leaves",
     "tests": "k_tests",
     "pair_filter": "k_filter_pairs",
     "face_planes": "k_planes + k_big_polygons",
@@ -70,9 +70,9 @@ def stage_bytes(name, n):
         # source leaves (float box and face id) and the cut tree (float node
         # boxes, leaf face ids) read once, raw pairs written
         "traversal": 28 * n["Fs"] + 24 * n["nodes_cut"] + 4 * (F - n["Fs"]) + 8 * CR,
-        # raw pairs and both shifted boxes read; pairs, pair hash and
-        # candidate faces written
-        "pair_filter": CR * (8 + 96) + 16 * C + 4 * FC,
+        # raw pairs and both shifted boxes read; pairs and candidate faces
+        # written
+        "pair_filter": CR * (8 + 96) + 8 * C + 4 * FC,
         # candidate faces: face list and vertices read, plane written
         "face_planes": FC * (72 + 40),
         # pairs read, tests written, per test: edge endpoints and face box

@@ -501,16 +501,6 @@ __global__ void k_batch_shift_params(Params* P, const unsigned long long (*rbox)
     }
 }
 
-__global__ void k_set_perturbation(Params* P, int has_pert, double p0, double p1, double p2)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        P->has_pert = has_pert;
-        P->pert[0] = p0;
-        P->pert[1] = p1;
-        P->pert[2] = p2;
-    }
-}
-
 // Per-axis tolerance that makes the raw-space broad phase find every pair
 // whose shifted boxes overlap.  With u = 2^-53 and, per axis, E the extent of
 // both meshes' raw box, W its largest magnitude and n the larger vertex count:
@@ -669,37 +659,9 @@ struct OffsetMesh {
 };
 __global__ void __launch_bounds__(1024) k_small_offsets(OffsetMesh m0, OffsetMesh m1)
 {
-    __shared__ uint32_t wsum[16];
     const OffsetMesh M = blockIdx.x ? m1 : m0;
     if (!M.sizes) return; // whole block
-    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    uint32_t base = 0;
-    for (uint32_t f0 = 0; f0 < M.nf; f0 += 4096) {
-        uint32_t v[4], own = 0;
-        const uint32_t f = f0 + 4 * threadIdx.x;
-#pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) v[q] = f + q < M.nf ? M.sizes[f + q] : 0u;
-#pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) own += v[q];
-        uint32_t x = own;
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t y = __shfl_up(x, o, 64);
-            if (lane >= (uint32_t)o) x += y;
-        }
-        if (lane == 63) wsum[wid] = x;
-        __syncthreads();
-        x += base - own;
-        for (uint32_t q = 0; q < 16; ++q) {
-            if (q < wid) x += wsum[q];
-            base += wsum[q];
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) {
-            if (f + q < M.nf) M.off[f + q] = x;
-            x += v[q];
-        }
-        __syncthreads();
-    }
+    const uint32_t base = scan_by_block(M.sizes, M.off, M.nf);
     if (threadIdx.x == 0) M.off[M.nf] = base;
 }
 

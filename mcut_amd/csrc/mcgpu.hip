@@ -333,9 +333,11 @@ inline unsigned grid_for(uint64_t n, unsigned block = kBlock, unsigned maxg = 40
     return (unsigned)g;
 }
 
-__global__ void k_reset_narrow(Counters* C)
+__global__ void k_reset_narrow(Counters* C, Params* P, double p0, double p1, double p2)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
+        P->has_pert = 1;
+        P->pert[0] = p0, P->pert[1] = p1, P->pert[2] = p2;
         C->n_tests = C->n_esc = C->n_reg = C->n_big = C->n_trip = 0; // candidate faces are kept
         C->ov_trip = 0;
         C->n_f32 = C->n_f64 = 0;
@@ -1595,7 +1597,12 @@ mcgpu_result enqueue_state_copy(mcgpu_context ctx)
 {
     ctx->state_copied = false;
     if (!ctx->hstate) CK(hipHostMalloc((void**)&ctx->hstate, sizeof(DevState), hipHostMallocDefault));
-    CK(hipMemcpyAsync(ctx->hstate, ctx->state.p, sizeof(DevState), hipMemcpyDeviceToHost, ctx->s));
+    CopySegs S{};
+    S.from[0] = ctx->state.p;
+    S.to[0] = ctx->hstate;
+    S.bytes[0] = sizeof(DevState);
+    k_copy_segs<<<1, 256, 0, ctx->s>>>(S);
+    CK(hipGetLastError());
     ctx->state_copied = true;
     return MCGPU_SUCCESS;
 }
@@ -2718,9 +2725,7 @@ MCGPU_API mcgpu_result mcgpu_redispatch_perturbed(mcgpu_context ctx, const doubl
         ctx->last_timed = ctx->stage_timing || ctx->kernel_timing;
     ctx->last_kernel_only = !ctx->stage_timing && ctx->kernel_timing;
         (void)hipEventRecord(ctx->ev[EV_A0], s);
-        ctx->state_copied = false; // finish() copies the state after its wait
-        k_reset_narrow<<<1, 1, 0, s>>>(C);
-        k_set_perturbation<<<1, 1, 0, s>>>(&P_<DevState>(ctx->state)->P, 1, perturbation[0], perturbation[1], perturbation[2]);
+        k_reset_narrow<<<1, 1, 0, s>>>(C, &P_<DevState>(ctx->state)->P, perturbation[0], perturbation[1], perturbation[2]);
         stage_event(ctx, EV_A_PARAMS, s);
         k_shift_vertices<<<grid_for(3 * V), kBlock, 0, s>>>(ctx->dv[0], ctx->nv[0], ctx->dv[1], ctx->nv[1],
                                                             &P_<DevState>(ctx->state)->P, P_<double>(ctx->ps_v), 1);
@@ -2728,6 +2733,7 @@ MCGPU_API mcgpu_result mcgpu_redispatch_perturbed(mcgpu_context ctx, const doubl
         stage_event(ctx, EV_A_JOIN, s);
         stage_event(ctx, EV_A_FILTER, s);
         enqueue_narrow(ctx, make_soup(ctx), false, ctx->pairs_given ? kPairsGiven : kPairsMoved);
+        (void)enqueue_state_copy(ctx); // on failure finish() copies after its wait
         bool overflow = false;
         if ((r = finish(ctx, info, &overflow)) != MCGPU_SUCCESS) return r;
         if (!overflow) return MCGPU_SUCCESS;
@@ -3873,6 +3879,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_narrow(mcgpu_context ctx, const mcgpu_mesh
             P_<uint32_t>(ctx->cand_list), C);
         stage_event(ctx, EV_A_FILTER, s);
         enqueue_narrow(ctx, make_soup(ctx), false, kPairsGiven);
+        (void)enqueue_state_copy(ctx); // on failure finish() copies after its wait
         bool overflow = false;
         if ((r = finish(ctx, info, &overflow)) != MCGPU_SUCCESS) return r;
         if (!overflow) return MCGPU_SUCCESS;

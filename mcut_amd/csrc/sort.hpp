@@ -160,13 +160,60 @@ __global__ void __launch_bounds__(kScan1Block) k_scan_hist(uint32_t* __restrict_
     }
 }
 
+// exclusive scan of in[0, n) into out (may alias in) by one block of 1,024
+// threads, 4,096 elements a round; every thread returns the total
+__device__ __forceinline__ uint32_t scan_by_block(const uint32_t* in, uint32_t* out, uint64_t n)
+{
+    __shared__ uint32_t wsum[16];
+    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    uint32_t base = 0;
+    for (uint64_t i0 = 0; i0 < n; i0 += 4096) {
+        uint32_t v[4], own = 0;
+        const uint64_t i = i0 + 4 * threadIdx.x;
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) v[q] = i + q < n ? in[i + q] : 0u;
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) own += v[q];
+        uint32_t x = own;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o, 64);
+            if (lane >= (uint32_t)o) x += y;
+        }
+        if (lane == 63) wsum[wid] = x;
+        __syncthreads();
+        x += base - own;
+        for (uint32_t q = 0; q < 16; ++q) {
+            if (q < wid) x += wsum[q];
+            base += wsum[q];
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            if (i + q < n) out[i + q] = x;
+            x += v[q];
+        }
+        __syncthreads();
+    }
+    return base;
+}
+
+static __global__ void __launch_bounds__(1024) k_scan_small(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* total)
+{
+    const uint32_t t = scan_by_block(in, out, n);
+    if (total && threadIdx.x == 0) *total = t;
+}
+
+constexpr uint64_t kScanSmall = 16384; // elements one block scans in less time than two more launches take
+
 // Host launcher: exclusive scan of n (host-known) u32 into out (may alias in);
 // tmp needs ceil(n / kScanTile) entries; total (device) optional.
 inline void scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, uint32_t* total,
                            hipStream_t s)
 {
-    uint32_t ntiles = (uint32_t)((n + kScanTile - 1) / kScanTile);
-    if (ntiles == 0) ntiles = 1;
+    if (n <= kScanSmall) {
+        k_scan_small<<<1, 1024, 0, s>>>(in, out, n, total);
+        return;
+    }
+    const uint32_t ntiles = (uint32_t)((n + kScanTile - 1) / kScanTile);
     k_scan_reduce<<<ntiles, kScanBlock, 0, s>>>(in, tmp, n);
     k_scan_tiles<<<1, kScanBlock, 0, s>>>(tmp, ntiles, total);
     k_scan_apply<<<ntiles, kScanBlock, 0, s>>>(in, out, tmp, n);
