@@ -916,13 +916,15 @@ __device__ __forceinline__ void topo_corner(const TopoPart& P, const TopoSeg& g,
 
 // An edge's bucket by vertex ranges: that of one of its ends, the lower for
 // every other edge so that vertices numbered before their neighbours (coarse
-// ones of a subdivision) do not fill theirs.
+// ones of a subdivision) do not fill theirs.  An index past the mesh's
+// vertices (a face list that is being refused) lands in the last bucket.
 __device__ __forceinline__ uint32_t topo_range(const TopoSeg& g, uint32_t a, uint32_t d, uint32_t* own, uint32_t* oth)
 {
     const uint32_t lo = a < d ? a : d, hi = a < d ? d : a;
     *own = (lo ^ hi) & 1 ? hi : lo;
     *oth = (lo ^ hi) & 1 ? lo : hi;
-    return (uint32_t)(((uint64_t)*own * g.inv) >> 32);
+    const uint32_t b = (uint32_t)(((uint64_t)*own * g.inv) >> 32), last = (1u << g.bb) - 1;
+    return b < last ? b : last;
 }
 
 // corner q of a segment as a word; its bucket in *bucket

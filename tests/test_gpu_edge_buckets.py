@@ -124,3 +124,21 @@ def test_vertices_of_many_faces(ctx, rings, hub):
     R = ctx.dispatch(src, cut)
     v0, v1, f0, f1 = R.edges()
     assert v0.size == 3 * sum(rings) + 33 and int((f1 < 0).sum()) == 12
+
+
+@pytest.mark.parametrize("index", [0, 1, 2])
+@pytest.mark.parametrize("value", ["nv", "max"])
+def test_refused_lists_of_large_meshes(ctx, index, value):
+    # an index past the vertices, in meshes whose buckets are vertex ranges:
+    # refused, alone and in a batch, and the context goes on
+    from mcut_amd import frontend
+    V, F, _ = strip(174763)
+    bad = F.copy()
+    bad[3 * 1000 + index] = V.shape[0] if value == "nv" else 0xffffffff
+    with pytest.raises(frontend.McgpuError) as e:
+        ctx.dispatch((V, bad, None), blade(1.0))
+    assert e.value.code == -1
+    with pytest.raises(frontend.McgpuError) as e:
+        ctx.dispatch_batch([((V, F, None), blade(1.0)), ((V, bad, None), blade(1.0))])
+    assert e.value.code == -1
+    assert ctx.dispatch((V, F, None), blade(1.0)).counts["edges"] == 2 * 174763 + 1 + 33
