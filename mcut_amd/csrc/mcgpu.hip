@@ -886,6 +886,14 @@ void enqueue_validate(mcgpu_context ctx)
 // vertex and face, face lists checked against their own pair's vertex count
 // and rewritten as ids of the concatenated part, raw boxes of every (pair,
 // mesh), each pair's broad-phase tolerance, and the cell layout.
+// tiles of the batch's largest mesh
+uint32_t batch_box_tiles(mcgpu_context ctx)
+{
+    uint32_t nv = 1;
+    for (const BatchPair& q : ctx->hpairs) nv = std::max({nv, (uint32_t)q.nvs, (uint32_t)q.nvc});
+    return (nv + kBatchBoxTile - 1) / kBatchBoxTile;
+}
+
 void enqueue_validate_batch(mcgpu_context ctx)
 {
     ctx->state_copied = false;
@@ -924,9 +932,7 @@ void enqueue_validate_batch(mcgpu_context ctx)
         BF[m] = BatchFaces{ctx->bin_idx[m], off, ctx->dsz[m], ctx->nf[m], P_<uint32_t>(ctx->bidx[m])};
     }
     k_batch_globalize<<<grid_for((uint64_t)ctx->nf[0] + ctx->nf[1]), kBlock, 0, s>>>(BF[0], BF[1], fp, bp, C);
-    uint32_t nvmax = 1;
-    for (const BatchPair& q : ctx->hpairs) nvmax = std::max({nvmax, q.nvs, q.nvc});
-    k_batch_bbox<<<dim3(2 * np, (nvmax + kBatchBoxTile - 1) / kBatchBoxTile), 256, 0, s>>>(ctx->dv[0], ctx->dv[1], bp, brbox);
+    k_batch_bbox<<<dim3(2 * np, batch_box_tiles(ctx)), 256, 0, s>>>(ctx->dv[0], ctx->dv[1], bp, brbox);
     const bool absolute = (ctx->flags & MCGPU_DISPATCH_ENFORCE_GENERAL_POSITION_ABSOLUTE) != 0;
     k_batch_tolerance<<<grid_for(np), kBlock, 0, s>>>(Pb, brbox, bp, np, ctx->gp_constant, absolute ? 1 : 0, C);
     k_batch_layout<<<1, 1024, 0, s>>>(Pb, brbox, np);
@@ -957,7 +963,19 @@ mcgpu_result fetch(mcgpu_context ctx, std::initializer_list<Fetch> list)
     }
     small = at <= (1u << 20);
     if (!n) return MCGPU_SUCCESS;
-    CK(hipSetDevice(ctx->device));
+    struct Device { // the context's while launching; the caller's again after
+        int was = -1;
+        ~Device()
+        {
+            if (was >= 0) (void)hipSetDevice(was);
+        }
+    } device;
+    int cur = 0;
+    CK(hipGetDevice(&cur));
+    if (cur != ctx->device) {
+        CK(hipSetDevice(ctx->device));
+        device.was = cur;
+    }
     if (!small) {
         for (int q = 0; q < n; ++q) CK(hipMemcpyAsync(of[q]->to, of[q]->from, of[q]->bytes, hipMemcpyDeviceToHost, ctx->s));
         CK(hipStreamSynchronize(ctx->s));
@@ -1802,7 +1820,7 @@ std::vector<uint64_t> graph_key(mcgpu_context ctx)
     auto ptr = [&k](const void* p) { k.push_back((uint64_t)(uintptr_t)p); };
     put(ctx->batch), put(ctx->npairs), put(ctx->batch_mb), put(ctx->cc_check), put(ctx->batch ? ctx->sort_bits : leaf_bits(ctx)),
         put(ctx->shifted_bp), put(ctx->walk), put(ctx->trav.walk), put(ctx->want_trees), put(ctx->one_stream), put(ctx->forced), put(ctx->cap_nodes), put(ctx->topo_hash), put(ctx->topo_buckets), put(ctx->topo_tiles), put(ctx->topo_bits),
-        put(ctx->nseg),
+        put(ctx->nseg), put(ctx->topo_ranges), put(ctx->batch ? batch_box_tiles(ctx) : 0),
         put(ctx->gbits), put(ctx->kbits);
     for (int m = 0; m < 2; ++m) {
         put(ctx->nv[m]), put(ctx->nf[m]), put(ctx->ncorner[m]), put(ctx->depth[m]);
