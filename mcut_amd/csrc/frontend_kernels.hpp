@@ -55,10 +55,12 @@ constexpr int kSumRing = 16;
 
 // acc + v[0] + v[STRIDE] + ... + v[STRIDE (n - 1)], left to right, by one
 // wavefront (the whole wave returns it); rows (optional): the value after every
-// 16 of them
+// 16 of them.  at: this lane's element of a step's STRIDE, the same across a
+// row of 16 lanes; rows of lanes with elements of their own add chains of
+// their own (the broadcasts stay within a row).
 template <int STRIDE, bool ROWS>
 __device__ __forceinline__ double serial_chain(const double* __restrict__ v, uint32_t n, const double* __restrict__ zero,
-                                               double acc, double* __restrict__ rows)
+                                               double acc, double* __restrict__ rows, uint32_t at = 0)
 {
     const uint32_t c = threadIdx.x & 15;
     const uint32_t nfull = n / 64;
@@ -70,7 +72,7 @@ __device__ __forceinline__ double serial_chain(const double* __restrict__ v, uin
         for (int r = 0; r < kSumRing; ++r) {
             const double* vb = v + (uint64_t)(64 * STRIDE) * ((uint32_t)r < last ? (uint32_t)r : last); // uniform block base
 #pragma unroll
-            for (int q = 0; q < 4; ++q) X[r][q] = vb[STRIDE * (16 * q + c)];
+            for (int q = 0; q < 4; ++q) X[r][q] = vb[STRIDE * (16 * q + c) + at];
         }
         for (uint32_t b0 = 0; b0 < nfull; b0 += kSumRing) {
 #pragma unroll
@@ -89,7 +91,7 @@ __device__ __forceinline__ double serial_chain(const double* __restrict__ v, uin
                 const uint32_t nb = b0 + kSumRing + r;
                 const double* vb = v + (uint64_t)(64 * STRIDE) * (nb < last ? nb : last);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) X[r][q] = vb[STRIDE * (16 * q + c)];
+                for (int q = 0; q < 4; ++q) X[r][q] = vb[STRIDE * (16 * q + c) + at];
             }
         }
     }
@@ -98,7 +100,7 @@ __device__ __forceinline__ double serial_chain(const double* __restrict__ v, uin
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const uint32_t i = nfull * 64 + 16 * q + c;
-            T[q] = *(i < n ? v + (uint64_t)STRIDE * i : zero);
+            T[q] = *(i < n ? v + (uint64_t)STRIDE * i + at : zero);
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -431,15 +433,17 @@ __global__ void __launch_bounds__(384) k_sum_rest(SumBufs B, const double* __res
     if (threadIdx.x == 0) shift_params(P, C, A);
 }
 
-// Batches: the 6 chains of every pair (pair p, mesh m, coordinate j is chain
-// 6 p + 3 m + j), handed out longest first (order[]) by a work queue to a
-// persistent grid of waves, so that long chains start early and short ones
-// fill in behind them.
+// Batches: the chains of every pair's meshes (mesh m of pair p is 2 p + m),
+// handed out longest first (order[]) by a work queue to a persistent grid of
+// waves, so that long chains start early and short ones fill in behind them.  A
+// wave adds a mesh's three coordinates at once, one a row of 16 lanes: a wave a
+// coordinate took 22.7 ms for 4,096 uneven pairs, this 8.2.
 __global__ void __launch_bounds__(64) k_batch_sums(const double* __restrict__ vs, const double* __restrict__ vc,
                                                    const BatchPair* __restrict__ bp, const uint32_t* __restrict__ order,
-                                                   uint32_t nchains, Counters* C, Params* P)
+                                                   uint32_t nmeshes, Counters* C, Params* P)
 {
     __builtin_amdgcn_s_setprio(3);
+    const uint32_t row = threadIdx.x >> 4, j = row < 3 ? row : 2; // the last row adds z again
     for (;;) {
         // Everything that steers this loop is a scalar (readfirstlane) and the
         // body has no lane-dependent branch: with a chain index read back from
@@ -447,15 +451,15 @@ __global__ void __launch_bounds__(64) k_batch_sums(const double* __restrict__ vs
         // store, the compiler treats the exit as divergent and may structure
         // the loop so that lanes 1-63 keep iterating without lane 0, which
         // never ends.  Every lane issues the atomic (lane 0 adds 1, the others
-        // 0) and lane 0's result is the wave's chain.
+        // 0) and lane 0's result is the wave's mesh.
         const uint32_t w = __builtin_amdgcn_readfirstlane(atomicAdd(&C->sum_next, threadIdx.x == 0 ? 1u : 0u));
-        if (w >= nchains) break;
-        const uint32_t chain = __builtin_amdgcn_readfirstlane(order[w]);
-        const uint32_t p = chain / 6, m = (chain % 6) / 3, j = chain % 3;
+        if (w >= nmeshes) break;
+        const uint32_t mesh = __builtin_amdgcn_readfirstlane(order[w]);
+        const uint32_t p = mesh >> 1, m = mesh & 1;
         const uint32_t v0 = __builtin_amdgcn_readfirstlane(m ? bp[p].vc0 : bp[p].vs0);
         const uint32_t n = __builtin_amdgcn_readfirstlane(m ? bp[p].nvc : bp[p].nvs);
-        const double acc = serial_sum((m ? vc : vs) + 3ull * v0 + j, n, &C->zero);
-        P[p].sum[m][j] = acc; // the same value in every lane
+        const double acc = serial_chain<3, false>((m ? vc : vs) + 3ull * v0, n, &C->zero, 0.0, nullptr, j);
+        P[p].sum[m][j] = acc; // the same value across a row
     }
 }
 

@@ -559,7 +559,7 @@ mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
     CK(ensure(ctx->planes, F, &pl));
     (void)p;
     CK(ensure(ctx->scan_tmp, scan_need + 1024, &u));
-    if (!ctx->batch) { // coordinate sums from segments (k_sum_blocks .. k_sum_rest), for the chains computed here
+    if (!ctx->batch) { // coordinate sums from segments (k_sum_items .. k_sum_rest), for the chains computed here
         const uint64_t nmax = std::max<uint64_t>(ctx->res ? 0 : ctx->nv[0], ctx->nv[1]);
         const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, (nmax + kSumTile - 1) / kSumTile);
         ctx->sum_nblk = nblk;
@@ -1481,7 +1481,7 @@ void enqueue_frontend(mcgpu_context ctx)
     if (ctx->batch) {
         ev_wait(ctx, ssum, EV_FORK);
         stage_event(ctx, EV_S0, ssum);
-        const uint32_t nch = 6 * ctx->npairs;
+        const uint32_t nch = 2 * ctx->npairs;
         k_batch_sums<<<std::min<uint32_t>(nch, kBatchSumWaves), 64, 0, ssum>>>(
             ctx->dv[0], ctx->dv[1], P_<BatchPair>(ctx->bpairs), P_<uint32_t>(ctx->border), nch, C, Pb);
     } else {
@@ -2465,7 +2465,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
     // pair tables
     ctx->hpairs.assign(np, BatchPair{});
     ctx->hstarts.resize(4ull * np);
-    std::vector<uint32_t> len(6ull * np);
+    std::vector<uint32_t> len(2ull * np);
     for (uint32_t p = 0; p < np; ++p) {
         BatchPair& b = ctx->hpairs[p];
         b.fs0 = fo[0][p], b.nfs = fo[0][p + 1] - fo[0][p];
@@ -2476,7 +2476,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
         ctx->hstarts[np + p] = b.vc0;
         ctx->hstarts[2ull * np + p] = b.fs0;
         ctx->hstarts[3ull * np + p] = b.fc0;
-        for (int j = 0; j < 6; ++j) len[6ull * p + j] = j < 3 ? b.nvs : b.nvc;
+        len[2ull * p] = b.nvs, len[2ull * p + 1] = b.nvc;
     }
     // the edge numbering's segments: both meshes of every pair (corner counts
     // are known on the host for triangle meshes and host face sizes)
@@ -2505,8 +2505,8 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
         }
     }
     // serial-sum chains, longest first
-    ctx->horder.resize(6ull * np);
-    for (uint32_t c = 0; c < 6 * np; ++c) ctx->horder[c] = c;
+    ctx->horder.resize(2ull * np);
+    for (uint32_t c = 0; c < 2 * np; ++c) ctx->horder[c] = c;
     std::stable_sort(ctx->horder.begin(), ctx->horder.end(), [&](uint32_t a, uint32_t b) { return len[a] > len[b]; });
     const uint64_t F = (uint64_t)ctx->nf[0] + ctx->nf[1];
     const uint64_t V = (uint64_t)ctx->nv[0] + ctx->nv[1];
@@ -2522,7 +2522,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
         unsigned long long* ull;
         CK(ensure(ctx->bpairs, np, &bp));
         CK(ensure(ctx->bstarts, 4ull * np, &u));
-        CK(ensure(ctx->border, 6ull * np, &u));
+        CK(ensure(ctx->border, 2ull * np, &u));
         CK(ensure(ctx->pflags, np, &u));
         CK(ensure(ctx->rstart, np, &u));
         CK(ensure(ctx->rend, np, &u));
@@ -2537,7 +2537,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
         if ((r = upload_flush(ctx)) != MCGPU_SUCCESS) return r; // the meshes
         if ((r = upload(ctx, ctx->bpairs.p, ctx->hpairs.data(), sizeof(BatchPair) * np)) != MCGPU_SUCCESS) return r;
         if ((r = upload(ctx, ctx->bstarts.p, ctx->hstarts.data(), 16ull * np)) != MCGPU_SUCCESS) return r;
-        if ((r = upload(ctx, ctx->border.p, ctx->horder.data(), 24ull * np)) != MCGPU_SUCCESS) return r;
+        if ((r = upload(ctx, ctx->border.p, ctx->horder.data(), 8ull * np)) != MCGPU_SUCCESS) return r;
         if (!ctx->topo_hash && (r = upload(ctx, ctx->tseg.p, ctx->hseg.data(), sizeof(TopoSeg) * ctx->nseg)) != MCGPU_SUCCESS)
             return r;
         if ((r = upload_flush(ctx)) != MCGPU_SUCCESS) return r;
