@@ -3438,11 +3438,22 @@ __device__ __forceinline__ void status_insert(const Soup& S, uint32_t e, uint32_
 // through LDS.  That is about 50 instructions per element and pass; a bitonic
 // network spent 78 compare-exchange stages on the 4096 elements of one CU and
 // took 61 us even for a registry of a few hundred entries.
+//
+// A tile of up to kRegRunMax entries, as small registries have, needs no digit
+// counts: every element ranks itself among its 16 neighbours, then runs of 16,
+// 32, .. are merged two to one, an element's new place being its place in its
+// own run plus a binary search in the other.  Only keys pass through LDS, and
+// four barriers less a digit: a registry of a few hundred entries takes 4.9 us
+// in place of 17.4, one of 1,600 takes 15 in place of 25.  At 4,096 entries the
+// searches' LDS reads cost as much as the digit passes (icosphere-7, five
+// tiles: 562-576 us a pair with runs, 538-555 with digits), so those keep the
+// radix sort; so does a key that uses bit 63, which marks the padding here.
 constexpr int kRegTile = 4096;
 constexpr int kRegSortThreads = 1024;
 constexpr int kRegPer = kRegTile / kRegSortThreads; // 4
 constexpr int kRegWaves = kRegSortThreads / 64;     // 16
 constexpr uint64_t kRegMergeTiles = 64;
+constexpr uint32_t kRegRunMax = 2048;
 
 __global__ void __launch_bounds__(kRegSortThreads) k_reg_tile_sort(const unsigned long long* __restrict__ key,
                                                                    const uint32_t* __restrict__ val,
@@ -3495,6 +3506,50 @@ __global__ void __launch_bounds__(kRegSortThreads) k_reg_tile_sort(const unsigne
     for (int w = 0; w < kRegWaves; ++w) all |= wor[w];
     const int used = all ? 64 - __clzll((long long)all) : 1;
     const int nbits = used < kbits ? used : kbits;
+    if (cnt <= kRegRunMax && used < 64) { // the whole block
+        const uint32_t P = cnt <= 16 ? 16u : 1u << (32 - __clz(cnt - 1));
+        uint32_t pos[kRegPer];
+#pragma unroll
+        for (int r = 0; r < kRegPer; ++r) {
+            const uint32_t i = r * kRegSortThreads + t;
+            if (i >= cnt) K[r] = (1ull << 63) | i; // distinct, above every key
+            if (i < P) sk[i] = K[r];
+            pos[r] = i;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kRegPer; ++r) {
+            if (pos[r] >= P) continue;
+            const uint32_t g0 = pos[r] & ~15u;
+            uint32_t below = 0;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) below += sk[g0 + q] < K[r];
+            pos[r] = g0 + below;
+        }
+        for (uint32_t w = 16; w < cnt; w <<= 1) { // runs of w, two to one
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kRegPer; ++r)
+                if (pos[r] < P) sk[pos[r]] = K[r];
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kRegPer; ++r) {
+                if (pos[r] >= P) continue;
+                const unsigned long long* other = sk + ((pos[r] & ~(w - 1)) ^ w);
+                uint32_t lo = 0;
+                for (uint32_t h = w >> 1; h > 0; h >>= 1) lo += other[lo + h - 1] < K[r] ? h : 0u;
+                lo += other[lo] < K[r];
+                pos[r] = (pos[r] & ~(2 * w - 1)) + (pos[r] & (w - 1)) + lo;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kRegPer; ++r)
+            if (pos[r] < cnt) {
+                skey[t0 + pos[r]] = K[r];
+                sval[t0 + pos[r]] = V[r];
+            }
+        return;
+    }
     // the prefix step: thread t sums digit dg over the waves of row pr
     const uint32_t dg = t & (kRadix - 1), pr = t >> kRadixBits;
     for (int shift = 0; shift < nbits; shift += kRadixBits) {
@@ -3594,7 +3649,7 @@ __global__ void k_reg_merge(Soup S, const unsigned long long* __restrict__ skey,
         const uint64_t t = i / kRegTile;
         const unsigned long long k = skey[i];
         uint64_t rank = i - t * kRegTile;
-        for (uint64_t u0 = 0; u0 < ntiles; u0 += kRegMergeILP) {
+        for (uint64_t u0 = ntiles > 1 ? 0 : 1; u0 < ntiles; u0 += kRegMergeILP) {
             // entries below k in eight tiles at once: 13 halvings cover 4096,
             // every load unconditional (a load behind a branch is waited for at
             // once), so that the eight are in flight together
