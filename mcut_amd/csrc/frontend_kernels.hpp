@@ -122,9 +122,9 @@ __device__ __forceinline__ double serial_sum(const double* __restrict__ v, uint3
 // walks 64 values a thread (a chunk) into segments and single steps and writes
 // them with their adds, a tile's without gaps.  k_sum_chain, one block a chain
 // on the reserved CUs, runs the DPP chain over all adds, from LDS.
-// k_sum_verify checks every item on its real start, a thread a chunk, and
-// k_sum_rest takes the values one by one from the first chunk that found a
-// start its segment does not move with (as a rule there is none).
+// k_sum_verify checks every item on its real start, a thread a chunk, and takes
+// the values one by one from the first chunk that found a start its segment
+// does not move with (as a rule there is none).
 //
 // What bounds it: the walk (64 dependent steps of about 75 instructions on one
 // wave a SIMD) and the chain (2.44 ns an add); beside the tree build and the
@@ -144,6 +144,7 @@ constexpr int kSumKeep = 16;                         // adds of a thread kept in
 constexpr int kSumChain = 256;
 constexpr uint32_t kSumLdsAdds = 16384;              // adds of a chain in LDS at a time
 constexpr uint32_t kSumSerial = 4096;
+constexpr uint32_t kSumFail = 32; // words a chain: a line each, or the chains' atomics queue on one
 
 struct SumBufs {
     const double* v[2]; // vertex arrays (xyz), null when that mesh's sums are preset
@@ -156,7 +157,7 @@ struct SumBufs {
     double* adds;       // [6][kSumMaxAdds * nblk * kSumTile]: the tiles' adds
     double* past;       // the same places, for the adds LDS has none for
     double* rows;       // [6][kSumMaxAdds * nblk * kSumTile / 16]: the chain after every 16 adds
-    uint32_t* fail;     // [6]: first chunk whose start its segment does not move with
+    uint32_t* fail;     // [6][kSumFail]: first chunk whose start its segment does not move with; blocks that checked theirs
 };
 
 __device__ __forceinline__ bool sum_chain_active(const SumBufs& B, int ch) { return B.v[ch / 3] != nullptr && B.n[ch / 3] > 0; }
@@ -170,7 +171,10 @@ __device__ __forceinline__ bool sum_chain_items(const SumBufs& B, int ch)
 __device__ __forceinline__ void sum_block(const SumBufs& B, uint32_t b, int ch, double* red)
 {
     const int m = ch / 3, j = ch % 3;
-    if (b == 0 && threadIdx.x == 0) B.fail[ch] = 0xffffffffu;
+    if (b == 0 && threadIdx.x == 0) {
+        B.fail[kSumFail * ch] = 0xffffffffu;
+        B.fail[kSumFail * ch + 1] = 0u;
+    }
     if (!sum_chain_items(B, ch)) return;
     const uint32_t n = B.n[m];
     if ((uint64_t)b * kSumTile >= n) return;
@@ -389,48 +393,65 @@ __device__ __forceinline__ double sum_chunk_start(const SumBufs& B, int ch, uint
     return s;
 }
 
-__global__ void __launch_bounds__(kSumThreads) k_sum_verify(SumBufs B)
+// Checks every chunk; the block that ends a chain last adds its values one by
+// one from the first chunk that failed, if any did, and the last of the six
+// chains makes the shift.  What passes between blocks (fail, the count behind
+// it, a sum added again) does so by device-scope atomics, each waited for
+// before the next, so no cache has to be written back; a kernel of its own for
+// the rest and the shift cost its launch and 8-14 us of the sums' path.
+__global__ void __launch_bounds__(kSumThreads) k_sum_verify(SumBufs B, const double* __restrict__ zero, Params* P, Counters* C,
+                                                            ShiftArgs A)
 {
-    const int ch = blockIdx.y;
-    if (!sum_chain_items(B, ch)) return;
-    const uint32_t c = blockIdx.x * kSumThreads + threadIdx.x;
-    if ((uint64_t)c * kSumPer >= B.n[ch / 3]) return;
-    const uint64_t chunk = (uint64_t)ch * B.nblk * kSumThreads + c;
-    const SumItem* it = B.items + chunk * kSumPer;
-    const uint32_t k = B.chunk[chunk] >> 16;
-    double s = sum_chunk_start(B, ch, c);
-    bool ok = true;
-    for (uint32_t q0 = 0; q0 < k; q0 += 4) {
-        SumItem I[4];
+    static_assert(kSumThreads == 64, "one wave a block");
+    const int ch = blockIdx.y, m = ch / 3, j = ch % 3;
+    const bool items = sum_chain_items(B, ch);
+    const uint32_t n = B.n[m], blocks = items ? (n + kSumTile - 1) / kSumTile : 1u;
+    if (blockIdx.x >= blocks) return;
+    double acc = 0.0;
+    uint32_t from = 0xffffffffu; // first chunk of the chain that failed
+    if (items) {
+        uint32_t* fail = B.fail + kSumFail * ch;
+        const uint32_t c = blockIdx.x * kSumThreads + threadIdx.x;
+        bool ok = true;
+        if ((uint64_t)c * kSumPer < n) {
+            const uint64_t chunk = (uint64_t)ch * B.nblk * kSumThreads + c;
+            const SumItem* it = B.items + chunk * kSumPer;
+            const uint32_t k = B.chunk[chunk] >> 16;
+            double s = sum_chunk_start(B, ch, c);
+            for (uint32_t q0 = 0; q0 < k; q0 += 4) {
+                SumItem I[4];
 #pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) I[q] = it[q0 + q < k ? q0 + q : k - 1];
+                for (uint32_t q = 0; q < 4; ++q) I[q] = it[q0 + q < k ? q0 + q : k - 1];
 #pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) {
-            if (q0 + q >= k) break;
-            double end = s + I[q].p, d;
-            bool odd;
-            if (!sum_is_step(I[q])) ok &= sum_apply(I[q], s, &end, &d, &odd);
-            s = end;
+                for (uint32_t q = 0; q < 4; ++q) {
+                    if (q0 + q >= k) break;
+                    double end = s + I[q].p, d;
+                    bool odd;
+                    if (!sum_is_step(I[q])) ok &= sum_apply(I[q], s, &end, &d, &odd);
+                    s = end;
+                }
+            }
+        }
+        const unsigned long long bad = __ballot(!ok);
+        uint32_t last = 0;
+        if (threadIdx.x == 0) {
+            if (bad) {
+                const uint32_t old = atomicMin(fail, blockIdx.x * kSumThreads + (uint32_t)__builtin_ctzll(bad));
+                asm volatile("" : : "v"(old) : "memory"); // its result is here: it is done
+            }
+            last = atomicAdd(fail + 1, 1u) + 1 == blocks;
+            if (last) from = atomicAdd(fail, 0u);
+        }
+        if (!__builtin_amdgcn_readfirstlane(last)) return;
+        from = __builtin_amdgcn_readfirstlane(from);
+        if (from != 0xffffffffu) {
+            __builtin_amdgcn_s_setprio(3);
+            const uint32_t i0 = from * kSumPer;
+            const double start = sum_chunk_start(B, ch, from);
+            acc = serial_chain<3, false>(B.v[m] + j + 3ull * i0, n - i0, zero, start, nullptr);
         }
     }
-    if (!ok) atomicMin(&B.fail[ch], c);
-}
-
-// the rest of the chains that failed a check, a wave each, and the shift
-__global__ void __launch_bounds__(384) k_sum_rest(SumBufs B, const double* __restrict__ zero, Params* P, const Counters* C,
-                                                  ShiftArgs A)
-{
-    const int ch = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = ch / 3, j = ch % 3;
-    const uint32_t c = __builtin_amdgcn_readfirstlane(B.fail[ch]);
-    if (c != 0xffffffffu) {
-        __builtin_amdgcn_s_setprio(3);
-        const uint32_t i0 = c * kSumPer;
-        const double start = sum_chunk_start(B, ch, c);
-        const double acc = serial_chain<3, false>(B.v[m] + j + 3ull * i0, B.n[m] - i0, zero, start, nullptr);
-        if ((threadIdx.x & 63) == 0) P->sum[m][j] = acc;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) shift_params(P, C, A);
+    sum_done(acc, from != 0xffffffffu, m, j, P, C, A);
 }
 
 // Batches: the chains of every pair's meshes (mesh m of pair p is 2 p + m),

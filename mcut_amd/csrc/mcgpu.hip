@@ -559,7 +559,7 @@ mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
     CK(ensure(ctx->planes, F, &pl));
     (void)p;
     CK(ensure(ctx->scan_tmp, scan_need + 1024, &u));
-    if (!ctx->batch) { // coordinate sums from segments (k_sum_items .. k_sum_rest), for the chains computed here
+    if (!ctx->batch) { // coordinate sums from segments (k_sum_items .. k_sum_verify), for the chains computed here
         const uint64_t nmax = std::max<uint64_t>(ctx->res ? 0 : ctx->nv[0], ctx->nv[1]);
         const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, (nmax + kSumTile - 1) / kSumTile);
         ctx->sum_nblk = nblk;
@@ -569,7 +569,7 @@ mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
             SumItem* si;
             CK(ensure(ctx->sbsum, 6ull * nblk, &dp));
             CK(ensure(ctx->sitems, region, &si));
-            CK(ensure(ctx->snitem, region / kSumPer + 6ull * nblk + 8, &u));
+            CK(ensure(ctx->snitem, region / kSumPer + 6ull * nblk + 6 * kSumFail, &u));
             CK(ensure(ctx->sadds, 2 * kSumMaxAdds * region, &dp));
             CK(ensure(ctx->srows, kSumMaxAdds * region / 16, &dp));
         }
@@ -1497,10 +1497,7 @@ void enqueue_frontend(mcgpu_context ctx)
         k_sum_chain<<<6, kSumChain, 0, ssum>>>(SB, &C->zero, Pd, C, SA, ctx->sum_items ? 0 : 1);
         ev_record(ctx, EV_SUM_CHAIN, ssum);
         ev_wait(ctx, s, EV_SUM_CHAIN);
-        if (ctx->sum_items) {
-            k_sum_verify<<<grid, kSumThreads, 0, s>>>(SB);
-            k_sum_rest<<<1, 384, 0, s>>>(SB, &C->zero, Pd, C, SA);
-        }
+        if (ctx->sum_items) k_sum_verify<<<grid, kSumThreads, 0, s>>>(SB, &C->zero, Pd, C, SA);
         ev_record(ctx, EV_A_SUMS, s);
     }
     if (ctx->batch) {
