@@ -267,9 +267,8 @@ struct CopySegs {
     void* to[kCopySegs];
     unsigned long long bytes[kCopySegs];
 };
-__global__ void __launch_bounds__(256) k_copy_segs(CopySegs S)
+__device__ __forceinline__ void copy_seg(const CopySegs& S, int q)
 {
-    const int q = blockIdx.y;
     const uint64_t n = S.bytes[q], i0 = blockIdx.x * 256ull + threadIdx.x, stride = gridDim.x * 256ull;
     const auto* f = static_cast<const uint32_t*>(S.from[q]);
     auto* t = static_cast<uint32_t*>(S.to[q]);
@@ -281,5 +280,6 @@ __global__ void __launch_bounds__(256) k_copy_segs(CopySegs S)
     if (i0 < n % 4) // the last bytes of an array of bytes
         static_cast<uint8_t*>(S.to[q])[n - n % 4 + i0] = static_cast<const uint8_t*>(S.from[q])[n - n % 4 + i0];
 }
+__global__ void __launch_bounds__(256) k_copy_segs(CopySegs S) { copy_seg(S, blockIdx.y); }
 
 } // namespace mcgpu

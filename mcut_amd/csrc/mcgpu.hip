@@ -826,6 +826,16 @@ TolArgs tol_args(mcgpu_context ctx)
     return TolArgs{ctx->nv[0], ctx->nv[1], ctx->gp_constant, absolute ? 1 : 0, (ctx->allow_loose && !ctx->res) ? 1 : 0};
 }
 
+// blocks for the largest of the staged uploads
+unsigned stage_blocks(mcgpu_context ctx)
+{
+    uint64_t most = 0;
+    for (int q = 0; q < ctx->stage_count; ++q) most = std::max<uint64_t>(most, ctx->stage_segs.bytes[q]);
+    return (unsigned)grid_for(most / 4 + 1, 4 * 256, 256);
+}
+
+mcgpu_result upload_flush(mcgpu_context ctx);
+
 constexpr uint32_t kSmallOffsets = 1u << 16; // faces whose offsets one block scans
 
 void enqueue_validate(mcgpu_context ctx)
@@ -837,7 +847,14 @@ void enqueue_validate(mcgpu_context ctx)
     Counters* C = &P_<DevState>(ctx->state)->C;
     uint32_t* etotal = P_<uint32_t>(ctx->etotal);
     ev_record(ctx, EV_A0, s);
-    k_reset_counters<<<1, kBlock, 0, s>>>(C, &P_<DevState>(ctx->state)->P, ctx->res ? ctx->res->dres : nullptr);
+    Params* Pd = &P_<DevState>(ctx->state)->P;
+    const ResidentGpuView* res = ctx->res ? ctx->res->dres : nullptr;
+    if (ctx->stage_count && !ctx->recording) { // the meshes are still in the stage
+        k_upload_reset<<<dim3(stage_blocks(ctx), ctx->stage_count + 1), kBlock, 0, s>>>(ctx->stage_segs, C, Pd, res);
+        ctx->stage_count = 0;
+    } else {
+        k_reset_counters<<<1, kBlock, 0, s>>>(C, Pd, res);
+    }
     // polygon meshes' face offsets
     OffsetMesh om[2]{};
     for (int m = ctx->res ? 1 : 0; m < 2; ++m) {
@@ -1855,6 +1872,7 @@ mcgpu_result enqueue_dispatch(mcgpu_context ctx)
         enqueue_frontend(ctx);
         return enqueue_state_copy(ctx);
     }
+    if (const mcgpu_result r = upload_flush(ctx); r != MCGPU_SUCCESS) return r; // not part of a recording
     std::vector<uint64_t> key = graph_key(ctx);
     if (key != ctx->prog_key || ctx->prog.empty()) {
         graph_drop(ctx);
@@ -1900,9 +1918,7 @@ constexpr uint64_t kStageBytes = 1u << 20;
 mcgpu_result upload_flush(mcgpu_context ctx)
 {
     if (!ctx->stage_count) return MCGPU_SUCCESS;
-    uint64_t most = 0;
-    for (int q = 0; q < ctx->stage_count; ++q) most = std::max<uint64_t>(most, ctx->stage_segs.bytes[q]);
-    k_copy_segs<<<dim3((unsigned)grid_for(most / 4 + 1, 4 * 256, 256), ctx->stage_count), 256, 0, ctx->s>>>(ctx->stage_segs);
+    k_copy_segs<<<dim3(stage_blocks(ctx), ctx->stage_count), 256, 0, ctx->s>>>(ctx->stage_segs);
     ctx->stage_count = 0;
     CK(hipGetLastError());
     return MCGPU_SUCCESS;
@@ -2336,7 +2352,7 @@ static mcgpu_result frontend_prepare(mcgpu_context ctx, const mcgpu_mesh* src, c
     if ((r = upload_begin(ctx)) != MCGPU_SUCCESS) return r;
     if ((r = upload_mesh(ctx, 0, src, desc->input_on_device != 0)) != MCGPU_SUCCESS) return r;
     if ((r = upload_mesh(ctx, 1, cut, desc->input_on_device != 0)) != MCGPU_SUCCESS) return r;
-    if ((r = upload_flush(ctx)) != MCGPU_SUCCESS) return r;
+    // what the stage holds goes up with the dispatch's first launch (enqueue_validate)
     const uint64_t F = (uint64_t)ctx->nf[0] + ctx->nf[1];
     ctx->gbits = bits_for(F + 1);
     ctx->kbits = ctx->gbits + bits_for(ctx->ncorner[0] + ctx->ncorner[1] + 1);
@@ -3319,7 +3335,6 @@ mcgpu_result slot_bind(mcgpu_server srv, mcgpu_context ctx, const mcgpu_mesh* cu
     mcgpu_result rr;
     if ((rr = upload_begin(ctx)) != MCGPU_SUCCESS) return rr;
     if ((rr = upload_mesh(ctx, 1, cut, on_device)) != MCGPU_SUCCESS) return rr;
-    if ((rr = upload_flush(ctx)) != MCGPU_SUCCESS) return rr;
     const uint64_t F = (uint64_t)ctx->nf[0] + ctx->nf[1];
     ctx->gbits = bits_for(F + 1);
     ctx->kbits = ctx->gbits + bits_for(ctx->ncorner[0] + ctx->ncorner[1] + 1);
