@@ -5,6 +5,7 @@
 // dispatch is enqueued end to end without host synchronisation.
 #pragma once
 #include "kernels.hpp"
+#include "regrank.hpp"
 #include "sort.hpp"
 #include "sumseg.hpp"
 
@@ -3459,9 +3460,8 @@ __device__ __forceinline__ void status_insert(const Soup& S, uint32_t e, uint32_
 // Registry order for up to kRegMergeTiles tiles of kRegTile entries, in two
 // launches instead of a multi-pass radix sort.  k_reg_tile_sort sorts each
 // tile in LDS and clears the status hash; k_reg_merge ranks every entry by its
-// place in its own tile plus binary searches in the other tiles (registry keys
-// are distinct), writes (edge, face, point) to that rank and counts the
-// status face pairs.
+// place in its own tile plus binary searches in the other tiles, writes (edge,
+// face, point) to that rank and counts the status face pairs.
 //
 // The tile sort is an LSD radix sort over the key's kbits bits, 8 bits a
 // pass.  Element i of a tile sits in thread i % 1024 as its row i / 1024, so a
@@ -3545,7 +3545,7 @@ __global__ void __launch_bounds__(kRegSortThreads) k_reg_tile_sort(const unsigne
 #pragma unroll
         for (int r = 0; r < kRegPer; ++r) {
             const uint32_t i = r * kRegSortThreads + t;
-            if (i >= cnt) K[r] = (1ull << 63) | i; // distinct, above every key
+            if (i >= cnt) K[r] = (1ull << 63) | i; // above every key
             if (i < P) sk[i] = K[r];
             pos[r] = i;
         }
@@ -3554,10 +3554,7 @@ __global__ void __launch_bounds__(kRegSortThreads) k_reg_tile_sort(const unsigne
         for (int r = 0; r < kRegPer; ++r) {
             if (pos[r] >= P) continue;
             const uint32_t g0 = pos[r] & ~15u;
-            uint32_t below = 0;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) below += sk[g0 + q] < K[r];
-            pos[r] = g0 + below;
+            pos[r] = g0 + reg_rank16(sk + g0, pos[r] & 15u, K[r]);
         }
         for (uint32_t w = 16; w < cnt; w <<= 1) { // runs of w, two to one
             __syncthreads();
@@ -3568,11 +3565,8 @@ __global__ void __launch_bounds__(kRegSortThreads) k_reg_tile_sort(const unsigne
 #pragma unroll
             for (int r = 0; r < kRegPer; ++r) {
                 if (pos[r] >= P) continue;
-                const unsigned long long* other = sk + ((pos[r] & ~(w - 1)) ^ w);
-                uint32_t lo = 0;
-                for (uint32_t h = w >> 1; h > 0; h >>= 1) lo += other[lo + h - 1] < K[r] ? h : 0u;
-                lo += other[lo] < K[r];
-                pos[r] = (pos[r] & ~(2 * w - 1)) + (pos[r] & (w - 1)) + lo;
+                const uint32_t other = (pos[r] & ~(w - 1)) ^ w;
+                pos[r] = (pos[r] & ~(2 * w - 1)) + (pos[r] & (w - 1)) + reg_rank_run(sk + other, w, (other & w) == 0, K[r]);
             }
         }
 #pragma unroll
@@ -3663,9 +3657,7 @@ __global__ void __launch_bounds__(kRegSortThreads) k_reg_tile_sort(const unsigne
     }
 }
 
-// first index of tile u (sorted, cnt_u entries at skey + lo_u) whose key is not
-// below k, for up to 8 tiles at once so that their loads overlap
-constexpr int kRegMergeILP = 8;
+constexpr int kRegMergeILP = 8; // tiles an entry is ranked in at once, so that their loads overlap
 
 __global__ void k_reg_merge(Soup S, const unsigned long long* __restrict__ skey, const uint32_t* __restrict__ sval,
                             const unsigned long long* __restrict__ n_dev, uint64_t cap, const uint32_t* __restrict__ e_in,
@@ -3683,31 +3675,20 @@ __global__ void k_reg_merge(Soup S, const unsigned long long* __restrict__ skey,
         const unsigned long long k = skey[i];
         uint64_t rank = i - t * kRegTile;
         for (uint64_t u0 = ntiles > 1 ? 0 : 1; u0 < ntiles; u0 += kRegMergeILP) {
-            // entries below k in eight tiles at once: 13 halvings cover 4096,
-            // every load unconditional (a load behind a branch is waited for at
-            // once), so that the eight are in flight together
+            // entries that go before k in eight tiles at once
             const unsigned long long* tile[kRegMergeILP];
+            bool first[kRegMergeILP];
             uint32_t lo[kRegMergeILP], len[kRegMergeILP];
 #pragma unroll
             for (int q = 0; q < kRegMergeILP; ++q) {
                 const uint64_t u = u0 + q, base = u * kRegTile;
                 const bool other = u < ntiles && u != t;
                 tile[q] = skey + (other ? base : 0);
+                first[q] = u < t;
                 lo[q] = 0;
                 len[q] = other ? (uint32_t)((n - base) < (uint64_t)kRegTile ? (n - base) : kRegTile) : 0u;
             }
-            for (int step = 0; step < 13; ++step) {
-                unsigned long long v[kRegMergeILP];
-#pragma unroll
-                for (int q = 0; q < kRegMergeILP; ++q) v[q] = tile[q][len[q] ? lo[q] + (len[q] >> 1) : 0];
-#pragma unroll
-                for (int q = 0; q < kRegMergeILP; ++q) {
-                    const uint32_t half = len[q] >> 1;
-                    const bool right = len[q] && v[q] < k;
-                    lo[q] += right ? half + 1 : 0;
-                    len[q] = right ? len[q] - half - 1 : half;
-                }
-            }
+            reg_rank_tiles<kRegMergeILP>(tile, first, len, lo, k);
 #pragma unroll
             for (int q = 0; q < kRegMergeILP; ++q) rank += lo[q];
         }
