@@ -5,6 +5,7 @@
 // dispatch is enqueued end to end without host synchronisation.
 #pragma once
 #include "kernels.hpp"
+#include "pairgrid.hpp"
 #include "regrank.hpp"
 #include "sort.hpp"
 #include "sumseg.hpp"
@@ -2433,6 +2434,7 @@ struct PairStage {
 // 30 us for 1,280 x 1,280 nodes
 // where this takes 14).  With the face boxes in place of nodes (one level) it
 // tests all faces of two meshes.
+static_assert(kPairTileSrc == 256 && kPairTileCut == 32, "a thread a source item, a mask of 32 cut items");
 __global__ void __launch_bounds__(256) k_pairs_start(Tree src, Tree cut, int s0, int c0, unsigned long long* __restrict__ out,
                                                      uint64_t cap, unsigned long long* n, unsigned int* over)
 {
@@ -2440,7 +2442,9 @@ __global__ void __launch_bounds__(256) k_pairs_start(Tree src, Tree cut, int s0,
     __shared__ uint32_t wsum[4];
     __shared__ unsigned long long base;
     const uint32_t ns = level_nodes(src.n, src.D, s0), nc = level_nodes(cut.n, cut.D, c0);
-    const uint32_t s = blockIdx.x * 256 + threadIdx.x, c1 = blockIdx.y * 32, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    uint32_t s1, c1;
+    pair_tile(blockIdx.x, ns, &s1, &c1);
+    const uint32_t s = s1 + threadIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (threadIdx.x < 32) {
         float b[6];
         load_box(cut.nodes, c0, c1 + threadIdx.x < nc ? c1 + threadIdx.x : nc - 1, b);

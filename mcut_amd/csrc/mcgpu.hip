@@ -1125,7 +1125,7 @@ void launch_node_pairs(const BroadView& B, const Tree& src, const Tree& cut, Cou
     while ((uint64_t)level_nodes(src.n, src.D, ls) * level_nodes(cut.n, cut.D, lc) > kPairStart)
         if (level_nodes(src.n, src.D, ls) >= level_nodes(cut.n, cut.D, lc)) --ls;
         else --lc;
-    const dim3 g0((level_nodes(src.n, src.D, ls) + 255) / 256, (level_nodes(cut.n, cut.D, lc) + 31) / 32);
+    const dim3 g0((unsigned)pair_blocks(level_nodes(src.n, src.D, ls), level_nodes(cut.n, cut.D, lc)));
     launch_timed(k_pairs_start, g0, dim3(256), st, a, (hipEvent_t) nullptr, src, cut, ls, lc, B.node_pairs[0], B.cap_nodes,
                  &C->n_nodes[0], &C->ov_nodes);
     for (; ls < ts || lc < tc; ++step) {
@@ -1166,7 +1166,7 @@ void launch_all_pairs(mcgpu_context ctx, hipStream_t st, Counters* C)
     Tree T[2];
     for (int m = 0; m < 2; ++m)
         T[m] = Tree{nullptr, P_<float>(ctx->rawbox) + (m ? 6ull * ctx->nf[0] : 0), (int)ctx->nf[m], 0};
-    const dim3 g((ctx->nf[0] + 255) / 256, (ctx->nf[1] + 31) / 32);
+    const dim3 g((unsigned)pair_blocks(ctx->nf[0], ctx->nf[1]));
     launch_timed(k_pairs_start, g, dim3(256), st, kt ? ctx->ev[EV_TRAV_K0] : nullptr, kt ? ctx->ev[EV_TRAV_K1] : nullptr, T[0],
                  T[1], 0, 0, P_<unsigned long long>(ctx->raw_pairs), ctx->cap_pairs, &C->n_raw, &C->ov_pairs);
     ev_record(ctx, EV_B_TRAV, st);
