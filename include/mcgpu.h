@@ -20,8 +20,16 @@
  *     (kernel.cpp:2237-2331, 2532-2604, 3211-3229, 3439-3452).
  *
  * Plain C types only.  Every function returns an mcgpu_result; no exception
- * crosses this boundary.  A context owns one HIP stream and its device
- * buffers; it must not be used from two threads at once.
+ * crosses this boundary.  A context owns its HIP streams and device buffers;
+ * it must not be used from two threads at once.
+ *
+ * The null stream: the CU-masked streams of mcgpu_dispatch_frontend, its
+ * enqueued form, mcgpu_dispatch_batch, mcgpu_autotune and the server's requests
+ * synchronise with it, so such a call's kernels start after the work queued
+ * there before and hold up work queued there meanwhile.  Pairs of up to 8,192
+ * faces and 4,096 vertices a mesh, the last part of an enqueued dispatch (from
+ * the candidate pairs on), and every other call that takes a context run on a
+ * stream that does not.
  *
  * The front end is a superset of what MCUT computes in one place: its broad
  * phase runs on the unshifted coordinates with a rounding bound, overlapped
@@ -140,7 +148,7 @@ typedef struct {
 
 /* --- context (one per MCUT context / API thread) ---------------------------- */
 
-/* mcCreateContext (mcut.h:567) counterpart: binds a device and creates the stream. */
+/* mcCreateContext (mcut.h:567) counterpart: binds a device and creates the streams. */
 MCGPU_API mcgpu_result mcgpu_create_context(int device, mcgpu_context* out);
 /* mcReleaseContext (mcut.h:1377) counterpart. */
 MCGPU_API mcgpu_result mcgpu_release_context(mcgpu_context ctx);
@@ -440,7 +448,7 @@ MCGPU_API mcgpu_result mcgpu_get_cutpath_edges(mcgpu_context ctx, uint32_t* src,
  * between the cross-stream event records and waits, and replay them (each on
  * the stream, and CU mask, it was captured from) while the shape stays the
  * same; a different shape (sizes, capacities, flags, traversal shape, buffer
- * addresses) records anew.  Dispatches with stage timing on run eagerly.
+ * addresses; enqueued or not) records anew.  Dispatches with stage timing on run eagerly.
  * MCGPU_ERROR_UNSUPPORTED on a serving slot's context. */
 MCGPU_API mcgpu_result mcgpu_set_graphs(mcgpu_context ctx, int enable);
 /* programs recorded and replayed so far, and the graphs of the current one */
@@ -478,7 +486,8 @@ typedef struct mcgpu_tuning {
 MCGPU_API mcgpu_result mcgpu_autotune(mcgpu_context ctx, mcgpu_tuning* out);
 /* The CU split of a context's batch streams: broad_share_pct percent (10-90)
  * of the CUs outside the sums' reservation for the broad phase, the rest for
- * the edge numbering (default 58).  The streams are made with their masks by
+ * the edge numbering (default 70, the split of single pairs, whose streams
+ * batches then share).  Streams of another split are made with their masks by
  * the context's first batch, so this is accepted only before it
  * (MCGPU_ERROR_INVALID_VALUE after). */
 MCGPU_API mcgpu_result mcgpu_set_batch_split(mcgpu_context ctx, uint32_t broad_share_pct);

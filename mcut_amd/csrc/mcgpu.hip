@@ -5,6 +5,7 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <deque>
@@ -153,7 +154,9 @@ struct Resident {
 
 struct mcgpu_context_t {
     int device = 0;
-    hipStream_t s = nullptr, s2 = nullptr, s3 = nullptr, ssum = nullptr;
+    hipStream_t s = nullptr, s2 = nullptr, s3 = nullptr, ssum = nullptr; // s: stream A of the call in progress, one of
+    hipStream_t s_plain = nullptr, s_queue = nullptr;                    // these two (StreamA; a serving slot has neither)
+    bool on_queue = false;           // the last dispatch's stream A was s_queue
     hipStream_t s2b = nullptr, s3b = nullptr; // B and C of batched dispatches, made by the first one
     hipEvent_t ev[EV_COUNT];
     hipError_t last_error = hipSuccess;
@@ -1832,6 +1835,7 @@ std::vector<uint64_t> graph_key(mcgpu_context ctx)
     std::vector<uint64_t> k;
     auto put = [&k](uint64_t x) { k.push_back(x); };
     auto ptr = [&k](const void* p) { k.push_back((uint64_t)(uintptr_t)p); };
+    ptr(ctx->s); // the program holds its streams
     put(ctx->batch), put(ctx->npairs), put(ctx->batch_mb), put(ctx->cc_check), put(ctx->batch ? ctx->sort_bits : leaf_bits(ctx)),
         put(ctx->shifted_bp), put(ctx->walk), put(ctx->trav.walk), put(ctx->want_trees), put(ctx->one_stream), put(ctx->forced), put(ctx->cap_nodes), put(ctx->topo_hash), put(ctx->topo_buckets), put(ctx->topo_tiles), put(ctx->topo_bits),
         put(ctx->nseg), put(ctx->topo_ranges), put(ctx->batch ? batch_box_tiles(ctx) : 0),
@@ -2023,37 +2027,122 @@ MCGPU_API const char* mcgpu_result_string(mcgpu_result r)
     return "unknown";
 }
 
-// Stream A: a mask of every CU, which gives it a hardware queue of its own like
-// the other three.  On a queue of the runtime's pool its kernels waited while
-// a large grid of stream C was being placed (a one-thread kernel for 0.33 ms
-// on two 1.3 M triangle meshes, the whole dispatch 1.69 ms against 1.47).
-static hipError_t create_full_stream(int ncu, hipStream_t* s)
-{
-    std::vector<uint32_t> m((ncu + 31) / 32, 0u);
-    for (int i = 0; i < ncu; ++i) m[i / 32] |= 1u << (i % 32);
-    return hipExtStreamCreateWithCUMask(s, (uint32_t)m.size(), m.data());
-}
-
 // Streams B and C of a dispatch: disjoint CU sets outside the first kSumCUs,
 // B taking `share` of them; a device too small to partition gets no masks.
+static void split_masks(int ncu, double share, std::vector<uint32_t>* b, std::vector<uint32_t>* c)
+{
+    b->assign((ncu + 31) / 32, 0u);
+    c->assign((ncu + 31) / 32, 0u);
+    const int nb = kSumCUs + (int)(share * (ncu - kSumCUs) + 0.5);
+    for (int i = kSumCUs; i < ncu; ++i) (i < nb ? *b : *c)[i / 32] |= 1u << (i % 32);
+    if (ncu <= 4 * kSumCUs) {
+        std::fill(b->begin(), b->end(), ~0u);
+        std::fill(c->begin(), c->end(), ~0u);
+    }
+}
+
 static hipError_t create_split_streams(int ncu, double share, hipStream_t* b, hipStream_t* c)
 {
-    const int nw = (ncu + 31) / 32;
-    std::vector<uint32_t> mb(nw, 0u), mc(nw, 0u);
-    const int nb = kSumCUs + (int)(share * (ncu - kSumCUs) + 0.5);
-    for (int i = kSumCUs; i < ncu; ++i) (i < nb ? mb : mc)[i / 32] |= 1u << (i % 32);
-    if (ncu <= 4 * kSumCUs) {
-        std::fill(mb.begin(), mb.end(), ~0u);
-        std::fill(mc.begin(), mc.end(), ~0u);
-    }
-    hipError_t e = hipExtStreamCreateWithCUMask(b, nw, mb.data());
+    std::vector<uint32_t> mb, mc;
+    split_masks(ncu, share, &mb, &mc);
+    hipError_t e = hipExtStreamCreateWithCUMask(b, (uint32_t)mb.size(), mb.data());
     if (e != hipSuccess) return e;
-    if ((e = hipExtStreamCreateWithCUMask(c, nw, mc.data())) != hipSuccess) {
+    if ((e = hipExtStreamCreateWithCUMask(c, (uint32_t)mc.size(), mc.data())) != hipSuccess) {
         (void)hipStreamDestroy(*b);
         *b = nullptr;
     }
     return e;
 }
+
+// A context's streams.  A CU-masked stream has a hardware queue of its own,
+// and the queues are dealt to the device's four pipes in the order they are
+// made, so the four masked ones (s_queue with every CU) land on a pipe each.
+// Stream A on a plain stream, whose queue may share the pipe of one of them,
+// waits while a large grid of that one is being placed (a polygon pair 0.43 ms
+// against 0.34, two meshes of 1.3 M triangles 1.54 against 1.48).
+//
+// Every context starts at the next of the four: with one order for all, their
+// like streams share a pipe and run one after another.  Dispatches a second of
+// two contexts in two threads: 32,000 triangles a mesh 2,530 with one order,
+// 5,150 this way (one context 3,900); 72,000 2,360 and 4,260; eight contexts of
+// the latter 2,510 and 3,880.
+//
+// s_plain does not synchronise with the null stream, as masked streams do.
+constexpr unsigned kMaxDevices = 64;
+
+// The runtime makes the queues that plain streams share one by one, up to four
+// (GPU_MAX_HW_QUEUES), as plain streams are made.  All of them exist before the
+// first masked stream, so that none made later moves one context's masked
+// streams against another's.
+static void fill_plain_queues()
+{
+    const char* most = getenv("GPU_MAX_HW_QUEUES");
+    const int n = most ? std::max(1, std::min(32, atoi(most))) : 4;
+    std::vector<hipStream_t> st;
+    for (int i = 0; i < n; ++i) {
+        hipStream_t s = nullptr;
+        if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) break;
+        st.push_back(s);
+    }
+    for (hipStream_t s : st) (void)hipStreamDestroy(s);
+}
+
+static hipError_t create_streams(mcgpu_context ctx, int ncu)
+{
+    static std::atomic<unsigned> made[kMaxDevices]; // contexts of each device: where the next one starts
+    ctx->ncu = ncu;
+    // the first kSumCUs compute units for the serial sums, the rest for the
+    // streams that run beside them
+    std::vector<uint32_t> every((ncu + 31) / 32, 0u), sums((ncu + 31) / 32, 0u), mb, mc;
+    for (int i = 0; i < ncu; ++i) every[i / 32] |= 1u << (i % 32);
+    for (int i = 0; i < kSumCUs && i < ncu; ++i) sums[i / 32] |= 1u << (i % 32);
+    split_masks(ncu, kBroadShare, &mb, &mc);
+    hipStream_t* const st[4] = {&ctx->s_queue, &ctx->ssum, &ctx->s2, &ctx->s3};
+    const std::vector<uint32_t>* const mask[4] = {&every, &sums, &mb, &mc};
+    hipError_t e = hipStreamCreateWithFlags(&ctx->s_plain, hipStreamNonBlocking);
+    const unsigned first = made[(unsigned)ctx->device % kMaxDevices]++;
+    if (first == 0) fill_plain_queues();
+    for (unsigned q = 0; q < 4 && e == hipSuccess; ++q) {
+        const unsigned i = (first + q) % 4;
+        e = hipExtStreamCreateWithCUMask(st[i], (uint32_t)mask[i]->size(), mask[i]->data());
+    }
+    ctx->s = ctx->s_plain;
+    return e;
+}
+
+static void destroy_streams(mcgpu_context ctx)
+{
+    if (!ctx->own_streams) { // a serving slot's one stream
+        (void)hipStreamDestroy(ctx->s);
+        return;
+    }
+    if (ctx->s2b == ctx->s2) ctx->s2b = ctx->s3b = nullptr;
+    for (hipStream_t st : {ctx->ssum, ctx->s3, ctx->s2, ctx->s3b, ctx->s2b, ctx->s_plain, ctx->s_queue})
+        if (st) (void)hipStreamDestroy(st);
+}
+
+// Stream A of an entry point, which the caller waits for: s_queue for a
+// dispatch over four streams (three of them synchronise with the null stream
+// anyway), s_plain for all else, so that calls on stream A alone, and a
+// dispatch that goes on after its call returned, neither wait for a caller's
+// work on the null stream nor hold it up.  A pair on one stream is faster on
+// s_plain, too (960 against 192 faces 171 us, 205 on s_queue).
+struct StreamA {
+    mcgpu_context ctx;
+    bool done = false; // the host has waited for it
+    StreamA(mcgpu_context c, bool queue) : ctx(c)
+    {
+        if (ctx->s_plain) ctx->s = queue ? ctx->s_queue : ctx->s_plain;
+        ctx->on_queue = queue;
+    }
+    StreamA(const StreamA&) = delete;
+    ~StreamA()
+    {
+        if (!ctx->s_plain || ctx->s == ctx->s_plain) return;
+        if (!done) (void)hipStreamSynchronize(ctx->s);
+        ctx->s = ctx->s_plain;
+    }
+};
 
 // percent of the CUs outside the sums' reservation that the dispatch's
 // broad-phase stream holds (100: one stream for everything)
@@ -2275,22 +2364,8 @@ MCGPU_API mcgpu_result mcgpu_create_context(int device, mcgpu_context* out)
     ctx->device = device;
     hipDeviceProp_t prop;
     if (hipSetDevice(device) != hipSuccess || hipGetDeviceProperties(&prop, device) != hipSuccess ||
-        create_full_stream(prop.multiProcessorCount, &ctx->s) != hipSuccess) {
-        delete ctx;
-        return MCGPU_ERROR_DEVICE;
-    }
-    // CU masks: the first kSumCUs compute units for the serial sums, the rest
-    // for the streams that run beside them
-    const int ncu = prop.multiProcessorCount;
-    ctx->ncu = ncu;
-    const int nw = (ncu + 31) / 32;
-    std::vector<uint32_t> msum(nw, 0u);
-    for (int c = 0; c < kSumCUs && c < ncu; ++c) msum[c / 32] |= 1u << (c % 32);
-    if (hipExtStreamCreateWithCUMask(&ctx->ssum, nw, msum.data()) != hipSuccess ||
-        create_split_streams(ncu, kBroadShare, &ctx->s2, &ctx->s3) != hipSuccess) {
-        for (hipStream_t st : {ctx->ssum, ctx->s2, ctx->s3})
-            if (st) (void)hipStreamDestroy(st);
-        (void)hipStreamDestroy(ctx->s);
+        create_streams(ctx, prop.multiProcessorCount) != hipSuccess) {
+        destroy_streams(ctx);
         delete ctx;
         return MCGPU_ERROR_DEVICE;
     }
@@ -2305,7 +2380,7 @@ MCGPU_API mcgpu_result mcgpu_release_context(mcgpu_context ctx)
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->s);
     if (ctx->own_streams) {
-        for (hipStream_t st : {ctx->s2, ctx->s3, ctx->s2b, ctx->s3b, ctx->ssum})
+        for (hipStream_t st : {ctx->s2, ctx->s3, ctx->s2b, ctx->s3b, ctx->ssum, ctx->s_queue})
             if (st) (void)hipStreamSynchronize(st);
     }
     for (const GraphOp& op : ctx->prog)
@@ -2316,12 +2391,7 @@ MCGPU_API mcgpu_result mcgpu_release_context(mcgpu_context ctx)
         if (p) (void)hipHostFree(p);
     for (int i = 0; i < EV_COUNT; ++i) (void)hipEventDestroy(ctx->ev[i]);
     if (ctx->ev_user) (void)hipEventDestroy(ctx->ev_user);
-    if (ctx->own_streams) {
-        if (ctx->s2b == ctx->s2) ctx->s2b = ctx->s3b = nullptr;
-        for (hipStream_t st : {ctx->ssum, ctx->s3, ctx->s2, ctx->s3b, ctx->s2b})
-            if (st) (void)hipStreamDestroy(st);
-    }
-    (void)hipStreamDestroy(ctx->s);
+    destroy_streams(ctx);
     delete ctx;
     return MCGPU_SUCCESS;
 }
@@ -2390,17 +2460,25 @@ static mcgpu_result frontend_complete(mcgpu_context ctx, mcgpu_frontend_info* in
 MCGPU_API mcgpu_result mcgpu_dispatch_frontend(mcgpu_context ctx, const mcgpu_mesh* src, const mcgpu_mesh* cut,
                                                const mcgpu_dispatch_desc* desc, mcgpu_frontend_info* info)
 {
+    if (!ctx || ctx->pending || !src || !cut) return MCGPU_ERROR_INVALID_VALUE;
+    // four streams, unless the pair is as small as uses_one_stream() takes
+    StreamA a(ctx, (uint64_t)src->num_faces + cut->num_faces > kOneStream ||
+                       std::max(src->num_vertices, cut->num_vertices) > kSumSerial);
     mcgpu_result r;
     if ((r = frontend_prepare(ctx, src, cut, desc)) != MCGPU_SUCCESS) return r;
     if ((r = alloc_list_buffers(ctx)) != MCGPU_SUCCESS) return r;
     ctx->stage_mode = 0;
     if ((r = enqueue_dispatch(ctx)) != MCGPU_SUCCESS) return r;
-    return frontend_complete(ctx, info, 0);
+    r = frontend_complete(ctx, info, 0);
+    a.done = r == MCGPU_SUCCESS;
+    return r;
 }
 
 MCGPU_API mcgpu_result mcgpu_dispatch_frontend_async(mcgpu_context ctx, const mcgpu_mesh* src, const mcgpu_mesh* cut,
                                                      const mcgpu_dispatch_desc* desc, void* stream)
 {
+    if (!ctx || ctx->pending) return MCGPU_ERROR_INVALID_VALUE;
+    StreamA a(ctx, false);
     mcgpu_result r;
     if ((r = frontend_prepare(ctx, src, cut, desc)) != MCGPU_SUCCESS) return r;
     if ((r = alloc_list_buffers(ctx)) != MCGPU_SUCCESS) return r;
@@ -2455,6 +2533,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
     const int pb = bits_for(np);
     if (pb > 28) return MCGPU_ERROR_UNSUPPORTED;
     CK(hipSetDevice(ctx->device));
+    StreamA a(ctx, true);
     ctx->have = false;
     ctx->broad_only = false;
     ctx->batch = true;
@@ -2569,7 +2648,9 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
         if ((r = finish(ctx, info, &overflow)) != MCGPU_SUCCESS) return r;
         if (!overflow) {
             if ((r = finish_batch(ctx, info)) != MCGPU_SUCCESS) return r;
-            return autotune_first(ctx);
+            r = autotune_first(ctx);
+            a.done = r == MCGPU_SUCCESS;
+            return r;
         }
     }
     return MCGPU_ERROR_OUT_OF_MEMORY;
@@ -3005,7 +3086,10 @@ MCGPU_API mcgpu_result mcgpu_autotune(mcgpu_context ctx, mcgpu_tuning* out)
     if (!ctx) return MCGPU_ERROR_INVALID_VALUE;
     if (!ctx->have || ctx->broad_only || ctx->stage_mode != 0 || ctx->res) return MCGPU_ERROR_NO_RESULT;
     CK(hipSetDevice(ctx->device));
-    return autotune(ctx, out);
+    StreamA a(ctx, ctx->on_queue);
+    const mcgpu_result r = autotune(ctx, out);
+    a.done = r == MCGPU_SUCCESS;
+    return r;
 }
 
 MCGPU_API mcgpu_result mcgpu_cutpath_edges(mcgpu_context ctx, const uint32_t* order, mcgpu_cutpath_info* info)
