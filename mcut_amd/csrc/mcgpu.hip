@@ -902,10 +902,6 @@ void enqueue_validate(mcgpu_context ctx)
         k_tolerance<<<1, 1, 0, s>>>(&P_<DevState>(ctx->state)->P, C, tol_args(ctx));
 }
 
-// Batches: the same reset and validation, per pair: segment ids of every
-// vertex and face, face lists checked against their own pair's vertex count
-// and rewritten as ids of the concatenated part, raw boxes of every (pair,
-// mesh), each pair's broad-phase tolerance, and the cell layout.
 // tiles of the batch's largest mesh
 uint32_t batch_box_tiles(mcgpu_context ctx)
 {
@@ -914,6 +910,10 @@ uint32_t batch_box_tiles(mcgpu_context ctx)
     return (nv + kBatchBoxTile - 1) / kBatchBoxTile;
 }
 
+// Batches: the same reset and validation, per pair: segment ids of every
+// vertex and face, face lists checked against their own pair's vertex count
+// and rewritten as ids of the concatenated part, raw boxes of every (pair,
+// mesh), each pair's broad-phase tolerance, and the cell layout.
 void enqueue_validate_batch(mcgpu_context ctx)
 {
     ctx->state_copied = false;
@@ -958,8 +958,16 @@ void enqueue_validate_batch(mcgpu_context ctx)
     k_batch_layout<<<1, 1024, 0, s>>>(Pb, brbox, np);
 }
 
-// per-pair results of a batch, after finish(): status bits and registry
-// ranges read back, statuses decided as for one pair
+// The launch's own error: the thread's last error, which finish() reports, may
+// be another library's (a registry can be read all the same) or that of a
+// launch of this dispatch (which a check here would take from finish()).
+hipError_t launch_copies(const CopySegs& S, unsigned blocks, int n, hipStream_t st)
+{
+    CopySegs arg = S;
+    void* args[] = {&arg};
+    return hipLaunchKernel(reinterpret_cast<const void*>(k_copy_segs), dim3(blocks, n), dim3(256), args, 0, st);
+}
+
 // Device to host, ordered behind stream A's work and complete on return: up to
 // kStageBytes through the pinned stage by one launch, more by a copy each.
 struct Fetch {
@@ -1008,13 +1016,14 @@ mcgpu_result fetch(mcgpu_context ctx, std::initializer_list<Fetch> list)
         S.to[q] = ctx->stage_out + place[q];
         S.bytes[q] = of[q]->bytes;
     }
-    k_copy_segs<<<dim3((unsigned)grid_for(most / 4 + 1, 4 * 256, 256), n), 256, 0, ctx->s>>>(S);
-    CK(hipGetLastError());
+    CK(launch_copies(S, (unsigned)grid_for(most / 4 + 1, 4 * 256, 256), n, ctx->s));
     CK(hipStreamSynchronize(ctx->s));
     for (int q = 0; q < n; ++q) std::memcpy(of[q]->to, ctx->stage_out + place[q], of[q]->bytes);
     return MCGPU_SUCCESS;
 }
 
+// per-pair results of a batch, after finish(): status bits and registry
+// ranges read back, statuses decided as for one pair
 mcgpu_result finish_batch(mcgpu_context ctx, mcgpu_frontend_info* info)
 {
     const uint32_t np = ctx->npairs;
@@ -1636,8 +1645,7 @@ mcgpu_result enqueue_state_copy(mcgpu_context ctx)
     S.from[0] = ctx->state.p;
     S.to[0] = ctx->hstate;
     S.bytes[0] = sizeof(DevState);
-    k_copy_segs<<<1, 256, 0, ctx->s>>>(S);
-    CK(hipGetLastError());
+    CK(launch_copies(S, 1, 1, ctx->s));
     ctx->state_copied = true;
     return MCGPU_SUCCESS;
 }
@@ -1922,9 +1930,10 @@ constexpr uint64_t kStageBytes = 1u << 20;
 mcgpu_result upload_flush(mcgpu_context ctx)
 {
     if (!ctx->stage_count) return MCGPU_SUCCESS;
-    k_copy_segs<<<dim3(stage_blocks(ctx), ctx->stage_count), 256, 0, ctx->s>>>(ctx->stage_segs);
+    const unsigned blocks = stage_blocks(ctx);
+    const int n = ctx->stage_count;
     ctx->stage_count = 0;
-    CK(hipGetLastError());
+    CK(launch_copies(ctx->stage_segs, blocks, n, ctx->s));
     return MCGPU_SUCCESS;
 }
 
