@@ -1650,7 +1650,13 @@ mcgpu_result enqueue_state_copy(mcgpu_context ctx)
     return MCGPU_SUCCESS;
 }
 
-mcgpu_result finish(mcgpu_context ctx, mcgpu_frontend_info* info, bool* overflow)
+// What finish() found: the dispatch is whole; it has to run again another way
+// (each of them taken at most once a dispatch, so callers count no attempt);
+// or with lists that were too short and have been grown.
+enum class Again { kNo, kOtherPath, kLongerLists };
+constexpr int kListAttempts = 6; // runs with lists of new lengths: each finds what a shorter list before it hid
+
+mcgpu_result finish(mcgpu_context ctx, mcgpu_frontend_info* info, Again* again)
 {
     ctx->cp_have = false; // cut-path edges belong to the dispatch they were made from
     // stream A joins the other three before its last kernel, so it finishes last
@@ -1667,7 +1673,7 @@ mcgpu_result finish(mcgpu_context ctx, mcgpu_frontend_info* info, bool* overflow
     ctx->C = hs.C;
     ctx->P = hs.P;
     const Counters& C = ctx->C;
-    *overflow = false;
+    *again = Again::kNo;
     if (getenv("MCGPU_DEBUG"))
         fprintf(stderr,
                 "[mcgpu] raw=%llu pairs=%llu tests=%llu esc=%llu reg=%llu big=%llu cand=%llu edges=%llu+%llu ov=%u/%u/%u/%u/%u "
@@ -1692,23 +1698,22 @@ mcgpu_result finish(mcgpu_context ctx, mcgpu_frontend_info* info, bool* overflow
         if ((!ctx->res && C.ncc[0] != want) || C.ncc[1] != want) return MCGPU_ERROR_INVALID_VALUE;
     }
     if (C.unsupported & 2u) return MCGPU_ERROR_UNSUPPORTED;
-    if (C.loose && !ctx->shifted_bp) { // run again with the broad phase in shifted coordinates
+    if (C.loose && !ctx->shifted_bp) { // the broad phase in shifted coordinates
         ctx->shifted_bp = true;
-        *overflow = true;
-        return MCGPU_SUCCESS;
+        *again = Again::kOtherPath;
     }
-    if (C.ov_nodes) { // run again with the walk
+    if (C.ov_nodes) { // the walk
         node_pairs_overflowed(ctx, C);
-        *overflow = true;
-        return MCGPU_SUCCESS;
+        *again = Again::kOtherPath;
     }
-    if (C.ov_topo) { // run again with the edges numbered through the hash tables
+    if (C.ov_topo) { // the edges numbered through the hash tables
         ctx->topo_hash = true;
-        *overflow = true;
-        return alloc_edge_tables(ctx);
+        *again = Again::kOtherPath;
+        if (const mcgpu_result r = alloc_edge_tables(ctx); r != MCGPU_SUCCESS) return r;
     }
+    if (*again != Again::kNo) return MCGPU_SUCCESS; // the lists' counts are not that path's
     if (C.ov_pairs || C.ov_tests || C.ov_esc || C.ov_reg || C.ov_big || C.ov_trip) {
-        *overflow = true;
+        *again = Again::kLongerLists;
         // a refusal leaves the context's capacities as they were
         const uint64_t was[6] = {ctx->cap_pairs, ctx->cap_tests, ctx->cap_esc, ctx->cap_reg, ctx->cap_big,
                                  ctx->cap_trip};
@@ -2210,10 +2215,10 @@ static mcgpu_result rerun_dispatch(mcgpu_context ctx, float* ms)
     ctx->stage_mode = 0;
     mcgpu_result r = enqueue_dispatch(ctx);
     if (r != MCGPU_SUCCESS) return r;
-    bool overflow = false;
-    r = finish(ctx, nullptr, &overflow);
+    Again again;
+    r = finish(ctx, nullptr, &again);
     if (r != MCGPU_SUCCESS) return r;
-    if (overflow) return MCGPU_ERROR_DEVICE; // the same input cannot outgrow the lists it sized
+    if (again != Again::kNo) return MCGPU_ERROR_DEVICE; // the same input cannot outgrow the lists it sized
     if (ctx->batch && (r = finish_batch(ctx, nullptr)) != MCGPU_SUCCESS) return r;
     *ms = ctx->total_ms;
     return MCGPU_SUCCESS;
@@ -2452,14 +2457,14 @@ static mcgpu_result frontend_prepare(mcgpu_context ctx, const mcgpu_mesh* src, c
 
 // Completes an enqueued single-pair dispatch: waits, reads its counters, and
 // re-runs it with grown lists while one overflowed.
-static mcgpu_result frontend_complete(mcgpu_context ctx, mcgpu_frontend_info* info, int attempt)
+static mcgpu_result frontend_complete(mcgpu_context ctx, mcgpu_frontend_info* info)
 {
     mcgpu_result r;
-    for (;; ++attempt) {
-        bool overflow = false;
-        if ((r = finish(ctx, info, &overflow)) != MCGPU_SUCCESS) return r;
-        if (!overflow) return autotune_first(ctx);
-        if (attempt + 1 >= 6) return MCGPU_ERROR_OUT_OF_MEMORY;
+    for (int attempt = 1;;) {
+        Again again;
+        if ((r = finish(ctx, info, &again)) != MCGPU_SUCCESS) return r;
+        if (again == Again::kNo) return autotune_first(ctx);
+        if (again == Again::kLongerLists && ++attempt > kListAttempts) return MCGPU_ERROR_OUT_OF_MEMORY;
         if ((r = alloc_list_buffers(ctx)) != MCGPU_SUCCESS) return r;
         ctx->stage_mode = 0;
         if ((r = enqueue_dispatch(ctx)) != MCGPU_SUCCESS) return r;
@@ -2478,7 +2483,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_frontend(mcgpu_context ctx, const mcgpu_me
     if ((r = alloc_list_buffers(ctx)) != MCGPU_SUCCESS) return r;
     ctx->stage_mode = 0;
     if ((r = enqueue_dispatch(ctx)) != MCGPU_SUCCESS) return r;
-    r = frontend_complete(ctx, info, 0);
+    r = frontend_complete(ctx, info);
     a.done = r == MCGPU_SUCCESS;
     return r;
 }
@@ -2514,7 +2519,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_wait(mcgpu_context ctx, mcgpu_frontend_inf
     if (!ctx->pending) return MCGPU_ERROR_NO_RESULT;
     CK(hipSetDevice(ctx->device));
     ctx->pending = false;
-    const mcgpu_result r = frontend_complete(ctx, info, 0);
+    const mcgpu_result r = frontend_complete(ctx, info);
     if (r == MCGPU_SUCCESS && stream) // work queued on the caller's stream from now on sees the results
         CK(hipStreamWaitEvent((hipStream_t)stream, ctx->ev[EV_A_END], 0));
     return r;
@@ -2649,13 +2654,14 @@ MCGPU_API mcgpu_result mcgpu_dispatch_batch(mcgpu_context ctx, const mcgpu_batch
     if (ctx->cap_reg < ctx->cap_tests / 32) ctx->cap_reg = std::max<uint64_t>(1 << 14, ctx->cap_tests / 32);
     if (ctx->cap_big < 1024) ctx->cap_big = 1024;
     if (ctx->cap_trip < (1u << 16)) ctx->cap_trip = 1u << 16;
-    for (int attempt = 0; attempt < 6; ++attempt) {
+    for (int attempt = 0; attempt < kListAttempts;) {
         if ((r = alloc_list_buffers(ctx)) != MCGPU_SUCCESS) return r;
         ctx->stage_mode = 0;
         if ((r = enqueue_dispatch(ctx)) != MCGPU_SUCCESS) return r;
-        bool overflow = false;
-        if ((r = finish(ctx, info, &overflow)) != MCGPU_SUCCESS) return r;
-        if (!overflow) {
+        Again again;
+        if ((r = finish(ctx, info, &again)) != MCGPU_SUCCESS) return r;
+        attempt += again == Again::kLongerLists;
+        if (again == Again::kNo) {
             if ((r = finish_batch(ctx, info)) != MCGPU_SUCCESS) return r;
             r = autotune_first(ctx);
             a.done = r == MCGPU_SUCCESS;
@@ -2836,7 +2842,7 @@ MCGPU_API mcgpu_result mcgpu_redispatch_perturbed(mcgpu_context ctx, const doubl
     if (!ctx->have || ctx->broad_only || ctx->batch) return MCGPU_ERROR_NO_RESULT;
     CK(hipSetDevice(ctx->device));
     ctx->enforcement_count = enforcement_count;
-    for (int attempt = 0; attempt < 6; ++attempt) {
+    for (int attempt = 0; attempt < kListAttempts; ++attempt) {
         mcgpu_result r;
         if ((r = alloc_list_buffers(ctx)) != MCGPU_SUCCESS) return r;
         hipStream_t s = ctx->s;
@@ -2855,9 +2861,9 @@ MCGPU_API mcgpu_result mcgpu_redispatch_perturbed(mcgpu_context ctx, const doubl
         stage_event(ctx, EV_A_FILTER, s);
         enqueue_narrow(ctx, make_soup(ctx), false, ctx->pairs_given ? kPairsGiven : kPairsMoved);
         (void)enqueue_state_copy(ctx); // on failure finish() copies after its wait
-        bool overflow = false;
-        if ((r = finish(ctx, info, &overflow)) != MCGPU_SUCCESS) return r;
-        if (!overflow) return MCGPU_SUCCESS;
+        Again again;
+        if ((r = finish(ctx, info, &again)) != MCGPU_SUCCESS) return r;
+        if (again == Again::kNo) return MCGPU_SUCCESS;
         // a list overflowed: the pairs are intact, so only the narrow part reruns
     }
     return MCGPU_ERROR_OUT_OF_MEMORY;
@@ -3641,10 +3647,10 @@ MCGPU_API mcgpu_result mcgpu_server_run(mcgpu_server srv, const mcgpu_mesh* cuts
             const uint32_t i = (uint32_t)busy[s];
             mcgpu_context c = srv->slots[s];
             mcgpu_frontend_info info;
-            bool overflow = false;
-            mcgpu_result r = finish(c, &info, &overflow);
-            if (r == MCGPU_SUCCESS && overflow) { // a list outgrew its capacity: grow and run it again
-                if (++reruns[s] > 5) r = MCGPU_ERROR_OUT_OF_MEMORY;
+            Again again;
+            mcgpu_result r = finish(c, &info, &again);
+            if (r == MCGPU_SUCCESS && again != Again::kNo) {
+                if (again == Again::kLongerLists && ++reruns[s] >= kListAttempts) r = MCGPU_ERROR_OUT_OF_MEMORY;
                 else if ((r = alloc_list_buffers(c)) == MCGPU_SUCCESS) {
                     slot_enqueue(c, srv->done[s]);
                     continue;
@@ -3957,7 +3963,7 @@ MCGPU_API mcgpu_result mcgpu_dispatch_narrow(mcgpu_context ctx, const mcgpu_mesh
     if (ctx->cap_trip < (1u << 16)) ctx->cap_trip = 1u << 16;
     std::vector<unsigned long long> keys(num_pairs);
     for (uint64_t i = 0; i < num_pairs; ++i) keys[i] = ((unsigned long long)pairs[2 * i] << 32) | pairs[2 * i + 1];
-    for (int attempt = 0; attempt < 6; ++attempt) {
+    for (int attempt = 0; attempt < kListAttempts;) {
         if ((r = alloc_list_buffers(ctx)) != MCGPU_SUCCESS) return r;
         hipStream_t s = ctx->s;
         ctx->stage_mode = 1;
@@ -4003,9 +4009,10 @@ MCGPU_API mcgpu_result mcgpu_dispatch_narrow(mcgpu_context ctx, const mcgpu_mesh
         stage_event(ctx, EV_A_FILTER, s);
         enqueue_narrow(ctx, make_soup(ctx), false, kPairsGiven);
         (void)enqueue_state_copy(ctx); // on failure finish() copies after its wait
-        bool overflow = false;
-        if ((r = finish(ctx, info, &overflow)) != MCGPU_SUCCESS) return r;
-        if (!overflow) return MCGPU_SUCCESS;
+        Again again;
+        if ((r = finish(ctx, info, &again)) != MCGPU_SUCCESS) return r;
+        if (again == Again::kNo) return MCGPU_SUCCESS;
+        attempt += again == Again::kLongerLists;
     }
     return MCGPU_ERROR_OUT_OF_MEMORY;
 }
