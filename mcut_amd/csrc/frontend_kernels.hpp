@@ -139,8 +139,9 @@ __device__ __forceinline__ double serial_sum(const double* __restrict__ v, uint3
 // 1 M vertex terrain of whole coordinates, whose sums meet powers of two and
 // were added serially in 6.4 ms beside the other streams.  Chains of up to kSumSerial values are added
 // serially at once: the walks cost that much in launches.
-constexpr int kSumThreads = 64, kSumPer = 64;
+constexpr int kSumThreads = 64, kSumPer = kSumChunk;
 constexpr uint32_t kSumTile = kSumThreads * kSumPer; // values per block
+constexpr uint32_t kSumTileAdds = kSumThreads * kSumChunkAdds;
 constexpr int kSumLds = kSumPer + 1;                 // LDS stride of a thread's values (no bank conflicts)
 constexpr int kSumKeep = 16;                         // adds of a thread kept in LDS
 constexpr int kSumChain = 256;
@@ -151,18 +152,24 @@ constexpr uint32_t kSumFail = 32; // words a chain: a line each, or the chains' 
 struct SumBufs {
     const double* v[2]; // vertex arrays (xyz), null when that mesh's sums are preset
     uint32_t n[2];      // vertex counts
-    uint32_t nblk;      // tiles per chain (of the larger mesh)
-    double* bsum;       // [6][nblk]
-    SumItem* items;     // [6][nblk * kSumTile]: kSumPer places a chunk
-    uint32_t* chunk;    // [6][nblk * kSumThreads]: items << 16 | first add in the tile
-    uint32_t* nadd;     // [6][nblk]: adds of each tile (padded to 16), then its first add in the chain
-    double* adds;       // [6][kSumMaxAdds * nblk * kSumTile]: the tiles' adds
+    uint32_t tiles[2];  // tiles of each mesh's three chains (0: no items)
+    // for the tiles of all six chains (sum_tile0)
+    double* bsum;       // [tile]
+    SumItem* items;     // [tile][kSumTile]: kSumPer places a chunk
+    uint32_t* chunk;    // [tile][kSumThreads]: items << 16 | first add in the tile
+    uint32_t* nadd;     // [tile]: adds of each tile (padded to 16), then its first add in the chain
+    double* adds;       // [tile][kSumTileAdds]: the tiles' adds
     double* past;       // the same places, for the adds LDS has none for
-    double* rows;       // [6][kSumMaxAdds * nblk * kSumTile / 16]: the chain after every 16 adds
+    double* rows;       // [tile][kSumTileAdds / 16]: the chain after every 16 adds
     uint32_t* fail;     // [6][kSumFail]: first chunk whose start its segment does not move with; blocks that checked theirs
 };
 
 __device__ __forceinline__ bool sum_chain_active(const SumBufs& B, int ch) { return B.v[ch / 3] != nullptr && B.n[ch / 3] > 0; }
+// a chain's first tile
+__device__ __forceinline__ uint64_t sum_tile0(const SumBufs& B, int ch)
+{
+    return ch < 3 ? (uint64_t)ch * B.tiles[0] : 3ull * B.tiles[0] + (uint64_t)(ch - 3) * B.tiles[1];
+}
 // whether a chain goes through items
 __device__ __forceinline__ bool sum_chain_items(const SumBufs& B, int ch)
 {
@@ -193,7 +200,7 @@ __device__ __forceinline__ void sum_block(const SumBufs& B, uint32_t b, int ch, 
     for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
     __syncthreads();
-    if (threadIdx.x == 0) B.bsum[(uint64_t)ch * B.nblk + b] = (red[0] + red[1]) + (red[2] + red[3]);
+    if (threadIdx.x == 0) B.bsum[sum_tile0(B, ch) + b] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 __global__ void __launch_bounds__(kSumThreads) k_sum_items(SumBufs B)
@@ -223,7 +230,7 @@ __global__ void __launch_bounds__(kSumThreads) k_sum_items(SumBufs B)
         }
     }
     double a0 = 0.0; // the tiles before this one
-    for (uint32_t q = t; q < b; q += kSumThreads) a0 += B.bsum[(uint64_t)ch * B.nblk + q];
+    for (uint32_t q = t; q < b; q += kSumThreads) a0 += B.bsum[sum_tile0(B, ch) + q];
     for (int o = 32; o > 0; o >>= 1) a0 += __shfl_xor(a0, o, 64);
     __syncthreads();
     const double* x = xs + t * kSumLds;
@@ -237,10 +244,10 @@ __global__ void __launch_bounds__(kSumThreads) k_sum_items(SumBufs B)
     }
     y = __shfl_up(y, 1, 64);
     const uint32_t k0 = t * kSumPer, cnt = k0 < nb ? (nb - k0 < (uint32_t)kSumPer ? nb - k0 : (uint32_t)kSumPer) : 0u;
-    const uint64_t tile = ((uint64_t)ch * B.nblk + b) * kSumTile;
-    SumItem* out = B.items + tile + k0; // every item covers a value
-    double* tadds = B.adds + kSumMaxAdds * tile;
-    double* past = B.past + kSumMaxAdds * (tile + k0); // the adds LDS has no place for, until they are copied below
+    const uint64_t tile = sum_tile0(B, ch) + b;
+    SumItem* out = B.items + tile * kSumTile + k0; // every item covers a value
+    double* tadds = B.adds + tile * kSumTileAdds;
+    double* past = B.past + tile * kSumTileAdds + t * kSumChunkAdds; // the adds LDS has no place for, until they are copied below
     uint32_t k = 0, na = 0;
     {
         auto emit = [&](const SumItem& it) {
@@ -266,10 +273,10 @@ __global__ void __launch_bounds__(kSumThreads) k_sum_items(SumBufs B)
         if (t >= (uint32_t)o) off += z;
     }
     const uint32_t tot = __shfl(off, 63, 64), padded = (tot + 15u) & ~15u; // rows do not straddle tiles
-    if (t == 0) B.nadd[(uint64_t)ch * B.nblk + b] = padded;
+    if (t == 0) B.nadd[tile] = padded;
     if (t < padded - tot) tadds[tot + t] = 0.0; // adding +0.0 changes no partial sum
     off -= na;
-    B.chunk[((uint64_t)ch * B.nblk + b) * kSumThreads + t] = k << 16 | off; // at most 64 items, 320 * 64 adds
+    B.chunk[tile * kSumThreads + t] = k << 16 | off; // at most 64 items, 192 * 64 adds
     for (uint32_t q = 0; q < na && q < (uint32_t)kSumKeep; ++q) tadds[off + q] = kept[q][t];
     for (uint32_t q = kSumKeep; q < na; ++q) tadds[off + q] = past[q]; // the lane's own stores
 }
@@ -330,8 +337,8 @@ __global__ void __launch_bounds__(kSumChain) k_sum_chain(SumBufs B, const double
         return;
     }
     const uint32_t tiles = (n + kSumTile - 1) / kSumTile;
-    uint32_t* nadd = B.nadd + (uint64_t)ch * B.nblk;
-    const uint64_t base = kSumMaxAdds * (uint64_t)ch * B.nblk * kSumTile;
+    uint32_t* nadd = B.nadd + sum_tile0(B, ch);
+    const uint64_t base = sum_tile0(B, ch) * kSumTileAdds;
     double* rows = B.rows + base / 16;
     // the tiles' first adds: thread t takes `per` consecutive tiles
     const uint32_t per = (tiles + kSumChain - 1) / kSumChain;
@@ -362,7 +369,7 @@ __global__ void __launch_bounds__(kSumChain) k_sum_chain(SumBufs B, const double
         for (uint32_t b = wid; b < tiles; b += kWaves) { // the tiles' adds in [r0, r1), a wave a tile
             const uint32_t o = nadd[b], e = b + 1 < tiles ? nadd[b + 1] : tot;
             if (e <= r0 || o >= r1) continue;
-            const double* src = B.adds + base + (uint64_t)kSumMaxAdds * b * kSumTile;
+            const double* src = B.adds + base + (uint64_t)b * kSumTileAdds;
             const uint32_t q0 = o < r0 ? r0 : o, q1 = e < r1 ? e : r1;
 #pragma unroll 4
             for (uint32_t q = q0 + lane; q < q1; q += 64) ladds[q - r0] = src[q - o];
@@ -382,10 +389,10 @@ __global__ void __launch_bounds__(kSumChain) k_sum_chain(SumBufs B, const double
 // the chain's value before chunk c: the row before its first add, and the adds since
 __device__ __forceinline__ double sum_chunk_start(const SumBufs& B, int ch, uint32_t c)
 {
-    const uint32_t b = c / kSumThreads, off = B.chunk[(uint64_t)ch * B.nblk * kSumThreads + c] & 0xffffu, o16 = off & ~15u;
-    const uint64_t base = kSumMaxAdds * (uint64_t)ch * B.nblk * kSumTile;
-    const uint32_t row = (B.nadd[(uint64_t)ch * B.nblk + b] + o16) / 16;
-    const double* adds = B.adds + base + (uint64_t)kSumMaxAdds * b * kSumTile + o16; // a row's worth is there
+    const uint64_t tile0 = sum_tile0(B, ch), base = tile0 * kSumTileAdds;
+    const uint32_t b = c / kSumThreads, off = B.chunk[tile0 * kSumThreads + c] & 0xffffu, o16 = off & ~15u;
+    const uint32_t row = (B.nadd[tile0 + b] + o16) / 16;
+    const double* adds = B.adds + base + (uint64_t)b * kSumTileAdds + o16; // a row's worth is there
     double X[15];
 #pragma unroll
     for (uint32_t q = 0; q < 15; ++q) X[q] = adds[q];
@@ -416,7 +423,7 @@ __global__ void __launch_bounds__(kSumThreads) k_sum_verify(SumBufs B, const dou
         const uint32_t c = blockIdx.x * kSumThreads + threadIdx.x;
         bool ok = true;
         if ((uint64_t)c * kSumPer < n) {
-            const uint64_t chunk = (uint64_t)ch * B.nblk * kSumThreads + c;
+            const uint64_t chunk = sum_tile0(B, ch) * kSumThreads + c;
             const SumItem* it = B.items + chunk * kSumPer;
             const uint32_t k = B.chunk[chunk] >> 16;
             double s = sum_chunk_start(B, ch, c);
@@ -1481,7 +1488,7 @@ struct Head {
     uint32_t* to[4];
     uint32_t ncopy;
     SumBufs sums;
-    uint32_t box, face, fill, copy; // blocks of each kind; the rest: 6 sums.nblk tile sums
+    uint32_t box, face, fill, copy; // blocks of each kind; the rest: the sums' tiles
 };
 
 // both raw boxes, one atomic per block and coordinate after an LDS reduction
@@ -1577,7 +1584,9 @@ __global__ void __launch_bounds__(256) k_head(Head H, Counters* C)
         return;
     }
     b -= H.copy;
-    sum_block(H.sums, b / 6, (int)(b % 6), &red[0][0][0]);
+    const int m = b >= 3 * H.sums.tiles[0];
+    if (m) b -= 3 * H.sums.tiles[0];
+    sum_block(H.sums, b % H.sums.tiles[m], 3 * m + (int)(b / H.sums.tiles[m]), &red[0][0][0]);
 }
 
 // 21-bit Morton codes (128 cells per axis) of raw face-box centres with the

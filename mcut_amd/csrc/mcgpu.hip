@@ -199,7 +199,7 @@ struct mcgpu_context_t {
     Buf pqs, prs, pcounts; // predicate stage: per-test signs, stage counts
     Buf scan_tmp, scan_tmp_c, hist;
     Buf sbsum, sitems, snitem, sadds, srows; // coordinate sums from segments
-    uint32_t sum_nblk = 0;
+    uint32_t sum_tiles[2] = {0, 0};  // of each of a mesh's chains
     bool sum_items = false;          // a mesh's chains are long enough to go through segments
 
     uint64_t cap_pairs = 0, cap_tests = 0, cap_esc = 0, cap_reg = 0, cap_big = 0, cap_trip = 0;
@@ -515,6 +515,9 @@ uint64_t topo_counters(mcgpu_context ctx) { return ctx->topo_hash ? 0 : 2ull * c
 
 uint32_t topo_rank_tiles(uint64_t corners) { return (uint32_t)((corners + kTopoTile - 1) / kTopoTile); }
 
+// tiles of the coordinate sums' six chains
+uint64_t sum_tiles(mcgpu_context ctx) { return 3ull * ((uint64_t)ctx->sum_tiles[0] + ctx->sum_tiles[1]); }
+
 mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
 {
     const uint64_t F = (uint64_t)ctx->nf[0] + ctx->nf[1];
@@ -563,18 +566,19 @@ mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
     (void)p;
     CK(ensure(ctx->scan_tmp, scan_need + 1024, &u));
     if (!ctx->batch) { // coordinate sums from segments (k_sum_items .. k_sum_verify), for the chains computed here
-        const uint64_t nmax = std::max<uint64_t>(ctx->res ? 0 : ctx->nv[0], ctx->nv[1]);
-        const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, (nmax + kSumTile - 1) / kSumTile);
-        ctx->sum_nblk = nblk;
-        ctx->sum_items = nmax > kSumSerial;
+        for (int m = 0; m < 2; ++m) {
+            const uint64_t n = ctx->pairs_given || (ctx->res && m == 0) ? 0 : ctx->nv[m]; // given pairs take no sums
+            ctx->sum_tiles[m] = n > kSumSerial ? (uint32_t)((n + kSumTile - 1) / kSumTile) : 0u;
+        }
+        ctx->sum_items = ctx->sum_tiles[0] || ctx->sum_tiles[1];
         if (ctx->sum_items) {
-            const uint64_t region = 6ull * nblk * kSumTile;
+            const uint64_t tiles = sum_tiles(ctx);
             SumItem* si;
-            CK(ensure(ctx->sbsum, 6ull * nblk, &dp));
-            CK(ensure(ctx->sitems, region, &si));
-            CK(ensure(ctx->snitem, region / kSumPer + 6ull * nblk + 6 * kSumFail, &u));
-            CK(ensure(ctx->sadds, 2 * kSumMaxAdds * region, &dp));
-            CK(ensure(ctx->srows, kSumMaxAdds * region / 16, &dp));
+            CK(ensure(ctx->sbsum, tiles, &dp));
+            CK(ensure(ctx->sitems, tiles * kSumTile, &si));
+            CK(ensure(ctx->snitem, tiles * kSumThreads + tiles + 6 * kSumFail, &u));
+            CK(ensure(ctx->sadds, 2 * tiles * kSumTileAdds, &dp));
+            CK(ensure(ctx->srows, tiles * kSumTileAdds / 16, &dp));
         }
     }
     if (ctx->cc_check) CK(ensure(ctx->cc_parent, (uint64_t)ctx->nv[0] + ctx->nv[1] + 8, &u));
@@ -671,15 +675,15 @@ SumBufs sum_bufs(mcgpu_context ctx)
     B.v[1] = ctx->dv[1];
     B.n[0] = ctx->nv[0];
     B.n[1] = ctx->nv[1];
-    B.nblk = ctx->sum_nblk;
+    for (int m = 0; m < 2; ++m) B.tiles[m] = ctx->sum_tiles[m];
     B.bsum = P_<double>(ctx->sbsum);
     B.items = P_<SumItem>(ctx->sitems);
-    const uint64_t region = 6ull * ctx->sum_nblk * kSumTile;
+    const uint64_t tiles = sum_tiles(ctx);
     B.chunk = P_<uint32_t>(ctx->snitem);
-    B.nadd = B.chunk + region / kSumPer;
-    B.fail = B.nadd + 6ull * ctx->sum_nblk;
+    B.nadd = B.chunk + tiles * kSumThreads;
+    B.fail = B.nadd + tiles;
     B.adds = P_<double>(ctx->sadds);
-    B.past = B.adds + kSumMaxAdds * region;
+    B.past = B.adds + tiles * kSumTileAdds;
     B.rows = P_<double>(ctx->srows);
     return B;
 }
@@ -896,7 +900,7 @@ void enqueue_validate(mcgpu_context ctx)
     H.face = (uint32_t)grid_for(nf, kBlock, 1024);
     H.fill = (uint32_t)grid_for(H.nzero, 8 * kBlock, 128);
     H.copy = H.ncopy ? (uint32_t)grid_for(H.ncopy, 4 * kBlock, 128) : 0;
-    const uint32_t tiles = ctx->sum_items && !ctx->pairs_given ? 6 * H.sums.nblk : 0;
+    const uint32_t tiles = (uint32_t)sum_tiles(ctx);
     k_head<<<H.box + H.face + H.fill + H.copy + tiles, kBlock, 0, s>>>(H, C);
     if (ctx->pairs_given || ctx->shifted_bp) // k_morton_raw finds it otherwise
         k_tolerance<<<1, 1, 0, s>>>(&P_<DevState>(ctx->state)->P, C, tol_args(ctx));
@@ -1518,7 +1522,7 @@ void enqueue_frontend(mcgpu_context ctx)
         // reserved CUs, the values one by one only where a check failed
         stage_event(ctx, EV_S0, s);
         const SumBufs SB = sum_bufs(ctx);
-        const dim3 grid(SB.nblk, 6);
+        const dim3 grid(std::max(SB.tiles[0], SB.tiles[1]), 6);
         const ShiftArgs SA{ctx->nv[0], ctx->nv[1], ctx->gp_constant, absolute ? 1 : 0};
         if (ctx->sum_items) k_sum_items<<<grid, kSumThreads, 0, s>>>(SB);
         ev_record(ctx, EV_SUM_ITEMS, s);
@@ -1858,7 +1862,7 @@ std::vector<uint64_t> graph_key(mcgpu_context ctx)
         ptr(ctx->dv[m]), ptr(ctx->didx[m]), ptr(ctx->dsz[m]), ptr(ctx->bin_idx[m]);
     }
     put(ctx->cap_pairs), put(ctx->cap_tests), put(ctx->cap_esc), put(ctx->cap_reg), put(ctx->cap_big),
-        put(ctx->cap_trip), put(ctx->sum_nblk);
+        put(ctx->cap_trip), put(ctx->sum_tiles[0]), put(ctx->sum_tiles[1]);
     uint64_t gp;
     std::memcpy(&gp, &ctx->gp_constant, 8);
     put(ctx->flags), put(gp), put(ctx->enforcement_count), put(ctx->keep_tests);

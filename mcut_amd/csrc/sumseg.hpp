@@ -185,6 +185,10 @@ __host__ __device__ inline bool sum_apply(const SumItem& it, double s, double* e
 // on its side: d + tie G / 2 is rounded to one by adding and taking away 1.5 2^53 G
 // (e < kSumExpLo holds the predicted start alone: d = 0).
 constexpr int kSumMaxAdds = 5;
+// Adds of a chunk of 64 values, at most: a segment ends before a step or with
+// the chunk, and every item covers a value, so there are up to 32 segments and
+// 32 steps.
+constexpr int kSumChunk = 64, kSumChunkAdds = kSumChunk / 2 * (kSumMaxAdds + 1);
 __host__ __device__ inline int sum_add_list(const SumItem& it, double* a)
 {
     if (sum_is_step(it)) {
