@@ -259,12 +259,13 @@ __device__ __forceinline__ int orient3d_staged(const double* pa, const double* p
 
 // --- exact orient3d sign: expansions of the coordinate differences ----------
 
-__device__ inline int grow_zeroelim(int n, const double* e, double b, double* h)
+// h + b, in place: component i is read before any place up to i is written
+__device__ inline int grow_zeroelim(int n, double* h, double b)
 {
     double q = b, qn, hh;
     int hi = 0;
     for (int i = 0; i < n; ++i) {
-        two_sum(q, e[i], qn, hh);
+        two_sum(q, h[i], qn, hh);
         q = qn;
         if (hh != 0.0) h[hi++] = hh;
     }
@@ -289,14 +290,10 @@ __device__ inline int scale_zeroelim(int n, const double* e, double b, double* h
     return hi;
 }
 
-// h = e + f (in place into h; tmp is scratch of the same capacity)
-__device__ inline int add_into(int n, double* h, int m, const double* f, double* tmp)
+// h + f, in place
+__device__ inline int add_into(int n, double* h, int m, const double* f)
 {
-    for (int i = 0; i < m; ++i) {
-        int l = grow_zeroelim(n, h, f[i], tmp);
-        for (int k = 0; k < l; ++k) h[k] = tmp[k];
-        n = l;
-    }
+    for (int i = 0; i < m; ++i) n = grow_zeroelim(n, h, f[i]);
     return n;
 }
 
@@ -324,36 +321,37 @@ __device__ inline int orient3d_exact_sign(const double* pa, const double* pb, co
         ny[i] = diff_expansion(P[i][1], pd[1], Y[i]);
         nz[i] = diff_expansion(P[i][2], pd[2], Z[i]);
     }
-    double acc[200], tmp[200], prod[16], t1[8], t2[8], part[8], m[64];
+    // Private memory: a queue keeps it for every wave the device holds, 1.0 GB
+    // for these 1.9 KB a lane (2.4 GB with a second accumulator and the terms of
+    // one coordinate summed apart).  Components, at most: 4 of a difference times
+    // a component of another, 8 of the two differences' product, 16 of a minor,
+    // 32 of that times a component of the third difference, 192 of the six of
+    // those.
+    double acc[192], prod[16], t2[8], part[4], sc[32];
     int alen = 1;
     acc[0] = 0.0;
     for (int i = 0; i < 3; ++i) {
         int j = (i + 1) % 3, k = (i + 2) % 3;
-        // t1 = X_j * Y_k
-        int l1 = 1;
-        t1[0] = 0.0;
+        // prod = X_j * Y_k
+        int lm = 1;
+        prod[0] = 0.0;
         for (int q = 0; q < ny[k]; ++q) {
             int pl = scale_zeroelim(nx[j], X[j], Y[k][q], part);
-            l1 = add_into(l1, t1, pl, part, tmp);
+            lm = add_into(lm, prod, pl, part);
         }
         // t2 = -(X_k * Y_j)
         int l2 = 1;
         t2[0] = 0.0;
         for (int q = 0; q < ny[j]; ++q) {
             int pl = scale_zeroelim(nx[k], X[k], -Y[j][q], part);
-            l2 = add_into(l2, t2, pl, part, tmp);
+            l2 = add_into(l2, t2, pl, part);
         }
-        for (int q = 0; q < l1; ++q) prod[q] = t1[q];
-        int lm = add_into(l1, prod, l2, t2, tmp);
-        // m = prod * Z_i
-        int ml = 1;
-        m[0] = 0.0;
+        lm = add_into(lm, prod, l2, t2);
+        // acc += prod * Z_i
         for (int q = 0; q < nz[i]; ++q) {
-            double sc[40];
             int pl = scale_zeroelim(lm, prod, Z[i][q], sc);
-            ml = add_into(ml, m, pl, sc, tmp);
+            alen = add_into(alen, acc, pl, sc);
         }
-        alen = add_into(alen, acc, ml, m, tmp);
     }
     double top = acc[alen - 1];
     return top > 0.0 ? 1 : (top < 0.0 ? -1 : 0);

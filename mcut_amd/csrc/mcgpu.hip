@@ -157,6 +157,7 @@ struct mcgpu_context_t {
     hipStream_t s = nullptr, s2 = nullptr, s3 = nullptr, ssum = nullptr; // s: stream A of the call in progress, one of
     hipStream_t s_plain = nullptr, s_queue = nullptr;                    // these two (StreamA; a serving slot has neither)
     bool on_queue = false;           // the last dispatch's stream A was s_queue
+    std::atomic<int>* queues = nullptr; // counts it among the device's contexts with an s_queue
     hipStream_t s2b = nullptr, s3b = nullptr; // B and C of batched dispatches, made by the first one
     hipEvent_t ev[EV_COUNT];
     hipError_t last_error = hipSuccess;
@@ -2086,7 +2087,17 @@ static hipError_t create_split_streams(int ncu, double share, hipStream_t* b, hi
 // the latter 2,510 and 3,880.
 //
 // s_plain does not synchronise with the null stream, as masked streams do.
+//
+// A queue keeps the private memory of the kernels it has run, for as many waves
+// as the device holds: 1.0 GB once it has run k_narrow_exact.  The runtime has
+// only so much of it for a process: with a queue for every context, at 2.4 GB
+// each, a dispatch of 16 contexts ended as out of resources with 260 GB free.
+// The plain streams of all contexts share four queues, so the first kOwnQueues
+// contexts alive on a device have an s_queue, and the others' stream A is
+// s_plain.  Dispatches a second of 12 contexts, 72,000 triangles a mesh: 2,620
+// (3,600 with a queue each, 400 with four).
 constexpr unsigned kMaxDevices = 64;
+constexpr int kOwnQueues = 8;
 
 // The runtime makes the queues that plain streams share one by one, up to four
 // (GPU_MAX_HW_QUEUES), as plain streams are made.  All of them exist before the
@@ -2108,6 +2119,8 @@ static void fill_plain_queues()
 static hipError_t create_streams(mcgpu_context ctx, int ncu)
 {
     static std::atomic<unsigned> made[kMaxDevices]; // contexts of each device: where the next one starts
+    static std::atomic<int> queues[kMaxDevices];    // those alive with an s_queue
+    const unsigned d = (unsigned)ctx->device % kMaxDevices;
     ctx->ncu = ncu;
     // the first kSumCUs compute units for the serial sums, the rest for the
     // streams that run beside them
@@ -2118,10 +2131,13 @@ static hipError_t create_streams(mcgpu_context ctx, int ncu)
     hipStream_t* const st[4] = {&ctx->s_queue, &ctx->ssum, &ctx->s2, &ctx->s3};
     const std::vector<uint32_t>* const mask[4] = {&every, &sums, &mb, &mc};
     hipError_t e = hipStreamCreateWithFlags(&ctx->s_plain, hipStreamNonBlocking);
-    const unsigned first = made[(unsigned)ctx->device % kMaxDevices]++;
+    const unsigned first = made[d]++;
+    if (++queues[d] <= kOwnQueues) ctx->queues = &queues[d];
+    else --queues[d];
     if (first == 0) fill_plain_queues();
     for (unsigned q = 0; q < 4 && e == hipSuccess; ++q) {
         const unsigned i = (first + q) % 4;
+        if (i == 0 && !ctx->queues) continue;
         e = hipExtStreamCreateWithCUMask(st[i], (uint32_t)mask[i]->size(), mask[i]->data());
     }
     ctx->s = ctx->s_plain;
@@ -2134,6 +2150,7 @@ static void destroy_streams(mcgpu_context ctx)
         (void)hipStreamDestroy(ctx->s);
         return;
     }
+    if (ctx->queues) --*ctx->queues;
     if (ctx->s2b == ctx->s2) ctx->s2b = ctx->s3b = nullptr;
     for (hipStream_t st : {ctx->ssum, ctx->s3, ctx->s2, ctx->s3b, ctx->s2b, ctx->s_plain, ctx->s_queue})
         if (st) (void)hipStreamDestroy(st);
@@ -2150,8 +2167,8 @@ struct StreamA {
     bool done = false; // the host has waited for it
     StreamA(mcgpu_context c, bool queue) : ctx(c)
     {
-        if (ctx->s_plain) ctx->s = queue ? ctx->s_queue : ctx->s_plain;
-        ctx->on_queue = queue;
+        ctx->on_queue = queue && ctx->s_queue;
+        if (ctx->on_queue) ctx->s = ctx->s_queue;
     }
     StreamA(const StreamA&) = delete;
     ~StreamA()

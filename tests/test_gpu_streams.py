@@ -1,6 +1,7 @@
 """Streams of a context beside others' work: calls that run on stream A alone
-return while a caller's work on the null stream still runs, and two contexts
-in two threads dispatch more pairs a second than one."""
+return while a caller's work on the null stream still runs, two contexts
+in two threads dispatch more pairs a second than one, and the private memory
+of queues does not grow with every context."""
 import ctypes as C
 import threading
 import time
@@ -119,3 +120,33 @@ def test_two_contexts_overlap(hip, n):
             c.close()
         for p in keep:
             hip.hipFree(p)
+
+
+def test_private_memory_of_many_contexts(hip):
+    """A queue that has run the exact predicates keeps 1 GB: only so many
+    contexts have one of their own, the others share four."""
+    from mcut_amd import frontend
+    src, cut = spheres(40)
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    cs, held, want = [], [], None
+    try:
+        for _ in range(16):
+            at = free()
+            cs.append(frontend.Context(0))
+            R = cs[-1].dispatch(src, cut)
+            got = R.status, R.counts, *R.registry()
+            held.append((at - free()) / 1e9)
+            want = want or got
+            assert got[:2] == want[:2]
+            for x, y in zip(got[2:], want[2:]):
+                assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+        print("GB a context:", " ".join("%.2f" % h for h in held), flush=True)
+        assert held[-1] < 0.5
+    finally:
+        for c in cs:
+            c.close()
