@@ -3859,9 +3859,9 @@ __global__ void k_batch_globalize(BatchFaces M0, BatchFaces M1, const uint32_t* 
     }
 }
 
-// raw box of every (pair, mesh) segment: one block each, order keys out
-// raw boxes, a tile of a mesh's vertices a block (a block a mesh took 0.20 ms of a
-// batch whose largest mesh has 100k vertices)
+// raw box of every (pair, mesh) segment as order keys: a tile of a mesh's vertices
+// a block, or several (batch_box_rows; a block a mesh took 0.20 ms of a batch
+// whose largest mesh has 100k vertices)
 constexpr uint32_t kBatchBoxTile = 4096;
 __global__ void __launch_bounds__(256) k_batch_bbox(const double* __restrict__ vs, const double* __restrict__ vc,
                                                     const BatchPair* __restrict__ bp, unsigned long long (*rbox)[2][6])
@@ -3870,17 +3870,20 @@ __global__ void __launch_bounds__(256) k_batch_bbox(const double* __restrict__ v
     const uint32_t p = blockIdx.x >> 1, m = blockIdx.x & 1;
     const BatchPair b = bp[p];
     const double* v = m ? vc + 3ull * b.vc0 : vs + 3ull * b.vs0;
-    const uint32_t n = m ? b.nvc : b.nvs, i0 = blockIdx.y * kBatchBoxTile;
+    const uint32_t n = m ? b.nvc : b.nvs;
+    uint64_t i0 = (uint64_t)blockIdx.y * kBatchBoxTile;
     if (i0 >= n && i0) return; // whole block
-    const uint32_t i1 = n - i0 < kBatchBoxTile ? n : i0 + kBatchBoxTile;
     double lo[3] = {1.7976931348623157e308, 1.7976931348623157e308, 1.7976931348623157e308};
     double hi[3] = {-1.7976931348623157e308, -1.7976931348623157e308, -1.7976931348623157e308};
-    for (uint32_t i = i0 + threadIdx.x; i < i1; i += blockDim.x)
-        for (int j = 0; j < 3; ++j) {
-            const double x = v[3ull * i + j];
-            lo[j] = x < lo[j] ? x : lo[j];
-            hi[j] = x > hi[j] ? x : hi[j];
-        }
+    for (; i0 < n; i0 += (uint64_t)gridDim.y * kBatchBoxTile) {
+        const uint64_t i1 = n - i0 < kBatchBoxTile ? n : i0 + kBatchBoxTile;
+        for (uint64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x)
+            for (int j = 0; j < 3; ++j) {
+                const double x = v[3ull * i + j];
+                lo[j] = x < lo[j] ? x : lo[j];
+                hi[j] = x > hi[j] ? x : hi[j];
+            }
+    }
     for (int o = 32; o > 0; o >>= 1)
         for (int j = 0; j < 3; ++j) {
             const double a = __shfl_xor(lo[j], o, 64), c = __shfl_xor(hi[j], o, 64);

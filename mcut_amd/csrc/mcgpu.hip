@@ -957,7 +957,7 @@ void enqueue_validate_batch(mcgpu_context ctx)
         BF[m] = BatchFaces{ctx->bin_idx[m], off, ctx->dsz[m], ctx->nf[m], P_<uint32_t>(ctx->bidx[m])};
     }
     k_batch_globalize<<<grid_for((uint64_t)ctx->nf[0] + ctx->nf[1]), kBlock, 0, s>>>(BF[0], BF[1], fp, bp, C);
-    k_batch_bbox<<<dim3(2 * np, batch_box_tiles(ctx)), 256, 0, s>>>(ctx->dv[0], ctx->dv[1], bp, brbox);
+    k_batch_bbox<<<dim3(2 * np, batch_box_rows(np, batch_box_tiles(ctx))), 256, 0, s>>>(ctx->dv[0], ctx->dv[1], bp, brbox);
     const bool absolute = (ctx->flags & MCGPU_DISPATCH_ENFORCE_GENERAL_POSITION_ABSOLUTE) != 0;
     k_batch_tolerance<<<grid_for(np), kBlock, 0, s>>>(Pb, brbox, bp, np, ctx->gp_constant, absolute ? 1 : 0, C);
     k_batch_layout<<<1, 1024, 0, s>>>(Pb, brbox, np);

@@ -1,7 +1,8 @@
 // Host check of mcut_amd/csrc/pairgrid.hpp: the launches of k_pairs_start stay
 // within the device's grid (2^31 - 1 blocks and 2^32 - 1 threads in x; all the
 // blocks are in x, as y holds 65,535) for every pair of counts whose product its launchers allow, and
-// its blocks cover every pair of items once.
+// its blocks cover every pair of items once; and those of k_batch_bbox do not
+// grow with the product of the pairs and the largest mesh.
 #include <cstdio>
 #include <vector>
 
@@ -36,6 +37,15 @@ int main()
                     for (uint32_t c = c0; c < c0 + kPairTileCut && c < nc; ++c) ++seen[(size_t)s * nc + c];
             }
             for (int n : seen) bad += n != 1;
+        }
+    // raw boxes of a batch: every mesh has a block, few are empty, y holds them
+    for (uint32_t np : {1u, 2u, 96u, 320u, 4096u, 40000u, 1u << 20})
+        for (uint32_t tiles : {1u, 2u, 25u, 245u, 2442u, 60000u, 300000u}) {
+            const uint64_t rows = batch_box_rows(np, tiles), blocks = 2ull * np * rows;
+            if (rows < 1 || rows > tiles || rows > 65535u || blocks > (2ull * np > (1u << 16) ? 2ull * np : 1u << 16)) {
+                if (bad < 8) printf("%u pairs, %u tiles: %llu blocks\n", np, tiles, (unsigned long long)blocks);
+                ++bad;
+            }
         }
     printf("bad %d\n", bad);
     return bad != 0;

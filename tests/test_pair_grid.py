@@ -1,11 +1,12 @@
 """The grid of the broad phase's first launch (k_pairs_start) for a mesh of few
-faces against one of millions, whichever of them is the source.
+faces against one of millions, whichever of them is the source, and of a batch's
+raw boxes (k_batch_bbox) for one large mesh among thousands of small ones.
 
 CPU: the launch sizes (mcut_amd/csrc/pairgrid.hpp, compiled for the host)
 against the device's limits, and the blocks' cover of the pairs.
 
 GPU: a box of 12 faces against a sheet of 2.2 M, in both orders, against the
-walk of the trees."""
+walk of the trees; and such a batch, whose large pair must equal the pair alone."""
 import os
 import subprocess
 
@@ -48,5 +49,28 @@ def test_few_faces_against_millions(box_first):
         assert (W.status, W.counts) == got[:2]
         for x, y in zip(got[2:], W.registry()):
             assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+    finally:
+        c.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("at", [0, 2300, 4199])
+def test_one_large_mesh_among_thousands(at):
+    from mcut_amd import frontend
+    # 66,049 vertices: 17 tiles of 4,096, a block takes three
+    V, F, _ = mg.grid_patch(256, 3.0)
+    sheet = (V + [0.0113, 0.0071, 0.0137], np.asarray(F).ravel(), None)
+    B, Fb, _ = mg.tessellated_box((0.0, 0.0, 0.0), 1.0, 3, rotation=mg.random_rotation(5))
+    G, Fg, _ = mg.grid_patch(2, 3.0)
+    small = (B, Fb, None), (G + [0.0113, 0.0071, 0.0137], np.asarray(Fg).ravel(), None)
+    large = (B, Fb, None), sheet
+    c = frontend.Context(0)
+    try:
+        want = [[np.array(x) for x in c.dispatch(*p).registry()] for p in (small, large)]
+        assert len(want[1][0]) > 0
+        R = c.dispatch_batch([large if i == at else small for i in range(4200)])
+        for i in (0, at, at - 1 if at else 1, 4199):
+            for x, y in zip(R.pair_registry(i), want[i == at]):
+                assert np.array_equal(np.ascontiguousarray(x).view(np.uint8), y.view(np.uint8)), i
     finally:
         c.close()
