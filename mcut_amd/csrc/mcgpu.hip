@@ -547,7 +547,7 @@ mcgpu_result alloc_mesh_buffers(mcgpu_context ctx)
         const uint64_t nk = ctx->ncorner[m], nf = ctx->nf[m];
         CK(ensure(ctx->off[m], nf + 1, &u));
         CK(ensure(ctx->cface[m], nk, &u));
-        CK(ensure(ctx->cedge[m], nk, &u));
+        CK(ensure(ctx->cedge[m], nk + 2, &u)); // k_batch_edge_bases reads a last face's second corner, also of an empty one
         int D = 0;
         while ((1ull << D) < nf) ++D;
         ctx->depth[m] = D;
