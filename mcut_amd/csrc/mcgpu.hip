@@ -37,7 +37,7 @@ struct Buf {
 // polygon-soup edges.  B and C are masked off the reserved CUs: a serial FP64
 // chain that shares its CU with memory- or atomic-heavy waves runs 4-8 times
 // slower.  B and C also get disjoint CU sets: sharing all of them, the tree
-// build's small launches queue behind the edge numbering's large hash grids
+// build's small launches queue behind the edge numbering's large grids
 // and the sort stretches from 0.12 to 0.25 ms.  B takes kBroadShare of the
 // CUs left after the sums (174 of 248 on the 256-CU part): it is the longest
 // of the three paths up to a subdivision-7 icosphere pair (0.464 ms with 0.70,
@@ -1683,12 +1683,12 @@ mcgpu_result finish(mcgpu_context ctx, mcgpu_frontend_info* info, Again* again)
         fprintf(stderr,
                 "[mcgpu] raw=%llu pairs=%llu tests=%llu esc=%llu reg=%llu big=%llu cand=%llu edges=%llu+%llu ov=%u/%u/%u/%u/%u "
                 "gp=%u bad=%u/%u unsup=%u nonman=%u badin=%u pairfail=%u partial=%u caps=%llu/%llu/%llu/%llu "
-                "trav splits=%llu lane_walks=%llu\n",
+                "trav splits=%llu lane_walks=%llu ov_nodes=%u ov_topo=%u walk=%d hash=%d shifted=%d\n",
                 C.n_raw, C.n_pairs, C.n_tests, C.n_esc, C.n_reg, C.n_big, C.n_cand, C.n_edges_src, C.n_edges_cut, C.ov_pairs,
                 C.ov_tests, C.ov_esc, C.ov_reg, C.ov_big, C.gp, C.bad_src, C.bad_cut, C.unsupported, C.nonmanifold,
                 C.bad_input, C.pair_fail, C.partial, (unsigned long long)ctx->cap_pairs,
                 (unsigned long long)ctx->cap_tests, (unsigned long long)ctx->cap_esc, (unsigned long long)ctx->cap_reg,
-                C.n_fallback, C.n_lane_walks);
+                C.n_fallback, C.n_lane_walks, C.ov_nodes, C.ov_topo, ctx->walk, ctx->topo_hash, ctx->shifted_bp);
     if (C.bad_input || C.nonmanifold) return MCGPU_ERROR_INVALID_VALUE;
     if (ctx->cc_check) { // check_input_mesh: one component per mesh (per pair of a batch)
         // rounds until no edge crosses two components (each round removes a root)

@@ -23,11 +23,13 @@
 // later tie resolves as predicted.  So the first tie alone counts: an odd d
 // ends at b + d + tie G, tie being the side the prediction rounded away from.
 // A climb, a sum on a power of two that neither rule covers, and sums outside
-// [2^-900, 2^1000] stay single steps.  The items of a stretch are again a sequence of such
-// steps, so the same walk composes them: two levels leave a few dozen items a
-// chain, which one wave adds with the checks made on the real start.  An item
-// whose check fails is replayed value by value, so a bad prediction costs time
-// and never a bit.
+// [2^-900, 2^1000] stay single steps.  The kernels add the items of all chunks
+// (7k for 164k values of a sphere) as one chain and check each on the start that
+// it then has; from the first chunk with an item that does not move with its
+// start the values are added one by one, so a bad prediction costs time and
+// never a bit.  The items of a stretch are again a sequence of such steps, which
+// the same walk could compose (sum_compose): on the device that cost what the
+// shorter chain saved, so only a host test does it.
 //
 // Usable on the host, where a test holds it to the sequential sum.
 #pragma once
@@ -209,7 +211,7 @@ __host__ __device__ inline int sum_add_list(const SumItem& it, double* a)
     return 5;
 }
 
-// one item of the level below
+// one item of the level below (no kernel composes items)
 template <class Emit>
 __host__ __device__ inline void sum_compose(SumWalk& W, const SumItem& it, Emit emit)
 {
