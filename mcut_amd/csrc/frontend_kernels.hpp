@@ -408,8 +408,26 @@ __device__ __forceinline__ double sum_chunk_start(const SumBufs& B, int ch, uint
 // it, a sum added again) does so by device-scope atomics, each waited for
 // before the next, so no cache has to be written back; a kernel of its own for
 // the rest and the shift cost its launch and 8-14 us of the sums' path.
+// apart: k_sum_rest does both, for meshes of more than kSumApart vertices, whose
+// values one by one take milliseconds, and longer beside the other streams'
+// blocks (4.4 ns a value on 3.1 M, 2.44 on the reserved CUs).
+constexpr uint32_t kSumApart = 1u << 21;
+__device__ __forceinline__ double sum_rest(const SumBufs& B, const double* __restrict__ zero, int ch, uint32_t from)
+{
+    __builtin_amdgcn_s_setprio(3);
+    const uint32_t i0 = from * kSumPer;
+    const double start = sum_chunk_start(B, ch, from);
+    return serial_chain<3, false>(B.v[ch / 3] + ch % 3 + 3ull * i0, B.n[ch / 3] - i0, zero, start, nullptr);
+}
+__global__ void __launch_bounds__(64) k_sum_rest(SumBufs B, const double* __restrict__ zero, Params* P, Counters* C, ShiftArgs A)
+{
+    const int ch = blockIdx.x;
+    const uint32_t from = __builtin_amdgcn_readfirstlane(sum_chain_items(B, ch) ? B.fail[kSumFail * ch] : 0xffffffffu);
+    const double acc = from != 0xffffffffu ? sum_rest(B, zero, ch, from) : 0.0;
+    sum_done(acc, from != 0xffffffffu, ch / 3, ch % 3, P, C, A);
+}
 __global__ void __launch_bounds__(kSumThreads) k_sum_verify(SumBufs B, const double* __restrict__ zero, Params* P, Counters* C,
-                                                            ShiftArgs A)
+                                                            ShiftArgs A, int apart)
 {
     static_assert(kSumThreads == 64, "one wave a block");
     const int ch = blockIdx.y, m = ch / 3, j = ch % 3;
@@ -448,18 +466,14 @@ __global__ void __launch_bounds__(kSumThreads) k_sum_verify(SumBufs B, const dou
                 const uint32_t old = atomicMin(fail, blockIdx.x * kSumThreads + (uint32_t)__builtin_ctzll(bad));
                 asm volatile("" : : "v"(old) : "memory"); // its result is here: it is done
             }
-            last = atomicAdd(fail + 1, 1u) + 1 == blocks;
+            last = !apart && atomicAdd(fail + 1, 1u) + 1 == blocks;
             if (last) from = atomicAdd(fail, 0u);
         }
         if (!__builtin_amdgcn_readfirstlane(last)) return;
         from = __builtin_amdgcn_readfirstlane(from);
-        if (from != 0xffffffffu) {
-            __builtin_amdgcn_s_setprio(3);
-            const uint32_t i0 = from * kSumPer;
-            const double start = sum_chunk_start(B, ch, from);
-            acc = serial_chain<3, false>(B.v[m] + j + 3ull * i0, n - i0, zero, start, nullptr);
-        }
+        if (from != 0xffffffffu) acc = sum_rest(B, zero, ch, from);
     }
+    if (apart) return;
     sum_done(acc, from != 0xffffffffu, m, j, P, C, A);
 }
 
@@ -862,7 +876,7 @@ constexpr uint32_t kNoCorner = 0xffffffffu;
 constexpr int kTopoCapLog = 12;                    // words a bucket holds
 constexpr uint32_t kTopoCap = 1u << kTopoCapLog;
 constexpr uint32_t kTopoFill = kTopoCap / 2;       // mean words of a bucket, at most: 4096 lies 6 sigma above
-constexpr int kTopoMaxBits = 12;                   // buckets a segment may have: 16 KB of counters a scatter block
+constexpr int kTopoMaxBits = 13;                   // buckets a segment may have: 32 KB of counters a scatter block
 constexpr int kTopoBlock = 512;
 constexpr int kTopoScatterBlock = 256, kTopoItems = 16; // corners of a scatter tile
 constexpr uint32_t kTopoTile = 4096;               // ranks per counting tile

@@ -76,7 +76,7 @@ const char* kStageNames[ST_COUNT] = {"coordinate_sums", "shift_params", "shift_b
 
 // event slots: stage boundaries on the three streams
 enum Ev { EV_A0, EV_S0, EV_A_SUMS, EV_A_PARAMS, EV_A_SHIFT, EV_A_BOXES, EV_A_JOIN, EV_A_FILTER, EV_A_PLANES, EV_A_JOIN2, EV_A_TESTS, EV_A_NARROW,
-          EV_A_END, EV_FORK, EV_B0, EV_B_SORT, EV_B_REFIT, EV_B_TRAV, EV_C0, EV_C_WORDS, EV_C_TOPO, EV_SUM_ITEMS, EV_SUM_CHAIN,
+          EV_A_END, EV_FORK, EV_B0, EV_B_SORT, EV_B_REFIT, EV_B_TRAV, EV_C0, EV_C_WORDS, EV_C_TOPO, EV_SUM_ITEMS, EV_SUM_CHAIN, EV_SUM_CHECK, EV_SUM_REST,
           EV_TRAV_K0, EV_TRAV_K1, EV_B_CC, EV_COUNT };
 
 // Launch shape of the traversal kernel, chosen per workload class by the
@@ -457,10 +457,10 @@ bool topo_plan(mcgpu_context ctx)
     }
     uint32_t kmax = 0;
     for (uint32_t i = 0; i < ctx->nseg; ++i) kmax = std::max(kmax, seg[i].k);
-    // counters of a scatter block: 1, 4 or 16 KB of LDS.  Meshes of at most 256
+    // counters of a scatter block: 1, 4, 16 or 32 KB of LDS.  Meshes of at most 256
     // buckets keep to the hash: their words stay in the caches, and counting the
     // ranges first would cost what they save.
-    ctx->topo_bits = kmax <= (kTopoFill << 8) ? 8 : kmax <= (kTopoFill << 10) ? 10 : kTopoMaxBits;
+    ctx->topo_bits = kmax <= (kTopoFill << 8) ? 8 : kmax <= (kTopoFill << 10) ? 10 : kmax <= (kTopoFill << 12) ? 12 : kTopoMaxBits;
     constexpr uint32_t tile = kTopoScatterBlock * kTopoItems;
     uint64_t words = 0, buckets = 0, tiles = 0;
     ctx->topo_ranges = true;
@@ -1374,6 +1374,16 @@ Topo topo_view(mcgpu_context ctx)
 
 void enqueue_topology_hash(mcgpu_context ctx, hipStream_t s3);
 
+// words into buckets of vertex ranges, and of hashes for the segments that have
+// no ranges or one that holds too many
+template <int BITS>
+void scatter_words(const Topo& T, dim3 g, dim3 gh, dim3 b, Counters* C, hipStream_t st)
+{
+    k_topo_ranges<BITS><<<g, b, 0, st>>>(T);
+    k_topo_scatter<false, BITS><<<g, b, 0, st>>>(T, g.x, C);
+    k_topo_scatter<true, BITS><<<gh, b, 0, st>>>(T, g.x, C);
+}
+
 // Polygon-soup edge numbering in two parts, the corners' words into their
 // buckets and the edges from those: both on stream C for one pair, the second
 // on stream A for a batch (on one pair stream A's part gained nothing:
@@ -1396,17 +1406,10 @@ void enqueue_topology_words(mcgpu_context ctx, hipStream_t s3)
         const dim3 g(n), b(kTopoScatterBlock);
         // a few blocks look whether a segment is hashed: most dispatches have none
         const dim3 gh(ctx->topo_ranges ? std::min<uint32_t>(n, 2 * ctx->ncu) : n);
-        if (ctx->topo_bits == 8) {
-            k_topo_scatter<true, 8><<<gh, b, 0, s3>>>(T, n, C);
-        } else if (ctx->topo_bits == 10) {
-            k_topo_ranges<10><<<g, b, 0, s3>>>(T);
-            k_topo_scatter<false, 10><<<g, b, 0, s3>>>(T, n, C);
-            k_topo_scatter<true, 10><<<gh, b, 0, s3>>>(T, n, C);
-        } else {
-            k_topo_ranges<kTopoMaxBits><<<g, b, 0, s3>>>(T);
-            k_topo_scatter<false, kTopoMaxBits><<<g, b, 0, s3>>>(T, n, C);
-            k_topo_scatter<true, kTopoMaxBits><<<gh, b, 0, s3>>>(T, n, C);
-        }
+        if (ctx->topo_bits == 8) k_topo_scatter<true, 8><<<gh, b, 0, s3>>>(T, n, C);
+        else if (ctx->topo_bits == 10) scatter_words<10>(T, g, gh, b, C, s3);
+        else if (ctx->topo_bits == 12) scatter_words<12>(T, g, gh, b, C, s3);
+        else scatter_words<kTopoMaxBits>(T, g, gh, b, C, s3);
     }
     if (ctx->batch) ev_record(ctx, EV_C_WORDS, s3);
 }
@@ -1531,7 +1534,15 @@ void enqueue_frontend(mcgpu_context ctx)
         k_sum_chain<<<6, kSumChain, 0, ssum>>>(SB, &C->zero, Pd, C, SA, ctx->sum_items ? 0 : 1);
         ev_record(ctx, EV_SUM_CHAIN, ssum);
         ev_wait(ctx, s, EV_SUM_CHAIN);
-        if (ctx->sum_items) k_sum_verify<<<grid, kSumThreads, 0, s>>>(SB, &C->zero, Pd, C, SA);
+        const int apart = (uint64_t)std::max(SB.tiles[0], SB.tiles[1]) * kSumTile > kSumApart;
+        if (ctx->sum_items) k_sum_verify<<<grid, kSumThreads, 0, s>>>(SB, &C->zero, Pd, C, SA, apart);
+        if (apart) {
+            ev_record(ctx, EV_SUM_CHECK, s);
+            ev_wait(ctx, ssum, EV_SUM_CHECK);
+            k_sum_rest<<<6, 64, 0, ssum>>>(SB, &C->zero, Pd, C, SA);
+            ev_record(ctx, EV_SUM_REST, ssum);
+            ev_wait(ctx, s, EV_SUM_REST);
+        }
         ev_record(ctx, EV_A_SUMS, s);
     }
     if (ctx->batch) {
