@@ -2179,7 +2179,10 @@ struct StreamA {
     StreamA(mcgpu_context c, bool queue) : ctx(c)
     {
         ctx->on_queue = queue && ctx->s_queue;
-        if (ctx->on_queue) ctx->s = ctx->s_queue;
+        if (!ctx->on_queue) return;
+        // a call that failed may have left work on s_plain that uses the same buffers
+        if (hipStreamQuery(ctx->s_plain) != hipSuccess) (void)hipStreamSynchronize(ctx->s_plain);
+        ctx->s = ctx->s_queue;
     }
     StreamA(const StreamA&) = delete;
     ~StreamA()
