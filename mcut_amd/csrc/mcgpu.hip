@@ -1168,7 +1168,8 @@ bool tests_all_pairs(mcgpu_context ctx)
 
 // One stream for a pair whose kernels are all shorter than a launch and than
 // the 5-10 us that a wait across streams takes (960 against 192 faces: 0.25 ms
-// with four streams, 0.21 with one; 2^14 to 2^16 faces: no gain).
+// with four streams, 0.21 with one, 0.17 on the plain one; 2^14 to 2^16 faces:
+// no gain).
 constexpr uint64_t kOneStream = 1ull << 13; // faces
 bool uses_one_stream(mcgpu_context ctx)
 {
