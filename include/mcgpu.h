@@ -27,9 +27,11 @@
  * enqueued form, mcgpu_dispatch_batch, mcgpu_autotune and the server's requests
  * synchronise with it, so such a call's kernels start after the work queued
  * there before and hold up work queued there meanwhile.  Pairs of up to 8,192
- * faces and 4,096 vertices a mesh, the last part of an enqueued dispatch (from
- * the candidate pairs on), and every other call that takes a context run on a
- * stream that does not.
+ * faces and 4,096 vertices a mesh do so only if work is queued there when they
+ * are called.  The last part of an enqueued dispatch (from the candidate pairs
+ * on) and every other call that takes a context run on a stream that does not
+ * synchronise with it.  A dispatch therefore overwrites a context's results only
+ * after null-stream work queued before it, which may still read them.
  *
  * The front end is a superset of what MCUT computes in one place: its broad
  * phase runs on the unshifted coordinates with a rounding bound, overlapped

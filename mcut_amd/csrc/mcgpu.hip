@@ -77,7 +77,7 @@ const char* kStageNames[ST_COUNT] = {"coordinate_sums", "shift_params", "shift_b
 // event slots: stage boundaries on the three streams
 enum Ev { EV_A0, EV_S0, EV_A_SUMS, EV_A_PARAMS, EV_A_SHIFT, EV_A_BOXES, EV_A_JOIN, EV_A_FILTER, EV_A_PLANES, EV_A_JOIN2, EV_A_TESTS, EV_A_NARROW,
           EV_A_END, EV_FORK, EV_B0, EV_B_SORT, EV_B_REFIT, EV_B_TRAV, EV_C0, EV_C_WORDS, EV_C_TOPO, EV_SUM_ITEMS, EV_SUM_CHAIN, EV_SUM_CHECK, EV_SUM_REST,
-          EV_TRAV_K0, EV_TRAV_K1, EV_B_CC, EV_COUNT };
+          EV_TRAV_K0, EV_TRAV_K1, EV_B_CC, EV_NULL, EV_COUNT };
 
 // Launch shape of the traversal kernel, chosen per workload class by the
 // autotuner (mcgpu_autotune) or set by the caller (mcgpu_set_tuning).
@@ -1167,9 +1167,9 @@ bool tests_all_pairs(mcgpu_context ctx)
 }
 
 // One stream for a pair whose kernels are all shorter than a launch and than
-// the 5-10 us that a wait across streams takes (960 against 192 faces: 0.25 ms
-// with four streams, 0.21 with one, 0.17 on the plain one; 2^14 to 2^16 faces:
-// no gain).
+// the 5-10 us that a wait across streams takes (960 against 192 faces behind
+// null-stream work: 0.25 ms with four streams, 0.20 with one; 2^14 to 2^16
+// faces: no gain).
 constexpr uint64_t kOneStream = 1ull << 13; // faces
 bool uses_one_stream(mcgpu_context ctx)
 {
@@ -1899,6 +1899,13 @@ void graph_drop(mcgpu_context ctx)
 mcgpu_result enqueue_dispatch(mcgpu_context ctx)
 {
     ctx->one_stream = uses_one_stream(ctx);
+    // A dispatch's outputs are overwritten only after the null stream's work
+    // queued before the call, which may read the last ones where they lie: with
+    // four streams B and C wait for it, on the plain stream alone B's event does.
+    if (ctx->one_stream && ctx->s == ctx->s_plain && hipStreamQuery(nullptr) != hipSuccess) {
+        CK(hipEventRecord(ctx->ev[EV_NULL], ctx->s2));
+        CK(hipStreamWaitEvent(ctx->s, ctx->ev[EV_NULL], 0));
+    }
     ctx->state_copied = false;
     if (!ctx->graphs || ctx->stage_timing || ctx->kernel_timing || !ctx->own_streams) {
         if (ctx->batch) enqueue_validate_batch(ctx);
@@ -2172,8 +2179,9 @@ static void destroy_streams(mcgpu_context ctx)
 // dispatch over four streams (three of them synchronise with the null stream
 // anyway), s_plain for all else, so that calls on stream A alone, and a
 // dispatch that goes on after its call returned, neither wait for a caller's
-// work on the null stream nor hold it up.  A pair on one stream is faster on
-// s_plain, too (960 against 192 faces 171 us, 205 on s_queue).
+// work on the null stream nor hold it up.  A pair on one stream runs on s_plain
+// while the null stream is idle, and goes behind its work on s_queue otherwise
+// (960 against 192 faces 150 us, and 197 behind a short kernel there).
 struct StreamA {
     mcgpu_context ctx;
     bool done = false; // the host has waited for it
@@ -2511,9 +2519,10 @@ MCGPU_API mcgpu_result mcgpu_dispatch_frontend(mcgpu_context ctx, const mcgpu_me
                                                const mcgpu_dispatch_desc* desc, mcgpu_frontend_info* info)
 {
     if (!ctx || ctx->pending || !src || !cut) return MCGPU_ERROR_INVALID_VALUE;
-    // four streams, unless the pair is as small as uses_one_stream() takes
+    // four streams, unless the pair is as small as uses_one_stream() takes, which
+    // goes behind the null stream's work if there is any (enqueue_dispatch)
     StreamA a(ctx, (uint64_t)src->num_faces + cut->num_faces > kOneStream ||
-                       std::max(src->num_vertices, cut->num_vertices) > kSumSerial);
+                       std::max(src->num_vertices, cut->num_vertices) > kSumSerial || hipStreamQuery(nullptr) != hipSuccess);
     mcgpu_result r;
     if ((r = frontend_prepare(ctx, src, cut, desc)) != MCGPU_SUCCESS) return r;
     if ((r = alloc_list_buffers(ctx)) != MCGPU_SUCCESS) return r;

@@ -150,3 +150,54 @@ def test_private_memory_of_many_contexts(hip):
     finally:
         for c in cs:
             c.close()
+
+
+@pytest.mark.parametrize("n", [3, 10, 40])
+@pytest.mark.parametrize("enqueued", [False, True])
+def test_a_dispatch_waits_for_null_stream_reads_of_the_last_registry(hip, n, enqueued):
+    """A program copies a registry from where it lies on the null stream, behind
+    other work there, and dispatches the next pair: its registry may only be
+    overwritten once it has been read."""
+    from mcut_amd import frontend
+    hip.hipMemcpyAsync.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_void_p]
+    lib = frontend.lib()
+    src, cut = spheres(n)
+    other = (cut[0] + [0.1, 0.05, 0.02], cut[1], None)
+    c = frontend.Context(0)
+    out = C.c_void_p()
+    release = threading.Event()
+
+    @C.CFUNCTYPE(None, C.c_void_p)
+    def work(_):
+        release.wait(1.0)
+
+    def dispatch(a, b):
+        if not enqueued:
+            return c.dispatch(a, b)
+        c.dispatch_async(a, b)
+        return c.wait()
+
+    try:
+        want = dispatch(src, other).registry()[2]
+        dispatch(src, cut)  # buffers, stages
+        R = dispatch(src, cut)
+        first = R.registry()[2]
+        assert len(first) > 0 and not np.array_equal(first, want)
+        e, f, p, k = C.c_void_p(), C.c_void_p(), C.c_void_p(), C.c_uint64()
+        assert lib.mcgpu_registry_device(c.h, C.byref(e), C.byref(f), C.byref(p), C.byref(k)) == 0 and k.value == len(first)
+        assert hip.hipMalloc(C.byref(out), first.nbytes) == 0 and hip.hipDeviceSynchronize() == 0
+        assert hip.hipLaunchHostFunc(None, work, None) == 0
+        assert hip.hipMemcpyAsync(out, p, first.nbytes, 3, None) == 0  # device to device, on the null stream
+        t = threading.Thread(target=dispatch, args=(src, other))
+        t.start()
+        time.sleep(0.15)  # long enough for a dispatch that does not wait
+        release.set()
+        t.join()
+        got = np.zeros_like(first)
+        assert hip.hipDeviceSynchronize() == 0 and hip.hipMemcpy(got.ctypes.data, out, got.nbytes, 2) == 0
+        assert np.array_equal(got, first)
+    finally:
+        release.set()
+        hip.hipDeviceSynchronize()
+        hip.hipFree(out)
+        c.close()
